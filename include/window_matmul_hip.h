@@ -72,6 +72,16 @@ typedef struct wm_operand {
   int64_t stride_c;
 } wm_operand;
 
+/* Rank-3 operand whose batch has two levels, for the wm_grouped_* entry points: with heads >= 1 element
+ * (b, r, c) lives at data + (b / heads)*stride_g + (b % heads)*stride_b + r*stride_r + c*stride_c, which is
+ * how a (batch, M, heads * N) projection is read as batch * heads elements of (M, N) in place: stride_g =
+ * M * heads * N, stride_b = N, stride_r = heads * N.  heads = 0: the plain operand in `op`. */
+typedef struct wm_grouped_operand {
+  wm_operand op;
+  int64_t heads;
+  int64_t stride_g;
+} wm_grouped_operand;
+
 /* A[b,i,j] = sum_h q[b,i,h] * k[b,h,i+j-w]  (0 <= i+j-w < M, else +0.0)
  *   q (B,M,N), k (B,N,M) -- the reference's orientation: K transposed -- , a (B,M,2w+1).
  * Replaces window_matmul_fw_cuda (reference cuda/window_matmul_cuda.cu:224-270),
@@ -209,6 +219,36 @@ int wm_window_attention_backward_static(const wm_operand *q, const wm_operand *k
  * overlap or run backwards), B <= 65535 and N <= 64 * 65535 (any M).  Callers fall back to their
  * own copy on that status, as the PyTorch extension does. */
 int wm_key_rows(const wm_operand *k, void *rows, int64_t B, int64_t N, int64_t M, int dtype, void *stream);
+
+/* The six entry points of the products and of the fused attention with operands whose batch may have two
+ * levels (wm_grouped_operand).  Same kernels, results, status codes and remaining arguments as the functions
+ * without `grouped` in their names.  Grouped operands of a call have the same `heads` (WM_ERR_BAD_SHAPE
+ * otherwise); plain ones (heads = 0) may stand beside them.  Band operands (a, grad_a) are always plain. */
+int wm_grouped_window_matmul_forward(const wm_grouped_operand *q, const wm_grouped_operand *k,
+                                     const wm_operand *a, int64_t B, int64_t M, int64_t N, int64_t w,
+                                     int dtype, unsigned flags, void *stream);
+int wm_grouped_window_matmul_backward(const wm_grouped_operand *q, const wm_grouped_operand *k,
+                                      const wm_operand *grad_a, const wm_grouped_operand *grad_q,
+                                      const wm_grouped_operand *grad_k, int64_t B, int64_t M, int64_t N,
+                                      int64_t w, int dtype, unsigned flags, void *stream);
+int wm_grouped_unwindow_matmul_forward(const wm_operand *a, const wm_grouped_operand *v,
+                                       const wm_grouped_operand *o, int64_t B, int64_t M, int64_t N,
+                                       int64_t w, int dtype, unsigned flags, void *stream);
+int wm_grouped_unwindow_matmul_backward(const wm_operand *a, const wm_grouped_operand *v,
+                                        const wm_grouped_operand *grad_o, const wm_operand *grad_a,
+                                        const wm_grouped_operand *grad_v, int64_t B, int64_t M, int64_t N,
+                                        int64_t w, int dtype, unsigned flags, void *stream);
+int wm_grouped_window_attention_forward(const wm_grouped_operand *q, const wm_grouped_operand *k,
+                                        const wm_grouped_operand *v, const wm_grouped_operand *o, float *lse,
+                                        int64_t B, int64_t M, int64_t N, int64_t w, double scale,
+                                        int mask_out_of_range, int dtype, unsigned flags, void *stream);
+int wm_grouped_window_attention_backward(const wm_grouped_operand *q, const wm_grouped_operand *k,
+                                         const wm_grouped_operand *v, const wm_grouped_operand *o,
+                                         const float *lse, const wm_grouped_operand *grad_o,
+                                         const wm_grouped_operand *grad_q, const wm_grouped_operand *grad_k,
+                                         const wm_grouped_operand *grad_v, float *delta, int64_t B,
+                                         int64_t M, int64_t N, int64_t w, double scale, int dtype,
+                                         unsigned flags, void *stream);
 
 /* 1 if the fused kernels exist for this shape, dtype and scale (layout aside), else 0. */
 int wm_window_attention_supported(int64_t M, int64_t N, int64_t w, int dtype, double scale);

@@ -44,19 +44,84 @@ int abi_dtype(const torch::Tensor &t, const char *op) {
 
 bool aligned16(const torch::Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 
-// Unit column stride and 16-byte aligned rows/batches, else a contiguous copy.
-torch::Tensor vector_friendly(const torch::Tensor &t) {
+// A tensor (..., R, C) is a batch of (R, C) matrices.  Its leading dimensions are read in place when they amount to
+// at most two levels of strides: contiguous leading dimensions are one, a (batch, M, heads * N) projection
+// seen as (batch, heads, M, N) is two.  False when there are more.
+bool batch_steps(const torch::Tensor &t, int64_t *step, int64_t *heads, int64_t *group) {
+  int64_t size[2] = {1, 1}, stride[2] = {0, 0};
+  int levels = 0;
+  for (int64_t d = t.dim() - 3; d >= 0; --d) {  // innermost level first
+    if (t.size(d) == 1) continue;
+    if (levels > 0 && t.stride(d) == stride[levels - 1] * size[levels - 1]) {
+      size[levels - 1] *= t.size(d);
+    } else {
+      if (levels == 2) return false;
+      size[levels] = t.size(d), stride[levels] = t.stride(d), ++levels;
+    }
+  }
+  *step = stride[0], *heads = levels == 2 ? size[0] : 0, *group = levels == 2 ? stride[1] : 0;
+  return true;
+}
+
+int64_t batch_of(const torch::Tensor &t) {
+  int64_t B = 1;
+  for (int64_t d = 0; d < t.dim() - 2; ++d) B *= t.size(d);
+  return B;
+}
+// Sizes of `like` with the last dimension replaced.
+std::vector<int64_t> with_columns(const torch::Tensor &like, int64_t columns) {
+  auto sizes = like.sizes().vec();
+  sizes.back() = columns;
+  return sizes;
+}
+
+// Unit column stride, 16-byte aligned rows and batch elements, at most two batch levels: what the kernels read in place.
+bool readable_in_place(const torch::Tensor &t) {
   const int64_t es = t.element_size();
-  const bool ok = t.stride(2) == 1 && (t.stride(1) * es) % 16 == 0 && (t.stride(0) * es) % 16 == 0 && aligned16(t);
-  if (ok || t.numel() == 0) return t;
+  int64_t step, heads, group;
+  return t.stride(-1) == 1 && (t.stride(-2) * es) % 16 == 0 && aligned16(t) && batch_steps(t, &step, &heads, &group) &&
+         (step * es) % 16 == 0 && (group * es) % 16 == 0;
+}
+
+// The operands of a call share one grouping of the batch (include/window_matmul_hip.h); the first tensor with two levels
+// of batch strides decides it.
+struct Heads {
+  int64_t heads = 0;
+  bool admit(const torch::Tensor &t) {
+    int64_t step, h, group;
+    if (!batch_steps(t, &step, &h, &group)) return false;
+    if (h != 0 && heads == 0) heads = h;
+    return h == 0 || h == heads;
+  }
+};
+
+// `t` where the kernels can read it in place, else a contiguous copy.
+torch::Tensor vector_friendly(const torch::Tensor &t) {
+  if (t.numel() == 0 || readable_in_place(t)) return t;
+  const bool alignable = (t.size(-1) * t.element_size()) % 16 == 0;
   if (t.is_contiguous()) {
     // rows that cannot be aligned (N * element size not a multiple of 16): the tile kernels take
     // the tensor as it is; alignable rows behind a misaligned pointer (a view at a storage offset)
     // move into a fresh allocation so that the tuned kernels apply
-    return (t.size(2) * es) % 16 == 0 ? t.clone(at::MemoryFormat::Contiguous) : t;
+    return alignable ? t.clone(at::MemoryFormat::Contiguous) : t;
   }
   auto c = t.contiguous();
-  return aligned16(c) || (t.size(2) * es) % 16 != 0 ? c : c.clone(at::MemoryFormat::Contiguous);
+  return aligned16(c) || !alignable ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+
+torch::Tensor vector_friendly(const torch::Tensor &t, Heads &heads) {
+  auto r = vector_friendly(t);
+  return heads.admit(r) ? r : r.contiguous();
+}
+
+// Storage for a result of the shape of `t`, in the memory layout of `t` where the kernels can write that (the
+// gradient of a projection view is then laid out like the projection and needs no copy on its way back).
+torch::Tensor empty_like_rows(const torch::Tensor &t, int64_t columns, Heads &heads) {
+  if (t.size(-1) == columns) {
+    auto g = torch::empty_like(t);
+    if (readable_in_place(g) && heads.admit(g)) return g;
+  }
+  return torch::empty(with_columns(t, columns), t.options());
 }
 
 // Band tensors (rows of odd length 2w+1) need to be contiguous and start on a 16-byte boundary.
@@ -77,7 +142,7 @@ constexpr int64_t kTileUpToWindowF32 = 256;
 bool tiles_preferred(const torch::Tensor &t, int64_t w) { return t.scalar_type() == at::kFloat && w <= kTileUpToWindowF32; }
 
 int64_t padded_width(const torch::Tensor &t, int64_t w) {
-  const int64_t N = t.size(2);
+  const int64_t N = t.size(-1);
   if (tiles_preferred(t, w)) return N;
   int64_t unit;
   switch (t.scalar_type()) {
@@ -90,13 +155,14 @@ int64_t padded_width(const torch::Tensor &t, int64_t w) {
   return N > 0 && Np <= 128 ? Np : N;
 }
 torch::Tensor pad_columns(const torch::Tensor &t, int64_t Np) {
-  if (t.size(2) == Np) return t;
-  auto padded = torch::zeros({t.size(0), t.size(1), Np}, t.options());
-  padded.narrow(2, 0, t.size(2)).copy_(t);
+  const int64_t N = t.size(-1);
+  if (N == Np) return t;
+  auto padded = torch::zeros(with_columns(t, Np), t.options());
+  padded.narrow(-1, 0, N).copy_(t);
   return padded;
 }
 torch::Tensor cut_columns(const torch::Tensor &t, int64_t N) {
-  return t.size(2) == N ? t : t.narrow(2, 0, N).contiguous();
+  return t.size(-1) == N ? t : t.narrow(-1, 0, N).contiguous();
 }
 
 // Head widths beyond 128 (the widest the tuned kernels take) are worked on in slices of 128 columns:
@@ -106,11 +172,20 @@ torch::Tensor cut_columns(const torch::Tensor &t, int64_t N) {
 // the sum is rounded once.  float64 is not sliced: its kernels take every head width.
 constexpr int64_t kMaxWidth = 128;
 bool sliced_width(const torch::Tensor &t, int64_t w) {
-  return t.size(2) > kMaxWidth && !tiles_preferred(t, w) && (t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat);
+  return t.size(-1) > kMaxWidth && !tiles_preferred(t, w) && (t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat);
 }
 
 wm_operand operand(const torch::Tensor &t) {
   return wm_operand{t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)};
+}
+// A contiguous band (..., M, W) as an operand.
+wm_operand band_operand(const torch::Tensor &t) {
+  return wm_operand{t.data_ptr(), t.size(-2) * t.size(-1), t.size(-1), 1};
+}
+wm_grouped_operand grouped(const torch::Tensor &t) {
+  wm_grouped_operand g{{t.data_ptr(), 0, t.stride(-2), t.stride(-1)}, 0, 0};
+  TORCH_CHECK(batch_steps(t, &g.op.stride_b, &g.heads, &g.stride_g), "more than two levels of batch strides");
+  return g;
 }
 
 void raise_on_error(int status, const char *op) {
@@ -121,34 +196,36 @@ void *current_stream(const torch::Tensor &t) {
   return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
-// K comes as (B,N,M).  The kernels want key rows contiguous, which is what a
-// transposed view of a row-major (B,M,N) tensor already is; anything else is
+// K comes as (...,N,M).  The kernels want key rows contiguous, which is what a
+// transposed view of a row-major (...,M,N) tensor already is; anything else is
 // copied into that layout once (the reference always copies: cuda:236).
 // A tensor that is laid out as (B,N,M) with unit stride along M goes through the library's own
 // transpose (one read and one write at memory speed; a general strided copy reaches a quarter of that).
-torch::Tensor key_rows(const torch::Tensor &k) {
-  auto view = k.transpose(1, 2);
-  if (view.stride(2) == 1 || k.stride(2) != 1 || k.numel() == 0 || !k.is_cuda()) return vector_friendly(view);
-  const int64_t es = k.element_size();
-  if (es != 2 && es != 4 && es != 8) return vector_friendly(view);
-  auto rows = torch::empty({k.size(0), k.size(2), k.size(1)}, k.options());
-  const wm_operand src{k.data_ptr(), k.stride(0), k.stride(1), k.stride(2)};
+torch::Tensor key_rows(const torch::Tensor &k, Heads &heads) {
+  auto view = k.transpose(-2, -1);
+  if (view.stride(-1) == 1 || k.stride(-1) != 1 || k.numel() == 0 || !k.is_cuda()) return vector_friendly(view, heads);
+  const int64_t es = k.element_size(), B = batch_of(k);
+  int64_t step, h, group;
+  if ((es != 2 && es != 4 && es != 8) || !batch_steps(k, &step, &h, &group) || h != 0) return vector_friendly(view, heads);
+  auto rows = torch::empty(view.sizes(), k.options());
+  const wm_operand src{k.data_ptr(), step, k.stride(-2), k.stride(-1)};
   const int dtype = es == 2 ? WM_DTYPE_BF16 : es == 4 ? WM_DTYPE_F32 : WM_DTYPE_F64;  // only the element size matters
-  const int status = wm_key_rows(&src, rows.data_ptr(), k.size(0), k.size(1), k.size(2), dtype,
-                                 current_stream(k));
-  if (status == WM_ERR_UNSUPPORTED) return vector_friendly(view);  // odd alignment: the general copy
+  const int status = wm_key_rows(&src, rows.data_ptr(), B, k.size(-2), k.size(-1), dtype, current_stream(k));
+  if (status == WM_ERR_UNSUPPORTED) return vector_friendly(view, heads);  // odd alignment: the general copy
   raise_on_error(status, "key rows");
   return rows;
 }
 
 
+// The operands may have any number of leading dimensions, which need not be the same as long as they amount to
+// the same number of batch elements.
 void check_window_inputs(const torch::Tensor &src, const torch::Tensor &other) {
   check_gpu(src, "A");
   check_gpu(other, "B");
-  TORCH_CHECK(src.dim() == 3 && other.dim() == 3, "Input mismatch");
-  TORCH_CHECK(src.size(0) == other.size(0), "Input mismatch");
-  TORCH_CHECK(src.size(2) == other.size(1), "Input mismatch");
-  TORCH_CHECK(src.size(1) == other.size(2), "Input mismatch");
+  TORCH_CHECK(src.dim() >= 2 && other.dim() >= 2, "Input mismatch");
+  TORCH_CHECK(batch_of(src) == batch_of(other), "Input mismatch");
+  TORCH_CHECK(src.size(-1) == other.size(-2), "Input mismatch");
+  TORCH_CHECK(src.size(-2) == other.size(-1), "Input mismatch");
   TORCH_CHECK(src.scalar_type() == other.scalar_type(), "Input mismatch");
   TORCH_CHECK(src.device() == other.device(), "Input mismatch");
 }
@@ -156,17 +233,18 @@ void check_window_inputs(const torch::Tensor &src, const torch::Tensor &other) {
 void check_unwindow_inputs(const torch::Tensor &src, const torch::Tensor &other, int64_t w) {
   check_gpu(src, "A");
   check_gpu(other, "B");
-  TORCH_CHECK(src.dim() == 3 && other.dim() == 3, "Input mismatch");
-  TORCH_CHECK(src.size(0) == other.size(0), "Input mismatch");
-  TORCH_CHECK(src.size(2) == 2 * w + 1, "Input mismatch");
-  TORCH_CHECK(src.size(1) == other.size(1), "Input mismatch");
+  TORCH_CHECK(src.dim() >= 2 && other.dim() >= 2, "Input mismatch");
+  TORCH_CHECK(batch_of(src) == batch_of(other), "Input mismatch");
+  TORCH_CHECK(src.size(-1) == 2 * w + 1, "Input mismatch");
+  TORCH_CHECK(src.size(-2) == other.size(-2), "Input mismatch");
   TORCH_CHECK(src.scalar_type() == other.scalar_type(), "Input mismatch");
   TORCH_CHECK(src.device() == other.device(), "Input mismatch");
 }
 
-void check_grad(const torch::Tensor &g, const torch::Tensor &like, std::vector<int64_t> sizes) {
+// `g` has the leading dimensions and rows of `like`, and this many columns.
+void check_grad(const torch::Tensor &g, const torch::Tensor &like, int64_t columns) {
   check_gpu(g, "grad_C");
-  TORCH_CHECK(g.dim() == 3 && g.sizes().vec() == sizes, "Input mismatch");
+  TORCH_CHECK(g.sizes().vec() == with_columns(like, columns), "Input mismatch");
   TORCH_CHECK(g.scalar_type() == like.scalar_type() && g.device() == like.device(), "Input mismatch");
 }
 
@@ -178,20 +256,21 @@ torch::Tensor window_matmul_forward(torch::Tensor src, torch::Tensor other, int6
   at::hip::HIPGuardMasqueradingAsCUDA guard(src.device());
   if (sliced_width(src, window_size)) {
     torch::Tensor band;
-    for (int64_t h = 0; h < src.size(2); h += kMaxWidth) {
-      const int64_t n = std::min(kMaxWidth, src.size(2) - h);
-      auto part = window_matmul_forward(src.narrow(2, h, n).to(at::kFloat), other.narrow(1, h, n).to(at::kFloat), window_size);
+    for (int64_t h = 0; h < src.size(-1); h += kMaxWidth) {
+      const int64_t n = std::min(kMaxWidth, src.size(-1) - h);
+      auto part = window_matmul_forward(src.narrow(-1, h, n).to(at::kFloat), other.narrow(-2, h, n).to(at::kFloat), window_size);
       if (h == 0) band = part; else band.add_(part);
     }
     return band.to(src.scalar_type());
   }
-  const int64_t B = src.size(0), M = src.size(1), N = padded_width(src, window_size);
-  auto q = vector_friendly(pad_columns(src, N));
-  auto krows = pad_columns(key_rows(other), N);  // (B,M,N) view or copy
-  auto kt = krows.transpose(1, 2);
-  auto out = torch::empty({B, M, 2 * window_size + 1}, src.options());
-  wm_operand oq = operand(q), ok = operand(kt), oa = operand(out);
-  raise_on_error(wm_window_matmul_forward(&oq, &ok, &oa, B, M, N, window_size, dtype, 0, current_stream(src)),
+  const int64_t B = batch_of(src), M = src.size(-2), N = padded_width(src, window_size);
+  Heads heads;
+  auto q = vector_friendly(pad_columns(src, N), heads);
+  auto kt = pad_columns(key_rows(other, heads), N).transpose(-2, -1);  // (...,N,M) view of key rows
+  auto out = torch::empty(with_columns(src, 2 * window_size + 1), src.options());
+  const wm_grouped_operand oq = grouped(q), ok = grouped(kt);
+  const wm_operand oa = band_operand(out);
+  raise_on_error(wm_grouped_window_matmul_forward(&oq, &ok, &oa, B, M, N, window_size, dtype, 0, current_stream(src)),
                  "window_matmul_forward");
   return out;
 }
@@ -204,40 +283,43 @@ std::tuple<c10::optional<torch::Tensor>, c10::optional<torch::Tensor>> window_ma
     bool need_other) {
   TORCH_CHECK(window_size >= 0, "Input mismatch");
   check_window_inputs(src, other);
-  const int64_t B = src.size(0), M = src.size(1), N = src.size(2);
-  check_grad(grad_output, src, {B, M, 2 * window_size + 1});
+  const int64_t B = batch_of(src), M = src.size(-2), N = src.size(-1);
+  check_grad(grad_output, src, 2 * window_size + 1);
   const int dtype = abi_dtype(src, "window_matmul_bw_cuda");
   at::hip::HIPGuardMasqueradingAsCUDA guard(src.device());
   if (sliced_width(src, window_size)) {
     std::vector<torch::Tensor> gq, gk;
     for (int64_t h = 0; h < N; h += kMaxWidth) {
       const int64_t n = std::min(kMaxWidth, N - h);
-      auto part = window_matmul_backward(src.narrow(2, h, n), other.narrow(1, h, n), window_size, grad_output, need_src, need_other);
+      auto part = window_matmul_backward(src.narrow(-1, h, n), other.narrow(-2, h, n), window_size, grad_output, need_src, need_other);
       if (need_src) gq.push_back(*std::get<0>(part));
       if (need_other) gk.push_back(*std::get<1>(part));
     }
     c10::optional<torch::Tensor> grad_q, grad_k;
-    if (need_src) grad_q = torch::cat(gq, 2);
-    if (need_other) grad_k = torch::cat(gk, 1);
+    if (need_src) grad_q = torch::cat(gq, -1);
+    if (need_other) grad_k = torch::cat(gk, -2);
     return std::make_tuple(grad_q, grad_k);
   }
   const int64_t Np = padded_width(src, window_size);
-  auto q = vector_friendly(pad_columns(src, Np));
-  auto kt = pad_columns(key_rows(other), Np).transpose(1, 2);
+  Heads heads;
+  auto q = vector_friendly(pad_columns(src, Np), heads);
+  auto kt = pad_columns(key_rows(other, heads), Np).transpose(-2, -1);
   auto ga = band_friendly(grad_output);
   c10::optional<torch::Tensor> grad_q, grad_k;
-  if (need_src) grad_q = torch::empty({B, M, Np}, src.options());
-  // grad_k is produced row-major per key row and handed back in the (B,N,M)
+  if (need_src) grad_q = empty_like_rows(src, Np, heads);
+  // grad_k is produced row-major per key row and handed back in the (...,N,M)
   // orientation of `other` as a transposed view, like the reference (cuda:318).
-  if (need_other) grad_k = torch::empty({B, M, Np}, src.options()).transpose(1, 2);
-  wm_operand oq = operand(q), ok = operand(kt), oga = operand(ga), ogq{}, ogk{};
-  if (need_src) ogq = operand(*grad_q);
-  if (need_other) ogk = operand(*grad_k);
-  raise_on_error(wm_window_matmul_backward(&oq, &ok, &oga, need_src ? &ogq : nullptr, need_other ? &ogk : nullptr, B,
-                                           M, Np, window_size, dtype, 0, current_stream(src)),
+  if (need_other) grad_k = empty_like_rows(other.transpose(-2, -1), Np, heads).transpose(-2, -1);
+  const wm_grouped_operand oq = grouped(q), ok = grouped(kt);
+  const wm_operand oga = band_operand(ga);
+  wm_grouped_operand ogq{}, ogk{};
+  if (need_src) ogq = grouped(*grad_q);
+  if (need_other) ogk = grouped(*grad_k);
+  raise_on_error(wm_grouped_window_matmul_backward(&oq, &ok, &oga, need_src ? &ogq : nullptr, need_other ? &ogk : nullptr,
+                                                   B, M, Np, window_size, dtype, 0, current_stream(src)),
                  "window_matmul_backward");
   if (need_src) grad_q = cut_columns(*grad_q, N);
-  if (need_other && Np != N) grad_k = grad_k->narrow(1, 0, N);
+  if (need_other && Np != N) grad_k = grad_k->narrow(-2, 0, N);
   return std::make_tuple(grad_q, grad_k);
 }
 
@@ -247,19 +329,21 @@ torch::Tensor unwindow_matmul_forward(torch::Tensor src, torch::Tensor other, in
   check_unwindow_inputs(src, other, window_size);
   const int dtype = abi_dtype(src, "unwindow_matmul_fw_cuda");
   at::hip::HIPGuardMasqueradingAsCUDA guard(src.device());
-  const int64_t B = other.size(0), M = other.size(1), N = other.size(2);
+  const int64_t B = batch_of(other), M = other.size(-2), N = other.size(-1);
   if (sliced_width(other, window_size)) {
     std::vector<torch::Tensor> parts;
     for (int64_t h = 0; h < N; h += kMaxWidth)
-      parts.push_back(unwindow_matmul_forward(src, other.narrow(2, h, std::min(kMaxWidth, N - h)), window_size));
-    return torch::cat(parts, 2);
+      parts.push_back(unwindow_matmul_forward(src, other.narrow(-1, h, std::min(kMaxWidth, N - h)), window_size));
+    return torch::cat(parts, -1);
   }
   const int64_t Np = padded_width(other, window_size);
   auto a = band_friendly(src);
-  auto v = vector_friendly(pad_columns(other, Np));
-  auto out = torch::empty({B, M, Np}, src.options());
-  wm_operand oa = operand(a), ov = operand(v), oo = operand(out);
-  raise_on_error(wm_unwindow_matmul_forward(&oa, &ov, &oo, B, M, Np, window_size, dtype, 0, current_stream(src)),
+  Heads heads;
+  auto v = vector_friendly(pad_columns(other, Np), heads);
+  auto out = torch::empty(with_columns(other, Np), src.options());
+  const wm_operand oa = band_operand(a);
+  const wm_grouped_operand ov = grouped(v), oo = grouped(out);
+  raise_on_error(wm_grouped_unwindow_matmul_forward(&oa, &ov, &oo, B, M, Np, window_size, dtype, 0, current_stream(src)),
                  "unwindow_matmul_forward");
   return cut_columns(out, N);
 }
@@ -270,8 +354,8 @@ std::tuple<c10::optional<torch::Tensor>, c10::optional<torch::Tensor>> unwindow_
     bool need_other) {
   TORCH_CHECK(window_size >= 0, "Input mismatch");
   check_unwindow_inputs(src, other, window_size);
-  const int64_t B = other.size(0), M = other.size(1), N = other.size(2);
-  check_grad(grad_output, src, {B, M, N});
+  const int64_t B = batch_of(other), M = other.size(-2), N = other.size(-1);
+  check_grad(grad_output, other, N);
   const int dtype = abi_dtype(src, "unwindow_matmul_bw_cuda");
   at::hip::HIPGuardMasqueradingAsCUDA guard(src.device());
   if (sliced_width(other, window_size)) {
@@ -280,28 +364,32 @@ std::tuple<c10::optional<torch::Tensor>, c10::optional<torch::Tensor>> unwindow_
     for (int64_t h = 0; h < N; h += kMaxWidth) {
       const int64_t n = std::min(kMaxWidth, N - h);
       if (need_other)
-        gv.push_back(*std::get<1>(unwindow_matmul_backward(src, other.narrow(2, h, n), window_size, grad_output.narrow(2, h, n), false, true)));
+        gv.push_back(*std::get<1>(unwindow_matmul_backward(src, other.narrow(-1, h, n), window_size, grad_output.narrow(-1, h, n), false, true)));
       if (need_src) {  // grad_a = band of grad_output against other: in float32, as in window_matmul_forward
-        auto part = window_matmul_forward(grad_output.narrow(2, h, n).to(at::kFloat), other.narrow(2, h, n).transpose(1, 2).to(at::kFloat), window_size);
+        auto part = window_matmul_forward(grad_output.narrow(-1, h, n).to(at::kFloat), other.narrow(-1, h, n).transpose(-2, -1).to(at::kFloat), window_size);
         if (h == 0) grad_a = part; else grad_a->add_(part);
       }
     }
-    if (need_src) grad_a = grad_a->to(src.scalar_type());
-    if (need_other) grad_v = torch::cat(gv, 2);
+    if (need_src) grad_a = grad_a->to(src.scalar_type()).view(src.sizes());
+    if (need_other) grad_v = torch::cat(gv, -1);
     return std::make_tuple(grad_a, grad_v);
   }
   const int64_t Np = padded_width(other, window_size);
   auto a = band_friendly(src);
-  auto v = vector_friendly(pad_columns(other, Np));
-  auto go = vector_friendly(pad_columns(grad_output, Np));
+  Heads heads;
+  auto v = vector_friendly(pad_columns(other, Np), heads);
+  auto go = vector_friendly(pad_columns(grad_output, Np), heads);
   c10::optional<torch::Tensor> grad_a, grad_v;
-  if (need_src) grad_a = torch::empty({B, M, 2 * window_size + 1}, src.options());
-  if (need_other) grad_v = torch::empty({B, M, Np}, src.options());
-  wm_operand oa = operand(a), ov = operand(v), ogo = operand(go), oga{}, ogv{};
-  if (need_src) oga = operand(*grad_a);
-  if (need_other) ogv = operand(*grad_v);
-  raise_on_error(wm_unwindow_matmul_backward(&oa, &ov, &ogo, need_src ? &oga : nullptr, need_other ? &ogv : nullptr, B,
-                                             M, Np, window_size, dtype, 0, current_stream(src)),
+  if (need_src) grad_a = torch::empty(src.sizes(), src.options());
+  if (need_other) grad_v = empty_like_rows(other, Np, heads);
+  const wm_operand oa = band_operand(a);
+  const wm_grouped_operand ov = grouped(v), ogo = grouped(go);
+  wm_operand oga{};
+  wm_grouped_operand ogv{};
+  if (need_src) oga = band_operand(*grad_a);
+  if (need_other) ogv = grouped(*grad_v);
+  raise_on_error(wm_grouped_unwindow_matmul_backward(&oa, &ov, &ogo, need_src ? &oga : nullptr, need_other ? &ogv : nullptr,
+                                                     B, M, Np, window_size, dtype, 0, current_stream(src)),
                  "unwindow_matmul_backward");
   if (need_other) grad_v = cut_columns(*grad_v, N);
   return std::make_tuple(grad_a, grad_v);
@@ -344,24 +432,24 @@ torch::Tensor band_softmax_backward(torch::Tensor probs, torch::Tensor grad_outp
 }
 
 // Fused window attention (no counterpart in the reference's native module): forward returns
-// (o, lse); q, k, v are (B, M, N) with k holding key rows.  Raises when the fused kernels do not
+// (o, lse); q, k, v are (..., M, N) with k holding key rows.  Raises when the fused kernels do not
 // cover the problem; window_attention_supported() lets the caller choose the separate ops first.
 bool window_attention_supported(torch::Tensor q, int64_t window_size, double scale) {
-  if (q.dim() != 3 || !q.device().is_cuda()) return false;
+  if (q.dim() < 2 || !q.device().is_cuda()) return false;
   int dtype;
   switch (q.scalar_type()) {
     case at::kHalf: dtype = WM_DTYPE_F16; break;
     case at::kBFloat16: dtype = WM_DTYPE_BF16; break;
     default: return false;
   }
-  return wm_window_attention_supported(q.size(1), q.size(2), window_size, dtype, scale) != 0;
+  return wm_window_attention_supported(q.size(-2), q.size(-1), window_size, dtype, scale) != 0;
 }
 
 void check_attention_inputs(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v) {
   check_gpu(q, "Q");
   check_gpu(k, "K");
   check_gpu(v, "V");
-  TORCH_CHECK(q.dim() == 3 && k.sizes() == q.sizes() && v.sizes() == q.sizes(), "Input mismatch");
+  TORCH_CHECK(q.dim() >= 2 && k.sizes() == q.sizes() && v.sizes() == q.sizes(), "Input mismatch");
   TORCH_CHECK(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type(), "Input mismatch");
   TORCH_CHECK(k.device() == q.device() && v.device() == q.device(), "Input mismatch");
 }
@@ -372,13 +460,14 @@ std::tuple<torch::Tensor, torch::Tensor> window_attention_forward(torch::Tensor 
   check_attention_inputs(q, k, v);
   const int dtype = abi_dtype(q, "window_attention_forward");
   at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-  const int64_t B = q.size(0), M = q.size(1), N = q.size(2);
-  auto qq = vector_friendly(q), kk = vector_friendly(k), vv = vector_friendly(v);
-  auto o = torch::empty({B, M, N}, q.options());
+  const int64_t B = batch_of(q), M = q.size(-2), N = q.size(-1);
+  Heads heads;
+  auto qq = vector_friendly(q, heads), kk = vector_friendly(k, heads), vv = vector_friendly(v, heads);
+  auto o = torch::empty(q.sizes(), q.options());
   auto lse = torch::empty({B, M}, q.options().dtype(at::kFloat));
-  wm_operand oq = operand(qq), ok = operand(kk), ov = operand(vv), oo = operand(o);
-  raise_on_error(wm_window_attention_forward(&oq, &ok, &ov, &oo, lse.data_ptr<float>(), B, M, N, window_size, scale,
-                                             mask_out_of_range, dtype, 0, current_stream(q)),
+  const wm_grouped_operand oq = grouped(qq), ok = grouped(kk), ov = grouped(vv), oo = grouped(o);
+  raise_on_error(wm_grouped_window_attention_forward(&oq, &ok, &ov, &oo, lse.data_ptr<float>(), B, M, N, window_size, scale,
+                                                     mask_out_of_range, dtype, 0, current_stream(q)),
                  "window_attention_forward");
   return std::make_tuple(o, lse);
 }
@@ -388,26 +477,28 @@ window_attention_backward(torch::Tensor q, torch::Tensor k, torch::Tensor v, tor
                           torch::Tensor grad_output, int64_t window_size, double scale, bool need_q, bool need_k,
                           bool need_v) {
   check_attention_inputs(q, k, v);
-  check_grad(grad_output, q, q.sizes().vec());
-  check_grad(o, q, q.sizes().vec());
+  const int64_t B = batch_of(q), M = q.size(-2), N = q.size(-1);
+  check_grad(grad_output, q, N);
+  check_grad(o, q, N);
   TORCH_CHECK(lse.device() == q.device() && lse.scalar_type() == at::kFloat && lse.dim() == 2 &&
-                  lse.size(0) == q.size(0) && lse.size(1) == q.size(1) && lse.is_contiguous(),
+                  lse.size(0) == B && lse.size(1) == M && lse.is_contiguous(),
               "Input mismatch");
   const int dtype = abi_dtype(q, "window_attention_backward");
   at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-  const int64_t B = q.size(0), M = q.size(1), N = q.size(2);
-  auto qq = vector_friendly(q), kk = vector_friendly(k), vv = vector_friendly(v), oo = vector_friendly(o),
-       go = vector_friendly(grad_output);
+  Heads heads;
+  auto qq = vector_friendly(q, heads), kk = vector_friendly(k, heads), vv = vector_friendly(v, heads),
+       oo = vector_friendly(o, heads), go = vector_friendly(grad_output, heads);
   c10::optional<torch::Tensor> gq, gk, gv;
-  wm_operand f{}, g{}, h{};
-  if (need_q) gq = torch::empty({B, M, N}, q.options()), f = operand(*gq);
-  if (need_k) gk = torch::empty({B, M, N}, q.options()), g = operand(*gk);
-  if (need_v) gv = torch::empty({B, M, N}, q.options()), h = operand(*gv);
+  wm_grouped_operand f{}, g{}, h{};
+  if (need_q) gq = empty_like_rows(q, N, heads), f = grouped(*gq);
+  if (need_k) gk = empty_like_rows(k, N, heads), g = grouped(*gk);
+  if (need_v) gv = empty_like_rows(v, N, heads), h = grouped(*gv);
   auto delta = torch::empty({2, B, M}, lse.options());  // row sums and log2-scaled log-sum-exp
-  wm_operand a = operand(qq), b = operand(kk), c = operand(vv), d = operand(oo), e = operand(go);
-  raise_on_error(wm_window_attention_backward(&a, &b, &c, &d, lse.data_ptr<float>(), &e, need_q ? &f : nullptr,
-                                              need_k ? &g : nullptr, need_v ? &h : nullptr, delta.data_ptr<float>(),
-                                              B, M, N, window_size, scale, dtype, 0, current_stream(q)),
+  const wm_grouped_operand a = grouped(qq), b = grouped(kk), c = grouped(vv), d = grouped(oo), e = grouped(go);
+  raise_on_error(wm_grouped_window_attention_backward(&a, &b, &c, &d, lse.data_ptr<float>(), &e, need_q ? &f : nullptr,
+                                                      need_k ? &g : nullptr, need_v ? &h : nullptr,
+                                                      delta.data_ptr<float>(), B, M, N, window_size, scale, dtype, 0,
+                                                      current_stream(q)),
                  "window_attention_backward");
   return std::make_tuple(gq, gk, gv);
 }

@@ -2,6 +2,7 @@
 // the mapping of the four ops onto the three banded primitives.
 #include "wm_common.hpp"
 
+#include <initializer_list>
 #include <mutex>
 
 // Workspace of wm_window_attention_backward_static: the two per-row values the first backward
@@ -40,7 +41,31 @@ int check_common(int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned
   return WM_OK;
 }
 
-bool missing(const wm_operand *op) { return op == nullptr || op->data == nullptr; }
+const void *data_of(const wm_operand *op) { return op->data; }
+const void *data_of(const wm_grouped_operand *g) { return g->op.data; }
+template <typename Op>
+bool missing(const Op *op) { return op == nullptr || data_of(op) == nullptr; }
+const View kNoView{nullptr, BatchStep{0, 0, 0}, 0, 0};
+template <typename Op>
+View view_or_none(const Op *op) {
+  return op != nullptr ? make_view(op) : kNoView;
+}
+
+// Gives all operands of a call the same `heads` (see batch_pos): a plain batch with step s is also groups of `heads`
+// elements with step heads * s from group to group.  False when two grouped operands differ.
+bool common_heads(std::initializer_list<View *> views) {
+  int heads = 0;
+  for (const View *v : views) {
+    if (v->data == nullptr || v->sb.heads == 0) continue;
+    if (v->sb.heads < 0 || (heads != 0 && v->sb.heads != heads)) return false;
+    heads = v->sb.heads;
+  }
+  for (View *v : views) {
+    if (v->sb.heads == 0) v->sb.group = heads * v->sb.step;
+    v->sb.heads = heads;
+  }
+  return true;
+}
 
 int to_status(hipError_t err) {
   if (err == hipSuccess) return WM_OK;
@@ -91,6 +116,116 @@ int p3(const Problem &p, const View &a, const View &y, const View &c) {
                        try_launch_tile_p3, launch_strided_p3, p, a, y, c);
 }
 
+// The entry points below, for operands of either kind: wm_operand or wm_grouped_operand.
+template <typename Op>
+int window_forward(const Op *q, const Op *k, const wm_operand *a, int64_t B, int64_t M, int64_t N, int64_t w, int dtype,
+                   unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (B == 0 || M == 0) return WM_OK;  // nothing to write
+  if (missing(a) || (N > 0 && (missing(q) || missing(k)))) return WM_ERR_NULL_POINTER;
+  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
+  View va = make_view(a);
+  // N == 0: operands are never dereferenced.  K arrives as (B,N,M); the primitives read it as rows c, columns h.
+  View vq = N > 0 ? make_view(q) : View{va.data, BatchStep{0, 0, 0}, 0, 0};
+  View vk = N > 0 ? transposed(make_view(k)) : vq;
+  if (!common_heads({&va, &vq, &vk})) return WM_ERR_BAD_SHAPE;
+  return p1(p, vq, vk, va);
+}
+
+template <typename Op>
+int window_backward(const Op *q, const Op *k, const wm_operand *grad_a, const Op *grad_q, const Op *grad_k, int64_t B,
+                    int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (B == 0 || M == 0 || N == 0) return WM_OK;
+  if (missing(q) || missing(k) || missing(grad_a)) return WM_ERR_NULL_POINTER;
+  if ((grad_q && missing(grad_q)) || (grad_k && missing(grad_k))) return WM_ERR_NULL_POINTER;
+  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
+  View vq = make_view(q), vk = transposed(make_view(k)), vga = make_view(grad_a), vgq = view_or_none(grad_q),
+       vgk = transposed(view_or_none(grad_k));
+  if (!common_heads({&vq, &vk, &vga, &vgq, &vgk})) return WM_ERR_BAD_SHAPE;
+  if (grad_q && grad_k && fused_backward_allowed(p)) {  // small problems: both products in one launch
+    hipError_t err = hipSuccess;
+    if (try_launch_vector_window_backward(p, vga, vk, vq, vgq, vgk, &err)) return to_status(err);
+  }
+  if (grad_q)
+    if (int st = p2(p, vga, vk, vgq)) return st;
+  if (grad_k)
+    if (int st = p3(p, vga, vq, vgk)) return st;
+  return WM_OK;
+}
+
+template <typename Op>
+int unwindow_forward(const wm_operand *a, const Op *v, const Op *o, int64_t B, int64_t M, int64_t N, int64_t w, int dtype,
+                     unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (B == 0 || M == 0 || N == 0) return WM_OK;
+  if (missing(a) || missing(v) || missing(o)) return WM_ERR_NULL_POINTER;
+  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
+  View va = make_view(a), vv = make_view(v), vo = make_view(o);
+  if (!common_heads({&va, &vv, &vo})) return WM_ERR_BAD_SHAPE;
+  return p2(p, va, vv, vo);
+}
+
+template <typename Op>
+int unwindow_backward(const wm_operand *a, const Op *v, const Op *grad_o, const wm_operand *grad_a, const Op *grad_v,
+                      int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (B == 0 || M == 0) return WM_OK;
+  if ((grad_a && missing(grad_a)) || (grad_v && missing(grad_v))) return WM_ERR_NULL_POINTER;
+  if (N > 0 && (missing(a) || missing(v) || missing(grad_o))) return WM_ERR_NULL_POINTER;
+  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
+  View va = view_or_none(a), vga = view_or_none(grad_a), vgv = view_or_none(grad_v);
+  // N == 0: grad_a is all +0.0 and the operands are never dereferenced
+  View vv = N > 0 ? make_view(v) : View{vga.data, BatchStep{0, 0, 0}, 0, 0};
+  View vgo = N > 0 ? make_view(grad_o) : vv;
+  if (!common_heads({&va, &vv, &vgo, &vga, &vgv})) return WM_ERR_BAD_SHAPE;
+  if (grad_a && grad_v && N > 0 && fused_backward_allowed(p)) {  // small problems: both products in one launch
+    hipError_t err = hipSuccess;
+    if (try_launch_vector_unwindow_backward(p, va, vv, vgo, vga, vgv, &err)) return to_status(err);
+  }
+  if (grad_a)
+    if (int st = p1(p, vgo, vv, vga)) return st;
+  if (grad_v && N > 0)
+    if (int st = p3(p, va, vgo, vgv)) return st;
+  return WM_OK;
+}
+
+template <typename Op>
+int attention_forward(const Op *q, const Op *k, const Op *v, const Op *o, float *lse, int64_t B, int64_t M, int64_t N,
+                      int64_t w, double scale, int mask_out_of_range, int dtype, unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
+  if (B == 0 || M == 0) return WM_OK;
+  if (missing(q) || missing(k) || missing(v) || missing(o)) return WM_ERR_NULL_POINTER;
+  const Problem prob{B, M, N, w, dtype, flags, static_cast<hipStream_t>(stream)};
+  View vq = make_view(q), vk = make_view(k), vv = make_view(v), vo = make_view(o);
+  if (!common_heads({&vq, &vk, &vv, &vo})) return WM_ERR_BAD_SHAPE;
+  hipError_t err = hipSuccess;
+  if (!try_launch_attention_forward(prob, vq, vk, vv, vo, lse, scale, mask_out_of_range, &err)) return WM_ERR_UNSUPPORTED;
+  return to_status(err);
+}
+
+template <typename Op>
+int attention_backward(const Op *q, const Op *k, const Op *v, const Op *o, const float *lse, const Op *grad_o,
+                       const Op *grad_q, const Op *grad_k, const Op *grad_v, float *delta, int64_t B, int64_t M,
+                       int64_t N, int64_t w, double scale, int dtype, unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
+  if (B == 0 || M == 0) return WM_OK;
+  if (missing(q) || missing(k) || missing(v) || missing(o) || missing(grad_o) || lse == nullptr || delta == nullptr)
+    return WM_ERR_NULL_POINTER;
+  if (grad_q == nullptr && grad_k == nullptr && grad_v == nullptr) return WM_OK;
+  if ((grad_q && missing(grad_q)) || (grad_k && missing(grad_k)) || (grad_v && missing(grad_v))) return WM_ERR_NULL_POINTER;
+  const Problem prob{B, M, N, w, dtype, flags, static_cast<hipStream_t>(stream)};
+  View vq = make_view(q), vk = make_view(k), vv = make_view(v), vo = make_view(o), vgo = make_view(grad_o),
+       vgq = view_or_none(grad_q), vgk = view_or_none(grad_k), vgv = view_or_none(grad_v);
+  if (!common_heads({&vq, &vk, &vv, &vo, &vgo, &vgq, &vgk, &vgv})) return WM_ERR_BAD_SHAPE;
+  hipError_t err = hipSuccess;
+  if (!try_launch_attention_backward(prob, vq, vk, vv, vo, vgo, lse, delta, vgq, vgk, vgv, scale, &err))
+    return WM_ERR_UNSUPPORTED;
+  return to_status(err);
+}
+
 }  // namespace
 }  // namespace wm
 
@@ -98,69 +233,20 @@ using namespace wm;
 
 extern "C" {
 
-int wm_window_matmul_forward(const wm_operand *q, const wm_operand *k, const wm_operand *a, int64_t B,
-                             int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
-  if (B == 0 || M == 0) return WM_OK;  // nothing to write
-  if (missing(a) || (N > 0 && (missing(q) || missing(k)))) return WM_ERR_NULL_POINTER;
-  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
-  const wm_operand none{a->data, 0, 0, 0};  // N == 0: operands are never dereferenced
-  // K arrives as (B,N,M); the primitives read it as rows c, columns h.
-  return p1(p, make_view(N > 0 ? q : &none), transposed(make_view(N > 0 ? k : &none)), make_view(a));
+int wm_window_matmul_forward(const wm_operand *q, const wm_operand *k, const wm_operand *a, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return window_forward(q, k, a, B, M, N, w, dtype, flags, stream);
 }
 
-int wm_window_matmul_backward(const wm_operand *q, const wm_operand *k, const wm_operand *grad_a,
-                              const wm_operand *grad_q, const wm_operand *grad_k, int64_t B, int64_t M,
-                              int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
-  if (B == 0 || M == 0 || N == 0) return WM_OK;
-  if (missing(q) || missing(k) || missing(grad_a)) return WM_ERR_NULL_POINTER;
-  if ((grad_q && !grad_q->data) || (grad_k && !grad_k->data)) return WM_ERR_NULL_POINTER;
-  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
-  if (grad_q && grad_k && fused_backward_allowed(p)) {  // small problems: both products in one launch
-    hipError_t err = hipSuccess;
-    if (try_launch_vector_window_backward(p, make_view(grad_a), transposed(make_view(k)), make_view(q), make_view(grad_q),
-                                          transposed(make_view(grad_k)), &err))
-      return to_status(err);
-  }
-  if (grad_q)
-    if (int st = p2(p, make_view(grad_a), transposed(make_view(k)), make_view(grad_q))) return st;
-  if (grad_k)
-    if (int st = p3(p, make_view(grad_a), make_view(q), transposed(make_view(grad_k)))) return st;
-  return WM_OK;
+int wm_window_matmul_backward(const wm_operand *q, const wm_operand *k, const wm_operand *grad_a, const wm_operand *grad_q, const wm_operand *grad_k, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return window_backward(q, k, grad_a, grad_q, grad_k, B, M, N, w, dtype, flags, stream);
 }
 
-int wm_unwindow_matmul_forward(const wm_operand *a, const wm_operand *v, const wm_operand *o, int64_t B,
-                               int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
-  if (B == 0 || M == 0 || N == 0) return WM_OK;
-  if (missing(a) || missing(v) || missing(o)) return WM_ERR_NULL_POINTER;
-  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
-  return p2(p, make_view(a), make_view(v), make_view(o));
+int wm_unwindow_matmul_forward(const wm_operand *a, const wm_operand *v, const wm_operand *o, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return unwindow_forward(a, v, o, B, M, N, w, dtype, flags, stream);
 }
 
-int wm_unwindow_matmul_backward(const wm_operand *a, const wm_operand *v, const wm_operand *grad_o,
-                                const wm_operand *grad_a, const wm_operand *grad_v, int64_t B, int64_t M,
-                                int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
-  if (B == 0 || M == 0) return WM_OK;
-  if ((grad_a && !grad_a->data) || (grad_v && !grad_v->data)) return WM_ERR_NULL_POINTER;
-  if (N > 0 && (missing(a) || missing(v) || missing(grad_o))) return WM_ERR_NULL_POINTER;
-  const Problem p{B, M, N, w, dtype, flags, (hipStream_t)stream};
-  if (grad_a && grad_v && N > 0 && fused_backward_allowed(p)) {  // small problems: both products in one launch
-    hipError_t err = hipSuccess;
-    if (try_launch_vector_unwindow_backward(p, make_view(a), make_view(v), make_view(grad_o), make_view(grad_a),
-                                            make_view(grad_v), &err))
-      return to_status(err);
-  }
-  if (grad_a) {
-    const wm_operand none{grad_a->data, 0, 0, 0};  // N == 0: grad_a is all +0.0
-    if (int st = p1(p, make_view(N > 0 ? grad_o : &none), make_view(N > 0 ? v : &none), make_view(grad_a)))
-      return st;
-  }
-  if (grad_v && N > 0)
-    if (int st = p3(p, make_view(a), make_view(grad_o), make_view(grad_v))) return st;
-  return WM_OK;
+int wm_unwindow_matmul_backward(const wm_operand *a, const wm_operand *v, const wm_operand *grad_o, const wm_operand *grad_a, const wm_operand *grad_v, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return unwindow_backward(a, v, grad_o, grad_a, grad_v, B, M, N, w, dtype, flags, stream);
 }
 
 int wm_band_softmax_forward(const wm_operand *a, const wm_operand *p, int64_t B, int64_t M, int64_t w, double scale,
@@ -185,41 +271,31 @@ int wm_band_softmax_backward(const wm_operand *p, const wm_operand *grad_p, cons
                                                 mask_out_of_range));
 }
 
-int wm_window_attention_forward(const wm_operand *q, const wm_operand *k, const wm_operand *v, const wm_operand *o,
-                                float *lse, int64_t B, int64_t M, int64_t N, int64_t w, double scale,
-                                int mask_out_of_range, int dtype, unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
-  if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
-  if (B == 0 || M == 0) return WM_OK;
-  if (missing(q) || missing(k) || missing(v) || missing(o)) return WM_ERR_NULL_POINTER;
-  const Problem prob{B, M, N, w, dtype, flags, static_cast<hipStream_t>(stream)};
-  hipError_t err = hipSuccess;
-  if (!try_launch_attention_forward(prob, make_view(q), make_view(k), make_view(v), make_view(o), lse, scale,
-                                    mask_out_of_range, &err))
-    return WM_ERR_UNSUPPORTED;
-  return to_status(err);
+int wm_window_attention_forward(const wm_operand *q, const wm_operand *k, const wm_operand *v, const wm_operand *o, float *lse, int64_t B, int64_t M, int64_t N, int64_t w, double scale, int mask_out_of_range, int dtype, unsigned flags, void *stream) {
+  return attention_forward(q, k, v, o, lse, B, M, N, w, scale, mask_out_of_range, dtype, flags, stream);
 }
 
-int wm_window_attention_backward(const wm_operand *q, const wm_operand *k, const wm_operand *v, const wm_operand *o,
-                                 const float *lse, const wm_operand *grad_o, const wm_operand *grad_q,
-                                 const wm_operand *grad_k, const wm_operand *grad_v, float *delta, int64_t B,
-                                 int64_t M, int64_t N, int64_t w, double scale, int dtype, unsigned flags,
-                                 void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
-  if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
-  if (B == 0 || M == 0) return WM_OK;
-  if (missing(q) || missing(k) || missing(v) || missing(o) || missing(grad_o) || lse == nullptr || delta == nullptr)
-    return WM_ERR_NULL_POINTER;
-  if (grad_q == nullptr && grad_k == nullptr && grad_v == nullptr) return WM_OK;
-  if ((grad_q && !grad_q->data) || (grad_k && !grad_k->data) || (grad_v && !grad_v->data)) return WM_ERR_NULL_POINTER;
-  const Problem prob{B, M, N, w, dtype, flags, static_cast<hipStream_t>(stream)};
-  const View none{nullptr, 0, 0, 0};
-  hipError_t err = hipSuccess;
-  if (!try_launch_attention_backward(prob, make_view(q), make_view(k), make_view(v), make_view(o), make_view(grad_o),
-                                     lse, delta, grad_q ? make_view(grad_q) : none, grad_k ? make_view(grad_k) : none,
-                                     grad_v ? make_view(grad_v) : none, scale, &err))
-    return WM_ERR_UNSUPPORTED;
-  return to_status(err);
+int wm_window_attention_backward(const wm_operand *q, const wm_operand *k, const wm_operand *v, const wm_operand *o, const float *lse, const wm_operand *grad_o, const wm_operand *grad_q, const wm_operand *grad_k, const wm_operand *grad_v, float *delta, int64_t B, int64_t M, int64_t N, int64_t w, double scale, int dtype, unsigned flags, void *stream) {
+  return attention_backward(q, k, v, o, lse, grad_o, grad_q, grad_k, grad_v, delta, B, M, N, w, scale, dtype, flags, stream);
+}
+
+int wm_grouped_window_matmul_forward(const wm_grouped_operand *q, const wm_grouped_operand *k, const wm_operand *a, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return window_forward(q, k, a, B, M, N, w, dtype, flags, stream);
+}
+int wm_grouped_window_matmul_backward(const wm_grouped_operand *q, const wm_grouped_operand *k, const wm_operand *grad_a, const wm_grouped_operand *grad_q, const wm_grouped_operand *grad_k, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return window_backward(q, k, grad_a, grad_q, grad_k, B, M, N, w, dtype, flags, stream);
+}
+int wm_grouped_unwindow_matmul_forward(const wm_operand *a, const wm_grouped_operand *v, const wm_grouped_operand *o, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return unwindow_forward(a, v, o, B, M, N, w, dtype, flags, stream);
+}
+int wm_grouped_unwindow_matmul_backward(const wm_operand *a, const wm_grouped_operand *v, const wm_grouped_operand *grad_o, const wm_operand *grad_a, const wm_grouped_operand *grad_v, int64_t B, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags, void *stream) {
+  return unwindow_backward(a, v, grad_o, grad_a, grad_v, B, M, N, w, dtype, flags, stream);
+}
+int wm_grouped_window_attention_forward(const wm_grouped_operand *q, const wm_grouped_operand *k, const wm_grouped_operand *v, const wm_grouped_operand *o, float *lse, int64_t B, int64_t M, int64_t N, int64_t w, double scale, int mask_out_of_range, int dtype, unsigned flags, void *stream) {
+  return attention_forward(q, k, v, o, lse, B, M, N, w, scale, mask_out_of_range, dtype, flags, stream);
+}
+int wm_grouped_window_attention_backward(const wm_grouped_operand *q, const wm_grouped_operand *k, const wm_grouped_operand *v, const wm_grouped_operand *o, const float *lse, const wm_grouped_operand *grad_o, const wm_grouped_operand *grad_q, const wm_grouped_operand *grad_k, const wm_grouped_operand *grad_v, float *delta, int64_t B, int64_t M, int64_t N, int64_t w, double scale, int dtype, unsigned flags, void *stream) {
+  return attention_backward(q, k, v, o, lse, grad_o, grad_q, grad_k, grad_v, delta, B, M, N, w, scale, dtype, flags, stream);
 }
 
 int wm_window_attention_backward_static(const wm_operand *q, const wm_operand *k, const wm_operand *v,
@@ -243,7 +319,7 @@ int wm_key_rows(const wm_operand *k, void *rows, int64_t B, int64_t N, int64_t M
   if (missing(k) || rows == nullptr) return WM_ERR_NULL_POINTER;
   if (k->stride_c != 1) return WM_ERR_UNSUPPORTED;
   hipError_t err = hipSuccess;
-  if (!try_launch_transpose(k->data, rows, B, N, M, k->stride_b, k->stride_r, (int)dtype_size(dtype),
+  if (!try_launch_transpose(k->data, rows, B, N, M, make_view(k).sb, k->stride_r, (int)dtype_size(dtype),
                             static_cast<hipStream_t>(stream), &err))
     return WM_ERR_UNSUPPORTED;
   return to_status(err);

@@ -64,8 +64,8 @@ __device__ __forceinline__ float across_halves_sum(float v) {
 template <typename T, int NK, bool MASK>  // N = 16 NK
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, int64_t qsb, int64_t qsr,
-    int64_t ksb, int64_t ksr, int64_t vsb, int64_t vsr, int64_t osb, int64_t osr) {
+    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, BatchStep qsb, int64_t qsr,
+    BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;  // NB blocks of 32 output columns; the last may be half used
   constexpr int KS = N + 8;         // key rows 16 (mod 128) bytes apart in banks: conflict-free b128 reads
   constexpr int VS = 32 * NB + 16;  // value rows 32 or 96 (mod 128) bytes apart: what the transposed reads want
@@ -76,17 +76,18 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ksb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
   const int i0 = blk * AT_TM;
   const int qw0 = i0 + 32 * wave;     // first query of this wavefront
   const int qi = qw0 + (lane & 31);   // this lane's query
-  const uint16_t *Kb = K + (int64_t)b * ksb;
-  const uint16_t *Vb = V + (int64_t)b * vsb;
+  const uint16_t *Kb = K + ksb.at(bp);
+  const uint16_t *Vb = V + vsb.at(bp);
 
   // B operand of the first product: the wavefront's 32 queries, all of N, in registers
   u32x4 qf[NK];
   {
-    const uint16_t *qr = Q + (int64_t)b * qsb + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) qf[ks] = load_row_chunk(qr + 16 * ks, Q, qi < M);
   }
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
   if (L != nullptr && half == 0 && qi < M) L[(int64_t)b * M + qi] = (m_used + __builtin_amdgcn_logf(l)) * kLn2F;
   // every wave is past the last barrier: the value buffers are free and stage the result rows
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * AT_KC * VS, "the four staging areas must fit the value buffers");
-  store_wave_rows<T, NB>(&v_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + (int64_t)b * osb, osr, qw0, M, N, lane);
+  store_wave_rows<T, NB>(&v_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + osb.at(bp), osr, qw0, M, N, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -237,10 +238,10 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
 // (keys for S^T, then values for the second product, then the output rows, which leave as whole
 // non-temporal lines).  What bounds this kernel is HBM: it reads q, k, v and writes o, nothing else.
 template <typename T, int NK, int NKB, bool MASK>
-__global__ __launch_bounds__(kThreads, 2) void attention_forward_narrow_kernel(
+__global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_narrow_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, int64_t qsb, int64_t qsr,
-    int64_t ksb, int64_t ksr, int64_t vsb, int64_t vsr, int64_t osb, int64_t osr) {
+    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, BatchStep qsb, int64_t qsr,
+    BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
   constexpr int PADW = 16 * (NKB - 1);         // keys staged before the first and after the last query
   constexpr int ROWS = AT_TM + 2 * PADW;       // key / value rows of the workgroup
@@ -253,6 +254,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_forward_narrow_kernel(
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, qsb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
   const int i0 = blk * AT_TM;
   const int qw0 = i0 + 32 * wave, qi = qw0 + (lane & 31);
@@ -262,10 +264,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_forward_narrow_kernel(
   // value rows as coalesced 16-byte pieces (rows outside the sequence read a safe address, zeroed later)
   u32x4 qf[NK], kreg[SLOTS], vreg[SLOTS];
   {
-    const uint16_t *qr = Q + (int64_t)b * qsb + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) qf[ks] = fetch_row_chunk(qr + 16 * ks, Q, qi < M);
-    const uint16_t *Kb = K + (int64_t)b * ksb, *Vb = V + (int64_t)b * vsb;
+    const uint16_t *Kb = K + ksb.at(bp), *Vb = V + vsb.at(bp);
 #pragma unroll
     for (int u = 0; u < SLOTS; ++u) {
       const int p = min(tid + kThreads * u, PIECES - 1);
@@ -367,7 +369,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_forward_narrow_kernel(
   for (int p = lane; p < 32 * PER_ROW; p += 64) {
     const int r = p / PER_ROW, hg = p - r * PER_ROW;
     if (qw0 + r < M)
-      store_chunk_streaming(O + (int64_t)b * osb + (int64_t)(qw0 + r) * osr + 8 * hg,
+      store_chunk_streaming(O + osb.at(bp) + (int64_t)(qw0 + r) * osr + 8 * hg,
                             *reinterpret_cast<const u32x4 *>(stage + r * SO + 8 * hg));
   }
 }
@@ -391,8 +393,8 @@ __global__ __launch_bounds__(kThreads, 2) void attention_forward_narrow_kernel(
 template <typename T, int NK, bool MASK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_dma_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, int64_t qsb, int64_t qsr,
-    int64_t ksb, int64_t ksr, int64_t vsb, int64_t vsr, int64_t osb, int64_t osr) {
+    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, BatchStep qsb, int64_t qsr,
+    BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr) {
   // tile rows of 128 bytes (N <= 64) or 256 bytes; the pieces of a row beyond column N are never
   // fetched (requested out of range: zeros, no memory traffic)
   constexpr int N = 16 * NK, NB = (NK + 1) / 2, ROWB = NK <= 4 ? 128 : 256, PPR = ROWB / 16;
@@ -405,14 +407,15 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ksb.heads);
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i0 = blk * AT_TM;
   const int qw0 = i0 + 32 * wave;     // first query of this wavefront (scalar)
   const int qi = qw0 + (lane & 31);   // this lane's query
 
-  const u32x4 k_rsrc = make_rsrc(K + (int64_t)b * ksb, (uint32_t)((M - 1) * ksr * 2 + 2 * N));
-  const u32x4 v_rsrc = make_rsrc(V + (int64_t)b * vsb, (uint32_t)((M - 1) * vsr * 2 + 2 * N));
+  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * N));
+  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * N));
   const bool piece_in_row = (((64 * wave + lane) % PPR) ^ swz<PPR>((64 * wave + lane) / PPR)) < N / 8;
   const uint32_t k_voff = piece_in_row ? dma_lane_offset<PPR>(wave, lane, ksr) : 0x80000000u;
   const uint32_t v_voff = piece_in_row ? dma_lane_offset<PPR>(wave, lane, vsr) : 0x80000000u;
@@ -431,7 +434,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   // B operand of the first product: the wavefront's 32 queries, all of N, in registers
   u32x4 qf[NK];
   {
-    const uint16_t *qr = Q + (int64_t)b * qsb + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) qf[ks] = load_row_chunk(qr + 16 * ks, Q, qi < M);
   }
@@ -600,7 +603,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * STAGES * TILE, "the four staging areas must fit the tiles");
-  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + (int64_t)b * osb, osr, qw0, M, N, lane);
+  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + osb.at(bp), osr, qw0, M, N, lane);
 }
 
 template <typename T, int NK>

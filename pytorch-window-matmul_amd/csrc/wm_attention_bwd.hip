@@ -79,9 +79,9 @@ template <typename T, int NK, bool WITH_DQ>  // N = 16 NK; WITH_DQ false: only D
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_query_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L,
-    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, float scale, int64_t qsb,
-    int64_t qsr, int64_t ksb, int64_t ksr, int64_t vsb, int64_t vsr, int64_t osb, int64_t osr, int64_t gsb, int64_t gsr,
-    int64_t dqsb, int64_t dqsr) {
+    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, float scale, BatchStep qsb,
+    int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr,
+    BatchStep dqsb, int64_t dqsr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
   constexpr int TS = 32 * NB + 16;  // tile rows 32 or 96 (mod 128) bytes apart: row reads and transposed reads
   constexpr int PIECES = AB_KC * N / 8;
@@ -91,22 +91,23 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ksb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
   const int i0 = blk * AB_TM;
   const int qw0 = i0 + 32 * wave;
   const int qi = qw0 + (lane & 31);
   const bool q_ok = qi < M;
-  const uint16_t *Kb = K + (int64_t)b * ksb;
-  const uint16_t *Vb = V + (int64_t)b * vsb;
+  const uint16_t *Kb = K + ksb.at(bp);
+  const uint16_t *Vb = V + vsb.at(bp);
   const float c = scale * 1.4426950408889634f;
 
   // stationary side in registers: the query rows and their upstream gradient rows (B operands)
   u32x4 qf[NK], gf[NK];
   float delta = 0.0f;
   {
-    const uint16_t *qr = Q + (int64_t)b * qsb + (int64_t)qi * qsr + 8 * half;
-    const uint16_t *gr = dO + (int64_t)b * gsb + (int64_t)qi * gsr + 8 * half;
-    const uint16_t *orow = O + (int64_t)b * osb + (int64_t)qi * osr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr + 8 * half;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
       qf[ks] = load_row_chunk(qr + 16 * ks, Q, q_ok);
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_
   }
   // every wave is past the last barrier: the key buffers are free and stage the result rows
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * AB_KC * TS, "the four staging areas must fit the key buffers");
-  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, 1.0f, dQ + (int64_t)b * dqsb, dqsr, qw0, M, N,
+  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, 1.0f, dQ + dqsb.at(bp), dqsr, qw0, M, N,
                          lane);
 }
 
@@ -226,9 +227,9 @@ template <typename T, int NK>  // N = 16 NK
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_key_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ dO, const float *__restrict__ L, const float *__restrict__ D,
-    uint16_t *__restrict__ dK, uint16_t *__restrict__ dV, int B, int M, int w, int nblk, float scale, int64_t qsb,
-    int64_t qsr, int64_t ksb, int64_t ksr, int64_t vsb, int64_t vsr, int64_t gsb, int64_t gsr, int64_t dksb,
-    int64_t dksr, int64_t dvsb, int64_t dvsr) {
+    uint16_t *__restrict__ dK, uint16_t *__restrict__ dV, int B, int M, int w, int nblk, float scale, BatchStep qsb,
+    int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep gsb, int64_t gsr, BatchStep dksb,
+    int64_t dksr, BatchStep dvsb, int64_t dvsr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
   constexpr int TS = 32 * NB + 16;
   constexpr int PIECES = AB_KC * N / 8;
@@ -240,21 +241,22 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, qsb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
   const int c0 = blk * AB_TM;
   const int kw0 = c0 + 32 * wave;     // first key of this wavefront
   const int kj = kw0 + (lane & 31);   // this lane's key
   const bool k_ok = kj < M;
-  const uint16_t *Qb = Q + (int64_t)b * qsb;
-  const uint16_t *Gb = dO + (int64_t)b * gsb;
+  const uint16_t *Qb = Q + qsb.at(bp);
+  const uint16_t *Gb = dO + gsb.at(bp);
   const float *Lb = L + (int64_t)b * M;
   const float *Db = D + (int64_t)b * M;
   const float c = scale * 1.4426950408889634f;
 
   u32x4 kf[NK], vf[NK];
   {
-    const uint16_t *kr = K + (int64_t)b * ksb + (int64_t)kj * ksr + 8 * half;
-    const uint16_t *vr = V + (int64_t)b * vsb + (int64_t)kj * vsr + 8 * half;
+    const uint16_t *kr = K + ksb.at(bp) + (int64_t)kj * ksr + 8 * half;
+    const uint16_t *vr = V + vsb.at(bp) + (int64_t)kj * vsr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
       kf[ks] = load_row_chunk(kr + 16 * ks, K, k_ok);
@@ -371,8 +373,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   // either output may be absent (gradient not requested)
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * AB_KC * TS, "the four staging areas must fit the query buffers");
   uint16_t *stage = &q_lds[0][0] + wave * RowStage<NB>::ELEMS;
-  if (dK != nullptr) store_wave_rows<T, NB>(stage, dk, 1.0f, dK + (int64_t)b * dksb, dksr, kw0, M, N, lane);
-  if (dV != nullptr) store_wave_rows<T, NB>(stage, dv, 1.0f, dV + (int64_t)b * dvsb, dvsr, kw0, M, N, lane);
+  if (dK != nullptr) store_wave_rows<T, NB>(stage, dk, 1.0f, dK + dksb.at(bp), dksr, kw0, M, N, lane);
+  if (dV != nullptr) store_wave_rows<T, NB>(stage, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, N, lane);
 }
 
 
@@ -429,14 +431,15 @@ struct BwdTile {
 template <typename T, int NK>
 __global__ __launch_bounds__(kThreads) void attention_backward_stats_kernel(
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L, float *__restrict__ D,
-    int B, int M, int nblk, int64_t osb, int64_t osr, int64_t gsb, int64_t gsr) {
+    int B, int M, int nblk, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr) {
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, gsb.heads);
   const int lane = threadIdx.x & 63, half = lane >> 5;
   const int qi = blk * AB_TM + 32 * (threadIdx.x >> 6) + (lane & 31);
   const bool q_ok = qi < M;
-  const uint16_t *gr = dO + (int64_t)b * gsb + (int64_t)qi * gsr + 8 * half;
-  const uint16_t *orow = O + (int64_t)b * osb + (int64_t)qi * osr + 8 * half;
+  const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr + 8 * half;
+  const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr + 8 * half;
   float delta = 0.0f;
 #pragma unroll
   for (int ks = 0; ks < NK; ++ks)
@@ -455,9 +458,9 @@ template <typename T, int NK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_query_dma_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L,
-    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, float scale, int64_t qsb,
-    int64_t qsr, int64_t ksb, int64_t ksr, int64_t vsb, int64_t vsr, int64_t osb, int64_t osr, int64_t gsb, int64_t gsr,
-    int64_t dqsb, int64_t dqsr) {
+    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, float scale, BatchStep qsb,
+    int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr,
+    BatchStep dqsb, int64_t dqsr) {
   typedef BwdTile<NK> TL;
   constexpr int N = TL::N, NB = TL::NB, PPR = TL::PPR, ROWB = TL::ROWB, TILE = TL::TILE;
   constexpr int STAGES = 2, DEPTH = STAGES - 1;
@@ -467,6 +470,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ksb.heads);
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i0 = blk * AB_TM;
@@ -475,8 +479,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
   const bool q_ok = qi < M;
   const float c = scale * kLog2e;
 
-  const u32x4 k_rsrc = make_rsrc(K + (int64_t)b * ksb, (uint32_t)((M - 1) * ksr * 2 + 2 * N));
-  const u32x4 v_rsrc = make_rsrc(V + (int64_t)b * vsb, (uint32_t)((M - 1) * vsr * 2 + 2 * N));
+  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * N));
+  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * N));
   const uint32_t k_voff = TL::load_offset(wave, lane, ksr), v_voff = TL::load_offset(wave, lane, vsr);
   const uint32_t k_step = (uint32_t)(256 / PPR * ksr * 2), v_step = (uint32_t)(256 / PPR * vsr * 2);
   const uint32_t k_chunk = (uint32_t)(AB_KC * ksr * 2), v_chunk = (uint32_t)(AB_KC * vsr * 2);
@@ -493,9 +497,9 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
   u32x4 qf[NK], gf[NK];
   float delta = 0.0f;
   {
-    const uint16_t *qr = Q + (int64_t)b * qsb + (int64_t)qi * qsr + 8 * half;
-    const uint16_t *gr = dO + (int64_t)b * gsb + (int64_t)qi * gsr + 8 * half;
-    const uint16_t *orow = O + (int64_t)b * osb + (int64_t)qi * osr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr + 8 * half;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
       qf[ks] = load_row_chunk(qr + 16 * ks, Q, q_ok);
@@ -598,7 +602,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
   wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * STAGES * TILE, "the four staging areas must fit the tiles");
-  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, scale, dQ + (int64_t)b * dqsb, dqsr, qw0, M, N,
+  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, scale, dQ + dqsb.at(bp), dqsr, qw0, M, N,
                          lane);
 }
 
@@ -606,8 +610,8 @@ template <typename T, int NK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_key_dma_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ dO, const float *__restrict__ D, uint16_t *__restrict__ dK,
-    uint16_t *__restrict__ dV, int B, int M, int w, int nblk, float scale, int64_t qsb, int64_t qsr, int64_t ksb,
-    int64_t ksr, int64_t vsb, int64_t vsr, int64_t gsb, int64_t gsr, int64_t dksb, int64_t dksr, int64_t dvsb,
+    uint16_t *__restrict__ dV, int B, int M, int w, int nblk, float scale, BatchStep qsb, int64_t qsr, BatchStep ksb,
+    int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep gsb, int64_t gsr, BatchStep dksb, int64_t dksr, BatchStep dvsb,
     int64_t dvsr) {
   typedef BwdTile<NK> TL;
   constexpr int N = TL::N, NB = TL::NB, PPR = TL::PPR, ROWB = TL::ROWB, TILE = TL::TILE;
@@ -619,6 +623,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, qsb.heads);
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c0 = blk * AB_TM;
@@ -627,8 +632,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   const bool k_ok = kj < M;
   const float c = scale * kLog2e;
 
-  const u32x4 q_rsrc = make_rsrc(Q + (int64_t)b * qsb, (uint32_t)((M - 1) * qsr * 2 + 2 * N));
-  const u32x4 g_rsrc = make_rsrc(dO + (int64_t)b * gsb, (uint32_t)((M - 1) * gsr * 2 + 2 * N));
+  const u32x4 q_rsrc = make_rsrc(Q + qsb.at(bp), (uint32_t)((M - 1) * qsr * 2 + 2 * N));
+  const u32x4 g_rsrc = make_rsrc(dO + gsb.at(bp), (uint32_t)((M - 1) * gsr * 2 + 2 * N));
   // waves 0 and 2 fetch D, waves 1 and 3 the log-sum-exp (twice the same 256 bytes each: every
   // wavefront then has the same number of loads in flight, which is what the waits count)
   const u32x4 s_rsrc = make_rsrc(D + ((int64_t)(wave & 1) * B + b) * M, (uint32_t)(M * 4));
@@ -647,8 +652,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
 
   u32x4 kf[NK], vf[NK];
   {
-    const uint16_t *kr = K + (int64_t)b * ksb + (int64_t)kj * ksr + 8 * half;
-    const uint16_t *vr = V + (int64_t)b * vsb + (int64_t)kj * vsr + 8 * half;
+    const uint16_t *kr = K + ksb.at(bp) + (int64_t)kj * ksr + 8 * half;
+    const uint16_t *vr = V + vsb.at(bp) + (int64_t)kj * vsr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
       kf[ks] = load_row_chunk(kr + 16 * ks, K, k_ok);
@@ -764,8 +769,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   __builtin_amdgcn_s_barrier();
   static_assert(4 * RowStage<NB>::ELEMS <= STAGES * TILE, "the four staging areas must fit the query tiles");
   uint16_t *stage_rows = &q_lds[0][0] + wave * RowStage<NB>::ELEMS;
-  if (dK != nullptr) store_wave_rows<T, NB>(stage_rows, dk, scale, dK + (int64_t)b * dksb, dksr, kw0, M, N, lane);
-  if (dV != nullptr) store_wave_rows<T, NB>(stage_rows, dv, 1.0f, dV + (int64_t)b * dvsb, dvsr, kw0, M, N, lane);
+  if (dK != nullptr) store_wave_rows<T, NB>(stage_rows, dk, scale, dK + dksb.at(bp), dksr, kw0, M, N, lane);
+  if (dV != nullptr) store_wave_rows<T, NB>(stage_rows, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, N, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -788,8 +793,8 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L,
     uint16_t *__restrict__ dQ, uint16_t *__restrict__ dK, uint16_t *__restrict__ dV, int B, int M, int w, int nblk,
-    float scale, int64_t qsb, int64_t qsr, int64_t ksb, int64_t ksr, int64_t vsb, int64_t vsr, int64_t osb, int64_t osr,
-    int64_t gsb, int64_t gsr, int64_t dqsb, int64_t dqsr, int64_t dksb, int64_t dksr, int64_t dvsb, int64_t dvsr) {
+    float scale, BatchStep qsb, int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr,
+    BatchStep gsb, int64_t gsr, BatchStep dqsb, int64_t dqsr, BatchStep dksb, int64_t dksr, BatchStep dvsb, int64_t dvsr) {
   static_assert(NK <= 4, "rows of 128 bytes: two tiles and the staging must fit 64 KB of LDS");
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
   constexpr int PADW = 16 * (NKB - 1);     // tile rows before the first and after the last own row
@@ -811,6 +816,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, qsb.heads);
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i0 = blk * AB_TM;
@@ -834,8 +840,8 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
       dma_piece(rsrc, lds + 4096 * j, wanted ? (uint32_t)(row * sr * 2 + piece * 16) : 0x80000000u, 0);
     }
   };
-  request(Q + (int64_t)b * qsb, qsr, tile_a);
-  request(dO + (int64_t)b * gsb, gsr, tile_b);
+  request(Q + qsb.at(bp), qsr, tile_a);
+  request(dO + gsb.at(bp), gsr, tile_b);
 
   const uint32_t row_at = TL::row_at(lane), tr_at = TL::tr_at(lane);
   const float ninf = -__builtin_huge_valf();
@@ -863,7 +869,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   {
     const int row = t0 + own_first + r32;
     const bool ok = row >= need_lo && row <= need_hi;
-    const uint16_t *orow = O + (int64_t)b * osb + (int64_t)row * osr + 8 * half;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)row * osr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) o_own[ks] = load_row_chunk(orow + 16 * ks, O, ok);
     l_own = ok ? L[(int64_t)b * M + row] * kLog2e : 0.0f;
@@ -871,7 +877,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   if (halo_wave) {
     const int row = t0 + halo_first + h32;
     const bool ok = row >= need_lo && row <= need_hi;
-    const uint16_t *orow = O + (int64_t)b * osb + (int64_t)row * osr + 8 * half;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)row * osr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) o_halo[ks] = load_row_chunk(orow + 16 * ks, O, ok);
     l_halo = ok ? L[(int64_t)b * M + row] * kLog2e : 0.0f;
@@ -879,8 +885,8 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   // own rows as keys: B operands of the first two products
   u32x4 kf[NK], vf[NK];
   if (want_kv) {
-    const uint16_t *kr = K + (int64_t)b * ksb + (int64_t)ri * ksr + 8 * half;
-    const uint16_t *vr = V + (int64_t)b * vsb + (int64_t)ri * vsr + 8 * half;
+    const uint16_t *kr = K + ksb.at(bp) + (int64_t)ri * ksr + 8 * half;
+    const uint16_t *vr = V + vsb.at(bp) + (int64_t)ri * vsr + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
       kf[ks] = load_row_chunk(kr + 16 * ks, K, r_ok);
@@ -980,13 +986,13 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   }
   __syncthreads();  // nobody reads the tiles any more
   // K replaces Q while dK and dV leave through the other tile; V follows when those rows are out
-  if (dQ != nullptr) request(K + (int64_t)b * ksb, ksr, tile_a);
+  if (dQ != nullptr) request(K + ksb.at(bp), ksr, tile_a);
   uint16_t *stage_rows = tile_b + wave * RowStage<NB>::ELEMS;
-  if (dK != nullptr) store_wave_rows<T, NB>(stage_rows, dk, scale, dK + (int64_t)b * dksb, dksr, rw0, M, N, lane);
-  if (dV != nullptr) store_wave_rows<T, NB>(stage_rows, dv, 1.0f, dV + (int64_t)b * dvsb, dvsr, rw0, M, N, lane);
+  if (dK != nullptr) store_wave_rows<T, NB>(stage_rows, dk, scale, dK + dksb.at(bp), dksr, rw0, M, N, lane);
+  if (dV != nullptr) store_wave_rows<T, NB>(stage_rows, dv, 1.0f, dV + dvsb.at(bp), dvsr, rw0, M, N, lane);
   if (dQ == nullptr) return;
   __syncthreads();
-  request(V + (int64_t)b * vsb, vsr, tile_b);
+  request(V + vsb.at(bp), vsr, tile_b);
   f32x16 dq[NB];
 #pragma unroll
   for (int hb = 0; hb < NB; ++hb)
@@ -1040,7 +1046,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
     }
   }
   __syncthreads();
-  store_wave_rows<T, NB>(tile_a + wave * RowStage<NB>::ELEMS, dq, scale, dQ + (int64_t)b * dqsb, dqsr, rw0, M, N, lane);
+  store_wave_rows<T, NB>(tile_a + wave * RowStage<NB>::ELEMS, dq, scale, dQ + dqsb.at(bp), dqsr, rw0, M, N, lane);
 }
 
 template <typename T, int NK>

@@ -81,8 +81,8 @@ template <int NT, bool TRANSPOSED>
 __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void f32_band_in_kernel(const float *__restrict__ A,
                                                                   const float *__restrict__ Y,
                                                                   float *__restrict__ C, int B, int M, int N, int w,
-                                                                  int nblk, int64_t asb, int64_t ysb, int64_t ysr,
-                                                                  int64_t csb, int64_t csr) {
+                                                                  int nblk, int64_t asb, BatchStep ysb, int64_t ysr,
+                                                                  BatchStep csb, int64_t csr) {
   constexpr int NP = 32 * NT;
   constexpr int ST = TRANSPOSED ? TM + 4 : KC + 4;  // T tile: [KC][TM] (P3) or [TM][KC] (P2), floats
   constexpr int TROWS = TRANSPOSED ? KC : TM;
@@ -93,6 +93,7 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void f32_band_in_kernel(
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = 2 * w + 1;
   const int o0 = blk * TM;                 // first output row of the block (i for P2, c for P3)
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void f32_band_in_kernel(
   // blockIdx.y selects which NP columns of Y and C this workgroup works on (one workgroup does all
   // of them unless the launch splits the columns to fill the chip)
   const int h0 = NP * blockIdx.y;
-  const float *Yb = Y + (int64_t)b * ysb + h0;
+  const float *Yb = Y + ysb.at(bp) + h0;
   const int ncg = min(N - h0, NP) >> 2, ychunks = KC * ncg;
   int y_row[NT], y_col[NT];  // this thread's pieces of a Y chunk; row KC = none
 #pragma unroll
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void f32_band_in_kernel(
   // of its rows at a time in a private area and the rows leave as 16-byte pieces, 8 consecutive
   // lanes on one 128-byte line (non-temporal: the result is not read again here).
   float *stage = &t_lds[0][0] + wave * (32 * kStage);
-  float *Cb = C + (int64_t)b * csb + h0;
+  float *Cb = C + csb.at(bp) + h0;
   N -= h0;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -294,7 +295,7 @@ template <int NK8>  // N = 8 NK8
 __global__ __launch_bounds__(kThreads, NK8 <= 8 ? 4 : 2) void f32_band_out_kernel(const float *__restrict__ X,
                                                                    const float *__restrict__ Y,
                                                                    float *__restrict__ C, int B, int M, int w,
-                                                                   int nblk, int64_t xsb, int64_t xsr, int64_t ysb,
+                                                                   int nblk, BatchStep xsb, int64_t xsr, BatchStep ysb,
                                                                    int64_t ysr, int64_t csb) {
   constexpr int N = 8 * NK8;
   constexpr int SY = N + 4;
@@ -305,6 +306,7 @@ __global__ __launch_bounds__(kThreads, NK8 <= 8 ? 4 : 2) void f32_band_out_kerne
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int half = lane >> 5, col = lane & 31;
   const int W = 2 * w + 1;
@@ -318,7 +320,7 @@ __global__ __launch_bounds__(kThreads, NK8 <= 8 ? 4 : 2) void f32_band_out_kerne
     c_lo += first * KC;
     nk = last - first;
   }
-  const float *Yb = Y + (int64_t)b * ysb;
+  const float *Yb = Y + ysb.at(bp);
   float *Cb = C + (int64_t)b * csb;
 
   // this lane's row of X, the k values of its half-wave: xop[u][j] = X[i][8u + 4 half + j]
@@ -326,7 +328,7 @@ __global__ __launch_bounds__(kThreads, NK8 <= 8 ? 4 : 2) void f32_band_out_kerne
   f32x4 xop[NK8];
 #pragma unroll
   for (int u = 0; u < NK8; ++u)
-    xop[u] = load_row4(X + (int64_t)b * xsb + (int64_t)i * xsr + 8 * u + 4 * half, X, i < M);
+    xop[u] = load_row4(X + xsb.at(bp) + (int64_t)i * xsr + 8 * u + 4 * half, X, i < M);
 
   int y_row[YS], y_col[YS];  // this thread's pieces of a Y chunk; row KC = none
 #pragma unroll
@@ -453,14 +455,14 @@ hipError_t launch_band_in(const Problem &p, const View &a, const View &y, const 
   if (nb > 1 && wgs < 2 * kCUs && (wgs * nb + kCUs - 1) / kCUs < nb * ((wgs + kCUs - 1) / kCUs)) {
     grid.y = (unsigned)nb;
     hipLaunchKernelGGL((f32_band_in_kernel<1, TRANSPOSED>), grid, block, 0, p.stream, (const float *)a.data,
-                       (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, a.sb, y.sb,
+                       (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, a.sb.step, y.sb,
                        y.sr, c.sb, c.sr);
     return hipGetLastError();
   }
 #define WM_F32_IN(NT)                                                                                        \
   hipLaunchKernelGGL((f32_band_in_kernel<NT, TRANSPOSED>), grid, block, 0, p.stream, (const float *)a.data,  \
                      (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk,   \
-                     a.sb, y.sb, y.sr, c.sb, c.sr)
+                     a.sb.step, y.sb, y.sr, c.sb, c.sr)
   switch ((p.N + 31) / 32) {
     case 1: WM_F32_IN(1); break;
     case 2: WM_F32_IN(2); break;
@@ -482,7 +484,7 @@ hipError_t launch_band_out(const Problem &p, const View &x, const View &y, const
   case NK8:                                                                                                 \
     hipLaunchKernelGGL((f32_band_out_kernel<NK8>), grid, block, 0, p.stream, (const float *)x.data,         \
                        (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, x.sb,    \
-                       x.sr, y.sb, y.sr, c.sb);                                                             \
+                       x.sr, y.sb, y.sr, c.sb.step);                                                             \
     break;
   switch (p.N / 8) {
     WM_F32_OUT(1) WM_F32_OUT(2) WM_F32_OUT(3) WM_F32_OUT(4) WM_F32_OUT(5) WM_F32_OUT(6) WM_F32_OUT(7) WM_F32_OUT(8)

@@ -99,7 +99,7 @@ __device__ __forceinline__ f32x16 mma_split(const u32x4 (&xa)[3], const u32x4 (&
 template <int NT, bool TRANSPOSED>
 __global__ __launch_bounds__(kThreads, 2) void f32_split_band_in_kernel(
     const float *__restrict__ A, const float *__restrict__ Y, float *__restrict__ C, int B, int M, int N, int w, int nblk,
-    int64_t asb, int64_t ysb, int64_t ysr, int64_t csb, int64_t csr) {
+    int64_t asb, BatchStep ysb, int64_t ysr, BatchStep csb, int64_t csr) {
   constexpr int NP = 32 * NT;
   constexpr int ST = TRANSPOSED ? TM + 4 : SKC + 4;  // T tile: [KC][TM] (P3) or [TM][KC] (P2), floats
   constexpr int TROWS = TRANSPOSED ? SKC : TM;
@@ -111,6 +111,7 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_in_kernel(
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = 2 * w + 1;
   const int o0 = blk * TM;                 // first output row of the block (i for P2, c for P3)
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_in_kernel(
   // blockIdx.y selects which NP columns of Y and C this workgroup works on (one workgroup does all
   // of them unless the launch splits the columns)
   const int h0 = NP * blockIdx.y;
-  const float *Yb = Y + (int64_t)b * ysb + h0;
+  const float *Yb = Y + ysb.at(bp) + h0;
   const int ncg = min(N - h0, NP) >> 2, ychunks = SKC * ncg;
   int y_row[NT], y_col[NT];  // this thread's pieces of a Y chunk; row SKC = none
 #pragma unroll
@@ -303,7 +304,7 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_in_kernel(
   // of its rows at a time in a private area and the rows leave as 16-byte pieces, 8 consecutive
   // lanes on one 128-byte line (non-temporal: the result is not read again here).
   float *stage = &t_lds[0][0] + wave * (32 * kStage);
-  float *Cb = C + (int64_t)b * csb + h0;
+  float *Cb = C + csb.at(bp) + h0;
   N -= h0;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -333,7 +334,7 @@ template <int NKG>  // 16 NKG - 8 <= N <= 16 NKG
 __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const float *__restrict__ X,
                                                                         const float *__restrict__ Y,
                                                                         float *__restrict__ C, int B, int M, int N, int w,
-                                                                        int nblk, int64_t xsb, int64_t xsr, int64_t ysb,
+                                                                        int nblk, BatchStep xsb, int64_t xsr, BatchStep ysb,
                                                                         int64_t ysr, int64_t csb) {
   constexpr int NP = 16 * NKG;
   constexpr int SY = NP + 8;  // plane rows an odd number of 16-byte slots apart: conflict-free 16-byte reads
@@ -344,6 +345,7 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const f
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int half = lane >> 5, col = lane & 31;
   const int W = 2 * w + 1;
@@ -357,7 +359,7 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const f
     c_lo += first * SKC;
     nk = last - first;
   }
-  const float *Yb = Y + (int64_t)b * ysb;
+  const float *Yb = Y + ysb.at(bp);
   float *Cb = C + (int64_t)b * csb;
   // columns N .. NP - 1 of the planes are never written by a piece and must read as zeros
   if (N < NP) {
@@ -369,7 +371,7 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const f
   const int i = i0 + wave * 32 + col;
   u32x4 xop[NKG][3];
   {
-    const float *xr = X + (int64_t)b * xsb + (int64_t)i * xsr;
+    const float *xr = X + xsb.at(bp) + (int64_t)i * xsr;
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int g = 0; g < NKG; ++g) {
@@ -500,7 +502,7 @@ hipError_t launch_split_band_in(const Problem &p, const View &a, const View &y, 
   const int64_t wgs = p.B * nblk, nb = (p.N + 31) / 32;
 #define WM_F32S_IN(NT)                                                                                          \
   hipLaunchKernelGGL((f32_split_band_in_kernel<NT, TRANSPOSED>), grid, block, 0, p.stream, (const float *)a.data, \
-                     (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, a.sb,  \
+                     (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, a.sb.step,  \
                      y.sb, y.sr, c.sb, c.sr)
   // When the workgroups do not fill the CUs once or twice, each 32-column block of Y gets workgroups
   // of its own (the rule of wm_f32.hip: the band tile is then fetched once per block, by workgroups
@@ -534,7 +536,7 @@ hipError_t launch_split_band_out(const Problem &p, const View &x, const View &y,
   case NKG:                                                                                                   \
     hipLaunchKernelGGL((f32_split_band_out_kernel<NKG>), grid, block, 0, p.stream, (const float *)x.data,     \
                        (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk,  \
-                       x.sb, x.sr, y.sb, y.sr, c.sb);                                                         \
+                       x.sb, x.sr, y.sb, y.sr, c.sb.step);                                                         \
     break;
   switch ((p.N + 15) / 16) {
     WM_F32S_OUT(1) WM_F32S_OUT(2) WM_F32S_OUT(3) WM_F32S_OUT(4) WM_F32S_OUT(5) WM_F32S_OUT(6) WM_F32S_OUT(7)

@@ -41,8 +41,8 @@ template <typename T, int NT, bool ALIGNED, int KCH>
 __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void mfma_p2_kernel(const uint16_t *__restrict__ A,
                                                               const uint16_t *__restrict__ Y,
                                                               uint16_t *__restrict__ C, int B, int M, int N, int w,
-                                                              int nblk, int galign, int64_t asb, int64_t ysb,
-                                                              int64_t ysr, int64_t csb, int64_t csr) {
+                                                              int nblk, int galign, int64_t asb, BatchStep ysb,
+                                                              int64_t ysr, BatchStep csb, int64_t csr) {
   constexpr int KC = KCH;                 // chunk length of this kernel (shadows the family default)
   constexpr int TS = TM * KC / 8 / kThreads;  // band chunks per thread per tile
   constexpr int GPR = KC / 8;              // 8-column groups per tile row
@@ -58,13 +58,14 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void mfma_p2_kernel(cons
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = 2 * w + 1;
   const int i0 = blk * TM;
   const int rows = min(TM, M - i0);
   const int c_lo = max(i0 - w, 0), c_hi = min(i0 + rows - 1 + w, M - 1);
   const uint16_t *Ab = A + (int64_t)b * asb;
-  const uint16_t *Yb = Y + (int64_t)b * ysb;
+  const uint16_t *Yb = Y + ysb.at(bp);
   const int c_start = ALIGNED ? c_lo - (int)(((int64_t)c_lo + (int64_t)b * asb + w) & (galign - 1)) : c_lo;
   const int nk = (c_hi - c_start + KC) / KC;
 
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void mfma_p2_kernel(cons
   // acc[nt][v]: h = 32 nt + 8 (v / 4) + 4 (lane / 32) + v % 4, row = wave * 32 + lane % 32; every
   // wave is past the last barrier, so the tile buffers are free
   static_assert(4 * RowStage<NT>::ELEMS <= 2 * TM * KC, "the four staging areas must fit the band tile buffers");
-  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + (int64_t)b * csb, csr,
+  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + csb.at(bp), csr,
                          i0 + wave * 32, M, N, lane);
 }
 
@@ -204,8 +205,8 @@ template <typename T, int NT, bool ALIGNED>
 __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void mfma_p3_kernel(const uint16_t *__restrict__ A,
                                                               const uint16_t *__restrict__ Y,
                                                               uint16_t *__restrict__ C, int B, int M, int N, int w,
-                                                              int nblk, int galign, int64_t asb, int64_t ysb,
-                                                              int64_t ysr, int64_t csb, int64_t csr) {
+                                                              int nblk, int galign, int64_t asb, BatchStep ysb,
+                                                              int64_t ysr, BatchStep csb, int64_t csr) {
   constexpr int NP = 32 * NT;
   constexpr int ST = TM;  // T tile [KC rows r][TM cols c], unpadded and swizzled (see lds_read_transposed_swz)
   constexpr int SY = lds_stride_tr(NP);
@@ -214,6 +215,7 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void mfma_p3_kernel(cons
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = 2 * w + 1;
   // block origin: aligned variant shifts it left so that every 8-column group is an aligned chunk
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void mfma_p3_kernel(cons
   const int r_lo = max(c_first - w, 0), r_hi = min(c_last + w, M - 1);
   const int nk = (r_hi - r_lo + KC) / KC;
   const uint16_t *Ab = A + (int64_t)b * asb;
-  const uint16_t *Yb = Y + (int64_t)b * ysb;
+  const uint16_t *Yb = Y + ysb.at(bp);
 
   const int ychunks = KC * (N >> 3), ncg = N >> 3;
   int y_r[NT], y_h[NT], y_off[NT];
@@ -320,7 +322,7 @@ __global__ __launch_bounds__(kThreads, NT <= 2 ? 3 : 2) void mfma_p3_kernel(cons
   if (k < nk) slot(k, t_reg[0], y_reg[0], t_reg[1], y_reg[1]);
 
   static_assert(4 * RowStage<NT>::ELEMS <= 2 * TM * KC, "the four staging areas must fit the band tile buffers");
-  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + (int64_t)b * csb, csr,
+  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + csb.at(bp), csr,
                          c0 + wave * 32, M, N, lane);
 }
 
@@ -345,8 +347,8 @@ template <typename T, int NK, bool ALIGNED, int RING = 0, bool LINES = false>  /
 __global__ __launch_bounds__(kThreads, RING && NK <= 4 ? 3 : 2) void mfma_p1_kernel(const uint16_t *__restrict__ X,
                                                               const uint16_t *__restrict__ Y,
                                                               uint16_t *__restrict__ C, int B, int M, int w,
-                                                              int nblk, int galign, int64_t xsb, int64_t xsr,
-                                                              int64_t ysb, int64_t ysr, int64_t csb) {
+                                                              int nblk, int galign, BatchStep xsb, int64_t xsr,
+                                                              BatchStep ysb, int64_t ysr, int64_t csb) {
   constexpr int N = 16 * NK;
   constexpr int SY = N + 8;   // Y chunk rows: 16 (mod 128) bytes apart in banks -> conflict-free b128 reads
   // per-wave staging rows: one chunk, padded; or a ring of two chunks, unpadded, the 16-byte piece p
@@ -365,6 +367,7 @@ __global__ __launch_bounds__(kThreads, RING && NK <= 4 ? 3 : 2) void mfma_p1_ker
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = 2 * w + 1;
   const int i0 = blk * TM;
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(kThreads, RING && NK <= 4 ? 3 : 2) void mfma_p1_ker
     c_start += k0 * KC;
     nk = (RING && last_share ? last - 1 : last) - k0;
   }
-  const uint16_t *Yb = Y + (int64_t)b * ysb;
+  const uint16_t *Yb = Y + ysb.at(bp);
   uint16_t *Cb = C + (int64_t)b * csb;
   // Head and tail pieces of neighbouring rows meet through the seam buffer when both rows belong
   // to this wave, or to any wave of the workgroup if a workgroup barrier is certain to separate
@@ -403,7 +406,7 @@ __global__ __launch_bounds__(kThreads, RING && NK <= 4 ? 3 : 2) void mfma_p1_ker
   u32x4 xop[NK];
   {
     const int i = i0 + wave * 32 + (lane & 31);
-    const uint16_t *xr = X + (int64_t)b * xsb + (int64_t)i * xsr + 8 * (lane >> 5);
+    const uint16_t *xr = X + xsb.at(bp) + (int64_t)i * xsr + 8 * (lane >> 5);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) xop[ks] = load_row_chunk(xr + 16 * ks, X, i < M);
   }
@@ -627,8 +630,8 @@ template <typename T, int NK, bool ALIGNED>  // NK = N / 16
 __global__ __launch_bounds__(kThreads, 3) void mfma_p1_dma_kernel(const uint16_t *__restrict__ X,
                                                               const uint16_t *__restrict__ Y,
                                                               uint16_t *__restrict__ C, int B, int M, int w,
-                                                              int nblk, int galign, int64_t xsb, int64_t xsr,
-                                                              int64_t ysb, int64_t ysr, int64_t csb) {
+                                                              int nblk, int galign, BatchStep xsb, int64_t xsr,
+                                                              BatchStep ysb, int64_t ysr, int64_t csb) {
   constexpr int N = 16 * NK, PPR = 2 * NK, ROWB = 2 * N;  // 16-byte pieces and bytes per tile row
   constexpr int SS = KC + 8;  // per-wave staging rows
   constexpr int LOADS = PPR / 4;  // loads per wavefront and chunk
@@ -643,6 +646,7 @@ __global__ __launch_bounds__(kThreads, 3) void mfma_p1_dma_kernel(const uint16_t
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);
   const int W = 2 * w + 1;
@@ -651,7 +655,7 @@ __global__ __launch_bounds__(kThreads, 3) void mfma_p1_dma_kernel(const uint16_t
   const int c_lo = i0 - w, c_hi = i0 + rows - 1 + w;  // not clipped: out-of-sequence entries are written as zeros
   const int c_start = ALIGNED ? c_lo - (int)(((int64_t)c_lo + (int64_t)b * csb + w) & (galign - 1)) : c_lo;
   const int nk = (c_hi - c_start + KC) / KC;
-  const uint16_t *Yb = Y + (int64_t)b * ysb;
+  const uint16_t *Yb = Y + ysb.at(bp);
   uint16_t *Cb = C + (int64_t)b * csb;
   // Head and tail pieces of neighbouring rows meet through the seam buffer when both rows belong
   // to this wave, or to any wave of the workgroup if a workgroup barrier is certain to separate
@@ -662,7 +666,7 @@ __global__ __launch_bounds__(kThreads, 3) void mfma_p1_dma_kernel(const uint16_t
   u32x4 xop[NK];
   {
     const int i = i0 + wave * 32 + (lane & 31);
-    const uint16_t *xr = X + (int64_t)b * xsb + (int64_t)i * xsr + 8 * (lane >> 5);
+    const uint16_t *xr = X + xsb.at(bp) + (int64_t)i * xsr + 8 * (lane >> 5);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) xop[ks] = load_row_chunk(xr + 16 * ks, X, i < M);
   }
@@ -855,7 +859,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KCH * (2 * TM + (
                                                  ? 3
                                                  : 160 * 1024 / (STAGES * KCH * (2 * TM + (NK <= 4 ? 128 : 256))) >= 2 ? 2 : 1)) void mfma_p3_dma_kernel(
     const uint16_t *__restrict__ A, const uint16_t *__restrict__ Y, uint16_t *__restrict__ C, int B, int M, int n_total, int w,
-    int nblk, int galign, int64_t asb, int64_t ysb, int64_t ysr, int64_t csb, int64_t csr) {
+    int nblk, int galign, int64_t asb, BatchStep ysb, int64_t ysr, BatchStep csb, int64_t csr) {
   constexpr int N = 16 * NK, NT = (NK + 1) / 2, CH = KCH, DEPTH = STAGES - 1;
   using TT = LdsTile<CH, TM / 8>;            // [CH rows r][TM columns c]
   using YT = LdsTile<CH, NK <= 4 ? 8 : 16>;  // [CH rows r][64 or 128 columns, of which N are fetched]
@@ -867,6 +871,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KCH * (2 * TM + (
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int W = 2 * w + 1;
@@ -890,7 +895,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KCH * (2 * TM + (
   // give every block of columns workgroups of its own; otherwise there is one block)
   const int h0 = N * (int)blockIdx.y;
   const int n_cols = min(N, n_total - h0);  // (the last block of a width that is no multiple of N is narrower)
-  const u32x4 y_rsrc = make_rsrc(Y + (int64_t)b * ysb + h0, (uint32_t)(((int64_t)(M - 1) * ysr + n_cols) * 2));
+  const u32x4 y_rsrc = make_rsrc(Y + ysb.at(bp) + h0, (uint32_t)(((int64_t)(M - 1) * ysr + n_cols) * 2));
   // (pieces of the Y tile beyond column N are requested out of range: zeros, no memory traffic)
   const uint32_t y_voff = YT::load_piece(wave, lane) < n_cols / 8 ? YT::lane_offset(wave, lane, ysr) : 0x80000000u;
   const uint32_t y_step = YT::step(ysr), y_row = (uint32_t)(ysr * 2);
@@ -962,7 +967,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KCH * (2 * TM + (
   wait_vmcnt<0>();
   __syncthreads();
   static_assert(4 * RowStage<NT>::ELEMS <= STAGES * TT::ELEMS, "the four staging areas must fit the band tile buffers");
-  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + (int64_t)b * csb + h0, csr, cw0, M,
+  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + csb.at(bp) + h0, csr, cw0, M,
                          n_cols, lane);
 }
 
@@ -978,7 +983,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KC * (2 * TM + (N
                                            ? 3
                                            : 160 * 1024 / (STAGES * KC * (2 * TM + (NK <= 4 ? 128 : 256))) >= 2 ? 2 : 1)) void mfma_p2_dma_kernel(
     const uint16_t *__restrict__ A, const uint16_t *__restrict__ Y, uint16_t *__restrict__ C, int B, int M, int n_total, int w,
-    int nblk, int galign, int64_t asb, int64_t ysb, int64_t ysr, int64_t csb, int64_t csr) {
+    int nblk, int galign, int64_t asb, BatchStep ysb, int64_t ysr, BatchStep csb, int64_t csr) {
   constexpr int N = 16 * NK, NT = (NK + 1) / 2, DEPTH = STAGES - 1;
   using TT = LdsTile<TM, KC / 8>;            // [TM rows i][KC dense columns c]
   using YT = LdsTile<KC, NK <= 4 ? 8 : 16>;  // [KC rows c][64 or 128 columns, of which N are fetched]
@@ -990,6 +995,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KC * (2 * TM + (N
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int W = 2 * w + 1;
@@ -1011,7 +1017,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KC * (2 * TM + (N
   // give every block of columns workgroups of its own; otherwise there is one block)
   const int h0 = N * (int)blockIdx.y;
   const int n_cols = min(N, n_total - h0);  // (the last block of a width that is no multiple of N is narrower)
-  const u32x4 y_rsrc = make_rsrc(Y + (int64_t)b * ysb + h0, (uint32_t)(((int64_t)(M - 1) * ysr + n_cols) * 2));
+  const u32x4 y_rsrc = make_rsrc(Y + ysb.at(bp) + h0, (uint32_t)(((int64_t)(M - 1) * ysr + n_cols) * 2));
   const bool y_piece = YT::load_piece(wave, lane) < n_cols / 8;  // else: beyond the block's columns, requested out of range
   const uint32_t y_voff = YT::lane_offset(wave, lane, ysr), y_step = YT::step(ysr), y_row = (uint32_t)(ysr * 2);
   // pieces of the band tile that hold no entry of the band (8 columns from c8 of row i with c8 - i
@@ -1083,7 +1089,7 @@ __global__ __launch_bounds__(kThreads, (160 * 1024 / (STAGES * KC * (2 * TM + (N
   wait_vmcnt<0>();
   __syncthreads();
   static_assert(4 * RowStage<NT>::ELEMS <= STAGES * TT::ELEMS, "the four staging areas must fit the band tile buffers");
-  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + (int64_t)b * csb + h0, csr, iw0, M,
+  store_wave_rows<T, NT>(&t_lds[0][0] + wave * RowStage<NT>::ELEMS, acc, 1.0f, C + csb.at(bp) + h0, csr, iw0, M,
                          n_cols, lane);
 }
 
@@ -1168,7 +1174,7 @@ hipError_t launch_p2(const Problem &p, const View &a, const View &y, const View 
   case NK:                                                                                                     \
     hipLaunchKernelGGL((mfma_p2_dma_kernel<T, NK, STAGES>), grid_c, block, 0, p.stream, (const uint16_t *)a.data, \
                        (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w,   \
-                       nblk, g, a.sb, y.sb, y.sr, c.sb, c.sr);                                                 \
+                       nblk, g, a.sb.step, y.sb, y.sr, c.sb, c.sr);                                                 \
     break;
     switch (nkb) {
       WM_P2_DMA(1, 2) WM_P2_DMA(2, 2) WM_P2_DMA(3, 2) WM_P2_DMA(4, 2) WM_P2_DMA(5, 2) WM_P2_DMA(6, 2) WM_P2_DMA(7, 2)
@@ -1180,7 +1186,7 @@ hipError_t launch_p2(const Problem &p, const View &a, const View &y, const View 
 #define WM_P2(NT)                                                                                              \
   hipLaunchKernelGGL((mfma_p2_kernel<T, NT, ALIGNED, WM_P2_KC>), grid, block, 0, p.stream, (const uint16_t *)a.data,     \
                      (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, \
-                     galign, a.sb, y.sb, y.sr, c.sb, c.sr)
+                     galign, a.sb.step, y.sb, y.sr, c.sb, c.sr)
   switch ((p.N + 31) / 32) {
     case 1: WM_P2(1); break;
     case 2: WM_P2(2); break;
@@ -1208,7 +1214,7 @@ hipError_t launch_p3(const Problem &p, const View &a, const View &y, const View 
   case NK:                                                                                                     \
     hipLaunchKernelGGL((mfma_p3_dma_kernel<T, NK, KCH, STAGES>), grid_g, block, 0, p.stream,                   \
                        (const uint16_t *)a.data, (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B,       \
-                       (int)p.M, (int)p.N, (int)p.w, nblk_g, g, a.sb, y.sb, y.sr, c.sb, c.sr);                 \
+                       (int)p.M, (int)p.N, (int)p.w, nblk_g, g, a.sb.step, y.sb, y.sr, c.sb, c.sr);                 \
     break;
     // A band of a few chunks only: chunks of 32 rows, three deep, fit four workgroups on a CU up to
     // N = 64 and overfetch less at the band's edges (B96 M16384 N64, 32- against 64-row chunks: 119
@@ -1230,7 +1236,7 @@ hipError_t launch_p3(const Problem &p, const View &a, const View &y, const View 
 #define WM_P3(NT)                                                                                              \
   hipLaunchKernelGGL((mfma_p3_kernel<T, NT, ALIGNED>), grid, block, 0, p.stream, (const uint16_t *)a.data,     \
                      (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, \
-                     galign, a.sb, y.sb, y.sr, c.sb, c.sr)
+                     galign, a.sb.step, y.sb, y.sr, c.sb, c.sr)
   switch ((p.N + 31) / 32) {
     case 1: WM_P3(1); break;
     case 2: WM_P3(2); break;
@@ -1267,7 +1273,7 @@ hipError_t launch_p1(const Problem &p, const View &x, const View &y, const View 
 #define WM_P1_LAUNCH(NK, AL, RING, LINES, G)                                                                 \
   hipLaunchKernelGGL((mfma_p1_kernel<T, NK, AL, RING, LINES>), grid, block, 0, p.stream,                     \
                      (const uint16_t *)x.data, (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B,       \
-                     (int)p.M, (int)p.w, nblk, G, x.sb, x.sr, y.sb, y.sr, c.sb)
+                     (int)p.M, (int)p.w, nblk, G, x.sb, x.sr, y.sb, y.sr, c.sb.step)
 #define WM_P1(NK)                                                                                            \
   if (!ALIGNED && ring_pays && ring_unaligned)                                                               \
     WM_P1_LAUNCH(NK, true, 2, false, 2);                                                                     \
@@ -1290,7 +1296,7 @@ hipError_t launch_p1(const Problem &p, const View &x, const View &y, const View 
     // equal at w = 256 and 512 and 8 % slower at w = 64)
     hipLaunchKernelGGL((mfma_p1_dma_kernel<T, 8, ALIGNED>), dim3(grid.x), block, 0, p.stream, (const uint16_t *)x.data,
                        (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, galign, x.sb,
-                       x.sr, y.sb, y.sr, c.sb);
+                       x.sr, y.sb, y.sr, c.sb.step);
     return hipGetLastError();
   }
   switch (p.N / 16) {

@@ -47,7 +47,7 @@ template <typename T, int NK, int NYT>  // N = 16 NK; NYT 16-row tiles of Y cove
 __global__ __launch_bounds__(kThreads) void small_p1_kernel(const uint16_t *__restrict__ X,
                                                               const uint16_t *__restrict__ Y,
                                                               uint16_t *__restrict__ C, int B, int M, int w, int nblk,
-                                                              int64_t xsb, int64_t xsr, int64_t ysb, int64_t ysr,
+                                                              BatchStep xsb, int64_t xsr, BatchStep ysb, int64_t ysr,
                                                               int64_t csb) {
   constexpr int ROWS = 256;  // band rows per workgroup, 64 per wave
   constexpr int NK2 = (NK + 1) / 2;  // 32-column steps
@@ -55,6 +55,7 @@ __global__ __launch_bounds__(kThreads) void small_p1_kernel(const uint16_t *__re
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, xsb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = 2 * w + 1;
   const int i0 = blk * ROWS, iw0 = i0 + 64 * wave;
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(kThreads) void small_p1_kernel(const uint16_t *__re
     const int l16 = lane & 15, kq = lane >> 4;  // row of a tile; 8-column group of a 32-column step
     auto has_columns = [&](int ks) { return 32 * ks + 8 * kq < 16 * NK; };  // false only in half a last step
     u32x4 xop[4][NK2], yop[NYT][NK2];
-    const uint16_t *Xb = X + (int64_t)b * xsb, *Yb = Y + (int64_t)b * ysb;
+    const uint16_t *Xb = X + xsb.at(bp), *Yb = Y + ysb.at(bp);
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
       const int i = iw0 + 16 * rb + l16;
@@ -158,13 +159,14 @@ template <int NK, int NYT>  // N = 16 NK; NYT 16-row tiles of Y cover 64 + 2w ro
 __global__ __launch_bounds__(kThreads) void small_p1_f32_kernel(const float *__restrict__ X,
                                                                 const float *__restrict__ Y,
                                                                 float *__restrict__ C, int B, int M, int w, int nblk,
-                                                                int64_t xsb, int64_t xsr, int64_t ysb, int64_t ysr,
+                                                                BatchStep xsb, int64_t xsr, BatchStep ysb, int64_t ysr,
                                                                 int64_t csb) {
   constexpr int ROWS = 256;  // band rows per workgroup, 64 per wave
   extern __shared__ __attribute__((aligned(16))) float flat_f32[];  // 4 + ROWS * W (+ slack) elements
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, xsb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int W = 2 * w + 1;
   const int i0 = blk * ROWS, iw0 = i0 + 64 * wave;
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(kThreads) void small_p1_f32_kernel(const float *__r
   if (iw0 < M) {
     const int l16 = lane & 15, kq = lane >> 4;
     f32x4 xop[4][NK], yop[NYT][NK];
-    const float *Xb = X + (int64_t)b * xsb, *Yb = Y + (int64_t)b * ysb;
+    const float *Xb = X + xsb.at(bp), *Yb = Y + ysb.at(bp);
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
       const int i = iw0 + 16 * rb + l16;
@@ -273,7 +275,7 @@ template <int NT, bool TRANSPOSED>  // N = 16 NT <= 64
 __global__ __launch_bounds__(kThreads) void small_in_f32_kernel(const float *__restrict__ A,
                                                                 const float *__restrict__ Y,
                                                                 float *__restrict__ C, int B, int M, int w, int nblk,
-                                                                int64_t asb, int64_t ysb, int64_t ysr, int64_t csb,
+                                                                int64_t asb, BatchStep ysb, int64_t ysr, BatchStep csb,
                                                                 int64_t csr) {
   constexpr int ROWS = 64, N = 16 * NT;
   constexpr int MAXC = TRANSPOSED ? 8 : 4;  // aligned 4-float chunks of band rows per thread (checked on the host)
@@ -287,9 +289,10 @@ __global__ __launch_bounds__(kThreads) void small_in_f32_kernel(const float *__r
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i0 = blk * ROWS;
-  const float *Ab = A + (int64_t)b * asb, *Yb = Y + (int64_t)b * ysb;
+  const float *Ab = A + (int64_t)b * asb, *Yb = Y + ysb.at(bp);
   const int cv0 = i0 - wp;
 
   // band rows r_s .. r_e, flat: aligned chunks of four floats, all requested before any is used
@@ -382,7 +385,7 @@ __global__ __launch_bounds__(kThreads) void small_in_f32_kernel(const float *__r
   }
   // acc[t][v]: column 16 t + 4 (lane / 16) + v of row i
   if (i < M) {
-    float *crow = C + (int64_t)b * csb + (int64_t)i * csr + 4 * kq;
+    float *crow = C + csb.at(bp) + (int64_t)i * csr + 4 * kq;
 #pragma unroll
     for (int t = 0; t < NT; ++t) __builtin_nontemporal_store(acc[t], reinterpret_cast<f32x4 *>(crow + 16 * t));
   }
@@ -442,8 +445,8 @@ template <typename T, int NT, int RW, bool RP>  // N <= 32 NT; RW rows per wave;
 __global__ __launch_bounds__(kThreads) void small_p2_kernel(const uint16_t *__restrict__ A,
                                                             const uint16_t *__restrict__ Y,
                                                             uint16_t *__restrict__ C, int B, int M, int N, int w,
-                                                            int nblk, int64_t asb, int64_t ysb, int64_t ysr,
-                                                            int64_t csb, int64_t csr) {
+                                                            int nblk, int64_t asb, BatchStep ysb, int64_t ysr,
+                                                            BatchStep csb, int64_t csr) {
   constexpr int ROWS = 4 * RW;
   constexpr int SY = lds_stride_tr(32 * NT);
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -455,11 +458,12 @@ __global__ __launch_bounds__(kThreads) void small_p2_kernel(const uint16_t *__re
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i0 = blk * ROWS;
   const int nrows = min(ROWS, M - i0);
   const uint16_t *Ab = A + (int64_t)b * asb + (int64_t)i0 * W;
-  const uint16_t *Yb = Y + (int64_t)b * ysb;
+  const uint16_t *Yb = Y + ysb.at(bp);
   const int delta = RP ? 0 : (int)((reinterpret_cast<uintptr_t>(Ab) >> 1) & 7);
 
   // band rows, flat: aligned chunks; the first and last chunk may hold neighbours' entries
@@ -555,7 +559,7 @@ __global__ __launch_bounds__(kThreads) void small_p2_kernel(const uint16_t *__re
     const int r = q / per_row, hg = q - r * per_row;
     const int i = i0 + RW * wave + r;
     if (i < M)  // whole 128-byte lines, written once and not read again here: non-temporal
-      store_chunk_streaming(C + (int64_t)b * csb + (int64_t)i * csr + 8 * hg,
+      store_chunk_streaming(C + csb.at(bp) + (int64_t)i * csr + 8 * hg,
                             *reinterpret_cast<const u32x4 *>(stage + r * SO + 8 * hg));
   }
 }
@@ -576,8 +580,8 @@ template <typename T, int NT, int RW, bool RP>  // N <= 32 NT; RW output rows pe
 __global__ __launch_bounds__(kThreads) void small_p3_kernel(const uint16_t *__restrict__ A,
                                                             const uint16_t *__restrict__ Y,
                                                             uint16_t *__restrict__ C, int B, int M, int N, int w,
-                                                            int nblk, int64_t asb, int64_t ysb, int64_t ysr,
-                                                            int64_t csb, int64_t csr) {
+                                                            int nblk, int64_t asb, BatchStep ysb, int64_t ysr,
+                                                            BatchStep csb, int64_t csr) {
   constexpr int ROWS = 4 * RW;
   constexpr int SY = lds_stride_tr(32 * NT);
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -592,6 +596,7 @@ __global__ __launch_bounds__(kThreads) void small_p3_kernel(const uint16_t *__re
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t base_el = (int64_t)(reinterpret_cast<uintptr_t>(A) >> 1) + (int64_t)b * asb;
   const int shift = RP ? 0 : (int)((base_el + w) & 7);
@@ -599,7 +604,7 @@ __global__ __launch_bounds__(kThreads) void small_p3_kernel(const uint16_t *__re
   if (c_first >= M) return;
   const int r_org = c_first - wp;          // band row that image row 0 stands for (may be < 0)
   const int r_s = max(r_org, 0), r_e = min(r_org + span - 1, M - 1);  // rows that exist
-  const uint16_t *Yb = Y + (int64_t)b * ysb;
+  const uint16_t *Yb = Y + ysb.at(bp);
   // global element index of image element 0, rounded down to a chunk: g0 = base + r_org * W - delta
   const int64_t g_org = base_el + (int64_t)r_org * W;
   const int delta = RP ? 0 : (int)(g_org & 7);
@@ -692,7 +697,7 @@ __global__ __launch_bounds__(kThreads) void small_p3_kernel(const uint16_t *__re
     const int r = q / per_row, hg = q - r * per_row;
     const int c = c_first + RW * wave + r;
     if (c >= 0 && c < M)
-      store_chunk_streaming(C + (int64_t)b * csb + (int64_t)c * csr + 8 * hg,
+      store_chunk_streaming(C + csb.at(bp) + (int64_t)c * csr + 8 * hg,
                             *reinterpret_cast<const u32x4 *>(stage + r * SO + 8 * hg));
   }
 }
@@ -726,7 +731,7 @@ hipError_t launch_small_p1(const Problem &p, const View &x, const View &y, const
 #define WM_SP1(NK, NYT)                                                                                      \
   hipLaunchKernelGGL((small_p1_kernel<T, NK, NYT>), grid, block, lds, p.stream, (const uint16_t *)x.data,      \
                      (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, x.sb,   \
-                     x.sr, y.sb, y.sr, c.sb)
+                     x.sr, y.sb, y.sr, c.sb.step)
 #define WM_SP1_N(NYT)                    \
   switch (p.N / 16) {                    \
     case 1: WM_SP1(1, NYT); break;       \
@@ -778,7 +783,7 @@ hipError_t launch_small_p1_f32(const Problem &p, const View &x, const View &y, c
 #define WM_SPF(NK, NYT)                                                                                      \
   hipLaunchKernelGGL((small_p1_f32_kernel<NK, NYT>), grid, block, lds, p.stream, (const float *)x.data,      \
                      (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, x.sb, x.sr, \
-                     y.sb, y.sr, c.sb)
+                     y.sb, y.sr, c.sb.step)
 #define WM_SPF_N(NYT)                    \
   switch (p.N / 16) {                    \
     case 1: WM_SPF(1, NYT); break;       \
@@ -821,7 +826,7 @@ hipError_t launch_small_in_f32(const Problem &p, const View &a, const View &y, c
   const size_t lds = small_in_f32_lds(p.w, p.N);
 #define WM_SIF(NT)                                                                                              \
   hipLaunchKernelGGL((small_in_f32_kernel<NT, TRANSPOSED>), grid, block, lds, p.stream, (const float *)a.data,  \
-                     (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, a.sb, y.sb,    \
+                     (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, a.sb.step, y.sb,    \
                      y.sr, c.sb, c.sr)
   switch (p.N / 16) {
     case 1: WM_SIF(1); break;
@@ -859,7 +864,7 @@ hipError_t launch_small_p2(const Problem &p, const View &a, const View &y, const
 #define WM_SP2(NT_, RW_, RP_)                                                                                  \
   hipLaunchKernelGGL((small_p2_kernel<T, NT_, RW_, RP_>), grid, block, lds, p.stream, (const uint16_t *)a.data, \
                      (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, \
-                     a.sb, y.sb, y.sr, c.sb, c.sr)
+                     a.sb.step, y.sb, y.sr, c.sb, c.sr)
 #define WM_SP2_N(RP_)                   \
   switch (NT) {                         \
     case 1: WM_SP2(1, 32, RP_); break;  \
@@ -896,7 +901,7 @@ hipError_t launch_small_p3(const Problem &p, const View &a, const View &y, const
 #define WM_SP3(NT_, RW_, RP_)                                                                                  \
   hipLaunchKernelGGL((small_p3_kernel<T, NT_, RW_, RP_>), grid, block, lds, p.stream, (const uint16_t *)a.data, \
                      (const uint16_t *)y.data, (uint16_t *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk, \
-                     a.sb, y.sb, y.sr, c.sb, c.sr)
+                     a.sb.step, y.sb, y.sr, c.sb, c.sr)
 #define WM_SP3_N(RP_)                   \
   switch (NT) {                         \
     case 1: WM_SP3(1, 32, RP_); break;  \

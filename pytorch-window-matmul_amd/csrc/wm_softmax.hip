@@ -370,10 +370,10 @@ __global__ __launch_bounds__(kSoftmaxThreads) void band_softmax_strided_kernel(V
   const int W = 2 * w + 1;
   lo = 0, hi = W;
   if (mask) valid_columns(i, M, w, &lo, &hi);
-  const GlobalRow<T> x{static_cast<const T *>(in0.data) + b * in0.sb + i * in0.sr, in0.sc};
-  const GlobalOut<T> o{static_cast<T *>(out.data) + b * out.sb + i * out.sr, out.sc};
+  const GlobalRow<T> x{static_cast<const T *>(in0.data) + b * in0.sb.step + i * in0.sr, in0.sc};
+  const GlobalOut<T> o{static_cast<T *>(out.data) + b * out.sb.step + i * out.sr, out.sc};
   if (BACKWARD) {
-    const GlobalRow<T> g{static_cast<const T *>(in1.data) + b * in1.sb + i * in1.sr, in1.sc};
+    const GlobalRow<T> g{static_cast<const T *>(in1.data) + b * in1.sb.step + i * in1.sr, in1.sc};
     softmax_row_backward<T>(x, g, o, W, lo, hi, gl, (A)scale);
   } else {
     softmax_row_forward<T>(x, o, W, lo, hi, gl, (A)(scale * 1.4426950408889634));
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(kSoftmaxThreads) void band_softmax_strided_kernel(V
 // Host side
 // ---------------------------------------------------------------------------------------------
 bool contiguous_band(const View &v, int64_t M, int64_t W) {
-  return v.sc == 1 && v.sr == W && v.sb == M * W && ((uintptr_t)v.data) % 16 == 0;
+  return v.sc == 1 && v.sr == W && v.sb.step == M * W && ((uintptr_t)v.data) % 16 == 0;
 }
 
 // Shape classes of the register variant, then the re-reading one.  Lanes per row: 64 for rows

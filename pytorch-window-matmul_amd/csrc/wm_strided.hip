@@ -16,8 +16,8 @@ constexpr int kThreads = 256;
 template <typename T>
 __global__ __launch_bounds__(kThreads) void strided_p1_kernel(const T *__restrict__ X, const T *__restrict__ Y,
                                                               T *__restrict__ C, int64_t total, int M, int N,
-                                                              int w, int64_t xsb, int64_t xsr, int64_t xsc,
-                                                              int64_t ysb, int64_t ysr, int64_t ysc, int64_t csb,
+                                                              int w, BatchStep xsb, int64_t xsr, int64_t xsc,
+                                                              BatchStep ysb, int64_t ysr, int64_t ysc, BatchStep csb,
                                                               int64_t csr, int64_t csc) {
   typedef typename Acc<T>::type acc_t;
   const int W = 2 * w + 1;
@@ -27,14 +27,15 @@ __global__ __launch_bounds__(kThreads) void strided_p1_kernel(const T *__restric
     const int64_t bi = idx / W;
     const int i = (int)(bi % M);
     const int64_t b = bi / M;
+    const BatchPos bp = batch_pos(b, csb.heads);
     const int c = i + j - w;
     acc_t acc = 0;
     if (c >= 0 && c < M) {
-      const T *xr = X + b * xsb + (int64_t)i * xsr;
-      const T *yr = Y + b * ysb + (int64_t)c * ysr;
+      const T *xr = X + xsb.at(bp) + (int64_t)i * xsr;
+      const T *yr = Y + ysb.at(bp) + (int64_t)c * ysr;
       for (int h = 0; h < N; ++h) acc += to_acc<T>(xr[(int64_t)h * xsc]) * to_acc<T>(yr[(int64_t)h * ysc]);
     }
-    C[b * csb + (int64_t)i * csr + (int64_t)j * csc] = from_acc<T>(acc);
+    C[csb.at(bp) + (int64_t)i * csr + (int64_t)j * csc] = from_acc<T>(acc);
   }
 }
 
@@ -42,8 +43,8 @@ __global__ __launch_bounds__(kThreads) void strided_p1_kernel(const T *__restric
 template <typename T>
 __global__ __launch_bounds__(kThreads) void strided_p2_kernel(const T *__restrict__ A, const T *__restrict__ Y,
                                                               T *__restrict__ C, int64_t total, int M, int N,
-                                                              int w, int64_t asb, int64_t asr, int64_t asc,
-                                                              int64_t ysb, int64_t ysr, int64_t ysc, int64_t csb,
+                                                              int w, BatchStep asb, int64_t asr, int64_t asc,
+                                                              BatchStep ysb, int64_t ysr, int64_t ysc, BatchStep csb,
                                                               int64_t csr, int64_t csc) {
   typedef typename Acc<T>::type acc_t;
   for (int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x; idx < total;
@@ -52,13 +53,14 @@ __global__ __launch_bounds__(kThreads) void strided_p2_kernel(const T *__restric
     const int64_t bi = idx / N;
     const int i = (int)(bi % M);
     const int64_t b = bi / M;
+    const BatchPos bp = batch_pos(b, csb.heads);
     const int lo = max(i - w, 0), hi = min(i + w, M - 1);
-    const T *ar = A + b * asb + (int64_t)i * asr;
-    const T *yb = Y + b * ysb + (int64_t)h * ysc;
+    const T *ar = A + asb.at(bp) + (int64_t)i * asr;
+    const T *yb = Y + ysb.at(bp) + (int64_t)h * ysc;
     acc_t acc = 0;
     for (int c = lo; c <= hi; ++c)
       acc += to_acc<T>(ar[(int64_t)(c - i + w) * asc]) * to_acc<T>(yb[(int64_t)c * ysr]);
-    C[b * csb + (int64_t)i * csr + (int64_t)h * csc] = from_acc<T>(acc);
+    C[csb.at(bp) + (int64_t)i * csr + (int64_t)h * csc] = from_acc<T>(acc);
   }
 }
 
@@ -66,8 +68,8 @@ __global__ __launch_bounds__(kThreads) void strided_p2_kernel(const T *__restric
 template <typename T>
 __global__ __launch_bounds__(kThreads) void strided_p3_kernel(const T *__restrict__ A, const T *__restrict__ Y,
                                                               T *__restrict__ C, int64_t total, int M, int N,
-                                                              int w, int64_t asb, int64_t asr, int64_t asc,
-                                                              int64_t ysb, int64_t ysr, int64_t ysc, int64_t csb,
+                                                              int w, BatchStep asb, int64_t asr, int64_t asc,
+                                                              BatchStep ysb, int64_t ysr, int64_t ysc, BatchStep csb,
                                                               int64_t csr, int64_t csc) {
   typedef typename Acc<T>::type acc_t;
   for (int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x; idx < total;
@@ -76,13 +78,14 @@ __global__ __launch_bounds__(kThreads) void strided_p3_kernel(const T *__restric
     const int64_t bc = idx / N;
     const int c = (int)(bc % M);
     const int64_t b = bc / M;
+    const BatchPos bp = batch_pos(b, csb.heads);
     const int lo = max(c - w, 0), hi = min(c + w, M - 1);
-    const T *ab = A + b * asb;
-    const T *yb = Y + b * ysb + (int64_t)h * ysc;
+    const T *ab = A + asb.at(bp);
+    const T *yb = Y + ysb.at(bp) + (int64_t)h * ysc;
     acc_t acc = 0;
     for (int r = lo; r <= hi; ++r)
       acc += to_acc<T>(ab[(int64_t)r * asr + (int64_t)(c - r + w) * asc]) * to_acc<T>(yb[(int64_t)r * ysr]);
-    C[b * csb + (int64_t)c * csr + (int64_t)h * csc] = from_acc<T>(acc);
+    C[csb.at(bp) + (int64_t)c * csr + (int64_t)h * csc] = from_acc<T>(acc);
   }
 }
 

@@ -142,7 +142,7 @@ template <class T>
 struct Rows {  // one batch element of a view
   T *p;
   int64_t sr, sc;
-  __device__ Rows(const View &v, int64_t b) : p((T *)v.data + b * v.sb), sr(v.sr), sc(v.sc) {}
+  __device__ Rows(const View &v, int64_t b) : p((T *)v.data + v.sb.at(batch_pos(b, v.sb.heads))), sr(v.sr), sc(v.sc) {}
   __device__ typename Acc<T>::type get(int64_t r, int64_t c) const { return to_acc<T>(p[r * sr + c * sc]); }
   __device__ void put(int64_t r, int64_t c, typename Acc<T>::type v) const { p[r * sr + c * sc] = from_acc<T>(v); }
 };

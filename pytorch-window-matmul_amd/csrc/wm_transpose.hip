@@ -20,14 +20,14 @@ constexpr int TR_T = 64;  // tile edge in elements
 
 template <typename E, bool VEC_IN>  // E: an unsigned integer of the element's size; VEC_IN: source rows are 16-byte aligned
 __global__ __launch_bounds__(256) void transpose_kernel(const E *__restrict__ src, E *__restrict__ dst, int R, int C,
-                                                        int64_t ssb, int64_t ssr) {
+                                                        BatchStep ssb, int64_t ssr) {
   constexpr int ES = sizeof(E), PER = 16 / ES;                // elements per 16-byte piece
   constexpr int PITCH = TR_T * ES + (ES == 8 ? 8 : 4);        // bytes per tile row
   constexpr int PPR = TR_T / PER;                             // pieces per tile row (either way)
   __shared__ __attribute__((aligned(16))) unsigned char tile[TR_T * PITCH];
   const int c0 = blockIdx.x * TR_T, r0 = blockIdx.y * TR_T;
   const int64_t b = blockIdx.z;
-  const E *sb = src + b * ssb;
+  const E *sb = src + ssb.at(batch_pos(b, ssb.heads));
   E *db = dst + b * (int64_t)R * C;
 
   if (VEC_IN) {
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void transpose_kernel(const E *__restrict__ sr
 }
 
 template <typename E>
-hipError_t launch(const void *src, void *dst, int64_t B, int64_t R, int64_t C, int64_t ssb, int64_t ssr, bool vec_in,
+hipError_t launch(const void *src, void *dst, int64_t B, int64_t R, int64_t C, BatchStep ssb, int64_t ssr, bool vec_in,
                   hipStream_t stream) {
   const dim3 grid((unsigned)((C + TR_T - 1) / TR_T), (unsigned)((R + TR_T - 1) / TR_T), (unsigned)B);
   if (vec_in)
@@ -110,14 +110,14 @@ hipError_t launch(const void *src, void *dst, int64_t B, int64_t R, int64_t C, i
 }  // namespace
 
 // false: the layout is not one this kernel takes (nothing launched)
-bool try_launch_transpose(const void *src, void *dst, int64_t B, int64_t R, int64_t C, int64_t ssb, int64_t ssr,
+bool try_launch_transpose(const void *src, void *dst, int64_t B, int64_t R, int64_t C, BatchStep ssb, int64_t ssr,
                           int elem_size, hipStream_t stream, hipError_t *err) {
   if (elem_size != 2 && elem_size != 4 && elem_size != 8) return false;
   const int64_t per = 16 / elem_size;
   // the destination leaves as 16-byte pieces along R; the source comes in as such pieces along C where
   // its rows allow it, element by element otherwise
   if (reinterpret_cast<uintptr_t>(dst) % 16 != 0 || R % per != 0 || reinterpret_cast<uintptr_t>(src) % elem_size != 0) return false;
-  const bool vec_in = reinterpret_cast<uintptr_t>(src) % 16 == 0 && ssb % per == 0 && ssr % per == 0;
+  const bool vec_in = reinterpret_cast<uintptr_t>(src) % 16 == 0 && ssb.step % per == 0 && (ssb.heads <= 0 || ssb.group % per == 0) && ssr % per == 0;
   if (ssr < C || B > 65535 || (R + TR_T - 1) / TR_T > 65535 || C > 0x7fffffff - TR_T || R > 0x7fffffff - TR_T) return false;
   *err = hipSuccess;
   if (B == 0 || R == 0 || C == 0) return true;

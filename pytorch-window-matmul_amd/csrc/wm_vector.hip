@@ -76,8 +76,8 @@ template <typename T, int NK, bool TRANSPOSED>  // N = 16 NK (16-bit) or 8 NK (f
 __device__ __forceinline__ void vector_band_in_body(const typename Elem<T>::type *__restrict__ A,
                                                     const typename Elem<T>::type *__restrict__ Y,
                                                     typename Elem<T>::type *__restrict__ C, int B, int M, int w,
-                                                    int nblk, int vrows, int64_t asb, int64_t ysb, int64_t ysr,
-                                                    int64_t csb, int64_t csr) {
+                                                    int nblk, int vrows, int64_t asb, BatchStep ysb, int64_t ysr,
+                                                    BatchStep csb, int64_t csr) {
   typedef typename Elem<T>::type E;
   constexpr int VEC = 16 / sizeof(E);       // elements per 16-byte piece
   constexpr int NCG = 2 * NK, N = NCG * VEC;  // 16-byte column groups per row
@@ -87,6 +87,7 @@ __device__ __forceinline__ void vector_band_in_body(const typename Elem<T>::type
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ysb.heads);
   const int tid = threadIdx.x;
   const int W = 2 * w + 1;
   const int o0 = blk * vrows;                      // first output row
@@ -98,7 +99,7 @@ __device__ __forceinline__ void vector_band_in_body(const typename Elem<T>::type
   const int a1 = TRANSPOSED ? min(o0 + orows - 1 + w, M - 1) : o0 + orows - 1;
   const int arows = a1 - a0 + 1;
   const E *Ab = A + (int64_t)b * asb + (int64_t)a0 * W;
-  const E *Yb = Y + (int64_t)b * ysb;
+  const E *Yb = Y + ysb.at(bp);
   // flat band image in whole aligned 16-byte chunks: image element e is band element e - delta
   const int delta = (int)((reinterpret_cast<uintptr_t>(Ab) / sizeof(E)) & (VEC - 1));
   const int n_el = arows * W;
@@ -164,7 +165,7 @@ __device__ __forceinline__ void vector_band_in_body(const typename Elem<T>::type
       out = u32x4{__builtin_bit_cast(uint32_t, acc[0]), __builtin_bit_cast(uint32_t, acc[1]),
                   __builtin_bit_cast(uint32_t, acc[2]), __builtin_bit_cast(uint32_t, acc[3])};
     }
-    __builtin_nontemporal_store(out, reinterpret_cast<u32x4 *>(C + (int64_t)b * csb + (int64_t)o * csr + VEC * hg));
+    __builtin_nontemporal_store(out, reinterpret_cast<u32x4 *>(C + csb.at(bp) + (int64_t)o * csr + VEC * hg));
   };
   const int npairs = (orows + 1) >> 1;
   for (int item = tid; item < npairs * NCG; item += kThreads) {
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void vector_band_in_kernel(const typename
                                                                   const typename Elem<T>::type *__restrict__ Y,
                                                                   typename Elem<T>::type *__restrict__ C, int B,
                                                                   int M, int w, int nblk, int vrows, int64_t asb,
-                                                                  int64_t ysb, int64_t ysr, int64_t csb, int64_t csr) {
+                                                                  BatchStep ysb, int64_t ysr, BatchStep csb, int64_t csr) {
   vector_band_in_body<T, NK, TRANSPOSED>(A, Y, C, B, M, w, nblk, vrows, asb, ysb, ysr, csb, csr);
 }
 
@@ -214,8 +215,8 @@ template <typename T, int NK>
 __global__ __launch_bounds__(kThreads) void vector_window_backward_kernel(
     const typename Elem<T>::type *__restrict__ GA, const typename Elem<T>::type *__restrict__ K,
     const typename Elem<T>::type *__restrict__ Q, typename Elem<T>::type *__restrict__ GQ,
-    typename Elem<T>::type *__restrict__ GK, int B, int M, int w, int nblk, int vrows, int64_t asb, int64_t ksb,
-    int64_t ksr, int64_t qsb, int64_t qsr, int64_t gqsb, int64_t gqsr, int64_t gksb, int64_t gksr) {
+    typename Elem<T>::type *__restrict__ GK, int B, int M, int w, int nblk, int vrows, int64_t asb, BatchStep ksb,
+    int64_t ksr, BatchStep qsb, int64_t qsr, BatchStep gqsb, int64_t gqsr, BatchStep gksb, int64_t gksr) {
   if (blockIdx.y == 0)
     vector_band_in_body<T, NK, false>(GA, K, GQ, B, M, w, nblk, vrows, asb, ksb, ksr, gqsb, gqsr);
   else
@@ -241,7 +242,7 @@ template <typename T, int NK>  // 2 NK 16-byte pieces per row: N = 16 NK (16-bit
 __device__ __forceinline__ void vector_band_out_body(const typename Elem<T>::type *__restrict__ X,
                                                      const typename Elem<T>::type *__restrict__ Y,
                                                      typename Elem<T>::type *__restrict__ C, int B, int M, int w,
-                                                     int nblk, int vrows, int64_t xsb, int64_t xsr, int64_t ysb,
+                                                     int nblk, int vrows, BatchStep xsb, int64_t xsr, BatchStep ysb,
                                                      int64_t ysr, int64_t csb) {
   typedef typename Elem<T>::type E;
   constexpr int VEC = 16 / sizeof(E);
@@ -253,11 +254,12 @@ __device__ __forceinline__ void vector_band_out_body(const typename Elem<T>::typ
 
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, xsb.heads);
   const int tid = threadIdx.x;
   const int W = 2 * w + 1;
   const int i0 = blk * vrows;
   const int rows = min(vrows, M - i0);
-  const E *Xb = X + (int64_t)b * xsb, *Yb = Y + (int64_t)b * ysb;
+  const E *Xb = X + xsb.at(bp), *Yb = Y + ysb.at(bp);
   const int xchunks = rows * NCG, ychunks = (rows + 2 * w) * NCG;
   constexpr int BATCH = 8;
   for (int base = 0; base < xchunks + ychunks; base += BATCH * kThreads) {
@@ -314,8 +316,8 @@ template <typename T, int NK>
 __global__ __launch_bounds__(kThreads) void vector_band_out_kernel(const typename Elem<T>::type *__restrict__ X,
                                                                    const typename Elem<T>::type *__restrict__ Y,
                                                                    typename Elem<T>::type *__restrict__ C, int B,
-                                                                   int M, int w, int nblk, int vrows, int64_t xsb,
-                                                                   int64_t xsr, int64_t ysb, int64_t ysr, int64_t csb) {
+                                                                   int M, int w, int nblk, int vrows, BatchStep xsb,
+                                                                   int64_t xsr, BatchStep ysb, int64_t ysr, int64_t csb) {
   vector_band_out_body<T, NK>(X, Y, C, B, M, w, nblk, vrows, xsb, xsr, ysb, ysr, csb);
 }
 
@@ -327,7 +329,7 @@ __global__ __launch_bounds__(kThreads) void vector_unwindow_backward_kernel(
     const typename Elem<T>::type *__restrict__ A, const typename Elem<T>::type *__restrict__ V,
     const typename Elem<T>::type *__restrict__ GO, typename Elem<T>::type *__restrict__ GA,
     typename Elem<T>::type *__restrict__ GV, int B, int M, int w, int oblk, int orows, int iblk, int irows,
-    int64_t asb, int64_t vsb, int64_t vsr, int64_t gosb, int64_t gosr, int64_t gasb, int64_t gvsb, int64_t gvsr) {
+    int64_t asb, BatchStep vsb, int64_t vsr, BatchStep gosb, int64_t gosr, int64_t gasb, BatchStep gvsb, int64_t gvsr) {
   if (blockIdx.y == 0)
     vector_band_out_body<T, NK>(GO, V, GA, B, M, w, oblk, orows, gosb, gosr, vsb, vsr, gasb);
   else
@@ -359,7 +361,7 @@ hipError_t launch_vector(const Problem &p, const View &a, const View &y, const V
 #define WM_VEC(NK)                                                                                              \
   case NK:                                                                                                      \
     hipLaunchKernelGGL((vector_band_in_kernel<T, NK, TRANSPOSED>), grid, block, lds, p.stream, (const E *)a.data, \
-                       (const E *)y.data, (E *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, vrows, a.sb, y.sb, y.sr, \
+                       (const E *)y.data, (E *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, vrows, a.sb.step, y.sb, y.sr, \
                        c.sb, c.sr);                                                                                   \
     break;
   switch (pieces / 2) {
@@ -383,7 +385,7 @@ hipError_t launch_vector_out(const Problem &p, const View &x, const View &y, con
   case NK:                                                                                                      \
     hipLaunchKernelGGL((vector_band_out_kernel<T, NK>), grid, block, lds, p.stream, (const E *)x.data,          \
                        (const E *)y.data, (E *)c.data, (int)p.B, (int)p.M, (int)p.w, nblk, vrows, x.sb, x.sr,   \
-                       y.sb, y.sr, c.sb);                                                                       \
+                       y.sb, y.sr, c.sb.step);                                                                       \
     break;
   switch (pieces / 2) {
     WM_VOUT(1) WM_VOUT(2) WM_VOUT(3) WM_VOUT(4) WM_VOUT(5) WM_VOUT(6) WM_VOUT(7) WM_VOUT(8)
@@ -440,7 +442,7 @@ bool try_launch_vector_window_backward(const Problem &p, const View &ga, const V
     hipLaunchKernelGGL((vector_window_backward_kernel<T, NK>), grid, block, lds, p.stream,                       \
                        (const typename Elem<T>::type *)ga.data, (const typename Elem<T>::type *)k.data,          \
                        (const typename Elem<T>::type *)q.data, (typename Elem<T>::type *)gq.data,                \
-                       (typename Elem<T>::type *)gk.data, (int)p.B, (int)p.M, (int)p.w, nblk, vrows, ga.sb, k.sb, \
+                       (typename Elem<T>::type *)gk.data, (int)p.B, (int)p.M, (int)p.w, nblk, vrows, ga.sb.step, k.sb, \
                        k.sr, q.sb, q.sr, gq.sb, gq.sr, gk.sb, gk.sr);                                             \
     break;
 #define WM_VWB_ALL(T)                                                                                  \
@@ -481,7 +483,7 @@ bool try_launch_vector_unwindow_backward(const Problem &p, const View &a, const 
                        (const typename Elem<T>::type *)a.data, (const typename Elem<T>::type *)v.data,           \
                        (const typename Elem<T>::type *)go.data, (typename Elem<T>::type *)ga.data,               \
                        (typename Elem<T>::type *)gv.data, (int)p.B, (int)p.M, (int)p.w, oblk, orows, iblk, irows, \
-                       a.sb, v.sb, v.sr, go.sb, go.sr, ga.sb, gv.sb, gv.sr);                                      \
+                       a.sb.step, v.sb, v.sr, go.sb, go.sr, ga.sb.step, gv.sb, gv.sr);                                      \
     break;
 #define WM_VUB_ALL(T)                                                                                  \
   switch (pieces / 2) {                                                                                \

@@ -40,7 +40,7 @@ def _chain_is_faster(window_size: int, width: int, elements: int) -> bool:
 
 
 class WindowAttentionFunc(torch.autograd.Function):
-    """Fused kernels on 3-D ``(B, M, N)`` operands; ``k`` holds key rows (not transposed)."""
+    """Fused kernels on ``(..., M, N)`` operands; ``k`` holds key rows (not transposed)."""
 
     @staticmethod
     def forward(ctx, q, k, v, window_size: int, scale: float, mask_out_of_range: bool):
@@ -77,13 +77,11 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
         # chain (reference tests/test_attention.py:75-87); kept differentiable through torch ops
         score = (query * key).sum(-1, keepdim=True) * scale
         return torch.softmax(score, -1) * value
-    q, k, v = (t.reshape(-1, t.shape[-2], t.shape[-1]) for t in (query, key, value))
     # With a very narrow band the recomputing backward of the fused kernels costs more than the
     # band it avoids writing, so training there goes through the separate ops.
-    training = torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v))
-    if _native.window_attention_supported(q, window_size, scale) and not (training and _chain_is_faster(window_size, q.shape[-1], q.numel())):
-        out = WindowAttentionFunc.apply(q, k, v, window_size, scale, bool(mask_out_of_range))
-    else:
-        att = window_matmul(q, k.transpose(-1, -2), window_size)
-        out = unwindow_matmul(band_softmax(att, scale, mask_out_of_range), v, window_size)
-    return out.reshape(query.shape)
+    training = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
+    if _native.window_attention_supported(query, window_size, scale) and not (
+            training and _chain_is_faster(window_size, query.shape[-1], query.numel())):
+        return WindowAttentionFunc.apply(query, key, value, window_size, scale, bool(mask_out_of_range))
+    att = window_matmul(query, key.transpose(-1, -2), window_size)
+    return unwindow_matmul(band_softmax(att, scale, mask_out_of_range), value, window_size)

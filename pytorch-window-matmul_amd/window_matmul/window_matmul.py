@@ -24,10 +24,12 @@ _amp_backward = torch.amp.custom_bwd(device_type="cuda")
 
 
 class WindowMatmulFunc(torch.autograd.Function):
-    """``A[b, i, j] = sum_h inp[b, i, h] * other[b, h, i + j - w]`` on 3-D operands.
+    """``A[b, i, j] = sum_h inp[b, i, h] * other[b, h, i + j - w]``.
 
-    ``inp`` is ``(B, M, N)``, ``other`` is ``(B, N, M)`` (the keys, transposed),
-    the result is ``(B, M, 2w+1)``.  reference window_matmul.py:7-27.
+    ``inp`` is ``(..., M, N)``, ``other`` is ``(..., N, M)`` (the keys, transposed), the result is
+    ``(..., M, 2w+1)`` with the leading dimensions of ``inp``.  Leading dimensions with at most two levels
+    of strides (a projection seen as ``(batch, heads, M, N)``) are read in place, and gradients are laid out
+    like the operand they belong to.  reference window_matmul.py:7-27.
     """
 
     @staticmethod
@@ -50,10 +52,10 @@ class WindowMatmulFunc(torch.autograd.Function):
 
 
 class UnwindowMatmulFunc(torch.autograd.Function):
-    """``O[b, i, h] = sum_j inp[b, i, j] * other[b, i + j - w, h]`` on 3-D operands.
+    """``O[b, i, h] = sum_j inp[b, i, j] * other[b, i + j - w, h]``.
 
-    ``inp`` is the band ``(B, M, 2w+1)``, ``other`` is ``(B, M, N)``, the result is
-    ``(B, M, N)``.  reference window_matmul.py:43-63.
+    ``inp`` is the band ``(..., M, 2w+1)``, ``other`` is ``(..., M, N)``, the result has the shape of
+    ``other``; leading dimensions as in :class:`WindowMatmulFunc`.  reference window_matmul.py:43-63.
     """
 
     @staticmethod
@@ -78,31 +80,27 @@ def window_matmul(inp: torch.Tensor, other: torch.Tensor, window_size: Optional[
 
     A falsy ``window_size`` keeps only the diagonal and is computed with plain
     torch ops, giving ``(..., M, 1)`` (reference window_matmul.py:33-34).  Any
-    number of leading dimensions is flattened into one batch dimension for the
-    kernel and restored afterwards (reference window_matmul.py:35-40).
+    number of leading dimensions counts as one batch dimension
+    (reference window_matmul.py:35-40 flattens them; here the kernels read them where they are).
     """
     if not window_size:
         return (inp * other.transpose(-1, -2)).sum(dim=-1, keepdim=True)
-    lead = inp.shape[:-2]
     seq_len, hidden_dim = inp.shape[-2:]
-    band = WindowMatmulFunc.apply(
-        inp.reshape(-1, seq_len, hidden_dim), other.reshape(-1, hidden_dim, seq_len), window_size
-    )
-    return band.reshape(*lead, seq_len, 2 * window_size + 1)
+    if other.shape[-2:] != (hidden_dim, seq_len):  # reshaped to the keys' shape like the reference does
+        other = other.reshape(-1, hidden_dim, seq_len)
+    return WindowMatmulFunc.apply(inp, other, window_size)
 
 
 def unwindow_matmul(inp: torch.Tensor, other: torch.Tensor, window_size: Optional[int]) -> torch.Tensor:
     """Band times values: ``(..., M, 2w+1) x (..., M, N) -> (..., M, N)``.
 
     A falsy ``window_size`` is the elementwise product ``inp * other``
-    (reference window_matmul.py:69-70); leading dimensions are flattened and
-    restored as in :func:`window_matmul` (reference window_matmul.py:71-76).
+    (reference window_matmul.py:69-70); leading dimensions as in
+    :func:`window_matmul` (reference window_matmul.py:71-76).
     """
     if not window_size:
         return inp * other
-    lead = other.shape[:-2]
-    seq_len, hidden_dim = other.shape[-2:]
-    out = UnwindowMatmulFunc.apply(
-        inp.reshape(-1, seq_len, 2 * window_size + 1), other.reshape(-1, seq_len, hidden_dim), window_size
-    )
-    return out.reshape(*lead, seq_len, hidden_dim)
+    band_shape = (other.shape[-2], 2 * window_size + 1)
+    if inp.shape[-2:] != band_shape:
+        inp = inp.reshape(-1, *band_shape)
+    return UnwindowMatmulFunc.apply(inp, other, window_size)

@@ -32,6 +32,12 @@ class Operand(ctypes.Structure):
     ]
 
 
+class GroupedOperand(ctypes.Structure):
+    """Operand whose batch may have two levels: groups of `heads` elements, stride_g apart (heads = 0: plain)."""
+
+    _fields_ = [("op", Operand), ("heads", ctypes.c_int64), ("stride_g", ctypes.c_int64)]
+
+
 def declared_symbols():
     text = open(HEADER).read()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
@@ -66,6 +72,15 @@ def lib():
                                                   ctypes.c_int, u32, vp]
         L.wm_window_attention_backward.argtypes = [P, P, P, P, vp, P, P, P, P, vp, i64, i64, i64, i64, ctypes.c_double,
                                                    ctypes.c_int, u32, vp]
+        G = ctypes.POINTER(GroupedOperand)
+        L.wm_grouped_window_matmul_forward.argtypes = [G, G, P] + tail
+        L.wm_grouped_window_matmul_backward.argtypes = [G, G, P, G, G] + tail
+        L.wm_grouped_unwindow_matmul_forward.argtypes = [P, G, G] + tail
+        L.wm_grouped_unwindow_matmul_backward.argtypes = [P, G, G, P, G] + tail
+        L.wm_grouped_window_attention_forward.argtypes = [G, G, G, G, vp, i64, i64, i64, i64, ctypes.c_double, ctypes.c_int,
+                                                          ctypes.c_int, u32, vp]
+        L.wm_grouped_window_attention_backward.argtypes = [G, G, G, G, vp, G, G, G, G, vp, i64, i64, i64, i64,
+                                                           ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_window_attention_backward_static.argtypes = [P, P, P, P, vp, P, P, P, P, i64, i64, i64, i64,
                                                           ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_window_attention_supported.argtypes = [i64, i64, i64, ctypes.c_int, ctypes.c_double]
