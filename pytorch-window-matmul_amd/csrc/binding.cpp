@@ -20,6 +20,10 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
 #include <tuple>
 
 #include "../../include/window_matmul_hip.h"
@@ -175,9 +179,6 @@ bool sliced_width(const torch::Tensor &t, int64_t w) {
   return t.size(-1) > kMaxWidth && !tiles_preferred(t, w) && (t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat);
 }
 
-wm_operand operand(const torch::Tensor &t) {
-  return wm_operand{t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)};
-}
 // A contiguous band (..., M, W) as an operand.
 wm_operand band_operand(const torch::Tensor &t) {
   return wm_operand{t.data_ptr(), t.size(-2) * t.size(-1), t.size(-1), 1};
@@ -399,13 +400,13 @@ std::tuple<c10::optional<torch::Tensor>, c10::optional<torch::Tensor>> unwindow_
 // (reference tests/test_attention.py:60-61); not part of the reference's native module.
 torch::Tensor band_softmax_forward(torch::Tensor src, double scale, bool mask_out_of_range) {
   check_gpu(src, "A");
-  TORCH_CHECK(src.dim() == 3 && src.size(2) % 2 == 1, "Input mismatch");
+  TORCH_CHECK(src.dim() >= 2 && src.size(-1) % 2 == 1, "Input mismatch");
   const int dtype = abi_dtype(src, "band_softmax_forward");
   at::hip::HIPGuardMasqueradingAsCUDA guard(src.device());
   auto a = band_friendly(src);
   auto out = torch::empty_like(a);
-  wm_operand oa = operand(a), oo = operand(out);
-  raise_on_error(wm_band_softmax_forward(&oa, &oo, a.size(0), a.size(1), a.size(2) / 2, scale, mask_out_of_range,
+  const wm_operand oa = band_operand(a), oo = band_operand(out);
+  raise_on_error(wm_band_softmax_forward(&oa, &oo, batch_of(a), a.size(-2), a.size(-1) / 2, scale, mask_out_of_range,
                                          dtype, 0, current_stream(src)),
                  "band_softmax_forward");
   return out;
@@ -415,7 +416,7 @@ torch::Tensor band_softmax_backward(torch::Tensor probs, torch::Tensor grad_outp
                                     bool mask_out_of_range) {
   check_gpu(probs, "P");
   check_gpu(grad_output, "grad_P");
-  TORCH_CHECK(probs.dim() == 3 && probs.size(2) % 2 == 1, "Input mismatch");
+  TORCH_CHECK(probs.dim() >= 2 && probs.size(-1) % 2 == 1, "Input mismatch");
   TORCH_CHECK(grad_output.sizes() == probs.sizes() && grad_output.scalar_type() == probs.scalar_type() &&
                   grad_output.device() == probs.device(),
               "Input mismatch");
@@ -424,8 +425,8 @@ torch::Tensor band_softmax_backward(torch::Tensor probs, torch::Tensor grad_outp
   auto p = band_friendly(probs);
   auto g = band_friendly(grad_output);
   auto out = torch::empty_like(p);
-  wm_operand op = operand(p), og = operand(g), oo = operand(out);
-  raise_on_error(wm_band_softmax_backward(&op, &og, &oo, p.size(0), p.size(1), p.size(2) / 2, scale,
+  const wm_operand op = band_operand(p), og = band_operand(g), oo = band_operand(out);
+  raise_on_error(wm_band_softmax_backward(&op, &og, &oo, batch_of(p), p.size(-2), p.size(-1) / 2, scale,
                                           mask_out_of_range, dtype, 0, current_stream(probs)),
                  "band_softmax_backward");
   return out;
@@ -503,6 +504,161 @@ window_attention_backward(torch::Tensor q, torch::Tensor k, torch::Tensor v, tor
   return std::make_tuple(gq, gk, gv);
 }
 
+// Differentiable forms of the functions above.  The public functions of the package call these: an autograd node in
+// Python costs 20-30 us of host time per call and direction, which a small problem cannot hide (a training
+// step of the fused attention at B 7, M 3001 keeps the GPU busy for 33 us).  The nodes carry the names of the Python
+// classes they stand in for.
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+struct SavingNode : torch::autograd::Node {
+  std::vector<SavedVariable> saved;
+  void save(const torch::Tensor &t, bool is_output = false) { saved.emplace_back(t, is_output); }
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (auto &s : saved) s.reset_data();
+  }
+  std::vector<torch::Tensor> unpack() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    std::vector<torch::Tensor> t;
+    for (auto &s : saved) t.push_back(s.unpack(shared_from_this()));
+    return t;
+  }
+  // The gradients of the inputs, for a defined gradient of the output.
+  virtual variable_list gradients(const std::vector<torch::Tensor> &saved_tensors, const torch::Tensor &grad) = 0;
+  variable_list apply(variable_list &&grads) override {
+    if (!grads[0].defined()) return variable_list(num_outputs());
+    at::NoGradGuard no_grad;  // no second derivative
+    return gradients(unpack(), grads[0]);
+  }
+};
+
+bool records(std::initializer_list<const torch::Tensor *> inputs) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const auto *t : inputs)
+    if (t->requires_grad()) return true;
+  return false;
+}
+
+template <typename N>
+std::shared_ptr<N> make_node(const variable_list &inputs) {
+  std::shared_ptr<N> node(new N(), torch::autograd::deleteNode);
+  torch::autograd::edge_list edges;
+  for (const auto &t : inputs) edges.push_back(torch::autograd::impl::gradient_edge(t));
+  node->set_next_edges(std::move(edges));
+  return node;
+}
+
+torch::Tensor or_none(const c10::optional<torch::Tensor> &t) { return t ? *t : torch::Tensor(); }
+
+struct WindowMatmulFuncBackward : SavingNode {
+  int64_t window_size = 0;
+  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
+    auto g = window_matmul_backward(t[0], t[1], window_size, grad, task_should_compute_output(0), task_should_compute_output(1));
+    return {or_none(std::get<0>(g)), or_none(std::get<1>(g))};
+  }
+};
+
+torch::Tensor window_matmul(const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
+  const bool record = records({&src, &other});
+  torch::Tensor out;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    out = window_matmul_forward(src, other, window_size);
+  }
+  if (record) {
+    auto node = make_node<WindowMatmulFuncBackward>({src, other});
+    node->window_size = window_size;
+    node->save(src), node->save(other);
+    torch::autograd::set_history(out, node);
+  }
+  return out;
+}
+
+struct UnwindowMatmulFuncBackward : SavingNode {
+  int64_t window_size = 0;
+  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
+    auto g = unwindow_matmul_backward(t[0], t[1], window_size, grad, task_should_compute_output(0), task_should_compute_output(1));
+    return {or_none(std::get<0>(g)), or_none(std::get<1>(g))};
+  }
+};
+
+torch::Tensor unwindow_matmul(const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
+  const bool record = records({&src, &other});
+  torch::Tensor out;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    out = unwindow_matmul_forward(src, other, window_size);
+  }
+  if (record) {
+    auto node = make_node<UnwindowMatmulFuncBackward>({src, other});
+    node->window_size = window_size;
+    node->save(src), node->save(other);
+    torch::autograd::set_history(out, node);
+  }
+  return out;
+}
+
+struct BandSoftmaxFuncBackward : SavingNode {
+  double scale = 1.0;
+  bool mask_out_of_range = false;
+  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
+    return {band_softmax_backward(t[0], grad, scale, mask_out_of_range)};
+  }
+};
+
+torch::Tensor band_softmax(const torch::Tensor &src, double scale, bool mask_out_of_range) {
+  const bool record = records({&src});
+  torch::Tensor out;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    out = band_softmax_forward(src, scale, mask_out_of_range);
+  }
+  if (record) {
+    auto node = make_node<BandSoftmaxFuncBackward>({src});
+    node->scale = scale, node->mask_out_of_range = mask_out_of_range;
+    torch::autograd::set_history(out, node);
+    node->save(out, true);
+  }
+  return out;
+}
+
+struct WindowAttentionFuncBackward : SavingNode {
+  int64_t window_size = 0;
+  double scale = 1.0;
+  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
+    auto g = window_attention_backward(t[0], t[1], t[2], t[3], t[4], grad, window_size, scale, task_should_compute_output(0),
+                                       task_should_compute_output(1), task_should_compute_output(2));
+    return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), or_none(std::get<2>(g))};
+  }
+};
+
+torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v, int64_t window_size,
+                               double scale, bool mask_out_of_range) {
+  const bool record = records({&q, &k, &v});
+  torch::Tensor out, lse;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    std::tie(out, lse) = window_attention_forward(q, k, v, window_size, scale, mask_out_of_range);
+  }
+  if (record) {
+    auto node = make_node<WindowAttentionFuncBackward>({q, k, v});
+    node->window_size = window_size, node->scale = scale;
+    torch::autograd::set_history(out, node);
+    node->save(q), node->save(k), node->save(v), node->save(out, true), node->save(lse);
+  }
+  return out;
+}
+
+// What Python shows as the grad_fn of a result: an object of a class with the node's name.
+template <typename N>
+void name_node(const char *name) {
+  using namespace torch::autograd;
+  static PyTypeObject type;
+  TORCH_CHECK(_initFunctionPyTypeObject(type, name, nullptr, nullptr) != nullptr, "no Python type for ", name);
+  registerCppFunction(typeid(N), &type);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -534,5 +690,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("lse"), py::arg("grad_output"),
         py::arg("window_size"), py::arg("scale"), py::arg("need_q") = true, py::arg("need_k") = true,
         py::arg("need_v") = true);
+  name_node<WindowMatmulFuncBackward>("WindowMatmulFuncBackward");
+  name_node<UnwindowMatmulFuncBackward>("UnwindowMatmulFuncBackward");
+  name_node<BandSoftmaxFuncBackward>("BandSoftmaxFuncBackward");
+  name_node<WindowAttentionFuncBackward>("WindowAttentionFuncBackward");
+  m.def("window_matmul", &window_matmul, "WindowMatmul, differentiable", py::arg("src"), py::arg("other"), py::arg("window_size"));
+  m.def("unwindow_matmul", &unwindow_matmul, "UnwindowMatmul, differentiable", py::arg("src"), py::arg("other"),
+        py::arg("window_size"));
+  m.def("band_softmax", &band_softmax, "softmax over the band dimension, differentiable", py::arg("src"), py::arg("scale"),
+        py::arg("mask_out_of_range"));
+  m.def("window_attention", &window_attention, "fused window attention, differentiable", py::arg("q"), py::arg("k"),
+        py::arg("v"), py::arg("window_size"), py::arg("scale"), py::arg("mask_out_of_range"));
   m.def("abi_version", []() { return wm_abi_version(); }, "ABI version of libwindow_matmul_hip.so");
 }

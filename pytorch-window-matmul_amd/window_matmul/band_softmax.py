@@ -43,6 +43,4 @@ def band_softmax(inp: torch.Tensor, scale: Optional[float] = None, mask_out_of_r
     """
     if inp.dim() < 2 or inp.shape[-1] % 2 != 1:
         raise RuntimeError("Input mismatch")
-    scale = 1.0 if scale is None else float(scale)
-    flat = inp.reshape(-1, inp.shape[-2], inp.shape[-1])
-    return BandSoftmaxFunc.apply(flat, scale, bool(mask_out_of_range)).reshape(inp.shape)
+    return _native.band_softmax(inp, 1.0 if scale is None else float(scale), bool(mask_out_of_range))

@@ -82,6 +82,6 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
     training = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
     if _native.window_attention_supported(query, window_size, scale) and not (
             training and _chain_is_faster(window_size, query.shape[-1], query.numel())):
-        return WindowAttentionFunc.apply(query, key, value, window_size, scale, bool(mask_out_of_range))
+        return _native.window_attention(query, key, value, window_size, scale, bool(mask_out_of_range))
     att = window_matmul(query, key.transpose(-1, -2), window_size)
     return unwindow_matmul(band_softmax(att, scale, mask_out_of_range), value, window_size)
