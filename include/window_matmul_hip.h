@@ -64,6 +64,8 @@ typedef enum wm_status {
 #define WM_FLAG_NO_LDS_DIRECT 0x8u   /* never use the kernels that load chunks straight into LDS (fused attention; band-out product at N = 128) */
 #define WM_FLAG_NO_SPLIT_F32 0x10u   /* float32: never use the kernels that run on the bf16 matrix instruction through an exact three-way split */
 
+#define WM_FLAG_ANY_HEAD_WIDTH 0x20u /* fused attention: also head widths N = 8 ... 128 that are no multiple of 16, rows of any alignment */
+
 /* Rank-3 operand: element (b, r, c) lives at data + b*stride_b + r*stride_r + c*stride_c. */
 typedef struct wm_operand {
   void *data;
@@ -163,7 +165,8 @@ const char *wm_band_softmax_kernel_choice(int64_t w, int dtype, int contiguous, 
  * the probabilities as rounded to the storage type, the values that multiply v.
  * Returns WM_ERR_UNSUPPORTED, having launched nothing, unless dtype is float16 / bfloat16,
  * N is a multiple of 16 up to 128, w >= 1, scale > 0 and all four operands have unit column
- * stride and 16-byte aligned rows (see wm_window_attention_supported). */
+ * stride and 16-byte aligned rows (see wm_window_attention_supported); with WM_FLAG_ANY_HEAD_WIDTH also
+ * for every other N from 8 on, with rows of any alignment (no byte outside the rows is touched). */
 int wm_window_attention_forward(const wm_operand *q, const wm_operand *k, const wm_operand *v,
                                 const wm_operand *o, float *lse, int64_t B, int64_t M, int64_t N,
                                 int64_t w, double scale, int mask_out_of_range, int dtype,

@@ -435,7 +435,8 @@ torch::Tensor band_softmax_backward(torch::Tensor probs, torch::Tensor grad_outp
 // Fused window attention (no counterpart in the reference's native module): forward returns
 // (o, lse); q, k, v are (..., M, N) with k holding key rows.  Raises when the fused kernels do not
 // cover the problem; window_attention_supported() lets the caller choose the separate ops first.
-bool window_attention_supported(torch::Tensor q, int64_t window_size, double scale) {
+// any_width: also head widths from 8 on that are no multiple of 16.
+bool window_attention_supported(torch::Tensor q, int64_t window_size, double scale, bool any_width) {
   if (q.dim() < 2 || !q.device().is_cuda()) return false;
   int dtype;
   switch (q.scalar_type()) {
@@ -443,7 +444,25 @@ bool window_attention_supported(torch::Tensor q, int64_t window_size, double sca
     case at::kBFloat16: dtype = WM_DTYPE_BF16; break;
     default: return false;
   }
-  return wm_window_attention_supported(q.size(-2), q.size(-1), window_size, dtype, scale) != 0;
+  const int64_t N = q.size(-1), unit = any_width && N >= 8 ? (N + 15) / 16 * 16 : N;
+  return wm_window_attention_supported(q.size(-2), unit, window_size, dtype, scale) != 0;
+}
+
+// Operands of the fused attention.  Its kernels for widths that 16 does not divide take rows of any alignment.
+bool ragged_width(const torch::Tensor &t) { return t.size(-1) % 16 != 0; }
+unsigned attention_flags(const torch::Tensor &t) { return ragged_width(t) ? WM_FLAG_ANY_HEAD_WIDTH : 0; }
+bool ragged_rows_in_place(const torch::Tensor &t) {
+  int64_t step, heads, group;
+  return t.stride(-1) == 1 && batch_steps(t, &step, &heads, &group);
+}
+torch::Tensor attention_operand(const torch::Tensor &t, Heads &heads) {
+  if (!ragged_width(t)) return vector_friendly(t, heads);
+  return ragged_rows_in_place(t) && heads.admit(t) ? t : t.contiguous();
+}
+torch::Tensor attention_gradient(const torch::Tensor &t, Heads &heads) {
+  if (!ragged_width(t)) return empty_like_rows(t, t.size(-1), heads);
+  auto g = torch::empty_like(t);
+  return ragged_rows_in_place(g) && heads.admit(g) ? g : torch::empty(t.sizes(), t.options());
 }
 
 void check_attention_inputs(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v) {
@@ -463,12 +482,12 @@ std::tuple<torch::Tensor, torch::Tensor> window_attention_forward(torch::Tensor 
   at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
   const int64_t B = batch_of(q), M = q.size(-2), N = q.size(-1);
   Heads heads;
-  auto qq = vector_friendly(q, heads), kk = vector_friendly(k, heads), vv = vector_friendly(v, heads);
+  auto qq = attention_operand(q, heads), kk = attention_operand(k, heads), vv = attention_operand(v, heads);
   auto o = torch::empty(q.sizes(), q.options());
   auto lse = torch::empty({B, M}, q.options().dtype(at::kFloat));
   const wm_grouped_operand oq = grouped(qq), ok = grouped(kk), ov = grouped(vv), oo = grouped(o);
   raise_on_error(wm_grouped_window_attention_forward(&oq, &ok, &ov, &oo, lse.data_ptr<float>(), B, M, N, window_size, scale,
-                                                     mask_out_of_range, dtype, 0, current_stream(q)),
+                                                     mask_out_of_range, dtype, attention_flags(q), current_stream(q)),
                  "window_attention_forward");
   return std::make_tuple(o, lse);
 }
@@ -487,19 +506,19 @@ window_attention_backward(torch::Tensor q, torch::Tensor k, torch::Tensor v, tor
   const int dtype = abi_dtype(q, "window_attention_backward");
   at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
   Heads heads;
-  auto qq = vector_friendly(q, heads), kk = vector_friendly(k, heads), vv = vector_friendly(v, heads),
-       oo = vector_friendly(o, heads), go = vector_friendly(grad_output, heads);
+  auto qq = attention_operand(q, heads), kk = attention_operand(k, heads), vv = attention_operand(v, heads),
+       oo = attention_operand(o, heads), go = attention_operand(grad_output, heads);
   c10::optional<torch::Tensor> gq, gk, gv;
   wm_grouped_operand f{}, g{}, h{};
-  if (need_q) gq = empty_like_rows(q, N, heads), f = grouped(*gq);
-  if (need_k) gk = empty_like_rows(k, N, heads), g = grouped(*gk);
-  if (need_v) gv = empty_like_rows(v, N, heads), h = grouped(*gv);
+  if (need_q) gq = attention_gradient(q, heads), f = grouped(*gq);
+  if (need_k) gk = attention_gradient(k, heads), g = grouped(*gk);
+  if (need_v) gv = attention_gradient(v, heads), h = grouped(*gv);
   auto delta = torch::empty({2, B, M}, lse.options());  // row sums and log2-scaled log-sum-exp
   const wm_grouped_operand a = grouped(qq), b = grouped(kk), c = grouped(vv), d = grouped(oo), e = grouped(go);
   raise_on_error(wm_grouped_window_attention_backward(&a, &b, &c, &d, lse.data_ptr<float>(), &e, need_q ? &f : nullptr,
                                                       need_k ? &g : nullptr, need_v ? &h : nullptr,
-                                                      delta.data_ptr<float>(), B, M, N, window_size, scale, dtype, 0,
-                                                      current_stream(q)),
+                                                      delta.data_ptr<float>(), B, M, N, window_size, scale, dtype,
+                                                      attention_flags(q), current_stream(q)),
                  "window_attention_backward");
   return std::make_tuple(gq, gk, gv);
 }
@@ -682,7 +701,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("band_softmax_backward", &band_softmax_backward, "backward of band_softmax_forward", py::arg("probs"),
         py::arg("grad_output"), py::arg("scale") = 1.0, py::arg("mask_out_of_range") = false);
   m.def("window_attention_supported", &window_attention_supported, "whether the fused attention kernels cover q",
-        py::arg("q"), py::arg("window_size"), py::arg("scale"));
+        py::arg("q"), py::arg("window_size"), py::arg("scale"), py::arg("any_width") = false);
   m.def("window_attention_forward", &window_attention_forward, "fused window attention forward -> (o, lse)",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("window_size"), py::arg("scale"),
         py::arg("mask_out_of_range") = false);

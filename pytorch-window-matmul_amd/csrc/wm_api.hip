@@ -193,7 +193,7 @@ int unwindow_backward(const wm_operand *a, const Op *v, const Op *grad_o, const 
 template <typename Op>
 int attention_forward(const Op *q, const Op *k, const Op *v, const Op *o, float *lse, int64_t B, int64_t M, int64_t N,
                       int64_t w, double scale, int mask_out_of_range, int dtype, unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (int st = check_common(B, M, N, w, dtype, flags & ~WM_FLAG_ANY_HEAD_WIDTH)) return st;
   if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
   if (B == 0 || M == 0) return WM_OK;
   if (missing(q) || missing(k) || missing(v) || missing(o)) return WM_ERR_NULL_POINTER;
@@ -209,7 +209,7 @@ template <typename Op>
 int attention_backward(const Op *q, const Op *k, const Op *v, const Op *o, const float *lse, const Op *grad_o,
                        const Op *grad_q, const Op *grad_k, const Op *grad_v, float *delta, int64_t B, int64_t M,
                        int64_t N, int64_t w, double scale, int dtype, unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (int st = check_common(B, M, N, w, dtype, flags & ~WM_FLAG_ANY_HEAD_WIDTH)) return st;
   if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
   if (B == 0 || M == 0) return WM_OK;
   if (missing(q) || missing(k) || missing(v) || missing(o) || missing(grad_o) || lse == nullptr || delta == nullptr)

@@ -22,13 +22,21 @@
 //                             ds_read_b64_tr_b16.
 // Blocks that lie entirely outside a wavefront's band are skipped, blocks entirely inside it run
 // without any masking arithmetic.
+//
+// Head widths: N = 16 ... 128 in steps of 16 in this translation unit, with RAGGED_WIDTH set (wm_attention_ragged.hip)
+// any other N = 8 ... 127, see HeadWidth.
 #include "wm_mfma_common.hpp"
 
 #include <type_traits>
 
+#ifndef RAGGED_WIDTH
+#define RAGGED_WIDTH 0
+#endif
+
 namespace wm {
 namespace {
 
+constexpr bool RAG = RAGGED_WIDTH != 0;
 constexpr int AT_TM = 128;  // queries per workgroup
 constexpr int AT_KC = 64;   // keys per chunk
 constexpr float kRaiseStep = 8.0f;
@@ -62,9 +70,9 @@ __device__ __forceinline__ float across_halves_sum(float v) {
 }
 
 template <typename T, int NK, bool MASK>  // N = 16 NK
-__global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_kernel(
+__global__ __launch_bounds__(kThreads, NK <= 4 ? (RAG ? 3 : 4) : 2) void attention_forward_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, BatchStep qsb, int64_t qsr,
+    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, int n, float c, BatchStep qsb, int64_t qsr,
     BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;  // NB blocks of 32 output columns; the last may be half used
   constexpr int KS = N + 8;         // key rows 16 (mod 128) bytes apart in banks: conflict-free b128 reads
@@ -74,6 +82,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
   __shared__ __attribute__((aligned(16))) uint16_t k_lds[2][AT_KC * KS];
   __shared__ __attribute__((aligned(16))) uint16_t v_lds[2][AT_KC * VS];
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, ksb.heads);
@@ -85,11 +94,12 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
   const uint16_t *Vb = V + vsb.at(bp);
 
   // B operand of the first product: the wavefront's 32 queries, all of N, in registers
+  const u32x4 tail = width.tail(half);
   u32x4 qf[NK];
   {
-    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) qf[ks] = load_row_chunk(qr + 16 * ks, Q, qi < M);
+    for (int ks = 0; ks < NK; ++ks) qf[ks] = width.load_operand(qr, Q, qi < M, ks, half, tail);
   }
 
   const int kc_lo = max(i0 - w, 0) / AT_KC;
@@ -112,8 +122,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
 #pragma unroll
     for (int u = 0; u < SLOTS; ++u) {
       const int key = min(base + l_row[u], M - 1);
-      kreg[u] = *reinterpret_cast<const u32x4 *>(Kb + (int64_t)key * ksr + l_col[u]);
-      vreg[u] = *reinterpret_cast<const u32x4 *>(Vb + (int64_t)key * vsr + l_col[u]);
+      kreg[u] = width.load16(Kb + (int64_t)key * ksr + width.column(l_col[u] / 8));
+      vreg[u] = width.load16(Vb + (int64_t)key * vsr + width.column(l_col[u] / 8));
     }
   };
   auto stash = [&](int buf) {
@@ -140,7 +150,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
     for (int v = 0; v < 16; ++v) s[v] = 0.0f;
     const uint16_t *krow = &k_lds[buf][(32 * kb + (lane & 31)) * KS + 8 * half];
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) s = Mma<T>::run(*reinterpret_cast<const u32x4 *>(krow + 16 * ks), qf[ks], s);
+    for (int ks = 0; ks < NK; ++ks) s = Mma<T>::run(width.tile_operand(*reinterpret_cast<const u32x4 *>(krow + 16 * ks), ks, tail), qf[ks], s);
     // accumulator v of this lane: key c0 + 8 (v / 4) + 4 half + v % 4, query qi
     if (EDGE) {
       // key offset ofs = 8 (v / 4) + v % 4 of this lane is inside the band and the sequence iff
@@ -225,7 +235,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
   if (L != nullptr && half == 0 && qi < M) L[(int64_t)b * M + qi] = (m_used + __builtin_amdgcn_logf(l)) * kLn2F;
   // every wave is past the last barrier: the value buffers are free and stage the result rows
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * AT_KC * VS, "the four staging areas must fit the value buffers");
-  store_wave_rows<T, NB>(&v_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + osb.at(bp), osr, qw0, M, N, lane);
+  store_wave_rows<T, NB, RAG>(&v_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + osb.at(bp), osr, qw0, M, width.cols(), lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -240,7 +250,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_k
 template <typename T, int NK, int NKB, bool MASK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_narrow_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, BatchStep qsb, int64_t qsr,
+    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, int n, float c, BatchStep qsb, int64_t qsr,
     BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
   constexpr int PADW = 16 * (NKB - 1);         // keys staged before the first and after the last query
@@ -252,6 +262,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_n
   __shared__ __attribute__((aligned(16))) uint16_t tile[ROWS * VS];
   static_assert(KS <= VS, "the key tile must fit the region of the value tile");
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, qsb.heads);
@@ -262,22 +273,23 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_n
 
   // every load of the workgroup is issued before the first use: queries in operand layout, key and
   // value rows as coalesced 16-byte pieces (rows outside the sequence read a safe address, zeroed later)
+  const u32x4 tail = width.tail(half);
   u32x4 qf[NK], kreg[SLOTS], vreg[SLOTS];
   {
-    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) qf[ks] = fetch_row_chunk(qr + 16 * ks, Q, qi < M);
+    for (int ks = 0; ks < NK; ++ks) qf[ks] = width.fetch_piece(qr, Q, qi < M, 2 * ks + half);
     const uint16_t *Kb = K + ksb.at(bp), *Vb = V + vsb.at(bp);
 #pragma unroll
     for (int u = 0; u < SLOTS; ++u) {
       const int p = min(tid + kThreads * u, PIECES - 1);
-      const int key = i0 - PADW + p / (N / 8), col = (p % (N / 8)) * 8;
+      const int key = i0 - PADW + p / (N / 8), piece = p % (N / 8);
       const bool ok = (key >= 0) & (key < M);
-      kreg[u] = fetch_row_chunk(Kb + (int64_t)key * ksr + col, K, ok);
-      vreg[u] = fetch_row_chunk(Vb + (int64_t)key * vsr + col, V, ok);
+      kreg[u] = width.fetch_piece(Kb + (int64_t)key * ksr, K, ok, piece);
+      vreg[u] = width.fetch_piece(Vb + (int64_t)key * vsr, V, ok, piece);
     }
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) qf[ks] = mask_row_chunk(qf[ks], qi < M);
+    for (int ks = 0; ks < NK; ++ks) qf[ks] = width.mask_operand(qf[ks], qi < M, ks, tail);
 #pragma unroll
     for (int u = 0; u < SLOTS; ++u) {
       const int p = min(tid + kThreads * u, PIECES - 1);
@@ -297,7 +309,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_n
     for (int v = 0; v < 16; ++v) s[j][v] = 0.0f;
     const uint16_t *krow = &tile[(32 * wave + 32 * j + (lane & 31)) * KS + 8 * half];
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) s[j] = Mma<T>::run(*reinterpret_cast<const u32x4 *>(krow + 16 * ks), qf[ks], s[j]);
+    for (int ks = 0; ks < NK; ++ks)
+      s[j] = Mma<T>::run(width.tile_operand(*reinterpret_cast<const u32x4 *>(krow + 16 * ks), ks, tail), qf[ks], s[j]);
     // valid key offsets of this lane in tile j: first..last (band and sequence), as in the wide kernel
     const int k0 = kw0 + 32 * j + 4 * half;  // key at offset 0
     const int first = max(qi - w, 0) - k0, last = min(qi + w, M - 1) - k0;
@@ -368,9 +381,13 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_n
   constexpr int PER_ROW = N / 8;
   for (int p = lane; p < 32 * PER_ROW; p += 64) {
     const int r = p / PER_ROW, hg = p - r * PER_ROW;
-    if (qw0 + r < M)
-      store_chunk_streaming(O + osb.at(bp) + (int64_t)(qw0 + r) * osr + 8 * hg,
-                            *reinterpret_cast<const u32x4 *>(stage + r * SO + 8 * hg));
+    if (qw0 + r >= M || hg >= width.pieces()) continue;
+    uint16_t *to = O + osb.at(bp) + (int64_t)(qw0 + r) * osr + width.column(hg);
+    const u32x4 piece = *reinterpret_cast<const u32x4 *>(stage + r * SO + 8 * hg);
+    if (RAG)
+      store_chunk<false>(to, piece);
+    else
+      store_chunk_streaming(to, piece);
   }
 }
 
@@ -393,11 +410,11 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_n
 template <typename T, int NK, bool MASK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_dma_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
-    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, float c, BatchStep qsb, int64_t qsr,
+    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, int n, float c, BatchStep qsb, int64_t qsr,
     BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr) {
   // tile rows of 128 bytes (N <= 64) or 256 bytes; the pieces of a row beyond column N are never
   // fetched (requested out of range: zeros, no memory traffic)
-  constexpr int N = 16 * NK, NB = (NK + 1) / 2, ROWB = NK <= 4 ? 128 : 256, PPR = ROWB / 16;
+  constexpr int NB = (NK + 1) / 2, ROWB = NK <= 4 ? 128 : 256, PPR = ROWB / 16;
   constexpr int STAGES = 2, DEPTH = STAGES - 1;
   constexpr int TILE = AT_KC * ROWB / 2;   // elements per tile
   constexpr int LOADS = 2 * (PPR / 4);     // loads per wavefront and chunk (K and V)
@@ -405,6 +422,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   __shared__ __attribute__((aligned(1024))) uint16_t kv_lds[2 * STAGES][TILE];  // key tiles, then value tiles
   uint16_t (*const k_lds)[TILE] = kv_lds, (*const v_lds)[TILE] = kv_lds + STAGES;
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, ksb.heads);
@@ -414,11 +432,10 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   const int qw0 = i0 + 32 * wave;     // first query of this wavefront (scalar)
   const int qi = qw0 + (lane & 31);   // this lane's query
 
-  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * N));
-  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * N));
-  const bool piece_in_row = (((64 * wave + lane) % PPR) ^ swz<PPR>((64 * wave + lane) / PPR)) < N / 8;
-  const uint32_t k_voff = piece_in_row ? dma_lane_offset<PPR>(wave, lane, ksr) : 0x80000000u;
-  const uint32_t v_voff = piece_in_row ? dma_lane_offset<PPR>(wave, lane, vsr) : 0x80000000u;
+  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * width.cols()));
+  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * width.cols()));
+  const uint32_t k_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, ksr);
+  const uint32_t v_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, vsr);
   const uint32_t k_step = (uint32_t)(256 / PPR * ksr * 2), v_step = (uint32_t)(256 / PPR * vsr * 2);
   const uint32_t k_chunk = (uint32_t)(AT_KC * ksr * 2), v_chunk = (uint32_t)(AT_KC * vsr * 2);
   auto request = [&](int kc, int stage) {
@@ -432,11 +449,12 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   for (int d = 0; d < DEPTH; ++d) request(kc_lo + d, d);
 
   // B operand of the first product: the wavefront's 32 queries, all of N, in registers
+  const u32x4 tail = width.tail(half);
   u32x4 qf[NK];
   {
-    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) qf[ks] = load_row_chunk(qr + 16 * ks, Q, qi < M);
+    for (int ks = 0; ks < NK; ++ks) qf[ks] = width.load_operand(qr, Q, qi < M, ks, half, tail);
   }
 
   // LDS byte offsets inside a tile.  Key rows as A operand: row lane % 32 of a block, pieces
@@ -477,7 +495,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
     for (int v = 0; v < 16; ++v) s[v] = 0.0f;
     u32x4 ka[NK];
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) ka[ks] = key_operand(kt, kb, ks);
+    for (int ks = 0; ks < NK; ++ks) ka[ks] = width.tile_operand(key_operand(kt, kb, ks), ks, tail);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) s = Mma<T>::run(ka[ks], qf[ks], s);
@@ -603,7 +621,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * STAGES * TILE, "the four staging areas must fit the tiles");
-  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + osb.at(bp), osr, qw0, M, N, lane);
+  store_wave_rows<T, NB, RAG>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + osb.at(bp), osr, qw0, M, width.cols(), lane);
 }
 
 template <typename T, int NK>
@@ -615,7 +633,7 @@ hipError_t launch_forward(const Problem &p, const View &q, const View &k, const 
   const float c = (float)(scale * 1.4426950408889634);
 #define WM_AT(KERNEL)                                                                                              \
   hipLaunchKernelGGL(KERNEL, grid, block, 0, p.stream, (const uint16_t *)q.data, (const uint16_t *)k.data,         \
-                     (const uint16_t *)v.data, (uint16_t *)o.data, lse, (int)p.B, (int)p.M, (int)p.w, nblk, c,     \
+                     (const uint16_t *)v.data, (uint16_t *)o.data, lse, (int)p.B, (int)p.M, (int)p.w, nblk, (int)p.N, c, \
                      q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr)
   // narrow windows take the one-pass kernel (two key tiles per wavefront up to w = 16, three up to 32)
   if (p.w <= 16 && !(p.flags & WM_FLAG_NO_NARROW_BAND)) {
@@ -631,7 +649,9 @@ hipError_t launch_forward(const Problem &p, const View &q, const View &k, const 
   } else {
     // the buffer loads of the LDS-direct kernel address a batch element with 32-bit byte offsets
     const int64_t lim = 0x7fffffff;
-    const bool fits = (p.M + 3 * AT_KC) * k.sr * 2 < lim && (p.M + 3 * AT_KC) * v.sr * 2 < lim && k.sr > 0 && v.sr > 0;
+    // and fetch pieces at dword addresses
+    const bool fits = (p.M + 3 * AT_KC) * k.sr * 2 < lim && (p.M + 3 * AT_KC) * v.sr * 2 < lim && k.sr > 0 && v.sr > 0 &&
+                      (!RAG || (dword_rows(k) && dword_rows(v)));
     if (fits && !(p.flags & WM_FLAG_NO_LDS_DIRECT)) {
       if (mask)
         WM_AT((attention_forward_dma_kernel<T, NK, true>));
@@ -650,7 +670,7 @@ hipError_t launch_forward(const Problem &p, const View &q, const View &k, const 
 template <typename T>
 hipError_t forward_by_width(const Problem &p, const View &q, const View &k, const View &v, const View &o, float *lse,
                             double scale, int mask) {
-  switch (p.N / 16) {
+  switch ((p.N + 15) / 16) {
     case 1: return launch_forward<T, 1>(p, q, k, v, o, lse, scale, mask);
     case 2: return launch_forward<T, 2>(p, q, k, v, o, lse, scale, mask);
     case 3: return launch_forward<T, 3>(p, q, k, v, o, lse, scale, mask);
@@ -664,6 +684,14 @@ hipError_t forward_by_width(const Problem &p, const View &q, const View &k, cons
 
 }  // namespace
 
+#if RAGGED_WIDTH
+bool try_launch_attention_forward_ragged(const Problem &p, const View &q, const View &k, const View &v, const View &o,
+                                         float *lse, double scale, int mask, hipError_t *err) {
+  if (!(p.flags & WM_FLAG_ANY_HEAD_WIDTH) || p.N < 8 || !attention_supports(p.M, (p.N + 15) / 16 * 16, p.w, p.dtype, scale))
+    return false;
+  for (const View *t : {&q, &k, &v, &o})
+    if (t->sc != 1 || (uintptr_t)t->data % 2 != 0) return false;
+#else
 bool attention_supports(int64_t M, int64_t N, int64_t w, int dtype, double scale) {
   if (dtype != WM_DTYPE_BF16 && dtype != WM_DTYPE_F16) return false;
   if (N % 16 != 0 || N < 16 || N > 128) return false;
@@ -675,9 +703,11 @@ bool attention_supports(int64_t M, int64_t N, int64_t w, int dtype, double scale
 bool try_launch_attention_forward(const Problem &p, const View &q, const View &k, const View &v, const View &o,
                                   float *lse, double scale, int mask, hipError_t *err) {
   if (p.flags & WM_FLAG_FORCE_STRIDED) return false;
+  if (p.N % 16 != 0) return try_launch_attention_forward_ragged(p, q, k, v, o, lse, scale, mask, err);
   if (!attention_supports(p.M, p.N, p.w, p.dtype, scale)) return false;
   if (!fast_layout(q, p.dtype) || !fast_layout(k, p.dtype) || !fast_layout(v, p.dtype) || !fast_layout(o, p.dtype))
     return false;
+#endif
   *err = p.dtype == WM_DTYPE_BF16 ? forward_by_width<bf16_t>(p, q, k, v, o, lse, scale, mask)
                                   : forward_by_width<f16_t>(p, q, k, v, o, lse, scale, mask);
   return true;

@@ -19,15 +19,21 @@
 // tiles are read from LDS both by rows (first products) and transposed (second products).
 // Narrow windows of heads up to 64 wide take a third kernel that does the work of both at once
 // (attention_backward_narrow_kernel below).
+// Head widths as in wm_attention.hip.
 #include "wm_mfma_common.hpp"
 
 #include <type_traits>
+
+#ifndef RAGGED_WIDTH
+#define RAGGED_WIDTH 0
+#endif
 
 namespace wm {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+constexpr bool RAG = RAGGED_WIDTH != 0;
 constexpr int AB_TM = 128;  // stationary rows per workgroup (32 per wavefront)
 constexpr int AB_KC = 64;   // streamed rows per chunk
 
@@ -76,10 +82,10 @@ __device__ __forceinline__ u32x4 pack8(const float *x) {
 // query kernel: dQ and D
 // ---------------------------------------------------------------------------------------------
 template <typename T, int NK, bool WITH_DQ>  // N = 16 NK; WITH_DQ false: only D is wanted (grad_q not requested)
-__global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_query_kernel(
+__global__ __launch_bounds__(kThreads, NK <= 4 ? (RAG ? 2 : 3) : 1) void attention_backward_query_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L,
-    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, float scale, BatchStep qsb,
+    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, int n, float scale, BatchStep qsb,
     int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr,
     BatchStep dqsb, int64_t dqsr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
@@ -89,6 +95,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_
   __shared__ __attribute__((aligned(16))) uint16_t k_lds[2][AB_KC * TS];
   __shared__ __attribute__((aligned(16))) uint16_t v_lds[2][AB_KC * TS];
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, ksb.heads);
@@ -101,18 +108,19 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_
   const uint16_t *Vb = V + vsb.at(bp);
   const float c = scale * 1.4426950408889634f;
 
+  const u32x4 tail = width.tail(half);
   // stationary side in registers: the query rows and their upstream gradient rows (B operands)
   u32x4 qf[NK], gf[NK];
   float delta = 0.0f;
   {
-    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
-    const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr + 8 * half;
-    const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
+    const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      qf[ks] = load_row_chunk(qr + 16 * ks, Q, q_ok);
-      gf[ks] = load_row_chunk(gr + 16 * ks, dO, q_ok);
-      delta += dot8<T>(gf[ks], load_row_chunk(orow + 16 * ks, O, q_ok));
+      qf[ks] = width.load_operand(qr, Q, q_ok, ks, half, tail);
+      gf[ks] = width.load_operand(gr, dO, q_ok, ks, half, tail);
+      delta += dot8<T>(gf[ks], width.load_operand(orow, O, q_ok, ks, half, tail));
     }
   }
   delta = halves_sum(delta);
@@ -138,8 +146,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_
 #pragma unroll
     for (int u = 0; u < SLOTS; ++u) {
       const int key = min(base + l_row[u], M - 1);
-      kreg[u] = *reinterpret_cast<const u32x4 *>(Kb + (int64_t)key * ksr + l_col[u]);
-      vreg[u] = *reinterpret_cast<const u32x4 *>(Vb + (int64_t)key * vsr + l_col[u]);
+      kreg[u] = width.load16(Kb + (int64_t)key * ksr + width.column(l_col[u] / 8));
+      vreg[u] = width.load16(Vb + (int64_t)key * vsr + width.column(l_col[u] / 8));
     }
   };
   auto stash = [&](int buf) {
@@ -165,8 +173,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_
     const int at = (32 * kb + (lane & 31)) * TS + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      s = Mma<T>::run(*reinterpret_cast<const u32x4 *>(&k_lds[buf][at + 16 * ks]), qf[ks], s);
-      dp = Mma<T>::run(*reinterpret_cast<const u32x4 *>(&v_lds[buf][at + 16 * ks]), gf[ks], dp);
+      s = Mma<T>::run(width.tile_operand(*reinterpret_cast<const u32x4 *>(&k_lds[buf][at + 16 * ks]), ks, tail), qf[ks], s);
+      dp = Mma<T>::run(width.tile_operand(*reinterpret_cast<const u32x4 *>(&v_lds[buf][at + 16 * ks]), ks, tail), gf[ks], dp);
     }
     // accumulator v of this lane: key c0 + 8 (v / 4) + 4 half + v % 4, query qi
     if (EDGE) {
@@ -216,7 +224,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 1) void attention_backward_
   }
   // every wave is past the last barrier: the key buffers are free and stage the result rows
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * AB_KC * TS, "the four staging areas must fit the key buffers");
-  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, 1.0f, dQ + dqsb.at(bp), dqsr, qw0, M, N,
+  store_wave_rows<T, NB, RAG>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, 1.0f, dQ + dqsb.at(bp), dqsr, qw0, M, width.cols(),
                          lane);
 }
 
@@ -227,7 +235,7 @@ template <typename T, int NK>  // N = 16 NK
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_key_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ dO, const float *__restrict__ L, const float *__restrict__ D,
-    uint16_t *__restrict__ dK, uint16_t *__restrict__ dV, int B, int M, int w, int nblk, float scale, BatchStep qsb,
+    uint16_t *__restrict__ dK, uint16_t *__restrict__ dV, int B, int M, int w, int nblk, int n, float scale, BatchStep qsb,
     int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep gsb, int64_t gsr, BatchStep dksb,
     int64_t dksr, BatchStep dvsb, int64_t dvsr) {
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
@@ -239,6 +247,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   __shared__ __attribute__((aligned(16))) float l_lds[2][AB_KC];  // L * log2(e) of the chunk's queries
   __shared__ __attribute__((aligned(16))) float d_lds[2][AB_KC];  // D * scale
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, qsb.heads);
@@ -253,14 +262,15 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   const float *Db = D + (int64_t)b * M;
   const float c = scale * 1.4426950408889634f;
 
+  const u32x4 tail = width.tail(half);
   u32x4 kf[NK], vf[NK];
   {
-    const uint16_t *kr = K + ksb.at(bp) + (int64_t)kj * ksr + 8 * half;
-    const uint16_t *vr = V + vsb.at(bp) + (int64_t)kj * vsr + 8 * half;
+    const uint16_t *kr = K + ksb.at(bp) + (int64_t)kj * ksr;
+    const uint16_t *vr = V + vsb.at(bp) + (int64_t)kj * vsr;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      kf[ks] = load_row_chunk(kr + 16 * ks, K, k_ok);
-      vf[ks] = load_row_chunk(vr + 16 * ks, V, k_ok);
+      kf[ks] = width.load_operand(kr, K, k_ok, ks, half, tail);
+      vf[ks] = width.load_operand(vr, V, k_ok, ks, half, tail);
     }
   }
 
@@ -281,8 +291,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
 #pragma unroll
     for (int u = 0; u < SLOTS; ++u) {
       const int r = min(base + l_row[u], M - 1);
-      qreg[u] = *reinterpret_cast<const u32x4 *>(Qb + (int64_t)r * qsr + l_col[u]);
-      greg[u] = *reinterpret_cast<const u32x4 *>(Gb + (int64_t)r * gsr + l_col[u]);
+      qreg[u] = width.load16(Qb + (int64_t)r * qsr + width.column(l_col[u] / 8));
+      greg[u] = width.load16(Gb + (int64_t)r * gsr + width.column(l_col[u] / 8));
     }
     const int r = min(base + (tid & 63), M - 1);
     stat = (tid < 64 ? Lb : Db)[r];
@@ -312,8 +322,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
     const int at = (32 * qb + (lane & 31)) * TS + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      s = Mma<T>::run(*reinterpret_cast<const u32x4 *>(&q_lds[buf][at + 16 * ks]), kf[ks], s);
-      dp = Mma<T>::run(*reinterpret_cast<const u32x4 *>(&g_lds[buf][at + 16 * ks]), vf[ks], dp);
+      s = Mma<T>::run(width.tile_operand(*reinterpret_cast<const u32x4 *>(&q_lds[buf][at + 16 * ks]), ks, tail), kf[ks], s);
+      dp = Mma<T>::run(width.tile_operand(*reinterpret_cast<const u32x4 *>(&g_lds[buf][at + 16 * ks]), ks, tail), vf[ks], dp);
     }
     // accumulator v of this lane: query r0 + 8 (v / 4) + 4 half + v % 4, key kj
     if (EDGE) {
@@ -373,8 +383,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   // either output may be absent (gradient not requested)
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * AB_KC * TS, "the four staging areas must fit the query buffers");
   uint16_t *stage = &q_lds[0][0] + wave * RowStage<NB>::ELEMS;
-  if (dK != nullptr) store_wave_rows<T, NB>(stage, dk, 1.0f, dK + dksb.at(bp), dksr, kw0, M, N, lane);
-  if (dV != nullptr) store_wave_rows<T, NB>(stage, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, N, lane);
+  if (dK != nullptr) store_wave_rows<T, NB, RAG>(stage, dk, 1.0f, dK + dksb.at(bp), dksr, kw0, M, width.cols(), lane);
+  if (dV != nullptr) store_wave_rows<T, NB, RAG>(stage, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, width.cols(), lane);
 }
 
 
@@ -395,11 +405,6 @@ template <int NK>
 struct BwdTile {
   // tile rows of 128 bytes (N <= 64) or 256 bytes; pieces of a row beyond column N are never fetched
   static constexpr int N = 16 * NK, NB = (NK + 1) / 2, ROWB = NK <= 4 ? 128 : 256, PPR = ROWB / 16, TILE = AB_KC * ROWB / 2;
-  // byte offset of the lane's piece for the loads of a chunk (dma_chunk), out of range for pieces beyond N
-  static __device__ __forceinline__ uint32_t load_offset(int wave, int lane, int64_t row_stride) {
-    const int slot = 64 * wave + lane;
-    return ((slot % PPR) ^ swz<PPR>(slot / PPR)) < N / 8 ? dma_lane_offset<PPR>(wave, lane, row_stride) : 0x80000000u;
-  }
   static constexpr int STAGES = NK <= 4 ? 3 : 2, DEPTH = STAGES - 1;
   typedef s16x4 __attribute__((address_space(3))) * lds_tr_ptr;
   // byte offsets inside a tile for the two ways a tile is read (see attention_forward_dma_kernel)
@@ -431,19 +436,21 @@ struct BwdTile {
 template <typename T, int NK>
 __global__ __launch_bounds__(kThreads) void attention_backward_stats_kernel(
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L, float *__restrict__ D,
-    int B, int M, int nblk, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr) {
+    int B, int M, int nblk, int n, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr) {
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, gsb.heads);
   const int lane = threadIdx.x & 63, half = lane >> 5;
   const int qi = blk * AB_TM + 32 * (threadIdx.x >> 6) + (lane & 31);
   const bool q_ok = qi < M;
-  const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr + 8 * half;
-  const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr + 8 * half;
+  const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr;
+  const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr;
+  const u32x4 tail = width.tail(half);
   float delta = 0.0f;
 #pragma unroll
   for (int ks = 0; ks < NK; ++ks)
-    delta += dot8<T>(load_row_chunk(gr + 16 * ks, dO, q_ok), load_row_chunk(orow + 16 * ks, O, q_ok));
+    delta += dot8<T>(width.load_operand(gr, dO, q_ok, ks, half, tail), width.load_operand(orow, O, q_ok, ks, half, tail));
   delta = halves_sum(delta);
   if (q_ok && half == 0) {
     D[(int64_t)b * M + qi] = -delta;
@@ -458,7 +465,7 @@ template <typename T, int NK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_query_dma_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L,
-    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, float scale, BatchStep qsb,
+    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, int n, float scale, BatchStep qsb,
     int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr,
     BatchStep dqsb, int64_t dqsr) {
   typedef BwdTile<NK> TL;
@@ -468,6 +475,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
   __shared__ __attribute__((aligned(1024))) uint16_t kv_lds[2 * STAGES][TILE];  // key tiles, then value tiles
   uint16_t (*const k_lds)[TILE] = kv_lds, (*const v_lds)[TILE] = kv_lds + STAGES;
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, ksb.heads);
@@ -479,9 +487,9 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
   const bool q_ok = qi < M;
   const float c = scale * kLog2e;
 
-  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * N));
-  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * N));
-  const uint32_t k_voff = TL::load_offset(wave, lane, ksr), v_voff = TL::load_offset(wave, lane, vsr);
+  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * width.cols()));
+  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * width.cols()));
+  const uint32_t k_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, ksr), v_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, vsr);
   const uint32_t k_step = (uint32_t)(256 / PPR * ksr * 2), v_step = (uint32_t)(256 / PPR * vsr * 2);
   const uint32_t k_chunk = (uint32_t)(AB_KC * ksr * 2), v_chunk = (uint32_t)(AB_KC * vsr * 2);
   auto request = [&](int kc, int stage) {
@@ -493,18 +501,19 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) request(kc_lo + d, d);
 
+  const u32x4 tail = width.tail(half);
   // stationary side in registers: the query rows and their upstream gradient rows (B operands)
   u32x4 qf[NK], gf[NK];
   float delta = 0.0f;
   {
-    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr + 8 * half;
-    const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr + 8 * half;
-    const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr + 8 * half;
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
+    const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      qf[ks] = load_row_chunk(qr + 16 * ks, Q, q_ok);
-      gf[ks] = load_row_chunk(gr + 16 * ks, dO, q_ok);
-      delta += dot8<T>(gf[ks], load_row_chunk(orow + 16 * ks, O, q_ok));
+      qf[ks] = width.load_operand(qr, Q, q_ok, ks, half, tail);
+      gf[ks] = width.load_operand(gr, dO, q_ok, ks, half, tail);
+      delta += dot8<T>(gf[ks], width.load_operand(orow, O, q_ok, ks, half, tail));
     }
   }
   delta = halves_sum(delta);
@@ -530,7 +539,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
     for (int v = 0; v < 16; ++v) s[v] = 0.0f, dp[v] = 0.0f;
     u32x4 ka[NK], va[NK];
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) ka[ks] = TL::rows(kt, row_at, kb, ks), va[ks] = TL::rows(vt, row_at, kb, ks);
+    for (int ks = 0; ks < NK; ++ks) ka[ks] = width.tile_operand(TL::rows(kt, row_at, kb, ks), ks, tail), va[ks] = width.tile_operand(TL::rows(vt, row_at, kb, ks), ks, tail);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
@@ -602,7 +611,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
   wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
   static_assert(4 * RowStage<NB>::ELEMS <= 2 * STAGES * TILE, "the four staging areas must fit the tiles");
-  store_wave_rows<T, NB>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, scale, dQ + dqsb.at(bp), dqsr, qw0, M, N,
+  store_wave_rows<T, NB, RAG>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, dq, scale, dQ + dqsb.at(bp), dqsr, qw0, M, width.cols(),
                          lane);
 }
 
@@ -610,7 +619,7 @@ template <typename T, int NK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_key_dma_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ dO, const float *__restrict__ D, uint16_t *__restrict__ dK,
-    uint16_t *__restrict__ dV, int B, int M, int w, int nblk, float scale, BatchStep qsb, int64_t qsr, BatchStep ksb,
+    uint16_t *__restrict__ dV, int B, int M, int w, int nblk, int n, float scale, BatchStep qsb, int64_t qsr, BatchStep ksb,
     int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep gsb, int64_t gsr, BatchStep dksb, int64_t dksr, BatchStep dvsb,
     int64_t dvsr) {
   typedef BwdTile<NK> TL;
@@ -621,6 +630,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   __shared__ __attribute__((aligned(1024))) uint16_t g_lds[STAGES][TILE];
   __shared__ __attribute__((aligned(256))) float stat_lds[STAGES][2][AB_KC];  // [0] -D, [1] log-sum-exp (log2 units)
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, qsb.heads);
@@ -632,12 +642,12 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   const bool k_ok = kj < M;
   const float c = scale * kLog2e;
 
-  const u32x4 q_rsrc = make_rsrc(Q + qsb.at(bp), (uint32_t)((M - 1) * qsr * 2 + 2 * N));
-  const u32x4 g_rsrc = make_rsrc(dO + gsb.at(bp), (uint32_t)((M - 1) * gsr * 2 + 2 * N));
+  const u32x4 q_rsrc = make_rsrc(Q + qsb.at(bp), (uint32_t)((M - 1) * qsr * 2 + 2 * width.cols()));
+  const u32x4 g_rsrc = make_rsrc(dO + gsb.at(bp), (uint32_t)((M - 1) * gsr * 2 + 2 * width.cols()));
   // waves 0 and 2 fetch D, waves 1 and 3 the log-sum-exp (twice the same 256 bytes each: every
   // wavefront then has the same number of loads in flight, which is what the waits count)
   const u32x4 s_rsrc = make_rsrc(D + ((int64_t)(wave & 1) * B + b) * M, (uint32_t)(M * 4));
-  const uint32_t q_voff = TL::load_offset(wave, lane, qsr), g_voff = TL::load_offset(wave, lane, gsr);
+  const uint32_t q_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, qsr), g_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, gsr);
   const uint32_t q_step = (uint32_t)(256 / PPR * qsr * 2), g_step = (uint32_t)(256 / PPR * gsr * 2);
   const uint32_t q_chunk = (uint32_t)(AB_KC * qsr * 2), g_chunk = (uint32_t)(AB_KC * gsr * 2);
   auto request = [&](int qc, int stage) {
@@ -650,14 +660,15 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) request(qc_lo + d, d);
 
+  const u32x4 tail = width.tail(half);
   u32x4 kf[NK], vf[NK];
   {
-    const uint16_t *kr = K + ksb.at(bp) + (int64_t)kj * ksr + 8 * half;
-    const uint16_t *vr = V + vsb.at(bp) + (int64_t)kj * vsr + 8 * half;
+    const uint16_t *kr = K + ksb.at(bp) + (int64_t)kj * ksr;
+    const uint16_t *vr = V + vsb.at(bp) + (int64_t)kj * vsr;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      kf[ks] = load_row_chunk(kr + 16 * ks, K, k_ok);
-      vf[ks] = load_row_chunk(vr + 16 * ks, V, k_ok);
+      kf[ks] = width.load_operand(kr, K, k_ok, ks, half, tail);
+      vf[ks] = width.load_operand(vr, V, k_ok, ks, half, tail);
     }
   }
 
@@ -681,7 +692,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
     u32x4 qa[NK], ga[NK];
     f32x4 l2[4];
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) qa[ks] = TL::rows(qt, row_at, qb, ks), ga[ks] = TL::rows(gt, row_at, qb, ks);
+    for (int ks = 0; ks < NK; ++ks) qa[ks] = width.tile_operand(TL::rows(qt, row_at, qb, ks), ks, tail), ga[ks] = width.tile_operand(TL::rows(gt, row_at, qb, ks), ks, tail);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       // the dP accumulator starts from -D of its sixteen queries: dP - D comes out of the matrix pipe
@@ -769,8 +780,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   __builtin_amdgcn_s_barrier();
   static_assert(4 * RowStage<NB>::ELEMS <= STAGES * TILE, "the four staging areas must fit the query tiles");
   uint16_t *stage_rows = &q_lds[0][0] + wave * RowStage<NB>::ELEMS;
-  if (dK != nullptr) store_wave_rows<T, NB>(stage_rows, dk, scale, dK + dksb.at(bp), dksr, kw0, M, N, lane);
-  if (dV != nullptr) store_wave_rows<T, NB>(stage_rows, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, N, lane);
+  if (dK != nullptr) store_wave_rows<T, NB, RAG>(stage_rows, dk, scale, dK + dksb.at(bp), dksr, kw0, M, width.cols(), lane);
+  if (dV != nullptr) store_wave_rows<T, NB, RAG>(stage_rows, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, width.cols(), lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -789,11 +800,11 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
 // Memory sees q, k, v, dO, O once each (plus the halo, which the neighbouring workgroup has
 // usually just brought into the L2) and dQ, dK, dV once: nothing else bounds this kernel.
 template <typename T, int NK, int NKB>
-__global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3) void attention_backward_narrow_kernel(
+__global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) || (RAG && NK == 4) ? 2 : 3) void attention_backward_narrow_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
     const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L,
     uint16_t *__restrict__ dQ, uint16_t *__restrict__ dK, uint16_t *__restrict__ dV, int B, int M, int w, int nblk,
-    float scale, BatchStep qsb, int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr,
+    int n, float scale, BatchStep qsb, int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr,
     BatchStep gsb, int64_t gsr, BatchStep dqsb, int64_t dqsr, BatchStep dksb, int64_t dksr, BatchStep dvsb, int64_t dvsr) {
   static_assert(NK <= 4, "rows of 128 bytes: two tiles and the staging must fit 64 KB of LDS");
   constexpr int N = 16 * NK, NB = (NK + 1) / 2;
@@ -814,6 +825,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
       DYN ? reinterpret_cast<float *>(narrow_dynamic_lds + 4 * TL::ELEMS) : stat_declared);
   static_assert(4 * RowStage<NB>::ELEMS <= TL::ELEMS, "the four staging areas must fit one tile");
 
+  const HeadWidth<RAG, NK> width{n};
   int b, blk;
   if (!decode_block(nblk, B, &b, &blk)) return;
   const BatchPos bp = batch_pos(b, qsb.heads);
@@ -831,13 +843,13 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   // column N are requested out of range (zeros, no traffic)
   const int piece = TL::load_piece(wave, lane);
   auto request = [&](const uint16_t *base, int64_t sr, const uint16_t *tile) __attribute__((always_inline)) {
-    const u32x4 rsrc = make_rsrc(base, (uint32_t)((M - 1) * sr * 2 + 2 * N));
+    const u32x4 rsrc = make_rsrc(base, (uint32_t)((M - 1) * sr * 2 + 2 * width.cols()));
     const uint32_t lds = lds_address(tile) + 1024 * wave;
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
       const int row = t0 + TL::load_row(wave, lane, j);
-      const bool wanted = row >= need_lo && row <= need_hi && piece < N / 8;
-      dma_piece(rsrc, lds + 4096 * j, wanted ? (uint32_t)(row * sr * 2 + piece * 16) : 0x80000000u, 0);
+      const bool wanted = row >= need_lo && row <= need_hi && piece < width.pieces();
+      dma_piece(rsrc, lds + 4096 * j, wanted ? (uint32_t)(row * sr * 2 + width.column(piece) * 2) : 0x80000000u, 0);
     }
   };
   request(Q + qsb.at(bp), qsr, tile_a);
@@ -864,33 +876,34 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   const int halo_rows = min(32, PADW - 32 * hp);
   const int h32 = r32 < halo_rows ? r32 : 0;                         // lanes beyond the halo repeat its first row
   const uint32_t halo_at = TL::row_at(32 * half + h32);
+  const u32x4 tail = width.tail(half);
   u32x4 o_own[NK], o_halo[NK];
   float l_own, l_halo = 0.0f;
   {
     const int row = t0 + own_first + r32;
     const bool ok = row >= need_lo && row <= need_hi;
-    const uint16_t *orow = O + osb.at(bp) + (int64_t)row * osr + 8 * half;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)row * osr;
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) o_own[ks] = load_row_chunk(orow + 16 * ks, O, ok);
+    for (int ks = 0; ks < NK; ++ks) o_own[ks] = width.load_operand(orow, O, ok, ks, half, tail);
     l_own = ok ? L[(int64_t)b * M + row] * kLog2e : 0.0f;
   }
   if (halo_wave) {
     const int row = t0 + halo_first + h32;
     const bool ok = row >= need_lo && row <= need_hi;
-    const uint16_t *orow = O + osb.at(bp) + (int64_t)row * osr + 8 * half;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)row * osr;
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) o_halo[ks] = load_row_chunk(orow + 16 * ks, O, ok);
+    for (int ks = 0; ks < NK; ++ks) o_halo[ks] = width.load_operand(orow, O, ok, ks, half, tail);
     l_halo = ok ? L[(int64_t)b * M + row] * kLog2e : 0.0f;
   }
   // own rows as keys: B operands of the first two products
   u32x4 kf[NK], vf[NK];
   if (want_kv) {
-    const uint16_t *kr = K + ksb.at(bp) + (int64_t)ri * ksr + 8 * half;
-    const uint16_t *vr = V + vsb.at(bp) + (int64_t)ri * vsr + 8 * half;
+    const uint16_t *kr = K + ksb.at(bp) + (int64_t)ri * ksr;
+    const uint16_t *vr = V + vsb.at(bp) + (int64_t)ri * vsr;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      kf[ks] = load_row_chunk(kr + 16 * ks, K, r_ok);
-      vf[ks] = load_row_chunk(vr + 16 * ks, V, r_ok);
+      kf[ks] = width.load_operand(kr, K, r_ok, ks, half, tail);
+      vf[ks] = width.load_operand(vr, V, r_ok, ks, half, tail);
     }
   }
   wait_vmcnt<0>();
@@ -899,14 +912,14 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   {
     float d = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) d += dot8<T>(own_rows(tile_b, own_first, row_at, ks), o_own[ks]);
+    for (int ks = 0; ks < NK; ++ks) d += dot8<T>(width.tile_operand(own_rows(tile_b, own_first, row_at, ks), ks, tail), o_own[ks]);
     d = halves_sum(d);
     if (half == 0) stat[0][own_first + r32] = d, stat[1][own_first + r32] = l_own;
   }
   if (halo_wave) {
     float d = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) d += dot8<T>(own_rows(tile_b, halo_first, halo_at, ks), o_halo[ks]);
+    for (int ks = 0; ks < NK; ++ks) d += dot8<T>(width.tile_operand(own_rows(tile_b, halo_first, halo_at, ks), ks, tail), o_halo[ks]);
     d = halves_sum(d);
     if (half == 0 && r32 < halo_rows) stat[0][halo_first + r32] = d, stat[1][halo_first + r32] = l_halo;
   }
@@ -928,7 +941,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
       for (int v = 0; v < 16; ++v) s[v] = 0.0f, dp[v] = 0.0f;
       u32x4 qa[NK], ga[NK];
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) qa[ks] = TL::rows(tile_a, row_at, rb, ks), ga[ks] = TL::rows(tile_b, row_at, rb, ks);
+      for (int ks = 0; ks < NK; ++ks) qa[ks] = width.tile_operand(TL::rows(tile_a, row_at, rb, ks), ks, tail), ga[ks] = width.tile_operand(TL::rows(tile_b, row_at, rb, ks), ks, tail);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < NK; ++ks) {
@@ -981,15 +994,18 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
   float delta = 0.0f, lse2 = 0.0f;
   if (dQ != nullptr) {
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) qf[ks] = own_rows(tile_a, own_first, row_at, ks), gf[ks] = own_rows(tile_b, own_first, row_at, ks);
+    for (int ks = 0; ks < NK; ++ks) {
+      qf[ks] = width.tile_operand(own_rows(tile_a, own_first, row_at, ks), ks, tail);
+      gf[ks] = width.tile_operand(own_rows(tile_b, own_first, row_at, ks), ks, tail);
+    }
     delta = stat[0][own_first + r32], lse2 = stat[1][own_first + r32];
   }
   __syncthreads();  // nobody reads the tiles any more
   // K replaces Q while dK and dV leave through the other tile; V follows when those rows are out
   if (dQ != nullptr) request(K + ksb.at(bp), ksr, tile_a);
   uint16_t *stage_rows = tile_b + wave * RowStage<NB>::ELEMS;
-  if (dK != nullptr) store_wave_rows<T, NB>(stage_rows, dk, scale, dK + dksb.at(bp), dksr, rw0, M, N, lane);
-  if (dV != nullptr) store_wave_rows<T, NB>(stage_rows, dv, 1.0f, dV + dvsb.at(bp), dvsr, rw0, M, N, lane);
+  if (dK != nullptr) store_wave_rows<T, NB, RAG>(stage_rows, dk, scale, dK + dksb.at(bp), dksr, rw0, M, width.cols(), lane);
+  if (dV != nullptr) store_wave_rows<T, NB, RAG>(stage_rows, dv, 1.0f, dV + dvsb.at(bp), dvsr, rw0, M, width.cols(), lane);
   if (dQ == nullptr) return;
   __syncthreads();
   request(V + vsb.at(bp), vsr, tile_b);
@@ -1010,7 +1026,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
     for (int v = 0; v < 16; ++v) s[v] = 0.0f, dp[v] = 0.0f;
     u32x4 ka[NK], va[NK];
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) ka[ks] = TL::rows(tile_a, row_at, rb, ks), va[ks] = TL::rows(tile_b, row_at, rb, ks);
+    for (int ks = 0; ks < NK; ++ks) ka[ks] = width.tile_operand(TL::rows(tile_a, row_at, rb, ks), ks, tail), va[ks] = width.tile_operand(TL::rows(tile_b, row_at, rb, ks), ks, tail);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
@@ -1046,7 +1062,7 @@ __global__ __launch_bounds__(kThreads, NKB >= 4 || (NK >= 3 && NKB == 3) ? 2 : 3
     }
   }
   __syncthreads();
-  store_wave_rows<T, NB>(tile_a + wave * RowStage<NB>::ELEMS, dq, scale, dQ + dqsb.at(bp), dqsr, rw0, M, N, lane);
+  store_wave_rows<T, NB, RAG>(tile_a + wave * RowStage<NB>::ELEMS, dq, scale, dQ + dqsb.at(bp), dqsr, rw0, M, width.cols(), lane);
 }
 
 template <typename T, int NK>
@@ -1062,7 +1078,9 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
     // the LDS-direct kernels address a batch element with 32-bit byte offsets
     const int64_t lim = 0x7fffffff;
     bool fits = !(p.flags & WM_FLAG_NO_LDS_DIRECT) && (p.M + 3 * AB_KC) * 4 < lim;
-    for (const View *t : {&q, &k, &v, &go}) fits = fits && t->sr > 0 && (p.M + 3 * AB_KC) * t->sr * 2 < lim;
+    // and fetch pieces at dword addresses
+    for (const View *t : {&q, &k, &v, &go})
+      fits = fits && t->sr > 0 && (p.M + 3 * AB_KC) * t->sr * 2 < lim && (!RAG || dword_rows(*t));
     if constexpr (NK <= 4) {
       // narrow windows: one kernel for all three gradients (two row blocks per wavefront up to w = 16, three up
       // to 32, four up to 48, five up to 64 where it still pays: B96 M16384 N64 w = 64: 490 against 555 us for
@@ -1071,7 +1089,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
 #define WM_ABN(NKB, LDS_BYTES)                                                                                        \
   hipLaunchKernelGGL((attention_backward_narrow_kernel<T, NK, NKB>), grid, block, LDS_BYTES, p.stream, (in_t)q.data,  \
                      (in_t)k.data, (in_t)v.data, (in_t)o.data, (in_t)go.data, lse, (out_t)gq.data, (out_t)gk.data,    \
-                     (out_t)gv.data, (int)p.B, (int)p.M, (int)p.w, nblk, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb,  \
+                     (out_t)gv.data, (int)p.B, (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb,  \
                      v.sr, o.sb, o.sr, go.sb, go.sr, gq.sb, gq.sr, gk.sb, gk.sr, gv.sb, gv.sr)
         if (p.w <= 16) {
           WM_ABN(2, 0);
@@ -1101,16 +1119,16 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
       if (gq.data != nullptr)
         hipLaunchKernelGGL((attention_backward_query_dma_kernel<T, NK>), grid, block, 0, p.stream, (in_t)q.data,
                            (in_t)k.data, (in_t)v.data, (in_t)o.data, (in_t)go.data, lse, (out_t)gq.data, delta, (int)p.B,
-                           (int)p.M, (int)p.w, nblk, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr, go.sb,
+                           (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr, go.sb,
                            go.sr, gq.sb, gq.sr);
       else
         hipLaunchKernelGGL((attention_backward_stats_kernel<T, NK>), grid, block, 0, p.stream, (in_t)o.data,
-                           (in_t)go.data, lse, delta, (int)p.B, (int)p.M, nblk, o.sb, o.sr, go.sb, go.sr);
+                           (in_t)go.data, lse, delta, (int)p.B, (int)p.M, nblk, (int)p.N, o.sb, o.sr, go.sb, go.sr);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess || (gk.data == nullptr && gv.data == nullptr)) return err;
       hipLaunchKernelGGL((attention_backward_key_dma_kernel<T, NK>), grid, block, 0, p.stream, (in_t)q.data,
                          (in_t)k.data, (in_t)v.data, (in_t)go.data, (const float *)delta, (out_t)gk.data,
-                         (out_t)gv.data, (int)p.B, (int)p.M, (int)p.w, nblk, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb,
+                         (out_t)gv.data, (int)p.B, (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb,
                          v.sr, go.sb, go.sr, gk.sb, gk.sr, gv.sb, gv.sr);
       return hipGetLastError();
     }
@@ -1118,7 +1136,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
 #define WM_ABQ(WITH_DQ)                                                                                              \
   hipLaunchKernelGGL((attention_backward_query_kernel<T, NK, WITH_DQ>), grid, block, 0, p.stream, (in_t)q.data,      \
                      (in_t)k.data, (in_t)v.data, (in_t)o.data, (in_t)go.data, lse, (out_t)gq.data, delta, (int)p.B,  \
-                     (int)p.M, (int)p.w, nblk, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr, go.sb,  \
+                     (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr, go.sb,  \
                      go.sr, gq.sb, gq.sr)
   // D is needed by the key kernel even when grad_q is not: the query kernel then stops after writing it
   if (gq.data != nullptr)
@@ -1131,7 +1149,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
   if (gk.data == nullptr && gv.data == nullptr) return hipSuccess;
   hipLaunchKernelGGL((attention_backward_key_kernel<T, NK>), grid, block, 0, p.stream, (in_t)q.data, (in_t)k.data,
                      (in_t)v.data, (in_t)go.data, lse, (const float *)delta, (out_t)gk.data, (out_t)gv.data, (int)p.B,
-                     (int)p.M, (int)p.w, nblk, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, go.sb, go.sr, gk.sb,
+                     (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, go.sb, go.sr, gk.sb,
                      gk.sr, gv.sb, gv.sr);
   return hipGetLastError();
 }
@@ -1140,7 +1158,7 @@ template <typename T>
 hipError_t backward_by_width(const Problem &p, const View &q, const View &k, const View &v, const View &o,
                              const View &go, const float *lse, float *delta, const View &gq, const View &gk,
                              const View &gv, double scale) {
-  switch (p.N / 16) {
+  switch ((p.N + 15) / 16) {
     case 1: return launch_backward<T, 1>(p, q, k, v, o, go, lse, delta, gq, gk, gv, scale);
     case 2: return launch_backward<T, 2>(p, q, k, v, o, go, lse, delta, gq, gk, gv, scale);
     case 3: return launch_backward<T, 3>(p, q, k, v, o, go, lse, delta, gq, gk, gv, scale);
@@ -1154,14 +1172,25 @@ hipError_t backward_by_width(const Problem &p, const View &q, const View &k, con
 
 }  // namespace
 
+#if RAGGED_WIDTH
+bool try_launch_attention_backward_ragged(const Problem &p, const View &q, const View &k, const View &v, const View &o,
+                                          const View &go, const float *lse, float *delta, const View &gq,
+                                          const View &gk, const View &gv, double scale, hipError_t *err) {
+  if (!(p.flags & WM_FLAG_ANY_HEAD_WIDTH) || p.N < 8 || !attention_supports(p.M, (p.N + 15) / 16 * 16, p.w, p.dtype, scale))
+    return false;
+  for (const View *t : {&q, &k, &v, &o, &go, &gq, &gk, &gv})
+    if (t->data != nullptr && (t->sc != 1 || (uintptr_t)t->data % 2 != 0)) return false;
+#else
 bool try_launch_attention_backward(const Problem &p, const View &q, const View &k, const View &v, const View &o,
                                    const View &go, const float *lse, float *delta, const View &gq, const View &gk,
                                    const View &gv, double scale, hipError_t *err) {
   if (p.flags & WM_FLAG_FORCE_STRIDED) return false;
+  if (p.N % 16 != 0) return try_launch_attention_backward_ragged(p, q, k, v, o, go, lse, delta, gq, gk, gv, scale, err);
   if (!attention_supports(p.M, p.N, p.w, p.dtype, scale)) return false;
   const View *all[] = {&q, &k, &v, &o, &go, &gq, &gk, &gv};
   for (const View *t : all)
     if (t->data != nullptr && !fast_layout(*t, p.dtype)) return false;  // absent outputs have no layout
+#endif
   *err = p.dtype == WM_DTYPE_BF16 ? backward_by_width<bf16_t>(p, q, k, v, o, go, lse, delta, gq, gk, gv, scale)
                                   : backward_by_width<f16_t>(p, q, k, v, o, go, lse, delta, gq, gk, gv, scale);
   return true;

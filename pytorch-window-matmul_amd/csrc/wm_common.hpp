@@ -153,6 +153,13 @@ bool attention_supports(int64_t M, int64_t N, int64_t w, int dtype, double scale
 bool try_launch_attention_forward(const Problem &p, const View &q, const View &k, const View &v, const View &o,
                                   float *lse, double scale, int mask, hipError_t *err);
 
+// The same pair for head widths that 16 does not divide (N >= 8, WM_FLAG_ANY_HEAD_WIDTH set): rows of any alignment.
+bool try_launch_attention_forward_ragged(const Problem &p, const View &q, const View &k, const View &v, const View &o,
+                                         float *lse, double scale, int mask, hipError_t *err);
+bool try_launch_attention_backward_ragged(const Problem &p, const View &q, const View &k, const View &v, const View &o,
+                                          const View &go, const float *lse, float *delta, const View &gq,
+                                          const View &gk, const View &gv, double scale, hipError_t *err);
+
 // Backward of the fused attention (wm_attention_bwd.hip): two kernels on p.stream; `delta` is a
 // float32 (B,M) workspace the first one fills and the second one reads.
 bool try_launch_attention_backward(const Problem &p, const View &q, const View &k, const View &v, const View &o,
@@ -181,6 +188,11 @@ inline bool fast_layout(const View &v, int dtype) {
   if (v.sc != 1) return false;
   if (((uintptr_t)v.data) % 16 != 0) return false;
   return (v.sr * es) % 16 == 0 && (v.sb.step * es) % 16 == 0 && (v.sb.heads <= 0 || (v.sb.group * es) % 16 == 0);
+}
+
+// 16-bit rows that all start on a multiple of 4 bytes: what loads straight into LDS need.
+inline bool dword_rows(const View &v) {
+  return (uintptr_t)v.data % 4 == 0 && v.sr % 2 == 0 && v.sb.step % 2 == 0 && (v.sb.heads <= 0 || v.sb.group % 2 == 0);
 }
 
 // Band operands are only required to be contiguous per batch (rows of odd

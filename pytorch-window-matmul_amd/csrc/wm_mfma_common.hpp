@@ -91,6 +91,49 @@ __device__ __forceinline__ u32x4 load_row_chunk(const uint16_t *p, const uint16_
   return mask_row_chunk(fetch_row_chunk(p, safe, valid), valid);
 }
 
+// Rows of a head width that the matrix instructions do not divide (N not a multiple of 16, N >= 8), worked on
+// where they lie, without padded copies: a row is ceil(N / 8) pieces of 16 bytes of which the last one is
+// moved back to start at column N - 8.  No piece crosses the end of a row, so nothing outside the tensor is
+// read; the elements that the last piece shares with the one before it (the first 8 pieces() - N) are cleared
+// wherever a product is contracted over the columns, in both operands, and pieces past the last one count as
+// zeros.  Where columns are results the shared ones come out twice, equal bit for bit, and are stored twice.
+// RAG false: N = 16 NK, every helper below folds to the plain piece arithmetic.
+// (A training step at B1x8 M4096 N60 w64 float16 took 207 us through the separate ops on padded copies, 29 launches,
+// and takes 92 us in two kernels; B4x12 M16384 bfloat16: 1015 / 368 us at N = 60, w = 1, 1511 / 578 at N = 41, w = 100,
+// 4481 / 2584 at N = 127, w = 300.)
+template <bool RAG, int NK>
+struct HeadWidth {
+  int n;
+  __device__ __forceinline__ int cols() const { return RAG ? n : 16 * NK; }
+  __device__ __forceinline__ int pieces() const { return RAG ? (n + 7) / 8 : 2 * NK; }
+  __device__ __forceinline__ int column(int piece) const { return RAG ? min(8 * piece, n - 8) : 8 * piece; }
+  // first element of a piece that no earlier piece holds; 8 past the last piece
+  __device__ __forceinline__ int first(int piece) const { return piece < pieces() ? 8 * piece - column(piece) : 8; }
+  // What remains of piece 2 (NK - 1) + half, the only pair that can be shared or absent, in a contraction over columns.
+  __device__ __forceinline__ u32x4 tail(int half) const {
+    const u32x4 ones = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
+    return RAG ? keep_range(ones, first(2 * (NK - 1) + half), 7) : ones;
+  }
+  // 16 bytes of a tensor; rows of such widths have no alignment beyond the element's
+  static __device__ __forceinline__ u32x4 load16(const uint16_t *p) {
+    return RAG ? reinterpret_cast<const Chunk2 *>(p)->v : *reinterpret_cast<const u32x4 *>(p);
+  }
+  __device__ __forceinline__ u32x4 fetch_piece(const uint16_t *row, const uint16_t *safe, bool valid, int piece) const {
+    return load16(valid ? row + column(piece) : safe);
+  }
+  // Pieces 2 ks + half of a row, as operand of a product contracted over the columns; zeros if not valid.
+  __device__ __forceinline__ u32x4 mask_operand(u32x4 v, bool valid, int ks, u32x4 tail) const {
+    v = mask_row_chunk(v, valid);
+    return RAG && ks == NK - 1 ? v & tail : v;
+  }
+  __device__ __forceinline__ u32x4 load_operand(const uint16_t *row, const uint16_t *safe, bool valid, int ks, int half,
+                                                u32x4 tail) const {
+    return mask_operand(fetch_piece(row, safe, valid, 2 * ks + half), valid, ks, tail);
+  }
+  // The same operand read from an LDS tile of whole pieces.
+  static __device__ __forceinline__ u32x4 tile_operand(u32x4 v, int ks, u32x4 tail) { return RAG && ks == NK - 1 ? v & tail : v; }
+};
+
 template <typename T>
 struct Mma;
 template <>
@@ -199,7 +242,8 @@ struct RowStage {
   static constexpr int STRIDE = SW + 8;         // staged rows 16 bytes apart mod 128 (SW = 64)
   static constexpr int ELEMS = 32 * STRIDE;     // per wave
 };
-template <typename T, int NB>
+// RAG: N is no multiple of 16, the last piece of a row is moved back as in HeadWidth.
+template <typename T, int NB, bool RAG = false>
 __device__ __forceinline__ void store_wave_rows(uint16_t *stage, const f32x16 (&acc)[NB], float mul, uint16_t *Cb,
                                                 int64_t csr, int row0, int M, int N, int lane) {
   constexpr int SW = RowStage<NB>::SW, STRIDE = RowStage<NB>::STRIDE;
@@ -221,9 +265,13 @@ __device__ __forceinline__ void store_wave_rows(uint16_t *stage, const f32x16 (&
     for (int s = 0; s < 32 / RPP; ++s) {
       const int rr = lane / CPR + RPP * s, piece = lane % CPR;
       const int row = row0 + rr, h = 32 * n0 + 8 * piece;
-      if (row >= 0 && row < M && h < N)
-        __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(stage + rr * STRIDE + 8 * piece),
-                                    reinterpret_cast<u32x4 *>(Cb + (int64_t)row * csr + h));
+      if (row >= 0 && row < M && h < N) {
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + rr * STRIDE + 8 * piece);
+        if (RAG)
+          store_chunk<false>(Cb + (int64_t)row * csr + min(h, N - 8), v);
+        else
+          __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(Cb + (int64_t)row * csr + h));
+      }
     }
   }
 }
@@ -323,6 +371,14 @@ template <int PPR>
 __device__ __forceinline__ uint32_t dma_lane_offset(int wave, int lane, int64_t row_stride_elems) {
   const int slot = 64 * wave + lane, row = slot / PPR, piece = (slot % PPR) ^ swz<PPR>(row);
   return (uint32_t)(row * row_stride_elems * 2 + piece * 16);
+}
+
+// The same for a tile of rows of a head width below 8 PPR: pieces beyond the row are requested out of range
+// (zeros, no traffic).
+template <int PPR, bool RAG, int NK>
+__device__ __forceinline__ uint32_t dma_lane_offset_in_row(HeadWidth<RAG, NK> width, int wave, int lane, int64_t row_stride_elems) {
+  const int slot = 64 * wave + lane, row = slot / PPR, piece = (slot % PPR) ^ swz<PPR>(row);
+  return piece < width.pieces() ? (uint32_t)(row * row_stride_elems * 2 + width.column(piece) * 2) : 0x80000000u;
 }
 
 // A swizzled tile of ROWS rows x PPR pieces as the loads above fill it, generalised to any row count

@@ -3,7 +3,7 @@
 The reference package stops at the two banded matmuls; its callers write the chain above
 themselves (reference tests/test_attention.py:57-63).  This function is that chain with the
 same semantics, as an addition next to the unchanged two-function API.  For float16 /
-bfloat16 inputs whose last dimension is a multiple of 16 up to 128 it runs fused kernels that
+bfloat16 inputs whose last dimension is 8 to 128 it runs fused kernels that
 never write the ``(…, M, 2w+1)`` band to memory (forward keeps only the log-sum-exp of every
 row, backward recomputes the probabilities); everything else runs the chain of the separate
 ops of this package, on the GPU as well.
@@ -33,8 +33,10 @@ def _chain_is_faster(window_size: int, width: int, elements: int) -> bool:
     0.426 at w = 36) and up to about w = 24 at N = 96 (B96 M4096: 0.251 / 0.294 at w = 16, 0.332 / 0.308 at
     w = 32).  Small problems are bound by the host, which issues seven launches for the chain and three
     for the fused step: at B7 M3001 the chain takes 0.21 ms and the fused step 0.085-0.09 ms whatever the
-    window and head width, so below about 32 M elements per tensor the fused kernels are always taken."""
-    if width <= 64 or elements < _HOST_BOUND_ELEMENTS:
+    window and head width, so below about 32 M elements per tensor the fused kernels are always taken.  Widths that 16 does not
+    divide always are: the separate ops pad every operand there (B4x12 M16384, chain / fused: 1271 / 806 us at N = 75,
+    w = 4; 1979 / 949 at N = 120, w = 4; 1015 / 368 at N = 60, w = 1)."""
+    if width <= 64 or width % 16 or elements < _HOST_BOUND_ELEMENTS:
         return False
     return window_size <= (24 if width <= 96 else 32)
 
@@ -80,7 +82,9 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
     # With a very narrow band the recomputing backward of the fused kernels costs more than the
     # band it avoids writing, so training there goes through the separate ops.
     training = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
-    if _native.window_attention_supported(query, window_size, scale) and not (
+    # Head widths that 16 does not divide: the chain computes in float16 inside an autocast region, so it stays there.
+    any_width = not torch.is_autocast_enabled("cuda")
+    if _native.window_attention_supported(query, window_size, scale, any_width) and not (
             training and _chain_is_faster(window_size, query.shape[-1], query.numel())):
         return _native.window_attention(query, key, value, window_size, scale, bool(mask_out_of_range))
     att = window_matmul(query, key.transpose(-1, -2), window_size)
