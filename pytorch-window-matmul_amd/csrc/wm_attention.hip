@@ -624,6 +624,235 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   store_wave_rows<T, NB, RAG>(&k_lds[0][0] + wave * RowStage<NB>::ELEMS, o, inv, O + osb.at(bp), osr, qw0, M, width.cols(), lane);
 }
 
+// ---------------------------------------------------------------------------------------------
+// Few tiles: the keys of a query shared out among wavefronts
+// ---------------------------------------------------------------------------------------------
+// A launch with fewer tiles of 128 queries than the chip has CUs leaves CUs idle and gives the others one
+// wavefront per SIMD, whose score products, exponentials and value products then follow one another with
+// nothing to fill the waits.  Here a workgroup of eight wavefronts owns 64 queries: wavefront (g, s) has the
+// queries 32 g .. + 31 and of every chunk of 128 keys the block 32 s .. + 31, with a running maximum, row sum
+// and output of its own.  At the end the four shares of a query group exchange their maxima, scale to the common
+// one, and share s adds up and stores output columns 32 s .. + 31.  Chunks, operand layouts and arithmetic
+// are those of attention_forward_dma_kernel.  What bounds it: per chunk and SIMD two wavefronts of 512 matrix, 375
+// vector and 500 LDS cycles each that start together at the chunk's barrier, 1.45 us per chunk at N = 128.
+// B1 M16384 N128 w1024: 46 us before, 27 now; B1 M4096 N128 w256: 17.8 / 12.5.
+constexpr int FS_TM = 64, FS_KC = 128, FS_SHARES = 4, FS_THREADS = 512;
+
+template <int NK>
+struct SplitForward {
+  static constexpr int NB = (NK + 1) / 2, ROWB = NK <= 4 ? 128 : 256, STAGES = 2;
+  static constexpr int TILE = FS_KC * ROWB / 2;                 // elements per tile
+  static constexpr int TILE_BYTES = 2 * STAGES * 2 * TILE;      // key and value tiles
+  static constexpr int OUT_BYTES = 8 * NB * 32 * 32 * 4;        // the shares' outputs, in the same place
+  static constexpr int MAIN = TILE_BYTES > OUT_BYTES ? TILE_BYTES : OUT_BYTES;
+  static constexpr int BYTES = MAIN + 2 * 8 * 32 * 4;           // plus maximum and row sum of every share
+};
+
+template <typename T, int NK, bool MASK>
+__global__ __launch_bounds__(FS_THREADS, 2) void attention_forward_split_kernel(
+    const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
+    uint16_t *__restrict__ O, float *__restrict__ L, int B, int M, int w, int nblk, int n, float c, BatchStep qsb, int64_t qsr,
+    BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr) {
+  typedef SplitForward<NK> SF;
+  constexpr int NB = SF::NB, ROWB = SF::ROWB, PPR = ROWB / 16, STAGES = SF::STAGES, TILE = SF::TILE;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char split_lds[];
+  uint16_t *const k_lds = reinterpret_cast<uint16_t *>(split_lds), *const v_lds = k_lds + STAGES * TILE;
+  float *const m_lds = reinterpret_cast<float *>(split_lds + SF::MAIN), *const l_lds = m_lds + 8 * 32;
+
+  const HeadWidth<RAG, NK> width{n};
+  int b, blk;
+  if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ksb.heads);
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), share = wave & 3;
+  const int i0 = blk * FS_TM;
+  const int qw0 = i0 + 32 * (wave >> 2);  // first query of this wavefront (scalar)
+  const int qi = qw0 + (lane & 31);       // this lane's query
+
+  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * width.cols()));
+  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * width.cols()));
+  const uint32_t k_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, ksr);
+  const uint32_t v_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, vsr);
+  const uint32_t k_step = (uint32_t)(512 / PPR * ksr * 2), v_step = (uint32_t)(512 / PPR * vsr * 2);
+  const uint32_t k_chunk = (uint32_t)(FS_KC * ksr * 2), v_chunk = (uint32_t)(FS_KC * vsr * 2);
+  auto request = [&](int kc, int stage) {
+    dma_chunk<PPR, 8, FS_KC>(k_rsrc, k_lds + stage * TILE, wave, k_voff, k_chunk * (uint32_t)kc, k_step);
+    dma_chunk<PPR, 8, FS_KC>(v_rsrc, v_lds + stage * TILE, wave, v_voff, v_chunk * (uint32_t)kc, v_step);
+  };
+  const int kc_lo = max(i0 - w, 0) / FS_KC;
+  const int kc_hi = min(i0 + FS_TM - 1 + w, M - 1) / FS_KC;
+  request(kc_lo, 0);
+
+  const u32x4 tail = width.tail(half);
+  u32x4 qf[NK];
+  {
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) qf[ks] = width.load_operand(qr, Q, qi < M, ks, half, tail);
+  }
+
+  // LDS byte offsets as in attention_forward_dma_kernel, for the block of this share
+  const int r32 = lane & 31;
+  const uint32_t k_at = (uint32_t)(r32 * ROWB + ((half ^ swz<PPR>(r32)) << 4));
+  const int s16 = lane & 15, grp = lane >> 4, rowl = 4 * (grp >> 1) + (s16 >> 2);
+  const uint32_t v_at = (uint32_t)(rowl * ROWB + (((2 * (grp & 1) + ((s16 & 3) >> 1)) ^ swz<PPR>(rowl)) << 4) + 8 * (s16 & 1));
+  typedef s16x4 __attribute__((address_space(3))) * lds_tr_ptr;
+
+  f32x16 o[NB];
+#pragma unroll
+  for (int hb = 0; hb < NB; ++hb)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[hb][v] = 0.0f;
+  float m_used = -1.0e30f, l_part = 0.0f;
+  const float ninf = -__builtin_huge_valf();
+
+  auto block = [&](int stage, int c0, auto edge) {
+    constexpr bool EDGE = decltype(edge)::value;
+    const char *kt = reinterpret_cast<const char *>(k_lds + stage * TILE) + 32 * share * ROWB;
+    const char *vt = reinterpret_cast<const char *>(v_lds + stage * TILE) + 32 * share * ROWB;
+    f32x16 s;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.0f;
+    u32x4 ka[NK];
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks)
+      ka[ks] = width.tile_operand(*reinterpret_cast<const u32x4 *>(kt + (k_at ^ (32 * ks))), ks, tail);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) s = Mma<T>::run(ka[ks], qf[ks], s);
+    u32x4 va[2][NB];  // in flight while the softmax arithmetic runs
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int hb = 0; hb < NB; ++hb) {
+        const char *p = vt + 16 * t * ROWB;
+        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(p + (v_at ^ (64 * hb)))));
+        const u32x2 hi = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(p + 8 * ROWB + (v_at ^ 32 ^ (64 * hb)))));
+        va[t][hb] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    if (EDGE) {
+      const int d0 = c0 + 4 * half - qi;
+      const int first = -w - d0, last = min(w - d0, M - 1 - c0 - 4 * half);
+      const int origin = last < first ? 0x100000 : first;
+      const unsigned span = last < first ? 0u : (unsigned)(last - first);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int ofs = 8 * (v / 4) + v % 4;
+        s[v] = (unsigned)(ofs - origin) <= span ? s[v] : ninf;
+      }
+    }
+    float bm = s[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) bm = fmaxf(bm, s[v]);
+    bm = across_halves_max(bm) * c;
+    const bool raise = bm > m_used + kRaiseStep;
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+      const float m_new = raise ? bm : m_used;
+      const float alpha = __builtin_amdgcn_exp2f(m_used - m_new);
+      m_used = m_new;
+      l_part *= alpha;
+#pragma unroll
+      for (int hb = 0; hb < NB; ++hb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[hb][v] *= alpha;
+    }
+    float p[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], c, -m_used));
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const u32x4 pf = {Mma<T>::pack2(p[8 * t + 0], p[8 * t + 1]), Mma<T>::pack2(p[8 * t + 2], p[8 * t + 3]),
+                        Mma<T>::pack2(p[8 * t + 4], p[8 * t + 5]), Mma<T>::pack2(p[8 * t + 6], p[8 * t + 7])};
+#pragma unroll
+      for (int d = 0; d < 4; ++d) l_part = Mma<T>::add_pair(pf[d], l_part);
+#pragma unroll
+      for (int hb = 0; hb < NB; ++hb) o[hb] = Mma<T>::run(va[t][hb], pf, o[hb]);
+    }
+  };
+
+  int stage = 0;
+  // Chunk kc has landed for everyone, nobody reads chunk kc - 1 any more: its tile takes chunk kc + 1 (beyond
+  // the sequence: zeros nobody reads).
+  auto open_chunk = [&](int kc) {
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    request(kc + 1, stage ^ 1);
+  };
+  auto edge_chunk = [&](int kc) {
+    open_chunk(kc);
+    const int cb = kc * FS_KC + 32 * share;
+    if (!(cb + 31 < qw0 - w || cb > qw0 + 31 + w || cb >= M)) block(stage, cb, std::true_type());  // scalar
+    stage ^= 1;
+  };
+  // The chunks whose block of this share lies wholly inside the wavefront's band and the sequence; every wavefront of
+  // the workgroup passes the same number of barriers.
+  const int in_lo = max(kc_lo, (qw0 + 31 - w - 32 * share + FS_KC - 1) >> 7);
+  const int in_hi = min(kc_hi, (min(qw0 + w, M - 1) - 31 - 32 * share) >> 7);
+  const int lead_end = in_lo <= in_hi ? in_lo : kc_hi + 1;
+  int kc = kc_lo;
+  for (; kc < lead_end; ++kc) edge_chunk(kc);
+  for (; kc <= in_hi; ++kc) {
+    open_chunk(kc);
+    block(stage, 0, std::false_type());
+    stage ^= 1;
+  }
+  for (; kc <= kc_hi; ++kc) edge_chunk(kc);
+
+  // The shares' maxima meet in LDS; every share scales to the common one.
+  float l = across_halves_sum(l_part);
+  if (half == 0) m_lds[32 * wave + r32] = m_used;
+  wait_vmcnt_lgkm0<0>();  // also: the chunk requested past the last one has landed before its tile is reused
+  __builtin_amdgcn_s_barrier();
+  const int mate = wave & 4;  // first wavefront of this query group
+  float m_all = m_lds[32 * mate + r32];
+#pragma unroll
+  for (int x = 1; x < FS_SHARES; ++x) m_all = fmaxf(m_all, m_lds[32 * (mate + x) + r32]);
+  const float to_all = __builtin_amdgcn_exp2f(m_used - m_all);
+  if (half == 0) l_lds[32 * wave + r32] = l * to_all;
+  f32x4 *const part = reinterpret_cast<f32x4 *>(split_lds);
+#pragma unroll
+  for (int hb = 0; hb < NB; ++hb)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      part[((wave * NB + hb) * 4 + g) * 64 + lane] = f32x4{o[hb][4 * g] * to_all, o[hb][4 * g + 1] * to_all,
+                                                         o[hb][4 * g + 2] * to_all, o[hb][4 * g + 3] * to_all};
+  wait_vmcnt_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();
+  l = 0.0f;
+#pragma unroll
+  for (int x = 0; x < FS_SHARES; ++x) l += l_lds[32 * (mate + x) + r32];
+  float alpha = 1.0f;
+  if (!MASK) {  // band entries outside the sequence: see attention_forward_dma_kernel
+    const int n_out = max(0, w - qi) + max(0, qi + w - (M - 1));
+    const float m_new = n_out > 0 ? fmaxf(m_all, 0.0f) : m_all;
+    alpha = __builtin_amdgcn_exp2f(m_all - m_new);
+    l = l * alpha + (float)n_out * __builtin_amdgcn_exp2f(-m_new);
+    m_all = m_new;
+  }
+  if (qi >= M) l = 1.0f;  // rows past the end: keep the arithmetic finite, nothing is stored
+  if (L != nullptr && share == 0 && half == 0 && qi < M) L[(int64_t)b * M + qi] = (m_all + __builtin_amdgcn_logf(l)) * kLn2F;
+  // share s owns columns 32 s .. + 31
+  f32x16 sum[1];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) sum[0][v] = 0.0f;
+  if (share < NB) {
+#pragma unroll
+    for (int x = 0; x < FS_SHARES; ++x)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 q4 = part[(((mate + x) * NB + share) * 4 + g) * 64 + lane];
+        sum[0][4 * g] += q4[0], sum[0][4 * g + 1] += q4[1], sum[0][4 * g + 2] += q4[2], sum[0][4 * g + 3] += q4[3];
+      }
+  }
+  wait_vmcnt_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();  // everyone has read the parts: their place stages the result rows
+  if (share < NB)
+    store_wave_rows<T, 1, RAG>(reinterpret_cast<uint16_t *>(split_lds) + wave * RowStage<1>::ELEMS, sum, alpha / l,
+                               O + osb.at(bp) + 32 * share, osr, qw0, M, width.cols() - 32 * share, lane);
+}
+
 template <typename T, int NK>
 hipError_t launch_forward(const Problem &p, const View &q, const View &k, const View &v, const View &o, float *lse,
                           double scale, int mask) {
@@ -653,6 +882,19 @@ hipError_t launch_forward(const Problem &p, const View &q, const View &k, const 
     const bool fits = (p.M + 3 * AT_KC) * k.sr * 2 < lim && (p.M + 3 * AT_KC) * v.sr * 2 < lim && k.sr > 0 && v.sr > 0 &&
                       (!RAG || (dword_rows(k) && dword_rows(v)));
     if (fits && !(p.flags & WM_FLAG_NO_LDS_DIRECT)) {
+      if (shares_pay(p.B, p.M, p.w, FS_TM)) {
+        const int nsplit = (int)((p.M + FS_TM - 1) / FS_TM);
+        const auto kernel = mask ? attention_forward_split_kernel<T, NK, true> : attention_forward_split_kernel<T, NK, false>;
+        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                SplitForward<NK>::BYTES) == hipSuccess) {
+          hipLaunchKernelGGL(kernel, dim3((unsigned)tiled_grid(p.B, nsplit)), dim3(FS_THREADS), SplitForward<NK>::BYTES,
+                             p.stream, (const uint16_t *)q.data, (const uint16_t *)k.data, (const uint16_t *)v.data,
+                             (uint16_t *)o.data, lse, (int)p.B, (int)p.M, (int)p.w, nsplit, (int)p.N, c, q.sb, q.sr, k.sb,
+                             k.sr, v.sb, v.sr, o.sb, o.sr);
+          return hipGetLastError();
+        }
+        (void)hipGetLastError();  // refused: the kernel below
+      }
       if (mask)
         WM_AT((attention_forward_dma_kernel<T, NK, true>));
       else

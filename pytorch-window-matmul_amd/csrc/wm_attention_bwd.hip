@@ -785,6 +785,382 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
 }
 
 // ---------------------------------------------------------------------------------------------
+// Few tiles: the streamed side shared out among wavefronts
+// ---------------------------------------------------------------------------------------------
+// The two kernels above for launches that leave CUs idle, as attention_forward_split_kernel (wm_attention.hip)
+// does it: wavefront (g, s) of a workgroup has the stationary rows 32 g .. + 31 and of every chunk of 128 streamed
+// rows the block 32 s .. + 31.  The four shares' sums are added up through LDS in a fixed order, share s
+// those of columns 32 s .. + 31.  GROUPS is 2 where two wavefronts of the kernel fit a SIMD, else 1.
+// B1 M4096 N128 w256: query kernel 22.5 us before, 16.7 now; key kernel 28.4 / 17.3.
+constexpr int BS_KC = 128, BS_SHARES = 4;
+
+template <int NK, int GROUPS, int RESULTS>
+struct SplitTile {
+  static constexpr int WAVES = 4 * GROUPS, THREADS = 64 * WAVES, TM = 32 * GROUPS;
+  static constexpr int NB = (NK + 1) / 2, ROWB = NK <= 4 ? 128 : 256, PPR = ROWB / 16, STAGES = 2;
+  static constexpr int TILE = BS_KC * ROWB / 2;             // elements per tile
+  static constexpr int TILE_BYTES = 2 * STAGES * 2 * TILE;  // two tensors
+  static constexpr int SUM_BYTES = WAVES * NB * 4096;       // one result of every wavefront
+  static constexpr int MAIN = TILE_BYTES > RESULTS * SUM_BYTES ? TILE_BYTES : RESULTS * SUM_BYTES;
+  static constexpr int BYTES = MAIN + STAGES * 2 * BS_KC * 4;  // and two statistics of the streamed rows
+  static_assert(BYTES <= 160 * 1024, "LDS of a CU");
+  static __device__ __forceinline__ uint32_t step(int64_t row_stride) { return (uint32_t)(THREADS / PPR * row_stride * 2); }
+  static __device__ __forceinline__ void request(u32x4 rsrc, const uint16_t *tile, int wave, uint32_t voff, uint32_t at, uint32_t step) {
+    dma_chunk<PPR, WAVES, BS_KC>(rsrc, tile, wave, voff, at, step);
+  }
+  // The wavefront's sums into the exchange area, and columns 32 share .. of its group's four back out of it.
+  static __device__ __forceinline__ void put(f32x4 *area, const f32x16 (&acc)[NB], int wave, int lane) {
+#pragma unroll
+    for (int hb = 0; hb < NB; ++hb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        area[((wave * NB + hb) * 4 + g) * 64 + lane] = f32x4{acc[hb][4 * g], acc[hb][4 * g + 1], acc[hb][4 * g + 2], acc[hb][4 * g + 3]};
+  }
+  static __device__ __forceinline__ void collect(const f32x4 *area, f32x16 &sum, int wave, int lane) {
+    const int mate = wave & ~3, share = wave & 3;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+    if (share >= NB) return;
+#pragma unroll
+    for (int x = 0; x < BS_SHARES; ++x)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 q = area[(((mate + x) * NB + share) * 4 + g) * 64 + lane];
+        sum[4 * g] += q[0], sum[4 * g + 1] += q[1], sum[4 * g + 2] += q[2], sum[4 * g + 3] += q[3];
+      }
+  }
+};
+
+template <typename T, int NK>
+__global__ __launch_bounds__(512, 2) void attention_backward_query_split_kernel(
+    const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
+    const uint16_t *__restrict__ O, const uint16_t *__restrict__ dO, const float *__restrict__ L,
+    uint16_t *__restrict__ dQ, float *__restrict__ D, int B, int M, int w, int nblk, int n, float scale, BatchStep qsb,
+    int64_t qsr, BatchStep ksb, int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep osb, int64_t osr, BatchStep gsb, int64_t gsr,
+    BatchStep dqsb, int64_t dqsr) {
+  typedef BwdTile<NK> TL;
+  typedef SplitTile<NK, 2, 1> ST;
+  constexpr int NB = ST::NB, PPR = ST::PPR, STAGES = ST::STAGES, TILE = ST::TILE;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char split_lds[];
+  uint16_t *const k_lds = reinterpret_cast<uint16_t *>(split_lds), *const v_lds = k_lds + STAGES * TILE;
+
+  const HeadWidth<RAG, NK> width{n};
+  int b, blk;
+  if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, ksb.heads);
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), share = wave & 3;
+  const int i0 = blk * ST::TM;
+  const int qw0 = i0 + 32 * (wave >> 2);  // scalar
+  const int qi = qw0 + (lane & 31);
+  const bool q_ok = qi < M;
+  const float c = scale * kLog2e;
+
+  const u32x4 k_rsrc = make_rsrc(K + ksb.at(bp), (uint32_t)((M - 1) * ksr * 2 + 2 * width.cols()));
+  const u32x4 v_rsrc = make_rsrc(V + vsb.at(bp), (uint32_t)((M - 1) * vsr * 2 + 2 * width.cols()));
+  const uint32_t k_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, ksr), v_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, vsr);
+  const uint32_t k_step = ST::step(ksr), v_step = ST::step(vsr);
+  const uint32_t k_chunk = (uint32_t)(BS_KC * ksr * 2), v_chunk = (uint32_t)(BS_KC * vsr * 2);
+  auto request = [&](int kc, int stage) {
+    ST::request(k_rsrc, k_lds + stage * TILE, wave, k_voff, k_chunk * (uint32_t)kc, k_step);
+    ST::request(v_rsrc, v_lds + stage * TILE, wave, v_voff, v_chunk * (uint32_t)kc, v_step);
+  };
+  const int kc_lo = max(i0 - w, 0) / BS_KC;
+  const int kc_hi = min(i0 + ST::TM - 1 + w, M - 1) / BS_KC;
+  request(kc_lo, 0);
+
+  const u32x4 tail = width.tail(half);
+  u32x4 qf[NK], gf[NK];
+  float delta = 0.0f;
+  {
+    const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
+    const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr;
+    const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr;
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      qf[ks] = width.load_operand(qr, Q, q_ok, ks, half, tail);
+      gf[ks] = width.load_operand(gr, dO, q_ok, ks, half, tail);
+      delta += dot8<T>(gf[ks], width.load_operand(orow, O, q_ok, ks, half, tail));
+    }
+  }
+  delta = halves_sum(delta);
+  const float l2 = (q_ok ? L[(int64_t)b * M + qi] : 0.0f) * kLog2e;
+  if (q_ok && half == 0 && share == 0) {
+    D[(int64_t)b * M + qi] = -delta;  // the key kernel's dP accumulators start from it
+    D[((int64_t)B + b) * M + qi] = l2;
+  }
+
+  const uint32_t row_at = TL::row_at(lane), tr_at = TL::tr_at(lane);
+  f32x16 dq[NB];
+#pragma unroll
+  for (int hb = 0; hb < NB; ++hb)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) dq[hb][v] = 0.0f;
+  const float ninf = -__builtin_huge_valf();
+
+  auto block = [&](int stage, int c0, auto edge) {
+    constexpr bool EDGE = decltype(edge)::value;
+    const uint16_t *kt = k_lds + stage * TILE, *vt = v_lds + stage * TILE;
+    f32x16 s, dp;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.0f, dp[v] = 0.0f;
+    u32x4 ka[NK], va[NK];
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      ka[ks] = width.tile_operand(TL::rows(kt, row_at, share, ks), ks, tail);
+      va[ks] = width.tile_operand(TL::rows(vt, row_at, share, ks), ks, tail);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      s = Mma<T>::run(ka[ks], qf[ks], s);
+      dp = Mma<T>::run(va[ks], gf[ks], dp);
+    }
+    u32x4 kc[2][NB];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int hb = 0; hb < NB; ++hb) kc[t][hb] = TL::cols(kt, tr_at, share, t, hb);
+    __builtin_amdgcn_sched_barrier(0);
+    if (EDGE) {
+      const int d0 = c0 + 4 * half - qi;  // key - query at offset 0; valid offsets: first..last
+      const int first = -w - d0, last = min(w - d0, M - 1 - c0 - 4 * half);
+      const int origin = last < first ? 0x100000 : first;
+      const unsigned span = last < first ? 0u : (unsigned)(last - first);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int ofs = 8 * (v / 4) + v % 4;
+        s[v] = (unsigned)(ofs - origin) <= span ? s[v] : ninf;
+      }
+    }
+    float ds[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) ds[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], c, -l2)) * (dp[v] - delta);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const u32x4 dsf = pack8<T>(ds + 8 * t);
+#pragma unroll
+      for (int hb = 0; hb < NB; ++hb) dq[hb] = Mma<T>::run(kc[t][hb], dsf, dq[hb]);
+    }
+  };
+
+  int stage = 0;
+  auto open_chunk = [&](int kc) {
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    request(kc + 1, stage ^ 1);
+  };
+  auto edge_chunk = [&](int kc) {
+    open_chunk(kc);
+    const int cb = kc * BS_KC + 32 * share;
+    if (!(cb + 31 < qw0 - w || cb > qw0 + 31 + w || cb >= M)) block(stage, cb, std::true_type());  // scalar
+    stage ^= 1;
+  };
+  const int in_lo = max(kc_lo, (qw0 + 31 - w - 32 * share + BS_KC - 1) >> 7);
+  const int in_hi = min(kc_hi, (min(qw0 + w, M - 1) - 31 - 32 * share) >> 7);
+  const int lead_end = in_lo <= in_hi ? in_lo : kc_hi + 1;
+  int kc = kc_lo;
+  for (; kc < lead_end; ++kc) edge_chunk(kc);
+  for (; kc <= in_hi; ++kc) {
+    open_chunk(kc);
+    block(stage, 0, std::false_type());
+    stage ^= 1;
+  }
+  for (; kc <= kc_hi; ++kc) edge_chunk(kc);
+
+  wait_vmcnt_lgkm0<0>();  // the chunk requested past the last one has landed before its tile is reused
+  __builtin_amdgcn_s_barrier();
+  f32x4 *const area = reinterpret_cast<f32x4 *>(split_lds);
+  ST::put(area, dq, wave, lane);
+  wait_vmcnt_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();
+  f32x16 sum[1];
+  ST::collect(area, sum[0], wave, lane);
+  wait_vmcnt_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();  // everyone has read the sums: their place stages the result rows
+  if (share < NB)
+    store_wave_rows<T, 1, RAG>(reinterpret_cast<uint16_t *>(split_lds) + wave * RowStage<1>::ELEMS, sum, scale,
+                               dQ + dqsb.at(bp) + 32 * share, dqsr, qw0, M, width.cols() - 32 * share, lane);
+}
+
+template <typename T, int NK>
+__global__ __launch_bounds__(NK <= 4 ? 512 : 256, NK <= 4 ? 2 : 1) void attention_backward_key_split_kernel(
+    const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
+    const uint16_t *__restrict__ dO, const float *__restrict__ D, uint16_t *__restrict__ dK,
+    uint16_t *__restrict__ dV, int B, int M, int w, int nblk, int n, float scale, BatchStep qsb, int64_t qsr, BatchStep ksb,
+    int64_t ksr, BatchStep vsb, int64_t vsr, BatchStep gsb, int64_t gsr, BatchStep dksb, int64_t dksr, BatchStep dvsb,
+    int64_t dvsr) {
+  typedef BwdTile<NK> TL;
+  typedef SplitTile<NK, (NK <= 4 ? 2 : 1), 2> ST;
+  constexpr int NB = ST::NB, PPR = ST::PPR, STAGES = ST::STAGES, TILE = ST::TILE;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char split_lds[];
+  uint16_t *const q_lds = reinterpret_cast<uint16_t *>(split_lds), *const g_lds = q_lds + STAGES * TILE;
+  float *const stat_lds = reinterpret_cast<float *>(split_lds + ST::MAIN);  // [stage][0: -D, 1: log-sum-exp][row]
+
+  const HeadWidth<RAG, NK> width{n};
+  int b, blk;
+  if (!decode_block(nblk, B, &b, &blk)) return;
+  const BatchPos bp = batch_pos(b, qsb.heads);
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), share = wave & 3;
+  const int c0 = blk * ST::TM;
+  const int kw0 = c0 + 32 * (wave >> 2);  // first key of this wavefront (scalar)
+  const int kj = kw0 + (lane & 31);
+  const bool k_ok = kj < M;
+  const float c = scale * kLog2e;
+
+  const u32x4 q_rsrc = make_rsrc(Q + qsb.at(bp), (uint32_t)((M - 1) * qsr * 2 + 2 * width.cols()));
+  const u32x4 g_rsrc = make_rsrc(dO + gsb.at(bp), (uint32_t)((M - 1) * gsr * 2 + 2 * width.cols()));
+  // share x fetches statistic x % 2 of rows 64 (x / 2) .. + 63 of a chunk (both groups the same)
+  const u32x4 s_rsrc = make_rsrc(D + ((int64_t)(share & 1) * B + b) * M, (uint32_t)(M * 4));
+  const uint32_t q_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, qsr), g_voff = dma_lane_offset_in_row<PPR>(width, wave, lane, gsr);
+  const uint32_t q_step = ST::step(qsr), g_step = ST::step(gsr);
+  const uint32_t q_chunk = (uint32_t)(BS_KC * qsr * 2), g_chunk = (uint32_t)(BS_KC * gsr * 2);
+  auto request = [&](int qc, int stage) {
+    ST::request(q_rsrc, q_lds + stage * TILE, wave, q_voff, q_chunk * (uint32_t)qc, q_step);
+    ST::request(g_rsrc, g_lds + stage * TILE, wave, g_voff, g_chunk * (uint32_t)qc, g_step);
+    dma_dword(s_rsrc, lds_address(stat_lds + (2 * stage + (share & 1)) * BS_KC + 64 * (share >> 1)), 4 * lane,
+              (uint32_t)((qc * BS_KC + 64 * (share >> 1)) * 4));
+  };
+  const int qc_lo = max(c0 - w, 0) / BS_KC;
+  const int qc_hi = min(c0 + ST::TM - 1 + w, M - 1) / BS_KC;
+  request(qc_lo, 0);
+
+  const u32x4 tail = width.tail(half);
+  u32x4 kf[NK], vf[NK];
+  {
+    const uint16_t *kr = K + ksb.at(bp) + (int64_t)kj * ksr;
+    const uint16_t *vr = V + vsb.at(bp) + (int64_t)kj * vsr;
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      kf[ks] = width.load_operand(kr, K, k_ok, ks, half, tail);
+      vf[ks] = width.load_operand(vr, V, k_ok, ks, half, tail);
+    }
+  }
+
+  const uint32_t row_at = TL::row_at(lane), tr_at = TL::tr_at(lane);
+  f32x16 dk[NB], dv[NB];
+#pragma unroll
+  for (int hb = 0; hb < NB; ++hb)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) dk[hb][v] = 0.0f, dv[hb][v] = 0.0f;
+  const float ninf = -__builtin_huge_valf();
+
+  auto block = [&](int stage, int r0, auto edge) {
+    constexpr bool EDGE = decltype(edge)::value;
+    const uint16_t *qt = q_lds + stage * TILE, *gt = g_lds + stage * TILE;
+    const float *st = stat_lds + 2 * stage * BS_KC + 32 * share;
+    f32x16 s, dp;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.0f;
+    u32x4 qa[NK], ga[NK];
+    f32x4 l2[4];
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      qa[ks] = width.tile_operand(TL::rows(qt, row_at, share, ks), ks, tail);
+      ga[ks] = width.tile_operand(TL::rows(gt, row_at, share, ks), ks, tail);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 nd = *reinterpret_cast<const f32x4 *>(st + 8 * g + 4 * half);
+      dp[4 * g] = nd[0], dp[4 * g + 1] = nd[1], dp[4 * g + 2] = nd[2], dp[4 * g + 3] = nd[3];
+      l2[g] = *reinterpret_cast<const f32x4 *>(st + BS_KC + 8 * g + 4 * half);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) {
+      s = Mma<T>::run(qa[ks], kf[ks], s);
+      dp = Mma<T>::run(ga[ks], vf[ks], dp);
+    }
+    u32x4 gc[2][NB], qc[2][NB];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int hb = 0; hb < NB; ++hb) gc[t][hb] = TL::cols(gt, tr_at, share, t, hb), qc[t][hb] = TL::cols(qt, tr_at, share, t, hb);
+    __builtin_amdgcn_sched_barrier(0);
+    if (EDGE) {
+      const int d0 = r0 + 4 * half - kj;  // query - key at offset 0; valid offsets: first..last
+      const int first = -w - d0, last = min(w - d0, M - 1 - r0 - 4 * half);
+      const int origin = last < first ? 0x100000 : first;
+      const unsigned span = last < first ? 0u : (unsigned)(last - first);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int ofs = 8 * (v / 4) + v % 4;
+        s[v] = (unsigned)(ofs - origin) <= span ? s[v] : ninf;
+      }
+    }
+    float p[16], ds[16];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int v = 4 * g + r;
+        p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], c, -l2[g][r]));
+        ds[v] = p[v] * dp[v];
+      }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const u32x4 pf = pack8<T>(p + 8 * t), dsf = pack8<T>(ds + 8 * t);
+#pragma unroll
+      for (int hb = 0; hb < NB; ++hb) {
+        dv[hb] = Mma<T>::run(gc[t][hb], pf, dv[hb]);
+        dk[hb] = Mma<T>::run(qc[t][hb], dsf, dk[hb]);
+      }
+    }
+  };
+
+  int stage = 0;
+  auto open_chunk = [&](int qc) {
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    request(qc + 1, stage ^ 1);
+  };
+  auto edge_chunk = [&](int qc) {
+    open_chunk(qc);
+    const int rb = qc * BS_KC + 32 * share;
+    if (!(rb + 31 < kw0 - w || rb > kw0 + 31 + w || rb >= M)) block(stage, rb, std::true_type());  // scalar
+    stage ^= 1;
+  };
+  const int in_lo = max(qc_lo, (kw0 + 31 - w - 32 * share + BS_KC - 1) >> 7);
+  const int in_hi = min(qc_hi, (min(kw0 + w, M - 1) - 31 - 32 * share) >> 7);
+  const int lead_end = in_lo <= in_hi ? in_lo : qc_hi + 1;
+  int qc = qc_lo;
+  for (; qc < lead_end; ++qc) edge_chunk(qc);
+  for (; qc <= in_hi; ++qc) {
+    open_chunk(qc);
+    block(stage, 0, std::false_type());
+    stage ^= 1;
+  }
+  for (; qc <= qc_hi; ++qc) edge_chunk(qc);
+
+  wait_vmcnt_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();
+  f32x4 *const k_area = reinterpret_cast<f32x4 *>(split_lds), *const v_area = k_area + ST::SUM_BYTES / 16;
+  ST::put(k_area, dk, wave, lane);
+  ST::put(v_area, dv, wave, lane);
+  wait_vmcnt_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();
+  f32x16 ksum[1], vsum[1];
+  ST::collect(k_area, ksum[0], wave, lane);
+  ST::collect(v_area, vsum[0], wave, lane);
+  wait_vmcnt_lgkm0<0>();
+  __builtin_amdgcn_s_barrier();
+  uint16_t *stage_rows = reinterpret_cast<uint16_t *>(split_lds) + wave * RowStage<1>::ELEMS;
+  if (share < NB) {
+    const int cols = width.cols() - 32 * share;
+    if (dK != nullptr) store_wave_rows<T, 1, RAG>(stage_rows, ksum, scale, dK + dksb.at(bp) + 32 * share, dksr, kw0, M, cols, lane);
+    if (dV != nullptr) store_wave_rows<T, 1, RAG>(stage_rows, vsum, 1.0f, dV + dvsb.at(bp) + 32 * share, dvsr, kw0, M, cols, lane);
+  }
+}
+
+// More LDS than a kernel gets without asking: the call changes an attribute of the function, it allocates nothing.
+inline bool allow_lds(const void *kernel, int bytes) {
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+// ---------------------------------------------------------------------------------------------
 // Narrow windows (w <= 16 (NKB - 1), N <= 64): one kernel for all three gradients
 // ---------------------------------------------------------------------------------------------
 // With a band of at most 65 entries the two kernels above read q, k, v and dO twice and exchange D
@@ -1116,7 +1492,17 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
       }
     }
     if (fits) {
-      if (gq.data != nullptr)
+      typedef SplitTile<NK, 2, 1> QT;
+      typedef SplitTile<NK, (NK <= 4 ? 2 : 1), 2> KT;
+      const auto query_split = attention_backward_query_split_kernel<T, NK>;
+      const auto key_split = attention_backward_key_split_kernel<T, NK>;
+      const int nq = (int)((p.M + QT::TM - 1) / QT::TM), nk = (int)((p.M + KT::TM - 1) / KT::TM);
+      if (gq.data != nullptr && shares_pay(p.B, p.M, p.w, QT::TM) && allow_lds(reinterpret_cast<const void *>(query_split), QT::BYTES))
+        hipLaunchKernelGGL(query_split, dim3((unsigned)tiled_grid(p.B, nq)), dim3(QT::THREADS), QT::BYTES, p.stream, (in_t)q.data,
+                           (in_t)k.data, (in_t)v.data, (in_t)o.data, (in_t)go.data, lse, (out_t)gq.data, delta, (int)p.B,
+                           (int)p.M, (int)p.w, nq, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr,
+                           go.sb, go.sr, gq.sb, gq.sr);
+      else if (gq.data != nullptr)
         hipLaunchKernelGGL((attention_backward_query_dma_kernel<T, NK>), grid, block, 0, p.stream, (in_t)q.data,
                            (in_t)k.data, (in_t)v.data, (in_t)o.data, (in_t)go.data, lse, (out_t)gq.data, delta, (int)p.B,
                            (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr, go.sb,
@@ -1126,6 +1512,13 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
                            (in_t)go.data, lse, delta, (int)p.B, (int)p.M, nblk, (int)p.N, o.sb, o.sr, go.sb, go.sr);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess || (gk.data == nullptr && gv.data == nullptr)) return err;
+      if (shares_pay(p.B, p.M, p.w, KT::TM) && allow_lds(reinterpret_cast<const void *>(key_split), KT::BYTES)) {
+        hipLaunchKernelGGL(key_split, dim3((unsigned)tiled_grid(p.B, nk)), dim3(KT::THREADS), KT::BYTES, p.stream, (in_t)q.data,
+                           (in_t)k.data, (in_t)v.data, (in_t)go.data, (const float *)delta, (out_t)gk.data, (out_t)gv.data,
+                           (int)p.B, (int)p.M, (int)p.w, nk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr,
+                           go.sb, go.sr, gk.sb, gk.sr, gv.sb, gv.sr);
+        return hipGetLastError();
+      }
       hipLaunchKernelGGL((attention_backward_key_dma_kernel<T, NK>), grid, block, 0, p.stream, (in_t)q.data,
                          (in_t)k.data, (in_t)v.data, (in_t)go.data, (const float *)delta, (out_t)gk.data,
                          (out_t)gv.data, (int)p.B, (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb,

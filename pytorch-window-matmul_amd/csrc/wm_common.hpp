@@ -190,6 +190,15 @@ inline bool fast_layout(const View &v, int dtype) {
   return (v.sr * es) % 16 == 0 && (v.sb.step * es) % 16 == 0 && (v.sb.heads <= 0 || (v.sb.group * es) % 16 == 0);
 }
 
+// The fused attention kernels that share the streamed side of a tile out among wavefronts (workgroups of `rows` rows)
+// are taken while all their workgroups start at once, one on a CU: up to there they are faster at every window from
+// 32 on, beyond it the second round makes them slower.  us without / with, tiles of 128 rows in the launch:
+//   forward (64 rows)       N = 128 w = 1024: 64 tiles 45 / 25, 128 46 / 27, 192 46 / 47;  w = 256: 128 tiles 18 / 13, 192 18.7 / 23.7
+//                           N = 64 w = 256: 128 tiles 12.5 / 9.4, 192 12.6 / 13.2;  w = 64: 128 tiles 8.0 / 7.2
+//   query kernel (64 rows)  N = 128 w = 256: 128 tiles 23.8 / 18.2, 192 26 / 33;  w = 64: 14.2 / 13.5;  N = 96 w = 20: 9.1 / 9.8
+//   key kernel (32 rows)    N = 128 w = 256: 64 tiles 29.5 / 18.2, 128 29.1 / 29.1, 192 30 / 42;  w = 64: 64 tiles 17.7 / 14.0
+inline bool shares_pay(int64_t B, int64_t M, int64_t w, int rows) { return w >= 32 && B * ((M + rows - 1) / rows) <= 256; }
+
 // 16-bit rows that all start on a multiple of 4 bytes: what loads straight into LDS need.
 inline bool dword_rows(const View &v) {
   return (uintptr_t)v.data % 4 == 0 && v.sr % 2 == 0 && v.sb.step % 2 == 0 && (v.sb.heads <= 0 || v.sb.group % 2 == 0);

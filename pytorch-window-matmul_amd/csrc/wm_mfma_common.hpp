@@ -358,13 +358,14 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
 // (LDS, 64 * PPR slots).  `voff` is the lane's byte offset inside a chunk for the first of the
 // wave's loads (row and swizzled piece of slot 64 wave + lane); the wave's further loads are
 // 256 / PPR rows apart, which is `step` bytes in memory and 4096 bytes in LDS.
-template <int PPR>
+// With other counts of wavefronts and rows the loads are 64 WAVES / PPR rows and 1024 WAVES bytes of LDS apart.
+template <int PPR, int WAVES = 4, int ROWS = 64>
 __device__ __forceinline__ void dma_chunk(u32x4 rsrc, const uint16_t *tile, int wave, uint32_t voff,
                                           uint32_t row_bytes0, uint32_t step) {
-  constexpr int LOADS = PPR / 4;  // per wave: 64 PPR pieces / 64 lanes / 4 waves
+  constexpr int LOADS = ROWS * PPR / (64 * WAVES);  // per wave: ROWS PPR pieces / 64 lanes / WAVES
   const uint32_t base = lds_address(tile) + 1024 * wave;
 #pragma unroll
-  for (int j = 0; j < LOADS; ++j) dma_piece(rsrc, base + 4096 * j, voff, row_bytes0 + step * j);
+  for (int j = 0; j < LOADS; ++j) dma_piece(rsrc, base + 1024 * WAVES * j, voff, row_bytes0 + step * j);
 }
 // The lane's offset for the above: slot 64 wave + lane of the tile -> row, logical piece.
 template <int PPR>
