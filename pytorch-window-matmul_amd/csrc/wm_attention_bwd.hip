@@ -744,6 +744,88 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
     }
   };
 
+  // Both blocks of an interior chunk together, the vector arithmetic of one among the matrix instructions of the
+  // other: above N = 64 a SIMD has one wavefront, and nothing else fills its waits (at B1x16 M32768 N128 w512
+  // a block of 32 rows took 2 500 cycles for 1 024 of matrix instructions; a training step 1 580 us, with this 1 511).
+  // Up to N = 64 two wavefronts share the SIMD and 256 registers each, which this would not fit.
+  auto pair = [&](const uint16_t *qt, const uint16_t *gt, const float *st) {
+    f32x16 s[2], dp[2];
+    f32x4 l2[2][4];
+    u32x4 qa[2][NK], ga[2][NK], gc[2][2][NB], qc[2][2][NB], pf[2][2], dsf[2][2];
+    auto read_rows = [&](int x) {
+#pragma unroll
+      for (int ks = 0; ks < NK; ++ks) {
+        qa[x][ks] = width.tile_operand(TL::rows(qt, row_at, x, ks), ks, tail);
+        ga[x][ks] = width.tile_operand(TL::rows(gt, row_at, x, ks), ks, tail);
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 nd = *reinterpret_cast<const f32x4 *>(st + 32 * x + 8 * g + 4 * half);
+        dp[x][4 * g] = nd[0], dp[x][4 * g + 1] = nd[1], dp[x][4 * g + 2] = nd[2], dp[x][4 * g + 3] = nd[3];
+        l2[x][g] = *reinterpret_cast<const f32x4 *>(st + AB_KC + 32 * x + 8 * g + 4 * half);
+      }
+    };
+    auto first_products = [&](int x) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) s[x][v] = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < NK; ++ks) {
+        s[x] = Mma<T>::run(qa[x][ks], kf[ks], s[x]);
+        dp[x] = Mma<T>::run(ga[x][ks], vf[ks], dp[x]);
+      }
+    };
+    auto read_cols = [&](int x) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int hb = 0; hb < NB; ++hb)
+          gc[x][t][hb] = TL::cols(gt, tr_at, x, t, hb), qc[x][t][hb] = TL::cols(qt, tr_at, x, t, hb);
+    };
+    auto probabilities = [&](int x) {
+      float p[16], ds[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[x][v], c, -l2[x][v / 4][v % 4]));
+        ds[v] = p[v] * dp[x][v];
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) pf[x][t] = pack8<T>(p + 8 * t), dsf[x][t] = pack8<T>(ds + 8 * t);
+    };
+    auto second_products = [&](int x) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int hb = 0; hb < NB; ++hb) {
+          dv[hb] = Mma<T>::run(gc[x][t][hb], pf[x][t], dv[hb]);
+          dk[hb] = Mma<T>::run(qc[x][t][hb], dsf[x][t], dk[hb]);
+        }
+    };
+    // one matrix instruction, then vector arithmetic while it runs
+    auto interleave = [&](auto count) {
+#pragma unroll
+      for (int i = 0; i < decltype(count)::value; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x402, 6, 0);  // vector and transcendental
+      }
+    };
+    read_rows(0);
+    __builtin_amdgcn_sched_barrier(0);
+    read_rows(1);
+    first_products(0);
+    __builtin_amdgcn_sched_barrier(0);
+    read_cols(0);
+    first_products(1);
+    probabilities(0);
+    interleave(std::integral_constant<int, 2 * NK>());
+    __builtin_amdgcn_sched_barrier(0);
+    read_cols(1);
+    second_products(0);
+    probabilities(1);
+    interleave(std::integral_constant<int, 4 * NB>());
+    __builtin_amdgcn_sched_barrier(0);
+    second_products(1);
+  };
+
   int stage = 0;
   auto open_chunk = [&](int qc) {
     wait_vmcnt<(DEPTH - 1) * LOADS>();
@@ -770,8 +852,12 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_backward_
   for (; qc < lead_end; ++qc) edge_chunk(qc);
   for (; qc <= pair_hi; ++qc) {
     open_chunk(qc);
-    block(q_lds[stage], g_lds[stage], stat_lds[stage][0], 0, 0, std::false_type());
-    block(q_lds[stage], g_lds[stage], stat_lds[stage][0], 1, 0, std::false_type());
+    if constexpr (NK > 4) {
+      pair(q_lds[stage], g_lds[stage], stat_lds[stage][0]);
+    } else {
+      block(q_lds[stage], g_lds[stage], stat_lds[stage][0], 0, 0, std::false_type());
+      block(q_lds[stage], g_lds[stage], stat_lds[stage][0], 1, 0, std::false_type());
+    }
     close_chunk();
   }
   for (; qc <= qc_hi; ++qc) edge_chunk(qc);
