@@ -253,6 +253,15 @@ int wm_grouped_window_attention_backward(const wm_grouped_operand *q, const wm_g
                                          int64_t M, int64_t N, int64_t w, double scale, int dtype,
                                          unsigned flags, void *stream);
 
+/* Gradient of the scores of o = unwindow_matmul(softmax(scale * scores), v, w) in one kernel:
+ *   grad_scores = scale * probs * (window_matmul(grad_o, v^T, w) - rowsum(grad_o * o))
+ * probs and grad_scores are (B, M, 2w+1) bands, grad_o, v, o (B, M, N) operands.  WM_ERR_UNSUPPORTED, nothing launched, unless
+ * dtype is float32, N a multiple of 8 up to 128, w >= 16 and the rows are 16-byte aligned with unit column stride. */
+int wm_grouped_score_gradient(const wm_grouped_operand *grad_o, const wm_grouped_operand *v,
+                              const wm_grouped_operand *o, const wm_operand *probs, const wm_operand *grad_scores,
+                              int64_t B, int64_t M, int64_t N, int64_t w, double scale, int dtype, unsigned flags,
+                              void *stream);
+
 /* 1 if the fused kernels exist for this shape, dtype and scale (layout aside), else 0. */
 int wm_window_attention_supported(int64_t M, int64_t N, int64_t w, int dtype, double scale);
 

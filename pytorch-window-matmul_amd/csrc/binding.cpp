@@ -669,6 +669,70 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
   return out;
 }
 
+// Window attention in float32, where the recomputing kernels would need three times the matrix work: the separate ops
+// forward, and a backward that forms the gradient of the scores in one kernel.
+bool window_attention_f32_supported(const torch::Tensor &q, int64_t window_size, double scale) {
+  // from w = 32 on: below, the separate ops have narrow-band kernels for the product
+  return q.dim() >= 2 && q.device().is_cuda() && q.scalar_type() == at::kFloat && q.size(-1) >= 8 && q.size(-1) <= kMaxWidth &&
+         q.size(-1) % 8 == 0 && window_size >= 32 && window_size <= (1 << 28) && scale == scale && q.numel() > 0;
+}
+
+// An undefined result: the kernel does not take these layouts.
+torch::Tensor score_gradient(const torch::Tensor &probs, const torch::Tensor &v, const torch::Tensor &o, const torch::Tensor &grad_output,
+                             int64_t window_size, double scale) {
+  at::hip::HIPGuardMasqueradingAsCUDA guard(v.device());
+  Heads heads;
+  auto vv = vector_friendly(v, heads), oo = vector_friendly(o, heads), go = vector_friendly(grad_output, heads);
+  auto p = band_friendly(probs), gs = torch::empty_like(p);
+  const wm_grouped_operand a = grouped(go), b = grouped(vv), c = grouped(oo);
+  const wm_operand d = band_operand(p), e = band_operand(gs);
+  const int status = wm_grouped_score_gradient(&a, &b, &c, &d, &e, batch_of(v), v.size(-2), v.size(-1), window_size, scale,
+                                               WM_DTYPE_F32, 0, current_stream(v));
+  if (status == WM_ERR_UNSUPPORTED) return torch::Tensor();
+  raise_on_error(status, "score_gradient");
+  return gs;
+}
+
+struct WindowAttentionF32FuncBackward : SavingNode {
+  int64_t window_size = 0;
+  double scale = 1.0;
+  bool mask_out_of_range = false;
+  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
+    const auto &q = t[0], &k = t[1], &v = t[2], &probs = t[3], &out = t[4];
+    const bool need_q = task_should_compute_output(0), need_k = task_should_compute_output(1), need_v = task_should_compute_output(2);
+    check_grad(grad, v, v.size(-1));
+    variable_list g(3);
+    if (need_v) g[2] = or_none(std::get<1>(unwindow_matmul_backward(probs, v, window_size, grad, false, true)));
+    if (!need_q && !need_k) return g;
+    auto gs = score_gradient(probs, v, out, grad, window_size, scale);
+    if (!gs.defined())
+      gs = band_softmax_backward(probs, *std::get<0>(unwindow_matmul_backward(probs, v, window_size, grad, true, false)), scale, mask_out_of_range);
+    auto qk = window_matmul_backward(q, k.transpose(-1, -2), window_size, gs, need_q, need_k);
+    if (need_q) g[0] = *std::get<0>(qk);
+    if (need_k) g[1] = std::get<1>(qk)->transpose(-1, -2);
+    return g;
+  }
+};
+
+torch::Tensor window_attention_f32(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v, int64_t window_size,
+                                   double scale, bool mask_out_of_range) {
+  const bool record = records({&q, &k, &v});
+  check_attention_inputs(q, k, v);
+  torch::Tensor out, probs;
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    probs = band_softmax_forward(window_matmul_forward(q, k.transpose(-1, -2), window_size), scale, mask_out_of_range);
+    out = unwindow_matmul_forward(probs, v, window_size);
+  }
+  if (record) {
+    auto node = make_node<WindowAttentionF32FuncBackward>({q, k, v});
+    node->window_size = window_size, node->scale = scale, node->mask_out_of_range = mask_out_of_range;
+    torch::autograd::set_history(out, node);
+    node->save(q), node->save(k), node->save(v), node->save(probs), node->save(out, true);
+  }
+  return out;
+}
+
 // What Python shows as the grad_fn of a result: an object of a class with the node's name.
 template <typename N>
 void name_node(const char *name) {
@@ -713,6 +777,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   name_node<UnwindowMatmulFuncBackward>("UnwindowMatmulFuncBackward");
   name_node<BandSoftmaxFuncBackward>("BandSoftmaxFuncBackward");
   name_node<WindowAttentionFuncBackward>("WindowAttentionFuncBackward");
+  name_node<WindowAttentionF32FuncBackward>("WindowAttentionF32FuncBackward");
+  m.def("window_attention_f32_supported", &window_attention_f32_supported, "whether window_attention_f32 covers q", py::arg("q"),
+        py::arg("window_size"), py::arg("scale"));
+  m.def("window_attention_f32", &window_attention_f32, "window attention in float32, differentiable", py::arg("q"), py::arg("k"),
+        py::arg("v"), py::arg("window_size"), py::arg("scale"), py::arg("mask_out_of_range"));
   m.def("window_matmul", &window_matmul, "WindowMatmul, differentiable", py::arg("src"), py::arg("other"), py::arg("window_size"));
   m.def("unwindow_matmul", &unwindow_matmul, "UnwindowMatmul, differentiable", py::arg("src"), py::arg("other"),
         py::arg("window_size"));

@@ -298,6 +298,18 @@ int wm_grouped_window_attention_backward(const wm_grouped_operand *q, const wm_g
   return attention_backward(q, k, v, o, lse, grad_o, grad_q, grad_k, grad_v, delta, B, M, N, w, scale, dtype, flags, stream);
 }
 
+int wm_grouped_score_gradient(const wm_grouped_operand *grad_o, const wm_grouped_operand *v, const wm_grouped_operand *o, const wm_operand *probs, const wm_operand *grad_scores, int64_t B, int64_t M, int64_t N, int64_t w, double scale, int dtype, unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
+  if (B == 0 || M == 0) return WM_OK;
+  if (missing(grad_o) || missing(v) || missing(o) || missing(probs) || missing(grad_scores)) return WM_ERR_NULL_POINTER;
+  const Problem prob{B, M, N, w, dtype, flags, static_cast<hipStream_t>(stream)};
+  View vgo = make_view(grad_o), vv = make_view(v), vo = make_view(o), vp = make_view(probs), vgs = make_view(grad_scores);
+  if (!common_heads({&vgo, &vv, &vo, &vp, &vgs})) return WM_ERR_BAD_SHAPE;
+  hipError_t err = hipSuccess;
+  if (!try_launch_f32_split_score_gradient(prob, vgo, vv, vo, vp, vgs, scale, &err)) return WM_ERR_UNSUPPORTED;
+  return to_status(err);
+}
 int wm_window_attention_backward_static(const wm_operand *q, const wm_operand *k, const wm_operand *v,
                                         const wm_operand *o, const float *lse, const wm_operand *grad_o,
                                         const wm_operand *grad_q, const wm_operand *grad_k, const wm_operand *grad_v,

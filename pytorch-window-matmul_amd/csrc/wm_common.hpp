@@ -129,6 +129,9 @@ bool f32_supports(int op, int64_t M, int64_t N, int64_t w, int dtype);
 bool try_launch_f32_split_p1(const Problem &p, const View &x, const View &y, const View &c, hipError_t *err);
 bool try_launch_f32_split_p2(const Problem &p, const View &a, const View &y, const View &c, hipError_t *err);
 bool try_launch_f32_split_p3(const Problem &p, const View &a, const View &y, const View &c, hipError_t *err);
+// dS = scale * P * (dO V^T - rowsum(dO * O)) in band form, by the band-out kernel of that family.
+bool try_launch_f32_split_score_gradient(const Problem &p, const View &go, const View &v, const View &o, const View &probs,
+                                         const View &gs, double scale, hipError_t *err);
 bool f32_split_supports(int op, int64_t M, int64_t N, int64_t w, int dtype, unsigned flags);
 // Tile family: float64, and whatever the families above decline in 16-bit and float32 storage;
 // 64 x 64 tiles on the 16x16x4 matrix instructions, any strides, any N and w.

@@ -329,13 +329,28 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_in_kernel(
 // ------------------------------------------------------------------------------------------
 // P1: band[b,i,c-i+w] = sum_h X[b,i,h] Y[b,c,h]   (+0.0 where c is outside the sequence)
 // acc(m = c, n = i): A operand Y planes [c][h] read by rows, B operand X rows, split once, in registers.
+//
+// SCORES: the backward of a softmax between the two products, done on the way out.  X are the rows of the upstream gradient
+// dO of O = P V and Y those of V, so that the product is dP, and the band written is that of the scores,
+//   dS = scale P (dP - D),   D_i = sum_h dO[i,h] O[i,h] = sum_j P[i,j] dP[i,j].
+// D of a lane's row comes from the rows of O, fetched like those of X, and the pieces of P are requested before
+// the products of their chunk.  Two passes over the band less than with dP written and read again: at B96 M4096 N64
+// w256 the band-out product took 295 us and the softmax backward 400; a training step 2 333 us, with this 2 172.
+// What bounds it is the band-out kernel's staging side plus one more 805 MB of reads.
 // ------------------------------------------------------------------------------------------
-template <int NKG>  // 16 NKG - 8 <= N <= 16 NKG
+struct ScoreGradient {
+  const float *P, *O;
+  int64_t psb;
+  BatchStep osb;
+  int64_t osr;
+  float scale;
+};
+template <int NKG, bool SCORES>  // 16 NKG - 8 <= N <= 16 NKG
 __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const float *__restrict__ X,
                                                                         const float *__restrict__ Y,
                                                                         float *__restrict__ C, int B, int M, int N, int w,
                                                                         int nblk, BatchStep xsb, int64_t xsr, BatchStep ysb,
-                                                                        int64_t ysr, int64_t csb) {
+                                                                        int64_t ysr, int64_t csb, ScoreGradient sg) {
   constexpr int NP = 16 * NKG;
   constexpr int SY = NP + 8;  // plane rows an odd number of 16-byte slots apart: conflict-free 16-byte reads
   constexpr int YPL = SKC * SY;
@@ -370,6 +385,7 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const f
   // this lane's row of X, split: xop[g][p] holds plane p of X[i][16 g + 8 half .. + 7]
   const int i = i0 + wave * 32 + col;
   u32x4 xop[NKG][3];
+  float delta = 0.f;
   {
     const float *xr = X + xsb.at(bp) + (int64_t)i * xsr;
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
@@ -378,10 +394,28 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const f
       const int h = 16 * g + 8 * half;
       const f32x4 lo = (i < M && h < N) ? *reinterpret_cast<const f32x4 *>(xr + h) : z;
       const f32x4 hi = (i < M && h + 4 < N) ? *reinterpret_cast<const f32x4 *>(xr + h + 4) : z;
+      if (SCORES) {
+        const float *orow = sg.O + sg.osb.at(bp) + (int64_t)i * sg.osr + h;
+        const f32x4 olo = (i < M && h < N) ? *reinterpret_cast<const f32x4 *>(orow) : z;
+        const f32x4 ohi = (i < M && h + 4 < N) ? *reinterpret_cast<const f32x4 *>(orow + 4) : z;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) delta += lo[e] * olo[e] + hi[e] * ohi[e];
+      }
       const Planes4 pl = split4(lo), ph = split4(hi);
 #pragma unroll
       for (int p = 0; p < 3; ++p) xop[g][p] = u32x4{pl.p[p][0], pl.p[p][1], ph.p[p][0], ph.p[p][1]};
     }
+  }
+
+  // D of the rows whose pieces this lane stores
+  float d_row[4];
+  const float *Pb = nullptr;
+  if (SCORES) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(delta), __float_as_uint(delta), false, false);
+    delta = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) d_row[s] = __shfl(delta, (lane >> 3) + 8 * s);
+    Pb = sg.P + (int64_t)b * sg.psb;
   }
 
   const int ncg = N >> 2, pieces = SKC * ncg;
@@ -433,6 +467,17 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const f
     // a wave whose 32 rows have no band entry among the chunk's 32 columns has nothing to compute or store
     const int iw = i0 + wave * 32;
     if (cb <= iw + 31 + w && cb + SKC - 1 >= iw - w) {
+      f32x4 prob[4];  // of the pieces stored below, in flight during the products
+      if (SCORES) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int i2 = iw + (lane >> 3) + 8 * s, c = cb + 4 * (lane & 7);
+          const int e_lo = (i2 - w) - c, e_hi = (i2 + w) - c;
+          const bool whole = (i2 < M) & (e_lo <= 0) & (e_hi >= 3);
+          prob[s] = load4(whole ? Pb + (int64_t)i2 * W + (w - i2) + c : Pb);  // W >= 4: a safe address
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
       f32x16 acc;
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[v] = 0.f;
@@ -465,14 +510,19 @@ __global__ __launch_bounds__(kThreads, 2) void f32_split_band_out_kernel(const f
         const int i2 = i0 + wave * 32 + rr, c = cb + 4 * (lane & 7);
         const int e_lo = (i2 - w) - c, e_hi = (i2 + w) - c;
         if (i2 < M && e_hi >= 0 && e_lo <= 3) {
-          const f32x4 out = *reinterpret_cast<const f32x4 *>(stage + rr * kStage + 4 * (lane & 7));
+          f32x4 out = *reinterpret_cast<const f32x4 *>(stage + rr * kStage + 4 * (lane & 7));
           float *dst = Cb + (int64_t)i2 * W + (w - i2) + c;
           if (e_lo <= 0 && e_hi >= 3) {
+            if (SCORES) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) out[e] = sg.scale * (prob[s][e] * (out[e] - d_row[s]));
+            }
             store4(dst, out);
           } else {
+            const float *src = SCORES ? Pb + (dst - Cb) : nullptr;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              if (e >= e_lo && e <= e_hi) dst[e] = out[e];
+              if (e >= e_lo && e <= e_hi) dst[e] = SCORES ? sg.scale * (src[e] * (out[e] - d_row[s])) : out[e];
           }
         }
       }
@@ -525,7 +575,8 @@ hipError_t launch_split_band_in(const Problem &p, const View &a, const View &y, 
   return hipGetLastError();
 }
 
-hipError_t launch_split_band_out(const Problem &p, const View &x, const View &y, const View &c) {
+template <bool SCORES>
+hipError_t launch_split_band_out(const Problem &p, const View &x, const View &y, const View &c, const ScoreGradient &sg) {
   const int nblk = (int)((p.M + TM - 1) / TM);
   dim3 grid((unsigned)tiled_grid(p.B, nblk)), block(kThreads);
   // too few workgroups to fill the chip: each takes a share of its tile's dense columns instead of
@@ -534,9 +585,9 @@ hipError_t launch_split_band_out(const Problem &p, const View &x, const View &y,
   if (wgs < 2 * kCUs) grid.y = (unsigned)std::max<int64_t>(1, std::min<int64_t>(2 * kCUs / wgs, chunks / 4));
 #define WM_F32S_OUT(NKG)                                                                                      \
   case NKG:                                                                                                   \
-    hipLaunchKernelGGL((f32_split_band_out_kernel<NKG>), grid, block, 0, p.stream, (const float *)x.data,     \
+    hipLaunchKernelGGL((f32_split_band_out_kernel<NKG, SCORES>), grid, block, 0, p.stream, (const float *)x.data,     \
                        (const float *)y.data, (float *)c.data, (int)p.B, (int)p.M, (int)p.N, (int)p.w, nblk,  \
-                       x.sb, x.sr, y.sb, y.sr, c.sb.step);                                                         \
+                       x.sb, x.sr, y.sb, y.sr, c.sb.step, sg);                                                      \
     break;
   switch ((p.N + 15) / 16) {
     WM_F32S_OUT(1) WM_F32S_OUT(2) WM_F32S_OUT(3) WM_F32S_OUT(4) WM_F32S_OUT(5) WM_F32S_OUT(6) WM_F32S_OUT(7)
@@ -569,7 +620,18 @@ bool f32_split_supports(int op, int64_t M, int64_t N, int64_t w, int dtype, unsi
 bool try_launch_f32_split_p1(const Problem &p, const View &x, const View &y, const View &c, hipError_t *err) {
   if (!f32_split_supports(1, p.M, p.N, p.w, p.dtype, p.flags)) return false;
   if (!fast_layout(x, p.dtype) || !fast_layout(y, p.dtype) || !split_band_ok(c, 2 * p.w + 1)) return false;
-  *err = launch_split_band_out(p, x, y, c);
+  *err = launch_split_band_out<false>(p, x, y, c, ScoreGradient{});
+  return true;
+}
+bool try_launch_f32_split_score_gradient(const Problem &p, const View &go, const View &v, const View &o, const View &probs,
+                                         const View &gs, double scale, hipError_t *err) {
+  if (!f32_split_supports(1, p.M, p.N, p.w, p.dtype, p.flags) || (p.flags & WM_FLAG_FORCE_STRIDED)) return false;
+  if (tiled_grid(p.B, (p.M + TM - 1) / TM) > 0x7fffffff) return false;
+  if (!fast_layout(go, p.dtype) || !fast_layout(v, p.dtype) || !fast_layout(o, p.dtype)) return false;
+  if (!split_band_ok(probs, 2 * p.w + 1) || !split_band_ok(gs, 2 * p.w + 1)) return false;
+  *err = launch_split_band_out<true>(p, go, v, gs,
+                                     ScoreGradient{(const float *)probs.data, (const float *)o.data, probs.sb.step, o.sb, o.sr,
+                                                   (float)scale});
   return true;
 }
 bool try_launch_f32_split_p2(const Problem &p, const View &a, const View &y, const View &c, hipError_t *err) {

@@ -87,5 +87,7 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
     if _native.window_attention_supported(query, window_size, scale, any_width) and not (
             training and _chain_is_faster(window_size, query.shape[-1], query.numel())):
         return _native.window_attention(query, key, value, window_size, scale, bool(mask_out_of_range))
+    if training and not torch.is_autocast_enabled("cuda") and _native.window_attention_f32_supported(query, window_size, scale):
+        return _native.window_attention_f32(query, key, value, window_size, scale, bool(mask_out_of_range))
     att = window_matmul(query, key.transpose(-1, -2), window_size)
     return unwindow_matmul(band_softmax(att, scale, mask_out_of_range), value, window_size)
