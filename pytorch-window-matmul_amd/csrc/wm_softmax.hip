@@ -27,6 +27,7 @@ constexpr int kSoftmaxThreads = 256;
 constexpr int kLoadsInFlight = 4;      // 16-byte loads a thread issues before it touches LDS
 constexpr int kSpanBytes = 16 * 1024;  // LDS image a workgroup aims for, per input tensor
 constexpr int kLdsLimit = 64 * 1024;
+constexpr int kMaxShortSlots = 20;     // elements per lane up to which a row counts as short
 constexpr float kLog2e = 1.4426950408889634f;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -133,6 +134,40 @@ __device__ __forceinline__ void softmax_row_forward_regs(const T *x, T *out, int
   }
   sum = group_reduce<LANES>(sum, SumOp());
   const float inv = __builtin_amdgcn_rcpf(sum);
+#pragma unroll
+  for (int k = 0; k < SLOTS; ++k) {
+    const int j = gl + k * LANES;
+    if (k < FULL || j < W) out[j] = narrow<T>(v[k] * inv);
+  }
+}
+
+// The same for the longest rows (more than kMaxShortSlots elements per lane), with the arithmetic of the re-reading variant
+// below that they took before: arguments of the exponential in one rounding, the sum divided by, not multiplied with an
+// approximate reciprocal.  The row is read once and exponentiated once, not three times and twice.
+template <typename T, bool MASK, int LANES, int SLOTS, int FULL>
+__device__ __forceinline__ void softmax_row_forward_long(const T *x, T *out, int W, int lo, int hi, int gl, float c) {
+  float v[SLOTS];
+#pragma unroll
+  for (int k = 0; k < SLOTS; ++k) v[k] = to_acc<T>(x[gl + k * LANES]);
+  auto counts = [&](int k) {
+    const int j = gl + k * LANES;
+    return MASK ? j >= lo && j < hi : k < FULL || j < W;
+  };
+  float m = minus_infinity<float>();
+#pragma unroll
+  for (int k = 0; k < SLOTS; ++k) {
+    const float s = v[k] * c;
+    m = counts(k) && s > m ? s : m;
+  }
+  m = group_reduce<LANES>(m, MaxOp());
+  float sum = 0;
+#pragma unroll
+  for (int k = 0; k < SLOTS; ++k) {
+    v[k] = counts(k) ? exp2_of(__builtin_fmaf(v[k], c, -m)) : 0.0f;
+    sum += v[k];
+  }
+  sum = group_reduce<LANES>(sum, SumOp());
+  const float inv = 1.0f / sum;
 #pragma unroll
   for (int k = 0; k < SLOTS; ++k) {
     const int j = gl + k * LANES;
@@ -326,6 +361,8 @@ __global__ __launch_bounds__(kSoftmaxThreads) void band_softmax_staged_kernel(
     if constexpr (SHAPE::slots > 0) {
       if (BACKWARD)
         softmax_row_backward_regs<T, MASK, LANES, SHAPE::slots, SHAPE::full>(row0, row1, row0, W, lo, hi, gl, scale);
+      else if constexpr (SHAPE::slots > kMaxShortSlots)
+        softmax_row_forward_long<T, MASK, LANES, SHAPE::slots, SHAPE::full>(row0, row0, W, lo, hi, gl, scale * kLog2e);
       else
         softmax_row_forward_regs<T, MASK, LANES, SHAPE::slots, SHAPE::full>(row0, row0, W, lo, hi, gl,
                                                                             scale * kLog2e);
@@ -389,14 +426,17 @@ bool contiguous_band(const View &v, int64_t M, int64_t W) {
 
 // Shape classes of the register variant, then the re-reading one.  Lanes per row: 64 for rows
 // longer than 128, else the power of two at or above W/4 (at least 4), which gives 3 or 4
-// elements per lane (1..4 for the shortest rows); long rows get 3..20 per lane in steps that
-// waste at most a quarter of the slots.
+// elements per lane (1..4 for the shortest rows); long rows get 3..48 per lane in steps that
+// waste at most a quarter of the slots.  Rows beyond 48 x 64 elements (w > 1535) are re-read.
+// (With register classes up to 20 slots only, B7 M3001 w1500 float32, 252 MB a band, took 126 us forward and 178 us
+// backward in the re-reading variant; now 96 and 131, 5.2 and 5.8 TB/s.)
 typedef std::tuple<Shape<4, 1, 0>, Shape<4, 2, 1>, Shape<4, 3, 2>, Shape<4, 4, 3>, Shape<8, 3, 2>, Shape<8, 4, 3>,
                    Shape<16, 3, 2>, Shape<16, 4, 3>, Shape<32, 3, 2>, Shape<32, 4, 3>, Shape<64, 3, 2>,
                    Shape<64, 4, 3>, Shape<64, 5, 4>, Shape<64, 6, 5>, Shape<64, 8, 6>, Shape<64, 10, 8>,
-                   Shape<64, 12, 10>, Shape<64, 16, 12>, Shape<64, 20, 16>, Shape<64, 0, 0>>
+                   Shape<64, 12, 10>, Shape<64, 16, 12>, Shape<64, 20, 16>, Shape<64, 24, 20>,
+                   Shape<64, 32, 24>, Shape<64, 40, 32>, Shape<64, 48, 40>, Shape<64, 0, 0>>
     Shapes;
-constexpr int kMaxSlots = 20;
+constexpr int kMaxSlots = 48;
 
 struct StagedPlan {
   int lanes, slots, slots_class;  // slots_class: SLOTS of the chosen class (0: re-reading variant)
@@ -407,6 +447,7 @@ struct StagedPlan {
 constexpr int class_slots(int lanes, int slots) {
   if (slots > kMaxSlots) return 0;
   if (lanes < 64 || slots <= 6) return slots < 3 && lanes > 4 ? 3 : slots;
+  if (slots > kMaxShortSlots) return slots <= 24 ? 24 : slots <= 32 ? 32 : slots <= 40 ? 40 : 48;
   return slots <= 8 ? 8 : slots <= 10 ? 10 : slots <= 12 ? 12 : slots <= 16 ? 16 : 20;
 }
 
