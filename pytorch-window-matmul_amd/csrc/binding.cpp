@@ -672,9 +672,12 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 // Window attention in float32, where the recomputing kernels would need three times the matrix work: the separate ops
 // forward, and a backward that forms the gradient of the scores in one kernel.
 bool window_attention_f32_supported(const torch::Tensor &q, int64_t window_size, double scale) {
-  // from w = 32 on: below, the separate ops have narrow-band kernels for the product
+  // From w = 128 on.  A training step through the separate ops / with the fused gradient of the scores, us, B96 M4096: N = 64
+  // 931 / 953 at w = 64, 1251 / 1257 at w = 100, 2313 / 2093 at w = 256; N = 128 1521 / 1572, 2044 / 2027, 3609 / 3438; B8 M3001
+  // N = 16 191 / 174 at w = 256.  In a narrow band the pieces at its two edges, read element by element, cost more than
+  // the passes that are saved (N = 80, w = 32: 802 / 880).
   return q.dim() >= 2 && q.device().is_cuda() && q.scalar_type() == at::kFloat && q.size(-1) >= 8 && q.size(-1) <= kMaxWidth &&
-         q.size(-1) % 8 == 0 && window_size >= 32 && window_size <= (1 << 28) && scale == scale && q.numel() > 0;
+         q.size(-1) % 8 == 0 && window_size >= 128 && window_size <= (1 << 28) && scale == scale && q.numel() > 0;
 }
 
 // An undefined result: the kernel does not take these layouts.

@@ -9,8 +9,8 @@ from conftest import seeded
 from oracle import attention_oracle as ao
 
 pytestmark = pytest.mark.gpu
-# batch, heads, M, N, w: around a tile (128) and a chunk (32), one column group to eight, windows from the rule's
-# lower end to beyond the sequence; column shares (few tiles) and none
+# batch, heads, M, N, w: around a tile (128) and a chunk (32), one column group to eight, windows from the kernel's
+# lower range to beyond the sequence; column shares (few tiles) and none
 CASES = [(1, 1, 5, 8, 40), (2, 3, 129, 64, 32), (1, 2, 300, 80, 33), (2, 1, 127, 24, 64), (1, 2, 515, 128, 100), (1, 1, 700, 40, 800),
          (40, 16, 130, 16, 35)]
 
@@ -28,7 +28,8 @@ def _error(got, want):
 @pytest.mark.parametrize("layout", ["heads", "flat"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "B%dx%d_M%d_N%d_w%d" % c)
 def test_step_keeps_the_accuracy_of_the_separate_ops(device, case, layout):
-    from window_matmul import band_softmax, unwindow_matmul, window_attention, window_matmul
+    import window_matmul_kernel as native
+    from window_matmul import band_softmax, unwindow_matmul, window_matmul
 
     batch, heads, M, N, w = case
     views = _views(batch, heads, M, N, device, layout)
@@ -40,7 +41,7 @@ def test_step_keeps_the_accuracy_of_the_separate_ops(device, case, layout):
         for fused in (True, False):
             q, k, v = (t.detach().requires_grad_(True) for t in views[:3])
             if fused:
-                out = window_attention(q, k, v, w, mask_out_of_range=mask)
+                out = native.window_attention_f32(q, k, v, w, scale, mask)
                 assert type(out.grad_fn).__name__ == "WindowAttentionF32FuncBackward"
             else:
                 out = unwindow_matmul(band_softmax(window_matmul(q, k.transpose(-1, -2), w), scale, mask), v, w)
@@ -59,7 +60,7 @@ def test_part_of_the_gradients_and_below_the_rule(device):
 
     def grads(need):
         leaves = [t.detach().requires_grad_(n) for t, n in zip(base[:3], need)]
-        window_attention(*leaves, 50).backward(base[3])
+        window_attention(*leaves, 130).backward(base[3])
         return [t.grad for t in leaves]
 
     full = grads((True, True, True))
@@ -67,5 +68,7 @@ def test_part_of_the_gradients_and_below_the_rule(device):
         for n, x, y in zip(need, grads(need), full):
             assert (x is None) == (not n)
             assert x is None or torch.equal(x, y)
-    out = window_attention(base[0].detach().requires_grad_(True), base[1], base[2], 31)
+    out = window_attention(base[0].detach().requires_grad_(True), base[1], base[2], 127)
     assert type(out.grad_fn).__name__ == "UnwindowMatmulFuncBackward"
+    out = window_attention(base[0].detach().requires_grad_(True), base[1], base[2], 128)
+    assert type(out.grad_fn).__name__ == "WindowAttentionF32FuncBackward"
