@@ -880,7 +880,7 @@ hipError_t launch_forward(const Problem &p, const View &q, const View &k, const 
     const int64_t lim = 0x7fffffff;
     // and fetch pieces at dword addresses
     const bool fits = (p.M + 3 * AT_KC) * k.sr * 2 < lim && (p.M + 3 * AT_KC) * v.sr * 2 < lim && k.sr > 0 && v.sr > 0 &&
-                      (!RAG || (dword_rows(k) && dword_rows(v)));
+                      (!RAG || (dword_pieces(k, p.N) && dword_pieces(v, p.N)));
     if (fits && !(p.flags & WM_FLAG_NO_LDS_DIRECT)) {
       if (shares_pay(p.B, p.M, p.w, FS_TM)) {
         const int nsplit = (int)((p.M + FS_TM - 1) / FS_TM);

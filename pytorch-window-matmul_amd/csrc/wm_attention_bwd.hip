@@ -1542,7 +1542,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
     bool fits = !(p.flags & WM_FLAG_NO_LDS_DIRECT) && (p.M + 3 * AB_KC) * 4 < lim;
     // and fetch pieces at dword addresses
     for (const View *t : {&q, &k, &v, &go})
-      fits = fits && t->sr > 0 && (p.M + 3 * AB_KC) * t->sr * 2 < lim && (!RAG || dword_rows(*t));
+      fits = fits && t->sr > 0 && (p.M + 3 * AB_KC) * t->sr * 2 < lim && (!RAG || dword_pieces(*t, p.N));
     if constexpr (NK <= 4) {
       // narrow windows: one kernel for all three gradients (two row blocks per wavefront up to w = 16, three up
       // to 32, four up to 48, five up to 64 where it still pays: B96 M16384 N64 w = 64: 490 against 555 us for

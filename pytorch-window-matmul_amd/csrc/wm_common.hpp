@@ -202,9 +202,11 @@ inline bool fast_layout(const View &v, int dtype) {
 //   key kernel (32 rows)    N = 128 w = 256: 64 tiles 29.5 / 18.2, 128 29.1 / 29.1, 192 30 / 42;  w = 64: 64 tiles 17.7 / 14.0
 inline bool shares_pay(int64_t B, int64_t M, int64_t w, int rows) { return w >= 32 && B * ((M + rows - 1) / rows) <= 256; }
 
-// 16-bit rows that all start on a multiple of 4 bytes: what loads straight into LDS need.
-inline bool dword_rows(const View &v) {
-  return (uintptr_t)v.data % 4 == 0 && v.sr % 2 == 0 && v.sb.step % 2 == 0 && (v.sb.heads <= 0 || v.sb.group % 2 == 0);
+// 16-bit rows of N elements whose pieces all start on a multiple of 4 bytes, which is what loads straight into LDS need: the
+// rows themselves, and the last piece, which starts at column N - 8 (HeadWidth), so an odd N never qualifies.
+inline bool dword_pieces(const View &v, int64_t N) {
+  return N % 2 == 0 && (uintptr_t)v.data % 4 == 0 && v.sr % 2 == 0 && v.sb.step % 2 == 0 &&
+         (v.sb.heads <= 0 || v.sb.group % 2 == 0);
 }
 
 // Band operands are only required to be contiguous per batch (rows of odd

@@ -57,6 +57,31 @@ def test_step_against_oracle(device, case, dtype):
         assert got[1].stride() == views[0].stride()  # gradients are laid out like their operands
 
 
+# B, M, N, w: narrow and wide windows, up to and above N = 64, few tiles and more than any rule for few tiles admits
+@pytest.mark.parametrize("B,M,N,w", [(2, 150, 41, 10), (2, 300, 41, 70), (2, 150, 75, 20), (2, 300, 75, 100), (1, 300, 127, 50),
+                                     (270, 40, 41, 70), (270, 40, 75, 33)])
+@pytest.mark.parametrize("rows", ["padded", "every second"])
+def test_odd_widths_in_rows_on_dword_addresses(device, B, M, N, w, rows):
+    """Rows that start on a multiple of 4 bytes although N is odd: their last piece does not, so they are no case for
+    the loads straight into LDS and give the bits of contiguous rows."""
+    def view(seed):
+        if rows == "padded":
+            return seeded((B, M, N + 5), seed, BF16).to(device)[..., :N]
+        return seeded((B, 2 * M, N), seed, BF16).to(device)[:, ::2]
+
+    views = [view(320 + s) for s in range(4)]
+    assert all(t.stride(1) % 2 == 0 and t.data_ptr() % 4 == 0 for t in views)
+    flat = [t.contiguous() for t in views]
+    got, same = _step(views, w, False), _step(flat, w, False)
+    host = [t[:2].cpu() for t in flat]
+    scale = 1.0 / math.sqrt(N)
+    want_o, _ = ao.window_attention_forward(*host[:3], w, scale, False)
+    want = [want_o, *ao.window_attention_backward(*host[:3], w, host[3], scale, False)]
+    for x, y, z in zip(got, same, want):
+        assert torch.equal(x, y)
+        close(x[:2], z)
+
+
 @pytest.mark.parametrize("N,w", [(60, 20), (60, 100), (75, 20), (75, 100), (41, 60)])
 def test_neighbours_in_memory_do_not_matter(device, N, w):
     """Row pieces never reach into the next head: with NaN in all other heads the first one keeps its bits."""
