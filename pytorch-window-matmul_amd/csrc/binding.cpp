@@ -552,7 +552,12 @@ struct SavingNode : torch::autograd::Node {
   }
 };
 
+// Whether a node has to be made.  There are no forward-mode derivatives: a tangent that an input carries would be
+// dropped without a trace, so such inputs are refused with the error type of an autograd.Function without a jvp.
 bool records(std::initializer_list<const torch::Tensor *> inputs) {
+  for (const auto *t : inputs)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(0).defined(), "no forward-mode derivative is implemented for the banded products, "
+                                "the band softmax and the window attention");
   if (!at::GradMode::is_enabled()) return false;
   for (const auto *t : inputs)
     if (t->requires_grad()) return true;
@@ -783,14 +788,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   name_node<WindowAttentionF32FuncBackward>("WindowAttentionF32FuncBackward");
   m.def("window_attention_f32_supported", &window_attention_f32_supported, "whether window_attention_f32 covers q", py::arg("q"),
         py::arg("window_size"), py::arg("scale"));
-  m.def("window_attention_f32", &window_attention_f32, "window attention in float32, differentiable", py::arg("q"), py::arg("k"),
+  m.def("window_attention_f32", torch::wrap_pybind_function(window_attention_f32), "window attention in float32, differentiable", py::arg("q"), py::arg("k"),
         py::arg("v"), py::arg("window_size"), py::arg("scale"), py::arg("mask_out_of_range"));
-  m.def("window_matmul", &window_matmul, "WindowMatmul, differentiable", py::arg("src"), py::arg("other"), py::arg("window_size"));
-  m.def("unwindow_matmul", &unwindow_matmul, "UnwindowMatmul, differentiable", py::arg("src"), py::arg("other"),
+  m.def("window_matmul", torch::wrap_pybind_function(window_matmul), "WindowMatmul, differentiable", py::arg("src"), py::arg("other"), py::arg("window_size"));
+  m.def("unwindow_matmul", torch::wrap_pybind_function(unwindow_matmul), "UnwindowMatmul, differentiable", py::arg("src"), py::arg("other"),
         py::arg("window_size"));
-  m.def("band_softmax", &band_softmax, "softmax over the band dimension, differentiable", py::arg("src"), py::arg("scale"),
+  m.def("band_softmax", torch::wrap_pybind_function(band_softmax), "softmax over the band dimension, differentiable", py::arg("src"), py::arg("scale"),
         py::arg("mask_out_of_range"));
-  m.def("window_attention", &window_attention, "fused window attention, differentiable", py::arg("q"), py::arg("k"),
+  m.def("window_attention", torch::wrap_pybind_function(window_attention), "fused window attention, differentiable", py::arg("q"), py::arg("k"),
         py::arg("v"), py::arg("window_size"), py::arg("scale"), py::arg("mask_out_of_range"));
   m.def("abi_version", []() { return wm_abi_version(); }, "ABI version of libwindow_matmul_hip.so");
 }

@@ -1,0 +1,51 @@
+"""What torch.autograd.Function does for its callers holds for the native nodes behind the public functions too."""
+import pytest
+import torch
+import torch.autograd.forward_ad as forward_ad
+
+from conftest import seeded
+
+B, M, N, W = 2, 40, 32, 6
+# name, columns of the inputs, dtype
+OPS = [("window_matmul", (N, N), torch.bfloat16), ("unwindow_matmul", (2 * W + 1, N), torch.bfloat16),
+       ("band_softmax", (2 * W + 1,), torch.bfloat16), ("window_attention", (N, N, N), torch.bfloat16),
+       ("window_attention", (44, 44, 44), torch.float16), ("window_attention", (N, N, N), torch.float32)]
+IDS = ["window_matmul", "unwindow_matmul", "band_softmax", "window_attention", "window_attention_N44", "window_attention_float32"]
+
+
+def call(name, dtype):
+    import window_matmul as wm
+
+    if name == "window_matmul":
+        return lambda q, k: wm.window_matmul(q, k.transpose(-1, -2), W)
+    if name == "unwindow_matmul":
+        return lambda a, v: wm.unwindow_matmul(a, v, W)
+    if name == "band_softmax":
+        return lambda a: wm.band_softmax(a, 0.5, True)
+    return lambda q, k, v: wm.window_attention(q, k, v, 130 if dtype == torch.float32 else W)
+
+
+def operands(columns, dtype, device="cpu"):
+    return [seeded((B, M, c), 700 + i, dtype).to(device) for i, c in enumerate(columns)]
+
+
+def refuses_tangents(name, columns, dtype, device):
+    fn = call(name, dtype)
+    for i in range(len(columns)):
+        for other_needs_grad in (False, True):
+            xs = [x.requires_grad_(other_needs_grad and j != i) for j, x in enumerate(operands(columns, dtype, device))]
+            with forward_ad.dual_level():
+                xs[i] = forward_ad.make_dual(xs[i], torch.ones_like(xs[i]))
+                with pytest.raises(NotImplementedError):
+                    fn(*xs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,columns,dtype", OPS, ids=IDS)
+def test_forward_mode_is_refused(device, name, columns, dtype):
+    refuses_tangents(name, columns, dtype, device)
+
+
+@pytest.mark.parametrize("name,columns", [("window_matmul", (N, N)), ("unwindow_matmul", (2 * W + 1, N)), ("band_softmax", (2 * W + 1,))])
+def test_forward_mode_is_refused_before_anything_else(name, columns):
+    refuses_tangents(name, columns, torch.float32, "cpu")
