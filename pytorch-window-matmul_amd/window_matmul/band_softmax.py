@@ -15,7 +15,8 @@ import window_matmul_kernel as _native
 
 
 class BandSoftmaxFunc(torch.autograd.Function):
-    """``softmax(scale * inp, dim=-1)`` on a 3-D band ``(B, M, 2w+1)``; saves only the result."""
+    """``softmax(scale * inp, dim=-1)`` on a band ``(..., M, 2w+1)``; saves only the result.  What
+    :func:`band_softmax` is under ``torch.jit.trace``; elsewhere the native module's own node does the same."""
 
     @staticmethod
     def forward(ctx, inp: torch.Tensor, scale: float, mask_out_of_range: bool) -> torch.Tensor:
@@ -43,4 +44,7 @@ def band_softmax(inp: torch.Tensor, scale: Optional[float] = None, mask_out_of_r
     """
     if inp.dim() < 2 or inp.shape[-1] % 2 != 1:
         raise RuntimeError("Input mismatch")
-    return _native.band_softmax(inp, 1.0 if scale is None else float(scale), bool(mask_out_of_range))
+    scale = 1.0 if scale is None else float(scale)
+    if torch.jit.is_tracing():
+        return BandSoftmaxFunc.apply(inp, scale, bool(mask_out_of_range))
+    return _native.band_softmax(inp, scale, bool(mask_out_of_range))

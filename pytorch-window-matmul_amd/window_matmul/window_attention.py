@@ -42,7 +42,8 @@ def _chain_is_faster(window_size: int, width: int, elements: int) -> bool:
 
 
 class WindowAttentionFunc(torch.autograd.Function):
-    """Fused kernels on ``(..., M, N)`` operands; ``k`` holds key rows (not transposed)."""
+    """Fused kernels on ``(..., M, N)`` operands; ``k`` holds key rows (not transposed).  What
+    :func:`window_attention` takes under ``torch.jit.trace``; elsewhere the native module's own node does the same."""
 
     @staticmethod
     def forward(ctx, q, k, v, window_size: int, scale: float, mask_out_of_range: bool):
@@ -82,12 +83,13 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
     # With a very narrow band the recomputing backward of the fused kernels costs more than the
     # band it avoids writing, so training there goes through the separate ops.
     training = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
+    autocast, tracing = torch.is_autocast_enabled("cuda"), torch.jit.is_tracing()
     # Head widths that 16 does not divide: the chain computes in float16 inside an autocast region, so it stays there.
-    any_width = not torch.is_autocast_enabled("cuda")
-    if _native.window_attention_supported(query, window_size, scale, any_width) and not (
+    if _native.window_attention_supported(query, window_size, scale, not autocast) and not (
             training and _chain_is_faster(window_size, query.shape[-1], query.numel())):
-        return _native.window_attention(query, key, value, window_size, scale, bool(mask_out_of_range))
-    if training and not torch.is_autocast_enabled("cuda") and _native.window_attention_f32_supported(query, window_size, scale):
+        fused = WindowAttentionFunc.apply if tracing else _native.window_attention
+        return fused(query, key, value, window_size, scale, bool(mask_out_of_range))
+    if training and not autocast and not tracing and _native.window_attention_f32_supported(query, window_size, scale):
         return _native.window_attention_f32(query, key, value, window_size, scale, bool(mask_out_of_range))
     att = window_matmul(query, key.transpose(-1, -2), window_size)
     return unwindow_matmul(band_softmax(att, scale, mask_out_of_range), value, window_size)

@@ -19,7 +19,8 @@ import window_matmul_kernel as _native
 
 # Inside a CUDA/HIP autocast region the operands are cast to float16 and the
 # body runs with autocast disabled (reference window_matmul.py:9,18,45,54).  The public functions take
-# the two classes below there, and the native module's own autograd nodes everywhere else.
+# the two classes below there and under torch.jit.trace, which records a Function as one operation but of a native call
+# only the allocation of its result, and the native module's own autograd nodes everywhere else.
 _amp_forward = torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.float16)
 _amp_backward = torch.amp.custom_bwd(device_type="cuda")
 
@@ -89,7 +90,7 @@ def window_matmul(inp: torch.Tensor, other: torch.Tensor, window_size: Optional[
     seq_len, hidden_dim = inp.shape[-2:]
     if other.shape[-2:] != (hidden_dim, seq_len):  # reshaped to the keys' shape like the reference does
         other = other.reshape(-1, hidden_dim, seq_len)
-    if torch.is_autocast_enabled("cuda"):
+    if torch.is_autocast_enabled("cuda") or torch.jit.is_tracing():
         return WindowMatmulFunc.apply(inp, other, window_size)
     return _native.window_matmul(inp, other, window_size)
 
@@ -106,6 +107,6 @@ def unwindow_matmul(inp: torch.Tensor, other: torch.Tensor, window_size: Optiona
     band_shape = (other.shape[-2], 2 * window_size + 1)
     if inp.shape[-2:] != band_shape:
         inp = inp.reshape(-1, *band_shape)
-    if torch.is_autocast_enabled("cuda"):
+    if torch.is_autocast_enabled("cuda") or torch.jit.is_tracing():
         return UnwindowMatmulFunc.apply(inp, other, window_size)
     return _native.unwindow_matmul(inp, other, window_size)

@@ -49,3 +49,24 @@ def test_forward_mode_is_refused(device, name, columns, dtype):
 @pytest.mark.parametrize("name,columns", [("window_matmul", (N, N)), ("unwindow_matmul", (2 * W + 1, N)), ("band_softmax", (2 * W + 1,))])
 def test_forward_mode_is_refused_before_anything_else(name, columns):
     refuses_tangents(name, columns, torch.float32, "cpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,columns,dtype", OPS, ids=IDS)
+def test_traced_calls_replay(device, name, columns, dtype):
+    """A trace holds the operation and not only the allocation of its result: other inputs give other results, with
+    and without a graph, and gradients flow through the replay."""
+    fn = call(name, dtype)
+    for needs_grad in (False, True):
+        first = [x.requires_grad_(needs_grad) for x in operands(columns, dtype, device)]
+        traced = torch.jit.trace(lambda *xs: fn(*xs) + 0, tuple(first), check_trace=False)
+        for factor in (1.0, 0.5):
+            xs = [(x.detach() * factor).requires_grad_(needs_grad) for x in first]
+            torch.empty(1 << 20, device=device).fill_(float("nan"))  # what a fresh allocation may find
+            got, want = traced(*xs), fn(*xs)
+            assert torch.equal(got, want)
+            if needs_grad:
+                grad = torch.ones_like(want)
+                for a, b in zip(torch.autograd.grad(got, xs, grad), torch.autograd.grad(want, xs, grad)):
+                    # float32 attention is traced as the chain of the separate ops: the same sums in another order
+                    assert torch.equal(a, b) if dtype != torch.float32 else torch.allclose(a, b, rtol=1e-4, atol=1e-5)
