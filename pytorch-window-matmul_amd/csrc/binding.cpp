@@ -543,12 +543,12 @@ struct SavingNode : torch::autograd::Node {
     for (auto &s : saved) t.push_back(s.unpack(shared_from_this()));
     return t;
   }
-  // The gradients of the inputs, for a defined gradient of the output.
+  // The gradients of the inputs.
   virtual variable_list gradients(const std::vector<torch::Tensor> &saved_tensors, const torch::Tensor &grad) = 0;
   variable_list apply(variable_list &&grads) override {
-    if (!grads[0].defined()) return variable_list(num_outputs());
     at::NoGradGuard no_grad;  // no second derivative
-    return gradients(unpack(), grads[0]);
+    // an undefined gradient of the result counts as zeros, so that the inputs get zeros and not nothing
+    return gradients(unpack(), grads[0].defined() ? grads[0] : input_metadata(0).zeros_like());
   }
 };
 

@@ -70,3 +70,22 @@ def test_traced_calls_replay(device, name, columns, dtype):
                 for a, b in zip(torch.autograd.grad(got, xs, grad), torch.autograd.grad(want, xs, grad)):
                     # float32 attention is traced as the chain of the separate ops: the same sums in another order
                     assert torch.equal(a, b) if dtype != torch.float32 else torch.allclose(a, b, rtol=1e-4, atol=1e-5)
+
+
+class StopsGradients(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,columns,dtype", OPS, ids=IDS)
+def test_an_undefined_gradient_counts_as_zeros(device, name, columns, dtype):
+    xs = [x.requires_grad_(True) for x in operands(columns, dtype, device)]
+    StopsGradients.apply(call(name, dtype)(*xs)).sum().backward()
+    for x in xs:
+        assert x.grad is not None and x.grad.shape == x.shape and not x.grad.any()
