@@ -20,9 +20,8 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
-#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_cpp_function.h>
-#include <torch/csrc/autograd/saved_variable.h>
 
 #include <tuple>
 
@@ -523,155 +522,112 @@ window_attention_backward(torch::Tensor q, torch::Tensor k, torch::Tensor v, tor
   return std::make_tuple(gq, gk, gv);
 }
 
-// Differentiable forms of the functions above.  The public functions of the package call these: an autograd node in
+// Differentiable forms of the functions above.  The public functions of the package call these: an autograd.Function in
 // Python costs 20-30 us of host time per call and direction, which a small problem cannot hide (a training
-// step of the fused attention at B 7, M 3001 keeps the GPU busy for 33 us).  The nodes carry the names of the Python
-// classes they stand in for.
-using torch::autograd::SavedVariable;
+// step of the fused attention at B 7, M 3001 keeps the GPU busy for 33 us).  They are torch's own C++ Functions, so that
+// saved-tensor hooks, compiled autograd, functorch's refusal and undefined gradients are dealt with as in Python; what a node
+// written by hand saves over that is 1.1 us a call.
+using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-struct SavingNode : torch::autograd::Node {
-  std::vector<SavedVariable> saved;
-  void save(const torch::Tensor &t, bool is_output = false) { saved.emplace_back(t, is_output); }
-  void release_variables() override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    for (auto &s : saved) s.reset_data();
-  }
-  std::vector<torch::Tensor> unpack() {
-    std::lock_guard<std::mutex> lock(mutex_);
-    std::vector<torch::Tensor> t;
-    for (auto &s : saved) t.push_back(s.unpack(shared_from_this()));
-    return t;
-  }
-  // The gradients of the inputs.
-  virtual variable_list gradients(const std::vector<torch::Tensor> &saved_tensors, const torch::Tensor &grad) = 0;
-  variable_list apply(variable_list &&grads) override {
-    at::NoGradGuard no_grad;  // no second derivative
-    // an undefined gradient of the result counts as zeros, so that the inputs get zeros and not nothing
-    return gradients(unpack(), grads[0].defined() ? grads[0] : input_metadata(0).zeros_like());
-  }
-};
-
-// Whether a node has to be made.  There are no forward-mode derivatives: a tangent that an input carries would be
-// dropped without a trace, so such inputs are refused with the error type of an autograd.Function without a jvp.
-bool records(std::initializer_list<const torch::Tensor *> inputs) {
+// There are no forward-mode derivatives: inputs that carry a tangent are refused with the error type of a Python Function
+// without a jvp.
+void refuse_tangents(std::initializer_list<const torch::Tensor *> inputs) {
   for (const auto *t : inputs)
     TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(0).defined(), "no forward-mode derivative is implemented for the banded products, "
                                 "the band softmax and the window attention");
-  if (!at::GradMode::is_enabled()) return false;
-  for (const auto *t : inputs)
-    if (t->requires_grad()) return true;
-  return false;
-}
-
-template <typename N>
-std::shared_ptr<N> make_node(const variable_list &inputs) {
-  std::shared_ptr<N> node(new N(), torch::autograd::deleteNode);
-  torch::autograd::edge_list edges;
-  for (const auto &t : inputs) edges.push_back(torch::autograd::impl::gradient_edge(t));
-  node->set_next_edges(std::move(edges));
-  return node;
 }
 
 torch::Tensor or_none(const c10::optional<torch::Tensor> &t) { return t ? *t : torch::Tensor(); }
 
-struct WindowMatmulFuncBackward : SavingNode {
-  int64_t window_size = 0;
-  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
-    auto g = window_matmul_backward(t[0], t[1], window_size, grad, task_should_compute_output(0), task_should_compute_output(1));
-    return {or_none(std::get<0>(g)), or_none(std::get<1>(g))};
+struct WindowMatmulFunc : torch::autograd::Function<WindowMatmulFunc> {
+  static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
+    ctx->saved_data["window_size"] = window_size;
+    ctx->save_for_backward({src, other});
+    at::AutoDispatchBelowADInplaceOrView below;
+    return window_matmul_forward(src, other, window_size);
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    at::NoGradGuard no_grad;  // no second derivative
+    const auto t = ctx->get_saved_variables();
+    auto g = window_matmul_backward(t[0], t[1], ctx->saved_data["window_size"].toInt(), grads[0], ctx->needs_input_grad(0),
+                                    ctx->needs_input_grad(1));
+    return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), torch::Tensor()};
   }
 };
 
 torch::Tensor window_matmul(const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
-  const bool record = records({&src, &other});
-  torch::Tensor out;
-  {
-    at::AutoDispatchBelowADInplaceOrView below;
-    out = window_matmul_forward(src, other, window_size);
-  }
-  if (record) {
-    auto node = make_node<WindowMatmulFuncBackward>({src, other});
-    node->window_size = window_size;
-    node->save(src), node->save(other);
-    torch::autograd::set_history(out, node);
-  }
-  return out;
+  refuse_tangents({&src, &other});
+  return WindowMatmulFunc::apply(src, other, window_size);
 }
 
-struct UnwindowMatmulFuncBackward : SavingNode {
-  int64_t window_size = 0;
-  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
-    auto g = unwindow_matmul_backward(t[0], t[1], window_size, grad, task_should_compute_output(0), task_should_compute_output(1));
-    return {or_none(std::get<0>(g)), or_none(std::get<1>(g))};
+struct UnwindowMatmulFunc : torch::autograd::Function<UnwindowMatmulFunc> {
+  static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
+    ctx->saved_data["window_size"] = window_size;
+    ctx->save_for_backward({src, other});
+    at::AutoDispatchBelowADInplaceOrView below;
+    return unwindow_matmul_forward(src, other, window_size);
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    at::NoGradGuard no_grad;
+    const auto t = ctx->get_saved_variables();
+    auto g = unwindow_matmul_backward(t[0], t[1], ctx->saved_data["window_size"].toInt(), grads[0], ctx->needs_input_grad(0),
+                                      ctx->needs_input_grad(1));
+    return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), torch::Tensor()};
   }
 };
 
 torch::Tensor unwindow_matmul(const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
-  const bool record = records({&src, &other});
-  torch::Tensor out;
-  {
-    at::AutoDispatchBelowADInplaceOrView below;
-    out = unwindow_matmul_forward(src, other, window_size);
-  }
-  if (record) {
-    auto node = make_node<UnwindowMatmulFuncBackward>({src, other});
-    node->window_size = window_size;
-    node->save(src), node->save(other);
-    torch::autograd::set_history(out, node);
-  }
-  return out;
+  refuse_tangents({&src, &other});
+  return UnwindowMatmulFunc::apply(src, other, window_size);
 }
 
-struct BandSoftmaxFuncBackward : SavingNode {
-  double scale = 1.0;
-  bool mask_out_of_range = false;
-  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
-    return {band_softmax_backward(t[0], grad, scale, mask_out_of_range)};
+struct BandSoftmaxFunc : torch::autograd::Function<BandSoftmaxFunc> {
+  static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &src, double scale, bool mask_out_of_range) {
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["mask_out_of_range"] = mask_out_of_range;
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto probs = band_softmax_forward(src, scale, mask_out_of_range);
+    ctx->save_for_backward({probs});
+    return probs;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    at::NoGradGuard no_grad;
+    const auto t = ctx->get_saved_variables();
+    return {band_softmax_backward(t[0], grads[0], ctx->saved_data["scale"].toDouble(), ctx->saved_data["mask_out_of_range"].toBool()),
+            torch::Tensor(), torch::Tensor()};
   }
 };
 
 torch::Tensor band_softmax(const torch::Tensor &src, double scale, bool mask_out_of_range) {
-  const bool record = records({&src});
-  torch::Tensor out;
-  {
-    at::AutoDispatchBelowADInplaceOrView below;
-    out = band_softmax_forward(src, scale, mask_out_of_range);
-  }
-  if (record) {
-    auto node = make_node<BandSoftmaxFuncBackward>({src});
-    node->scale = scale, node->mask_out_of_range = mask_out_of_range;
-    torch::autograd::set_history(out, node);
-    node->save(out, true);
-  }
-  return out;
+  refuse_tangents({&src});
+  return BandSoftmaxFunc::apply(src, scale, mask_out_of_range);
 }
 
-struct WindowAttentionFuncBackward : SavingNode {
-  int64_t window_size = 0;
-  double scale = 1.0;
-  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
-    auto g = window_attention_backward(t[0], t[1], t[2], t[3], t[4], grad, window_size, scale, task_should_compute_output(0),
-                                       task_should_compute_output(1), task_should_compute_output(2));
-    return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), or_none(std::get<2>(g))};
+struct WindowAttentionFunc : torch::autograd::Function<WindowAttentionFunc> {
+  static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v,
+                               int64_t window_size, double scale, bool mask_out_of_range) {
+    ctx->saved_data["window_size"] = window_size;
+    ctx->saved_data["scale"] = scale;
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto [out, lse] = window_attention_forward(q, k, v, window_size, scale, mask_out_of_range);
+    ctx->save_for_backward({q, k, v, out, lse});
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    at::NoGradGuard no_grad;
+    const auto t = ctx->get_saved_variables();
+    auto g = window_attention_backward(t[0], t[1], t[2], t[3], t[4], grads[0], ctx->saved_data["window_size"].toInt(),
+                                       ctx->saved_data["scale"].toDouble(), ctx->needs_input_grad(0), ctx->needs_input_grad(1),
+                                       ctx->needs_input_grad(2));
+    return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), or_none(std::get<2>(g)), torch::Tensor(), torch::Tensor(), torch::Tensor()};
   }
 };
 
 torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v, int64_t window_size,
                                double scale, bool mask_out_of_range) {
-  const bool record = records({&q, &k, &v});
-  torch::Tensor out, lse;
-  {
-    at::AutoDispatchBelowADInplaceOrView below;
-    std::tie(out, lse) = window_attention_forward(q, k, v, window_size, scale, mask_out_of_range);
-  }
-  if (record) {
-    auto node = make_node<WindowAttentionFuncBackward>({q, k, v});
-    node->window_size = window_size, node->scale = scale;
-    torch::autograd::set_history(out, node);
-    node->save(q), node->save(k), node->save(v), node->save(out, true), node->save(lse);
-  }
-  return out;
+  refuse_tangents({&q, &k, &v});
+  return WindowAttentionFunc::apply(q, k, v, window_size, scale, mask_out_of_range);
 }
 
 // Window attention in float32, where the recomputing kernels would need three times the matrix work: the separate ops
@@ -701,20 +657,34 @@ torch::Tensor score_gradient(const torch::Tensor &probs, const torch::Tensor &v,
   return gs;
 }
 
-struct WindowAttentionF32FuncBackward : SavingNode {
-  int64_t window_size = 0;
-  double scale = 1.0;
-  bool mask_out_of_range = false;
-  variable_list gradients(const std::vector<torch::Tensor> &t, const torch::Tensor &grad) override {
-    const auto &q = t[0], &k = t[1], &v = t[2], &probs = t[3], &out = t[4];
-    const bool need_q = task_should_compute_output(0), need_k = task_should_compute_output(1), need_v = task_should_compute_output(2);
+struct WindowAttentionF32Func : torch::autograd::Function<WindowAttentionF32Func> {
+  static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v,
+                               int64_t window_size, double scale, bool mask_out_of_range) {
+    check_attention_inputs(q, k, v);
+    ctx->saved_data["window_size"] = window_size;
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["mask_out_of_range"] = mask_out_of_range;
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto probs = band_softmax_forward(window_matmul_forward(q, k.transpose(-1, -2), window_size), scale, mask_out_of_range);
+    auto out = unwindow_matmul_forward(probs, v, window_size);
+    ctx->save_for_backward({q, k, v, probs, out});
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    at::NoGradGuard no_grad;
+    const auto t = ctx->get_saved_variables();
+    const auto &q = t[0], &k = t[1], &v = t[2], &probs = t[3], &out = t[4], &grad = grads[0];
+    const int64_t window_size = ctx->saved_data["window_size"].toInt();
+    const double scale = ctx->saved_data["scale"].toDouble();
+    const bool need_q = ctx->needs_input_grad(0), need_k = ctx->needs_input_grad(1), need_v = ctx->needs_input_grad(2);
     check_grad(grad, v, v.size(-1));
-    variable_list g(3);
+    variable_list g(6);
     if (need_v) g[2] = or_none(std::get<1>(unwindow_matmul_backward(probs, v, window_size, grad, false, true)));
     if (!need_q && !need_k) return g;
     auto gs = score_gradient(probs, v, out, grad, window_size, scale);
     if (!gs.defined())
-      gs = band_softmax_backward(probs, *std::get<0>(unwindow_matmul_backward(probs, v, window_size, grad, true, false)), scale, mask_out_of_range);
+      gs = band_softmax_backward(probs, *std::get<0>(unwindow_matmul_backward(probs, v, window_size, grad, true, false)), scale,
+                                 ctx->saved_data["mask_out_of_range"].toBool());
     auto qk = window_matmul_backward(q, k.transpose(-1, -2), window_size, gs, need_q, need_k);
     if (need_q) g[0] = *std::get<0>(qk);
     if (need_k) g[1] = std::get<1>(qk)->transpose(-1, -2);
@@ -724,30 +694,17 @@ struct WindowAttentionF32FuncBackward : SavingNode {
 
 torch::Tensor window_attention_f32(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v, int64_t window_size,
                                    double scale, bool mask_out_of_range) {
-  const bool record = records({&q, &k, &v});
-  check_attention_inputs(q, k, v);
-  torch::Tensor out, probs;
-  {
-    at::AutoDispatchBelowADInplaceOrView below;
-    probs = band_softmax_forward(window_matmul_forward(q, k.transpose(-1, -2), window_size), scale, mask_out_of_range);
-    out = unwindow_matmul_forward(probs, v, window_size);
-  }
-  if (record) {
-    auto node = make_node<WindowAttentionF32FuncBackward>({q, k, v});
-    node->window_size = window_size, node->scale = scale, node->mask_out_of_range = mask_out_of_range;
-    torch::autograd::set_history(out, node);
-    node->save(q), node->save(k), node->save(v), node->save(probs), node->save(out, true);
-  }
-  return out;
+  refuse_tangents({&q, &k, &v});
+  return WindowAttentionF32Func::apply(q, k, v, window_size, scale, mask_out_of_range);
 }
 
-// What Python shows as the grad_fn of a result: an object of a class with the node's name.
-template <typename N>
+// What Python shows as the grad_fn of a result: an object of a class of this name.
+template <typename Func>
 void name_node(const char *name) {
   using namespace torch::autograd;
   static PyTypeObject type;
   TORCH_CHECK(_initFunctionPyTypeObject(type, name, nullptr, nullptr) != nullptr, "no Python type for ", name);
-  registerCppFunction(typeid(N), &type);
+  registerCppFunction(typeid(CppNode<Func>), &type);
 }
 
 }  // namespace
@@ -781,11 +738,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("lse"), py::arg("grad_output"),
         py::arg("window_size"), py::arg("scale"), py::arg("need_q") = true, py::arg("need_k") = true,
         py::arg("need_v") = true);
-  name_node<WindowMatmulFuncBackward>("WindowMatmulFuncBackward");
-  name_node<UnwindowMatmulFuncBackward>("UnwindowMatmulFuncBackward");
-  name_node<BandSoftmaxFuncBackward>("BandSoftmaxFuncBackward");
-  name_node<WindowAttentionFuncBackward>("WindowAttentionFuncBackward");
-  name_node<WindowAttentionF32FuncBackward>("WindowAttentionF32FuncBackward");
+  name_node<WindowMatmulFunc>("WindowMatmulFuncBackward");
+  name_node<UnwindowMatmulFunc>("UnwindowMatmulFuncBackward");
+  name_node<BandSoftmaxFunc>("BandSoftmaxFuncBackward");
+  name_node<WindowAttentionFunc>("WindowAttentionFuncBackward");
+  name_node<WindowAttentionF32Func>("WindowAttentionF32FuncBackward");
   m.def("window_attention_f32_supported", &window_attention_f32_supported, "whether window_attention_f32 covers q", py::arg("q"),
         py::arg("window_size"), py::arg("scale"));
   m.def("window_attention_f32", torch::wrap_pybind_function(window_attention_f32), "window attention in float32, differentiable", py::arg("q"), py::arg("k"),

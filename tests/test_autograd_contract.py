@@ -89,3 +89,60 @@ def test_an_undefined_gradient_counts_as_zeros(device, name, columns, dtype):
     StopsGradients.apply(call(name, dtype)(*xs)).sum().backward()
     for x in xs:
         assert x.grad is not None and x.grad.shape == x.shape and not x.grad.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,columns,dtype", OPS, ids=IDS)
+def test_compiled_autograd(device, name, columns, dtype):
+    fn = call(name, dtype)
+    eager, compiled = ([x.requires_grad_(True) for x in operands(columns, dtype, device)] for _ in range(2))
+    fn(*eager).sum().backward()
+    out = fn(*compiled).sum()
+    torch._dynamo.reset()
+    with torch._dynamo.compiled_autograd._enable(torch.compile(backend="eager")):
+        out.backward()
+    for x, y in zip(eager, compiled):
+        assert torch.equal(x.grad, y.grad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,columns,dtype", OPS, ids=IDS)
+def test_saved_tensor_hooks_and_checkpoints(device, name, columns, dtype):
+    """Everything the backward reads goes through the hooks, their errors arrive as they are, and a checkpoint, which
+    stops its second forward from inside a hook, gives the gradients of the plain call."""
+    from torch.utils.checkpoint import checkpoint
+
+    fn = call(name, dtype)
+    xs, ys = ([x.requires_grad_(True) for x in operands(columns, dtype, device)] for _ in range(2))
+    fn(*xs).sum().backward()
+    with torch.autograd.graph.save_on_cpu():
+        out = fn(*ys)
+    out.sum().backward()
+    assert all(torch.equal(x.grad, y.grad) for x, y in zip(xs, ys))
+    for y in ys:
+        y.grad = None
+    checkpoint(fn, *ys, use_reentrant=False).sum().backward()
+    assert all(torch.equal(x.grad, y.grad) for x, y in zip(xs, ys))
+
+    def refuse(t):
+        raise KeyError("from the hook")
+
+    with torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t), pytest.raises(KeyError, match="from the hook"):
+        fn(*ys)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,columns,dtype", OPS, ids=IDS)
+def test_backward_on_a_side_stream(device, name, columns, dtype):
+    """The backward runs on the stream of its forward whatever stream calls for it, and its inputs stay alive for it."""
+    fn = call(name, dtype)
+    xs, ys = ([x.requires_grad_(True) for x in operands(columns, dtype, device)] for _ in range(2))
+    fn(*xs).sum().backward()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        out = fn(*ys).sum()
+    out.backward()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    assert all(torch.equal(x.grad, y.grad) for x, y in zip(xs, ys))
