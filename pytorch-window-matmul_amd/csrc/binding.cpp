@@ -540,6 +540,23 @@ void refuse_tangents(std::initializer_list<const torch::Tensor *> inputs) {
 
 torch::Tensor or_none(const c10::optional<torch::Tensor> &t) { return t ? *t : torch::Tensor(); }
 
+// A result that the backward reads although the caller may change it in place: what is kept has a version counter of its own,
+// and a tensor of no elements that shares the result's counter tells the backward whether the values are still those.
+torch::Tensor keep_changeable(AutogradContext *ctx, const torch::Tensor &out) {
+  if (!out.is_inference()) {
+    auto counter = torch::empty({0});
+    torch::autograd::impl::set_version_counter(counter, torch::autograd::impl::version_counter(out));
+    ctx->saved_data["counter"] = counter;
+    ctx->saved_data["version"] = static_cast<int64_t>(out._version());
+  }
+  return out.variable_data();
+}
+bool changed_since(AutogradContext *ctx) {
+  const auto counter = ctx->saved_data.find("counter");
+  return counter != ctx->saved_data.end() &&
+         static_cast<int64_t>(counter->second.toTensor()._version()) != ctx->saved_data["version"].toInt();
+}
+
 struct WindowMatmulFunc : torch::autograd::Function<WindowMatmulFunc> {
   static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
     ctx->saved_data["window_size"] = window_size;
@@ -609,17 +626,23 @@ struct WindowAttentionFunc : torch::autograd::Function<WindowAttentionFunc> {
                                int64_t window_size, double scale, bool mask_out_of_range) {
     ctx->saved_data["window_size"] = window_size;
     ctx->saved_data["scale"] = scale;
+    ctx->saved_data["mask_out_of_range"] = mask_out_of_range;
     at::AutoDispatchBelowADInplaceOrView below;
     auto [out, lse] = window_attention_forward(q, k, v, window_size, scale, mask_out_of_range);
-    ctx->save_for_backward({q, k, v, out, lse});
+    // The separate ops keep nothing of their last result, so it may be changed in place before the backward.  At the widths
+    // that ran through them until these kernels took rows of any width, that holds on.
+    ctx->save_for_backward({q, k, v, ragged_width(q) ? keep_changeable(ctx, out) : out, lse});
     return out;
   }
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     at::NoGradGuard no_grad;
-    const auto t = ctx->get_saved_variables();
-    auto g = window_attention_backward(t[0], t[1], t[2], t[3], t[4], grads[0], ctx->saved_data["window_size"].toInt(),
-                                       ctx->saved_data["scale"].toDouble(), ctx->needs_input_grad(0), ctx->needs_input_grad(1),
-                                       ctx->needs_input_grad(2));
+    auto t = ctx->get_saved_variables();
+    const int64_t window_size = ctx->saved_data["window_size"].toInt();
+    const double scale = ctx->saved_data["scale"].toDouble();
+    if (changed_since(ctx))  // made again, bit for bit
+      std::tie(t[3], t[4]) = window_attention_forward(t[0], t[1], t[2], window_size, scale, ctx->saved_data["mask_out_of_range"].toBool());
+    auto g = window_attention_backward(t[0], t[1], t[2], t[3], t[4], grads[0], window_size, scale, ctx->needs_input_grad(0),
+                                       ctx->needs_input_grad(1), ctx->needs_input_grad(2));
     return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), or_none(std::get<2>(g)), torch::Tensor(), torch::Tensor(), torch::Tensor()};
   }
 };
@@ -667,13 +690,13 @@ struct WindowAttentionF32Func : torch::autograd::Function<WindowAttentionF32Func
     at::AutoDispatchBelowADInplaceOrView below;
     auto probs = band_softmax_forward(window_matmul_forward(q, k.transpose(-1, -2), window_size), scale, mask_out_of_range);
     auto out = unwindow_matmul_forward(probs, v, window_size);
-    ctx->save_for_backward({q, k, v, probs, out});
+    ctx->save_for_backward({q, k, v, probs, keep_changeable(ctx, out)});
     return out;
   }
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     at::NoGradGuard no_grad;
     const auto t = ctx->get_saved_variables();
-    const auto &q = t[0], &k = t[1], &v = t[2], &probs = t[3], &out = t[4], &grad = grads[0];
+    const auto &q = t[0], &k = t[1], &v = t[2], &probs = t[3], &grad = grads[0];
     const int64_t window_size = ctx->saved_data["window_size"].toInt();
     const double scale = ctx->saved_data["scale"].toDouble();
     const bool need_q = ctx->needs_input_grad(0), need_k = ctx->needs_input_grad(1), need_v = ctx->needs_input_grad(2);
@@ -681,6 +704,7 @@ struct WindowAttentionF32Func : torch::autograd::Function<WindowAttentionF32Func
     variable_list g(6);
     if (need_v) g[2] = or_none(std::get<1>(unwindow_matmul_backward(probs, v, window_size, grad, false, true)));
     if (!need_q && !need_k) return g;
+    const auto out = changed_since(ctx) ? unwindow_matmul_forward(probs, v, window_size) : t[4];  // again, bit for bit
     auto gs = score_gradient(probs, v, out, grad, window_size, scale);
     if (!gs.defined())
       gs = band_softmax_backward(probs, *std::get<0>(unwindow_matmul_backward(probs, v, window_size, grad, true, false)), scale,

@@ -71,6 +71,9 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
     callers' chain exactly as they write it: neighbours that fall outside the sequence take part
     in the softmax with score 0 and add nothing to the output.  With ``True`` they are left out
     of the softmax, which is the usual definition of sliding-window attention.
+
+    The result may be changed in place before the backward (``out += residual``), except for float16 /
+    bfloat16 training whose last dimension is a multiple of 16: its backward may read the result, and then raises.
     """
     if query.shape != key.shape or query.shape != value.shape or query.dim() < 2:
         raise RuntimeError("Input mismatch")

@@ -146,3 +146,50 @@ def test_backward_on_a_side_stream(device, name, columns, dtype):
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
     assert all(torch.equal(x.grad, y.grad) for x, y in zip(xs, ys))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("compiled", [False, True], ids=["eager", "compiled"])
+@pytest.mark.parametrize("name,columns,dtype", [OPS[1], OPS[4], OPS[5]], ids=[IDS[1], IDS[4], IDS[5]])
+def test_result_changed_in_place(device, name, columns, dtype, compiled):
+    """The last result of the separate ops is not needed by their backward; the routes that took their place keep to that.
+    The same gradients bit for bit as without the change."""
+    fn = call(name, dtype)
+
+    def gradients(change):
+        xs = [x.requires_grad_(True) for x in operands(columns, dtype, device)]
+        out = fn(*xs)
+        loss = (change(out) * 1.0).sum()
+        torch._dynamo.reset()
+        if compiled:
+            with torch._dynamo.compiled_autograd._enable(torch.compile(backend="eager")):
+                loss.backward()
+        else:
+            loss.backward()
+        return [x.grad for x in xs]
+
+    plain = gradients(lambda out: out * 2)
+    for x, y in zip(plain, gradients(lambda out: out.mul_(2))):
+        assert torch.equal(x, y)
+    for x, y in zip(plain, gradients(lambda out: out.mul_(2).add_(float("inf")))):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
+def test_result_that_stays_as_it_was_given(device):
+    """float16 / bfloat16 training at multiples of 16: the backward reads the result and notices a change."""
+    name, columns, dtype = OPS[3]
+    out = call(name, dtype)(*(x.requires_grad_(True) for x in operands(columns, dtype, device)))
+    out.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("columns,dtype", [(44, torch.float16), (N, torch.float32), (N, torch.bfloat16)])
+def test_inference_mode(device, columns, dtype):
+    xs = operands((columns,) * 3, dtype, device)
+    want = call("window_attention", dtype)(*xs)
+    with torch.inference_mode():
+        got = call("window_attention", dtype)(*xs)
+    assert got.is_inference() and torch.equal(got, want)
