@@ -310,12 +310,13 @@ int wm_grouped_score_gradient(const wm_grouped_operand *grad_o, const wm_grouped
   if (!try_launch_f32_split_score_gradient(prob, vgo, vv, vo, vp, vgs, scale, &err)) return WM_ERR_UNSUPPORTED;
   return to_status(err);
 }
+
 int wm_window_attention_backward_static(const wm_operand *q, const wm_operand *k, const wm_operand *v,
                                         const wm_operand *o, const float *lse, const wm_operand *grad_o,
                                         const wm_operand *grad_q, const wm_operand *grad_k, const wm_operand *grad_v,
                                         int64_t B, int64_t M, int64_t N, int64_t w, double scale, int dtype,
                                         unsigned flags, void *stream) {
-  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (int st = check_common(B, M, N, w, dtype, flags & ~WM_FLAG_ANY_HEAD_WIDTH)) return st;
   if (B * M > (int64_t)WM_STATIC_SCRATCH_ROWS) return WM_ERR_SCRATCH_TOO_SMALL;
   if (B == 0 || M == 0) return WM_OK;
   // Every row of the workspace that the second kernel reads is written by the first one in the

@@ -21,6 +21,7 @@ NO_ALIGNED_BAND = 0x2
 NO_NARROW_BAND = 0x4
 NO_LDS_DIRECT = 0x8
 NO_SPLIT_F32 = 0x10
+ANY_HEAD_WIDTH = 0x20
 
 
 class Operand(ctypes.Structure):

@@ -46,6 +46,13 @@ def test_argument_validation_happens_on_the_host():
     assert L.wm_status_string(0) == b"ok"
 
 
+def test_both_backward_entry_points_know_the_same_flags():
+    L = abi.lib()
+    for flag, status in ((abi.ANY_HEAD_WIDTH, 0), (0x80, 4)):  # an empty problem: only the arguments are looked at
+        assert L.wm_window_attention_backward(*(None,) * 10, 0, 4, 60, 1, 1.0, 2, flag, None) == status
+        assert L.wm_window_attention_backward_static(*(None,) * 9, 0, 4, 60, 1, 1.0, 2, flag, None) == status
+
+
 def test_kernel_choice_names():
     L = abi.lib()
     assert L.wm_kernel_choice(1, 2, 128, 64, 4, 0, 1, abi.FORCE_STRIDED) == b"strided_p1"

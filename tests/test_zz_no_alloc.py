@@ -40,6 +40,18 @@ def test_static_workspace_matches_caller_workspace(device, dtype):
             assert torch.equal(g.view(torch.int16), wnt.view(torch.int16)), (name, B, M, N, w)
 
 
+@pytest.mark.parametrize("N,w", [(60, 100), (100, 20), (75, 100)])
+def test_head_widths_16_does_not_divide(device, N, w):
+    q, k, v, go = (seeded((2, 260, N), 970 + s, torch.bfloat16).to(device) for s in range(4))
+    o, lse = abi.attention_forward(q, k, v, w, 0.1, flags=abi.ANY_HEAD_WIDTH)
+    want = abi.attention_backward(q, k, v, o, lse, go, w, 0.1, flags=abi.ANY_HEAD_WIDTH)
+    got = [torch.full_like(q, float("nan")) for _ in range(3)]
+    assert abi.attention_backward_static(q, k, v, o, lse, go, *got, w, 0.1, flags=abi.ANY_HEAD_WIDTH) == 0
+    for g, wnt in zip(got, want):
+        assert torch.equal(g, wnt)
+    assert abi.attention_backward_static(q, k, v, o, lse, go, *got, w, 0.1) == abi.UNSUPPORTED  # without the flag, as ever
+
+
 def test_skipped_gradients_and_the_size_limit(device):
     B, M, N, w = 2, 300, 128, 70
     q, k, v, go = (seeded((B, M, N), 950 + s, torch.float16).to(device) for s in range(4))
