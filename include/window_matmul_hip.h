@@ -77,7 +77,8 @@ typedef struct wm_operand {
 /* Rank-3 operand whose batch has two levels, for the wm_grouped_* entry points: with heads >= 1 element
  * (b, r, c) lives at data + (b / heads)*stride_g + (b % heads)*stride_b + r*stride_r + c*stride_c, which is
  * how a (batch, M, heads * N) projection is read as batch * heads elements of (M, N) in place: stride_g =
- * M * heads * N, stride_b = N, stride_r = heads * N.  heads = 0: the plain operand in `op`. */
+ * M * heads * N, stride_b = N, stride_r = heads * N.  heads = 0: the plain operand in `op`.  heads below 0 or
+ * beyond 2^31 - 1: WM_ERR_BAD_SHAPE. */
 typedef struct wm_grouped_operand {
   wm_operand op;
   int64_t heads;

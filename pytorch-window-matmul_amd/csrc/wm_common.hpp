@@ -46,8 +46,10 @@ struct View {
 inline View make_view(const wm_operand *op) {
   return View{op->data, BatchStep{op->stride_b, 0, 0}, op->stride_r, op->stride_c};
 }
+// heads outside 0 ... 2^31 - 1 become -1, which no call accepts (common_heads).
 inline View make_view(const wm_grouped_operand *g) {
-  return View{g->op.data, BatchStep{g->op.stride_b, g->stride_g, (int)g->heads}, g->op.stride_r, g->op.stride_c};
+  const int heads = g->heads < 0 || g->heads > 0x7fffffff ? -1 : (int)g->heads;
+  return View{g->op.data, BatchStep{g->op.stride_b, g->stride_g, heads}, g->op.stride_r, g->op.stride_c};
 }
 // Same storage seen with rows and columns swapped: (B,N,M) <-> (B,M,N).
 inline View transposed(const View &v) { return View{v.data, v.sb, v.sc, v.sr}; }

@@ -83,3 +83,14 @@ def test_grouped_operands_of_a_call_share_their_heads():
     assert L.wm_grouped_window_matmul_forward(P(two), P(three), P(plain), *tail) == 2
     assert L.wm_grouped_unwindow_matmul_forward(P(plain), P(negative), P(two), *tail) == 2
     assert L.wm_grouped_window_attention_forward(P(two), P(two), P(two), P(three), None, 1, 4, 16, 1, 1.0, 0, 1, 0, None) == 2
+
+
+def test_heads_out_of_range_are_refused():
+    """64-bit counts that 32 bits would turn into another grouping (2^32 + 2: into pairs) or into none at all (2^32)."""
+    L, P = abi.lib(), ctypes.byref
+    plain = abi.Operand(ctypes.c_void_p(16), 0, 0, 0)
+    for heads in (2 ** 32 + 2, 2 ** 32, 2 ** 31, -1, -2 ** 32):
+        odd = abi.GroupedOperand(plain, heads, 0)
+        assert L.wm_grouped_window_matmul_forward(P(odd), P(odd), P(plain), 1, 4, 4, 1, 0, 0, None) == 2
+        assert L.wm_grouped_unwindow_matmul_forward(P(plain), P(odd), P(odd), 1, 4, 4, 1, 0, 0, None) == 2
+        assert L.wm_grouped_window_attention_forward(P(odd), P(odd), P(odd), P(odd), None, 1, 4, 16, 1, 1.0, 0, 1, 0, None) == 2
