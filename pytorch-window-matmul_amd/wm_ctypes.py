@@ -82,6 +82,7 @@ def lib():
                                                           ctypes.c_int, u32, vp]
         L.wm_grouped_window_attention_backward.argtypes = [G, G, G, G, vp, G, G, G, G, vp, i64, i64, i64, i64,
                                                            ctypes.c_double, ctypes.c_int, u32, vp]
+        L.wm_grouped_score_gradient.argtypes = [G, G, G, P, P, i64, i64, i64, i64, ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_window_attention_backward_static.argtypes = [P, P, P, P, vp, P, P, P, P, i64, i64, i64, i64,
                                                           ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_window_attention_supported.argtypes = [i64, i64, i64, ctypes.c_int, ctypes.c_double]
@@ -96,6 +97,12 @@ def op(t):
         return None
     assert t.dim() == 3
     return ctypes.byref(Operand(t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)))
+
+
+def grouped_op(t):
+    """Grouped operand for a rank-3 tensor, or a rank-4 one (batch, heads, rows, columns)."""
+    step, heads, group = (t.stride(0), 0, 0) if t.dim() == 3 else (t.stride(1), t.shape[1], t.stride(0))
+    return ctypes.byref(GroupedOperand(Operand(t.data_ptr(), step, t.stride(-2), t.stride(-1)), heads, group))
 
 
 def _stream():
@@ -165,6 +172,16 @@ def band_softmax_backward(p, gp, scale=1.0, mask=False, flags=0, out=None):
     _check(lib().wm_band_softmax_backward(op(p), op(gp), op(ga), B, M, W // 2, float(scale), int(mask),
                                          DTYPES[p.dtype], flags, _stream()), "wm_band_softmax_backward")
     return ga
+
+
+def score_gradient(go, v, o, probs, w, scale=1.0, flags=0):
+    """Gradient of the scores of o = unwindow(softmax(scale * scores), v) from the float32 probabilities (B,M,2w+1); go, v and
+    o are (B,M,N) or (batch,heads,M,N)."""
+    B, M, _ = probs.shape
+    gs = torch.empty_like(probs)
+    _check(lib().wm_grouped_score_gradient(grouped_op(go), grouped_op(v), grouped_op(o), op(probs), op(gs), B, M, v.shape[-1],
+                                           w, float(scale), DTYPES[probs.dtype], flags, _stream()), "wm_grouped_score_gradient")
+    return gs
 
 
 UNSUPPORTED = 7
