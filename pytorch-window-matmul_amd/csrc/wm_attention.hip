@@ -876,13 +876,11 @@ hipError_t launch_forward(const Problem &p, const View &q, const View &k, const 
     else
       WM_AT((attention_forward_narrow_kernel<T, NK, 3, false>));
   } else {
-    // the buffer loads of the LDS-direct kernel address a batch element with 32-bit byte offsets
-    const int64_t lim = 0x7fffffff;
-    // and fetch pieces at dword addresses
-    const bool fits = (p.M + 3 * AT_KC) * k.sr * 2 < lim && (p.M + 3 * AT_KC) * v.sr * 2 < lim && k.sr > 0 && v.sr > 0 &&
+    // the LDS-direct kernels request one chunk past the last and fetch pieces at dword addresses
+    const bool fits = rows_in_reach(k, p.M, 3 * AT_KC) && rows_in_reach(v, p.M, 3 * AT_KC) &&
                       (!RAG || (dword_pieces(k, p.N) && dword_pieces(v, p.N)));
     if (fits && !(p.flags & WM_FLAG_NO_LDS_DIRECT)) {
-      if (shares_pay(p.B, p.M, p.w, FS_TM)) {
+      if (shares_pay(p.B, p.M, p.w, FS_TM) && rows_in_reach(k, p.M, 2 * FS_KC) && rows_in_reach(v, p.M, 2 * FS_KC)) {
         const int nsplit = (int)((p.M + FS_TM - 1) / FS_TM);
         const auto kernel = mask ? attention_forward_split_kernel<T, NK, true> : attention_forward_split_kernel<T, NK, false>;
         if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,

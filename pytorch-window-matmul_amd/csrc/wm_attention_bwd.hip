@@ -1537,12 +1537,14 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
   typedef const uint16_t *in_t;
   typedef uint16_t *out_t;
   {
-    // the LDS-direct kernels address a batch element with 32-bit byte offsets
-    const int64_t lim = 0x7fffffff;
-    bool fits = !(p.flags & WM_FLAG_NO_LDS_DIRECT) && (p.M + 3 * AB_KC) * 4 < lim;
-    // and fetch pieces at dword addresses
-    for (const View *t : {&q, &k, &v, &go})
-      fits = fits && t->sr > 0 && (p.M + 3 * AB_KC) * t->sr * 2 < lim && (!RAG || dword_pieces(*t, p.N));
+    // the LDS-direct kernels request up to two chunks of 64 rows, the ones that share a tile out one of 128, past the last
+    // (and as many row statistics), and fetch pieces at dword addresses
+    bool fits = !(p.flags & WM_FLAG_NO_LDS_DIRECT) && (p.M + 3 * AB_KC) * 4 < 0x7fffffff;
+    bool split_fits = (p.M + 2 * BS_KC) * 4 < 0x7fffffff;
+    for (const View *t : {&q, &k, &v, &go}) {
+      fits = fits && rows_in_reach(*t, p.M, 3 * AB_KC) && (!RAG || dword_pieces(*t, p.N));
+      split_fits = split_fits && rows_in_reach(*t, p.M, 2 * BS_KC);
+    }
     if constexpr (NK <= 4) {
       // narrow windows: one kernel for all three gradients (two row blocks per wavefront up to w = 16, three up
       // to 32, four up to 48, five up to 64 where it still pays: B96 M16384 N64 w = 64: 490 against 555 us for
@@ -1583,7 +1585,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
       const auto query_split = attention_backward_query_split_kernel<T, NK>;
       const auto key_split = attention_backward_key_split_kernel<T, NK>;
       const int nq = (int)((p.M + QT::TM - 1) / QT::TM), nk = (int)((p.M + KT::TM - 1) / KT::TM);
-      if (gq.data != nullptr && shares_pay(p.B, p.M, p.w, QT::TM) && allow_lds(reinterpret_cast<const void *>(query_split), QT::BYTES))
+      if (gq.data != nullptr && split_fits && shares_pay(p.B, p.M, p.w, QT::TM) && allow_lds(reinterpret_cast<const void *>(query_split), QT::BYTES))
         hipLaunchKernelGGL(query_split, dim3((unsigned)tiled_grid(p.B, nq)), dim3(QT::THREADS), QT::BYTES, p.stream, (in_t)q.data,
                            (in_t)k.data, (in_t)v.data, (in_t)o.data, (in_t)go.data, lse, (out_t)gq.data, delta, (int)p.B,
                            (int)p.M, (int)p.w, nq, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr,
@@ -1598,7 +1600,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
                            (in_t)go.data, lse, delta, (int)p.B, (int)p.M, nblk, (int)p.N, o.sb, o.sr, go.sb, go.sr);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess || (gk.data == nullptr && gv.data == nullptr)) return err;
-      if (shares_pay(p.B, p.M, p.w, KT::TM) && allow_lds(reinterpret_cast<const void *>(key_split), KT::BYTES)) {
+      if (split_fits && shares_pay(p.B, p.M, p.w, KT::TM) && allow_lds(reinterpret_cast<const void *>(key_split), KT::BYTES)) {
         hipLaunchKernelGGL(key_split, dim3((unsigned)tiled_grid(p.B, nk)), dim3(KT::THREADS), KT::BYTES, p.stream, (in_t)q.data,
                            (in_t)k.data, (in_t)v.data, (in_t)go.data, (const float *)delta, (out_t)gk.data, (out_t)gv.data,
                            (int)p.B, (int)p.M, (int)p.w, nk, (int)p.N, (float)scale, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr,

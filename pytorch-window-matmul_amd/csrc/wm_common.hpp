@@ -204,6 +204,10 @@ inline bool fast_layout(const View &v, int dtype) {
 //   key kernel (32 rows)    N = 128 w = 256: 64 tiles 29.5 / 18.2, 128 29.1 / 29.1, 192 30 / 42;  w = 64: 64 tiles 17.7 / 14.0
 inline bool shares_pay(int64_t B, int64_t M, int64_t w, int rows) { return w >= 32 && B * ((M + rows - 1) / rows) <= 256; }
 
+// Whether 32-bit byte offsets reach `past` rows beyond the M rows of a 16-bit batch element: the kernels that load straight
+// into LDS address it so and request whole chunks up to some past the last one, each launch as many rows as its kernel says.
+inline bool rows_in_reach(const View &v, int64_t M, int64_t past) { return v.sr > 0 && (M + past) * v.sr * 2 < 0x7fffffff; }
+
 // 16-bit rows of N elements whose pieces all start on a multiple of 4 bytes, which is what loads straight into LDS need: the
 // rows themselves, and the last piece, which starts at column N - 8 (HeadWidth), so an odd N never qualifies.
 inline bool dword_pieces(const View &v, int64_t N) {

@@ -50,6 +50,24 @@ def test_shares_agree_with_oracle_and_with_large_batches(device, case, dtype):
             torch.testing.assert_close(x.float(), y[0].float(), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("M,N,w", [(100, 128, 40), (100, 64, 70)])
+def test_rows_far_apart_are_not_shared_out(device, M, N, w):
+    """Row strides at which 32-bit offsets reach the chunk past the last of the kernels that do not share, 192 rows beyond
+    the sequence, but not that of the ones that do, 256: the bits of the former."""
+    stride = (2 ** 30 // (M + 224)) // 64 * 64
+    assert (M + 192) * stride * 2 < 2 ** 31 - 1 <= (M + 256) * stride * 2
+    room = torch.empty(M * stride, dtype=torch.bfloat16, device=device)
+    host = [seeded((1, M, N), 540 + s, torch.bfloat16) for s in range(4)]
+    far = [room.as_strided((1, M, N), (M * stride, stride, 1), N * s).copy_(t) for s, t in enumerate(host)]
+    near = [t.to(device) for t in host]
+    times = 257
+    many = [x[0] for x in _run(*(t.repeat(times, 1, 1) for t in near), w, 0.1, False) if x.dim() == 3]
+    got = [x[0] for x in _run(*far, w, 0.1, False) if x.dim() == 3]
+    shared = [x[0] for x in _run(*near, w, 0.1, False) if x.dim() == 3]
+    assert all(torch.equal(x, y) for x, y in zip(got, many))
+    assert not all(torch.equal(x, y) for x, y in zip(shared, many))  # otherwise the above says nothing
+
+
 @pytest.mark.parametrize("N,w", [(60, 40), (76, 130), (127, 64)])
 def test_shares_at_widths_16_does_not_divide(device, N, w):
     from window_matmul import window_attention
