@@ -224,8 +224,8 @@ int wm_window_attention_backward_static(const wm_operand *q, const wm_operand *k
  * own copy on that status, as the PyTorch extension does. */
 int wm_key_rows(const wm_operand *k, void *rows, int64_t B, int64_t N, int64_t M, int dtype, void *stream);
 
-/* The six entry points of the products and of the fused attention with operands whose batch may have two
- * levels (wm_grouped_operand).  Same kernels, results, status codes and remaining arguments as the functions
+/* The six entry points of the products and of the fused attention, and wm_key_rows, with operands whose batch may have
+ * two levels (wm_grouped_operand).  Same kernels, results, status codes and remaining arguments as the functions
  * without `grouped` in their names.  Grouped operands of a call have the same `heads` (WM_ERR_BAD_SHAPE
  * otherwise); plain ones (heads = 0) may stand beside them.  Band operands (a, grad_a) are always plain. */
 int wm_grouped_window_matmul_forward(const wm_grouped_operand *q, const wm_grouped_operand *k,
@@ -253,6 +253,8 @@ int wm_grouped_window_attention_backward(const wm_grouped_operand *q, const wm_g
                                          const wm_grouped_operand *grad_v, float *delta, int64_t B,
                                          int64_t M, int64_t N, int64_t w, double scale, int dtype,
                                          unsigned flags, void *stream);
+
+int wm_grouped_key_rows(const wm_grouped_operand *k, void *rows, int64_t B, int64_t N, int64_t M, int dtype, void *stream);
 
 /* Gradient of the scores of o = unwindow_matmul(softmax(scale * scores), v, w) in one kernel:
  *   grad_scores = scale * probs * (window_matmul(grad_o, v^T, w) - rowsum(grad_o * o))

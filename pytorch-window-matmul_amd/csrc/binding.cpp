@@ -204,13 +204,13 @@ void *current_stream(const torch::Tensor &t) {
 torch::Tensor key_rows(const torch::Tensor &k, Heads &heads) {
   auto view = k.transpose(-2, -1);
   if (view.stride(-1) == 1 || k.stride(-1) != 1 || k.numel() == 0 || !k.is_cuda()) return vector_friendly(view, heads);
-  const int64_t es = k.element_size(), B = batch_of(k);
+  const int64_t es = k.element_size();
   int64_t step, h, group;
-  if ((es != 2 && es != 4 && es != 8) || !batch_steps(k, &step, &h, &group) || h != 0) return vector_friendly(view, heads);
+  if ((es != 2 && es != 4 && es != 8) || !batch_steps(k, &step, &h, &group)) return vector_friendly(view, heads);
   auto rows = torch::empty(view.sizes(), k.options());
-  const wm_operand src{k.data_ptr(), step, k.stride(-2), k.stride(-1)};
+  const wm_grouped_operand src = grouped(k);
   const int dtype = es == 2 ? WM_DTYPE_BF16 : es == 4 ? WM_DTYPE_F32 : WM_DTYPE_F64;  // only the element size matters
-  const int status = wm_key_rows(&src, rows.data_ptr(), B, k.size(-2), k.size(-1), dtype, current_stream(k));
+  const int status = wm_grouped_key_rows(&src, rows.data_ptr(), batch_of(k), k.size(-2), k.size(-1), dtype, current_stream(k));
   if (status == WM_ERR_UNSUPPORTED) return vector_friendly(view, heads);  // odd alignment: the general copy
   raise_on_error(status, "key rows");
   return rows;

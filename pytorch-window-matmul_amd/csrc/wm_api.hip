@@ -226,6 +226,19 @@ int attention_backward(const Op *q, const Op *k, const Op *v, const Op *o, const
   return to_status(err);
 }
 
+template <typename Op>
+int key_rows(const Op *k, void *rows, int64_t B, int64_t N, int64_t M, int dtype, void *stream) {
+  if (int st = check_common(B, M, N, 0, dtype, 0)) return st;
+  if (missing(k) || rows == nullptr) return WM_ERR_NULL_POINTER;
+  View vk = make_view(k);
+  if (!common_heads({&vk})) return WM_ERR_BAD_SHAPE;
+  if (vk.sc != 1) return WM_ERR_UNSUPPORTED;
+  hipError_t err = hipSuccess;
+  if (!try_launch_transpose(vk.data, rows, B, N, M, vk.sb, vk.sr, (int)dtype_size(dtype), static_cast<hipStream_t>(stream), &err))
+    return WM_ERR_UNSUPPORTED;
+  return to_status(err);
+}
+
 }  // namespace
 }  // namespace wm
 
@@ -328,14 +341,10 @@ int wm_window_attention_backward_static(const wm_operand *q, const wm_operand *k
 }
 
 int wm_key_rows(const wm_operand *k, void *rows, int64_t B, int64_t N, int64_t M, int dtype, void *stream) {
-  if (int st = check_common(B, M, N, 0, dtype, 0)) return st;
-  if (missing(k) || rows == nullptr) return WM_ERR_NULL_POINTER;
-  if (k->stride_c != 1) return WM_ERR_UNSUPPORTED;
-  hipError_t err = hipSuccess;
-  if (!try_launch_transpose(k->data, rows, B, N, M, make_view(k).sb, k->stride_r, (int)dtype_size(dtype),
-                            static_cast<hipStream_t>(stream), &err))
-    return WM_ERR_UNSUPPORTED;
-  return to_status(err);
+  return key_rows(k, rows, B, N, M, dtype, stream);
+}
+int wm_grouped_key_rows(const wm_grouped_operand *k, void *rows, int64_t B, int64_t N, int64_t M, int dtype, void *stream) {
+  return key_rows(k, rows, B, N, M, dtype, stream);
 }
 
 int wm_window_attention_supported(int64_t M, int64_t N, int64_t w, int dtype, double scale) {

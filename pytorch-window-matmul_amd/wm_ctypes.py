@@ -5,6 +5,7 @@ the benchmark's per-kernel timing, and as a template for bindings from other hos
 Tensors are only used as (pointer, strides) carriers; work is enqueued on torch's
 current stream."""
 import ctypes
+import math
 import os
 import re
 
@@ -87,6 +88,7 @@ def lib():
                                                           ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_window_attention_supported.argtypes = [i64, i64, i64, ctypes.c_int, ctypes.c_double]
         L.wm_key_rows.argtypes = [P, vp, i64, i64, i64, ctypes.c_int, vp]
+        L.wm_grouped_key_rows.argtypes = [G, vp, i64, i64, i64, ctypes.c_int, vp]
         _LIB = L
     return _LIB
 
@@ -124,10 +126,13 @@ def window_forward(q, k, w, flags=0, out=None):
 
 
 def key_rows(k):
-    """wm_key_rows: k (B,N,M) with unit stride along M -> contiguous key rows (B,M,N)."""
-    B, N, M = k.shape
+    """wm_key_rows: k (B,N,M), or for wm_grouped_key_rows (batch,heads,N,M), with unit stride along M -> contiguous key rows
+    (B,M,N)."""
+    *lead, N, M = k.shape
+    B = math.prod(lead)
     rows = torch.empty(B, M, N, dtype=k.dtype, device=k.device)
-    _check(lib().wm_key_rows(op(k), ctypes.c_void_p(rows.data_ptr()), B, N, M, DTYPES[k.dtype], _stream()), "wm_key_rows")
+    fn, operand = (lib().wm_key_rows, op(k)) if k.dim() == 3 else (lib().wm_grouped_key_rows, grouped_op(k))
+    _check(fn(operand, ctypes.c_void_p(rows.data_ptr()), B, N, M, DTYPES[k.dtype], _stream()), "wm_key_rows")
     return rows
 
 

@@ -74,11 +74,34 @@ def test_more_levels_and_different_groupings(device):
         assert torch.equal(got.flatten(0, 2), window_attention(flat(q), flat(kk), flat(vv), w))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, F16, BF16, F64])
+@pytest.mark.parametrize("batch,heads,N,M,w", [(3, 5, 64, 133, 20), (2, 2, 128, 64, 9), (1, 3, 16, 1000, 40), (2, 3, 80, 97, 5)])
+def test_keys_as_columns_of_a_channels_first_projection(device, dtype, batch, heads, N, M, w):
+    """(batch, heads, N, M) keys cut out of a (batch, 3 * heads * N, M) projection: two batch levels and unit stride along M,
+    made into key rows by the library's own transpose."""
+    from window_matmul import window_matmul
+
+    for pad in (0, 7):  # rows that start on a 16-byte boundary, and rows that do not
+        qkv = seeded((batch, 3 * heads, N, M + pad), 11, dtype).to(device)
+        k = qkv[:, heads:2 * heads, :, pad:]
+        want = flat(k.transpose(-1, -2))
+        assert torch.equal(abi.key_rows(k), want)
+        q = seeded((batch, heads, M, N), 12, dtype).to(device)
+        grad = seeded((batch, heads, M, 2 * w + 1), 13, dtype).to(device)
+        got = steps(lambda a, b: window_matmul(a, b, w), (q, k), grad)
+        same = steps(lambda a, b: window_matmul(a, b.transpose(-1, -2), w), (flat(q), want), flat(grad))
+        assert torch.equal(flat(got[0]), same[0]) and torch.equal(flat(got[1]), same[1])
+        assert torch.equal(flat(got[2].transpose(-1, -2)), same[2])
+
+
 def test_grouped_operands_of_a_call_share_their_heads():
     L, P = abi.lib(), ctypes.byref
     plain = abi.Operand(ctypes.c_void_p(16), 0, 0, 0)
     two, three = (abi.GroupedOperand(plain, h, 0) for h in (2, 3))
     negative = abi.GroupedOperand(plain, -1, 0)
+    assert L.wm_grouped_key_rows(P(negative), ctypes.c_void_p(16), 1, 8, 8, 2, None) == 2
+    assert L.wm_grouped_key_rows(P(two), ctypes.c_void_p(16), 1, 8, 8, 2, None) == 7  # no unit column stride
     tail = (1, 4, 4, 1, 0, 0, None)
     assert L.wm_grouped_window_matmul_forward(P(two), P(three), P(plain), *tail) == 2
     assert L.wm_grouped_unwindow_matmul_forward(P(plain), P(negative), P(two), *tail) == 2
