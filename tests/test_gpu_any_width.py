@@ -57,6 +57,22 @@ def test_step_against_oracle(device, case, dtype):
         assert got[1].stride() == views[0].stride()  # gradients are laid out like their operands
 
 
+# N, w of launches with more workgroups than any rule for few tiles admits: even widths, which take the kernels that load
+# straight into LDS in their streaming form, with chunks wholly inside the band from 2 w >= 94 + 32 on; one and two blocks
+# of 32 result columns, above N = 64 three and four
+@pytest.mark.parametrize("mask", [False, True], ids=["zero_filled", "masked"])
+@pytest.mark.parametrize("N,w", [(60, 64), (60, 100), (22, 70), (42, 130), (76, 130), (100, 90), (100, 130), (126, 40), (36, 33)])
+def test_streaming_kernels_against_oracle(device, N, w, mask):
+    host = [seeded((1, 300, N), 330 + s, BF16) for s in range(4)]
+    times = 257
+    got = _step([t.to(device).repeat(times, 1, 1) for t in host], w, mask)
+    scale = 1.0 / math.sqrt(N)
+    want_o, _ = ao.window_attention_forward(*host[:3], w, scale, mask)
+    for x, y in zip(got, [want_o, *ao.window_attention_backward(*host[:3], w, host[3], scale, mask)]):
+        assert torch.equal(x[0], x[-1]) and torch.equal(x[0], x[100])
+        close(x[:1], y)
+
+
 # B, M, N, w: narrow and wide windows, up to and above N = 64, few tiles and more than any rule for few tiles admits
 @pytest.mark.parametrize("B,M,N,w", [(2, 150, 41, 10), (2, 300, 41, 70), (2, 150, 75, 20), (2, 300, 75, 100), (1, 300, 127, 50),
                                      (270, 40, 41, 70), (270, 40, 75, 33)])

@@ -128,3 +128,48 @@ def test_one_kernel_attention_backward_on_a_long_sequence(device, shape):
         assert bool(torch.isfinite(x).all())
         torch.testing.assert_close(x[:, -1000:].float(), y[:, -1000:].float(), rtol=2e-2, atol=2e-2)
         torch.testing.assert_close(x[:, ::997].float(), y[:, ::997].float(), rtol=2e-2, atol=2e-2)
+
+
+# batch, heads, M, N, w, dtype: rows whose 32-bit byte offsets reach to the end of a batch element, and rows that are too far
+# apart for that
+@pytest.mark.parametrize("batch,heads,M,N,w,dtype", [(3, 6, 1 << 20, 128, 20, torch.bfloat16), (3, 6, 1 << 20, 128, 70, torch.float16),
+                                                     (3, 12, 1 << 20, 60, 70, torch.bfloat16), (2, 20, 1 << 20, 64, 4, torch.bfloat16),
+                                                     (2, 9, 1 << 21, 64, 40, torch.float32)])
+def test_last_head_of_a_large_projection(device, batch, heads, M, N, w, dtype):
+    """Batches of two levels: (batch, M, heads * N) projections read in place, checked at the last head of the last
+    sequence.  Which kernel takes a tensor may depend on its row stride, so not bit for bit."""
+    from window_matmul import unwindow_matmul, window_attention, window_matmul
+
+    assert batch * heads * M * N > LIMIT
+
+    def projection(seed):
+        return _rand((batch, M, heads * N), dtype, device, seed).view(batch, M, heads, N).transpose(1, 2)
+
+    q, k, v, go = (projection(s) for s in (41, 42, 43, 44))
+    if dtype != torch.float32:
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        alone = [t[-1:, -1:].contiguous().requires_grad_(True) for t in (q, k, v)]
+        for xs, grad in ((leaves, go), (alone, go[-1:, -1:].contiguous())):
+            out = window_attention(*xs, w)
+            out.backward(grad)
+            xs.append(out.detach())
+        for name, x, y in zip(("out", "grad_v", "grad_k", "grad_q"), [leaves[3]] + [t.grad for t in leaves[2::-1]],
+                              [alone[3]] + [t.grad for t in alone[2::-1]]):
+            _close(x[-1:, -1:], y, name)
+        del leaves, alone, out, xs, grad, x, y
+        torch.cuda.empty_cache()
+    if w <= 40:  # the separate ops, whose band still fits the card
+        def last(fn, *xs):
+            return fn(*xs)[-1:, -1:], fn(*(t[-1:, -1:].contiguous() for t in xs))
+
+        _close(*last(lambda a, b: window_matmul(a, b.transpose(-1, -2), w), q, k), "window_matmul")
+        a = _rand((batch, heads, M, 2 * w + 1), dtype, device, 45, 0.2)
+        _close(*last(lambda a, b: unwindow_matmul(a, b, w), a, v), "unwindow_matmul")
+        for fn, x in ((lambda a, b: window_matmul(a, b.transpose(-1, -2), w), q), (lambda a, b: unwindow_matmul(a, b, w), a)):
+            y = k.detach().requires_grad_(True)
+            y1 = k[-1:, -1:].contiguous().requires_grad_(True)
+            upstream = a if x is q else go
+            fn(x, y).backward(upstream)
+            fn(x[-1:, -1:].contiguous(), y1).backward(upstream[-1:, -1:].contiguous())
+            _close(y.grad[-1:, -1:], y1.grad, "grad of the right operand")
+    torch.cuda.empty_cache()
