@@ -541,25 +541,24 @@ void refuse_tangents(std::initializer_list<const torch::Tensor *> inputs) {
 torch::Tensor or_none(const c10::optional<torch::Tensor> &t) { return t ? *t : torch::Tensor(); }
 
 // A result that the backward reads although the caller may change it in place: what is kept has a version counter of its own,
-// and a tensor of no elements that shares the result's counter tells the backward whether the values are still those.
+// and a tensor of no elements that shares the result's counter, 0 for a fresh tensor, tells the backward whether the
+// values are still those.
 torch::Tensor keep_changeable(AutogradContext *ctx, const torch::Tensor &out) {
   if (!out.is_inference()) {
+    TORCH_INTERNAL_ASSERT(out._version() == 0);
     auto counter = torch::empty({0});
     torch::autograd::impl::set_version_counter(counter, torch::autograd::impl::version_counter(out));
-    ctx->saved_data["counter"] = counter;
-    ctx->saved_data["version"] = static_cast<int64_t>(out._version());
+    ctx->saved_data["counter"] = std::move(counter);
   }
   return out.variable_data();
 }
 bool changed_since(AutogradContext *ctx) {
   const auto counter = ctx->saved_data.find("counter");
-  return counter != ctx->saved_data.end() &&
-         static_cast<int64_t>(counter->second.toTensor()._version()) != ctx->saved_data["version"].toInt();
+  return counter != ctx->saved_data.end() && counter->second.toTensor()._version() != 0;
 }
 
 struct WindowMatmulFunc : torch::autograd::Function<WindowMatmulFunc> {
   static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
-    ctx->saved_data["window_size"] = window_size;
     ctx->save_for_backward({src, other});
     at::AutoDispatchBelowADInplaceOrView below;
     return window_matmul_forward(src, other, window_size);
@@ -567,8 +566,8 @@ struct WindowMatmulFunc : torch::autograd::Function<WindowMatmulFunc> {
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     at::NoGradGuard no_grad;  // no second derivative
     const auto t = ctx->get_saved_variables();
-    auto g = window_matmul_backward(t[0], t[1], ctx->saved_data["window_size"].toInt(), grads[0], ctx->needs_input_grad(0),
-                                    ctx->needs_input_grad(1));
+    const int64_t window_size = grads[0].size(-1) / 2;  // the band width fixes the window: W = 2w + 1
+    auto g = window_matmul_backward(t[0], t[1], window_size, grads[0], ctx->needs_input_grad(0), ctx->needs_input_grad(1));
     return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), torch::Tensor()};
   }
 };
@@ -580,7 +579,6 @@ torch::Tensor window_matmul(const torch::Tensor &src, const torch::Tensor &other
 
 struct UnwindowMatmulFunc : torch::autograd::Function<UnwindowMatmulFunc> {
   static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &src, const torch::Tensor &other, int64_t window_size) {
-    ctx->saved_data["window_size"] = window_size;
     ctx->save_for_backward({src, other});
     at::AutoDispatchBelowADInplaceOrView below;
     return unwindow_matmul_forward(src, other, window_size);
@@ -588,8 +586,7 @@ struct UnwindowMatmulFunc : torch::autograd::Function<UnwindowMatmulFunc> {
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     at::NoGradGuard no_grad;
     const auto t = ctx->get_saved_variables();
-    auto g = unwindow_matmul_backward(t[0], t[1], ctx->saved_data["window_size"].toInt(), grads[0], ctx->needs_input_grad(0),
-                                      ctx->needs_input_grad(1));
+    auto g = unwindow_matmul_backward(t[0], t[1], t[0].size(-1) / 2, grads[0], ctx->needs_input_grad(0), ctx->needs_input_grad(1));
     return {or_none(std::get<0>(g)), or_none(std::get<1>(g)), torch::Tensor()};
   }
 };

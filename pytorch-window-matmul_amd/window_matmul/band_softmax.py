@@ -13,6 +13,8 @@ import torch
 
 import window_matmul_kernel as _native
 
+from .window_matmul import _tracing
+
 
 class BandSoftmaxFunc(torch.autograd.Function):
     """``softmax(scale * inp, dim=-1)`` on a band ``(..., M, 2w+1)``; saves only the result.  What
@@ -45,6 +47,6 @@ def band_softmax(inp: torch.Tensor, scale: Optional[float] = None, mask_out_of_r
     if inp.dim() < 2 or inp.shape[-1] % 2 != 1:
         raise RuntimeError("Input mismatch")
     scale = 1.0 if scale is None else float(scale)
-    if torch.jit.is_tracing():
+    if _tracing():
         return BandSoftmaxFunc.apply(inp, scale, bool(mask_out_of_range))
     return _native.band_softmax(inp, scale, bool(mask_out_of_range))

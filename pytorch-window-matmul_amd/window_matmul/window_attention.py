@@ -16,7 +16,7 @@ import torch
 import window_matmul_kernel as _native
 
 from .band_softmax import band_softmax
-from .window_matmul import unwindow_matmul, window_matmul
+from .window_matmul import _tracing, unwindow_matmul, window_matmul
 
 
 # tensors below this many elements: the step is bound by the host's launches, of which the fused path has fewer
@@ -86,7 +86,7 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
     # With a very narrow band the recomputing backward of the fused kernels costs more than the
     # band it avoids writing, so training there goes through the separate ops.
     training = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
-    autocast, tracing = torch.is_autocast_enabled("cuda"), torch.jit.is_tracing()
+    autocast, tracing = torch.is_autocast_enabled("cuda"), _tracing()
     # Head widths that 16 does not divide: the chain computes in float16 inside an autocast region, so it stays there.
     if _native.window_attention_supported(query, window_size, scale, not autocast) and not (
             training and _chain_is_faster(window_size, query.shape[-1], query.numel())):

@@ -23,6 +23,7 @@ import window_matmul_kernel as _native
 # only the allocation of its result, and the native module's own autograd nodes everywhere else.
 _amp_forward = torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.float16)
 _amp_backward = torch.amp.custom_bwd(device_type="cuda")
+_tracing = torch._C._is_tracing  # what torch.jit.is_tracing asks, in a quarter of its time (0.4 us a call)
 
 
 class WindowMatmulFunc(torch.autograd.Function):
@@ -90,7 +91,7 @@ def window_matmul(inp: torch.Tensor, other: torch.Tensor, window_size: Optional[
     seq_len, hidden_dim = inp.shape[-2:]
     if other.shape[-2:] != (hidden_dim, seq_len):  # reshaped to the keys' shape like the reference does
         other = other.reshape(-1, hidden_dim, seq_len)
-    if torch.is_autocast_enabled("cuda") or torch.jit.is_tracing():
+    if torch.is_autocast_enabled("cuda") or _tracing():
         return WindowMatmulFunc.apply(inp, other, window_size)
     return _native.window_matmul(inp, other, window_size)
 
@@ -107,6 +108,6 @@ def unwindow_matmul(inp: torch.Tensor, other: torch.Tensor, window_size: Optiona
     band_shape = (other.shape[-2], 2 * window_size + 1)
     if inp.shape[-2:] != band_shape:
         inp = inp.reshape(-1, *band_shape)
-    if torch.is_autocast_enabled("cuda") or torch.jit.is_tracing():
+    if torch.is_autocast_enabled("cuda") or _tracing():
         return UnwindowMatmulFunc.apply(inp, other, window_size)
     return _native.unwindow_matmul(inp, other, window_size)
