@@ -2,10 +2,11 @@
 // reference's native module exports (reference csrc/window_matmul/window_matmul.cpp:100-106),
 // implemented as a thin layer over the C ABI in include/window_matmul_hip.h.
 //
-// What this layer does, and nothing more: argument checks with the reference's error
+// What this layer does: argument checks with the reference's error
 // texts (reference cuda/utils.cuh:3-4, cuda/window_matmul_cuda.cu:226-232, 323-329),
 // layout normalisation, output allocation with the input's dtype and device, device
-// guard, current-stream lookup, and the call into libwindow_matmul_hip.so.
+// guard, current-stream lookup, and the call into libwindow_matmul_hip.so; and, in its second half, the
+// differentiable forms of these functions, which the Python package calls.
 //
 // There is deliberately no CPU implementation behind this module: tensors that do not
 // live on the GPU raise, as the reference does for GPU tensors in a CPU-only build
@@ -200,7 +201,8 @@ void *current_stream(const torch::Tensor &t) {
 // transposed view of a row-major (...,M,N) tensor already is; anything else is
 // copied into that layout once (the reference always copies: cuda:236).
 // A tensor that is laid out as (B,N,M) with unit stride along M goes through the library's own
-// transpose (one read and one write at memory speed; a general strided copy reaches a quarter of that).
+// transpose (one read and one write at memory speed; a general strided copy reaches a quarter of that), with one level of
+// batch strides or two.
 torch::Tensor key_rows(const torch::Tensor &k, Heads &heads) {
   auto view = k.transpose(-2, -1);
   if (view.stride(-1) == 1 || k.stride(-1) != 1 || k.numel() == 0 || !k.is_cuda()) return vector_friendly(view, heads);
@@ -526,7 +528,7 @@ window_attention_backward(torch::Tensor q, torch::Tensor k, torch::Tensor v, tor
 // Python costs 20-30 us of host time per call and direction, which a small problem cannot hide (a training
 // step of the fused attention at B 7, M 3001 keeps the GPU busy for 33 us).  They are torch's own C++ Functions, so that
 // saved-tensor hooks, compiled autograd, functorch's refusal and undefined gradients are dealt with as in Python; what a node
-// written by hand saves over that is 1.1 us a call.
+// written by hand saves over that is about 1 us a call.
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
@@ -661,7 +663,7 @@ bool window_attention_f32_supported(const torch::Tensor &q, int64_t window_size,
          q.size(-1) % 8 == 0 && window_size >= 128 && window_size <= (1 << 28) && scale == scale && q.numel() > 0;
 }
 
-// An undefined result: the kernel does not take these layouts.
+// An undefined result: the kernel does not take the problem (more workgroups than a launch can have; layouts are made to fit).
 torch::Tensor score_gradient(const torch::Tensor &probs, const torch::Tensor &v, const torch::Tensor &o, const torch::Tensor &grad_output,
                              int64_t window_size, double scale) {
   at::hip::HIPGuardMasqueradingAsCUDA guard(v.device());

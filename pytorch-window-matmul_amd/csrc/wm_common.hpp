@@ -166,7 +166,7 @@ bool try_launch_attention_backward_ragged(const Problem &p, const View &q, const
                                           const View &gk, const View &gv, double scale, hipError_t *err);
 
 // Backward of the fused attention (wm_attention_bwd.hip): two kernels on p.stream; `delta` is a
-// float32 (B,M) workspace the first one fills and the second one reads.
+// float32 (2,B,M) workspace the first one fills and the second one reads (-D and the log-sum-exp in log2 units).
 bool try_launch_attention_backward(const Problem &p, const View &q, const View &k, const View &v, const View &o,
                                    const View &go, const float *lse, float *delta, const View &gq, const View &gk,
                                    const View &gv, double scale, hipError_t *err);
@@ -196,8 +196,8 @@ inline bool fast_layout(const View &v, int dtype) {
 }
 
 // The fused attention kernels that share the streamed side of a tile out among wavefronts (workgroups of `rows` rows)
-// are taken while all their workgroups start at once, one on a CU: up to there they are faster at every window from
-// 32 on, beyond it the second round makes them slower.  us without / with, tiles of 128 rows in the launch:
+// are taken while all their workgroups start at once, one on a CU: up to there they are faster at the windows from
+// 32 on, or as fast (the key kernel at exactly 256 workgroups), beyond it the second round makes them slower.  us without / with, tiles of 128 rows in the launch:
 //   forward (64 rows)       N = 128 w = 1024: 64 tiles 45 / 25, 128 46 / 27, 192 46 / 47;  w = 256: 128 tiles 18 / 13, 192 18.7 / 23.7
 //                           N = 64 w = 256: 128 tiles 12.5 / 9.4, 192 12.6 / 13.2;  w = 64: 128 tiles 8.0 / 7.2
 //   query kernel (64 rows)  N = 128 w = 256: 128 tiles 23.8 / 18.2, 192 26 / 33;  w = 64: 14.2 / 13.5;  N = 96 w = 20: 9.1 / 9.8

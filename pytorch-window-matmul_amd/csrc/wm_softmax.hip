@@ -142,8 +142,8 @@ __device__ __forceinline__ void softmax_row_forward_regs(const T *x, T *out, int
 }
 
 // The same for the longest rows (more than kMaxShortSlots elements per lane), with the arithmetic of the re-reading variant
-// below that they took before: arguments of the exponential in one rounding, the sum divided by, not multiplied with an
-// approximate reciprocal.  The row is read once and exponentiated once, not three times and twice.
+// below that they took before: arguments of the exponential in one rounding, values multiplied by the correctly
+// rounded reciprocal of the sum where the rows above take the hardware's approximate one.  The row is read once and exponentiated once, not three times and twice.
 template <typename T, bool MASK, int LANES, int SLOTS, int FULL>
 __device__ __forceinline__ void softmax_row_forward_long(const T *x, T *out, int W, int lo, int hi, int gl, float c) {
   float v[SLOTS];

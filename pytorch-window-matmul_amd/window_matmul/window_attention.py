@@ -19,22 +19,23 @@ from .band_softmax import band_softmax
 from .window_matmul import _tracing, unwindow_matmul, window_matmul
 
 
-# tensors below this many elements: the step is bound by the host's launches, of which the fused path has fewer
+# tensors below this many elements take the fused kernels: most of them are bound by the host's launches, of which those need fewer
 _HOST_BOUND_ELEMENTS = 32 << 20
 
 
 def _chain_is_faster(window_size: int, width: int, elements: int) -> bool:
     """Whether a training step is faster through the separate ops than through the fused kernels.
-    Up to N = 64 the fused backward is one kernel at narrow windows and the fused step wins or ties at
-    every window (N = 16, 32 at w <= 2: 0.67 / 0.69 and 0.48 / 0.48 ms, chain / fused, on 100 M elements:
-    a tie, left to the fused kernels).  Above N = 64 the recomputing two-kernel backward costs the same
-    at every narrow window, and the chain wins up to w = 32 at N = 128 (B16 M32768: 0.374 / 0.535 ms at
-    w = 4, 0.510 / 0.543 at w = 32, 0.588 / 0.580 at w = 36; B96 M4096: 0.378 / 0.395 at w = 32, 0.435 /
-    0.426 at w = 36) and up to about w = 24 at N = 96 (B96 M4096: 0.251 / 0.294 at w = 16, 0.332 / 0.308 at
-    w = 32).  Small problems are bound by the host, which issues seven launches for the chain and three
-    for the fused step: at B7 M3001 the chain takes 0.21 ms and the fused step 0.085-0.09 ms whatever the
-    window and head width, so below about 32 M elements per tensor the fused kernels are always taken.  Widths that 16 does not
-    divide always are: the separate ops pad every operand there (B4x12 M16384, chain / fused: 1271 / 806 us at N = 75,
+    Up to N = 64 the fused backward is one kernel at narrow windows and the fused step wins or nearly ties at
+    every window (chain / fused on 100 M elements, us: N = 16 650 / 691 at w = 1 and 687 / 693 at w = 2, N = 32
+    465 / 478 and 479 / 482).  Above N = 64 the recomputing two-kernel backward costs the same
+    at every narrow window, and the chain wins up to w = 32 at N = 128 (B16 M32768: 356 / 535 at
+    w = 4, 506 / 548 at w = 32, 597 / 583 at w = 40; B96 M4096: 372 / 396 at w = 32, 430 / 424 at w = 36, as
+    (8, 12) projection views 388 / 422 at w = 32) and up to about w = 24 at N = 96 (B96 M4096: 303 / 305 at w = 24, 328 / 304 at
+    w = 32; N = 80 232 / 252 at w = 16, 288 / 272 at w = 24).  Small problems are bound by the host, which issues seven
+    launches for the chain and three for the fused step: at B7 M3001 83-90 / 47 at N = 80 and 128, w = 4 and 24, so below
+    about 32 M elements per tensor the fused kernels are always taken.  (At 20 M elements neither side is bound by
+    the host any more: N = 80 124 / 171 at w = 4, 207 / 183 at w = 24; N = 128 196 / 242 and 243 / 251; at 8 M 121 / 76.)
+    Widths that 16 does not divide always are: the separate ops pad every operand there (B4x12 M16384: 1271 / 806 at N = 75,
     w = 4; 1979 / 949 at N = 120, w = 4; 1015 / 368 at N = 60, w = 1)."""
     if width <= 64 or width % 16 or elements < _HOST_BOUND_ELEMENTS:
         return False

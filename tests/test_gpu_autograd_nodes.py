@@ -1,5 +1,5 @@
-"""The native autograd nodes behind the public functions: the same gradients as the Python Function classes (which the
-autocast path uses), saved tensors that are released, checked for in-place changes and kept under
+"""The native autograd nodes behind the public functions: the same gradients as the Python Function classes (which
+torch.jit.trace and, for the two products, autocast take instead), saved tensors that are released, checked for in-place changes and kept under
 retain_graph, and gradients only of the inputs that ask for one."""
 import pytest
 import torch
