@@ -193,3 +193,18 @@ def test_inference_mode(device, columns, dtype):
     with torch.inference_mode():
         got = call("window_attention", dtype)(*xs)
     assert got.is_inference() and torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,columns,dtype", OPS, ids=IDS)
+def test_compiled_callers(device, name, columns, dtype):
+    """torch.compile around a call breaks its graph there and gives the eager results and gradients."""
+    fn = call(name, dtype)
+    xs, ys = ([x.requires_grad_(True) for x in operands(columns, dtype, device)] for _ in range(2))
+    want = fn(*xs) * 2
+    torch._dynamo.reset()
+    got = torch.compile(lambda *t: fn(*t) * 2, backend="eager")(*ys)
+    assert torch.equal(got, want)
+    want.sum().backward()
+    got.sum().backward()
+    assert all(torch.equal(x.grad, y.grad) for x, y in zip(xs, ys))

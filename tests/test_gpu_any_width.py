@@ -58,10 +58,10 @@ def test_step_against_oracle(device, case, dtype):
 
 
 # N, w of launches with more workgroups than any rule for few tiles admits: even widths, which take the kernels that load
-# straight into LDS in their streaming form, with chunks wholly inside the band from 2 w >= 94 + 32 on; one and two blocks
-# of 32 result columns, above N = 64 three and four
+# straight into LDS in their streaming form, certain from w = 79 on to have chunks of 64 rows wholly inside the band of a
+# wavefront's 32; one to four blocks of 32 result columns
 @pytest.mark.parametrize("mask", [False, True], ids=["zero_filled", "masked"])
-@pytest.mark.parametrize("N,w", [(60, 64), (60, 100), (22, 70), (42, 130), (76, 130), (100, 90), (100, 130), (126, 40), (36, 33)])
+@pytest.mark.parametrize("N,w", [(60, 64), (60, 100), (14, 70), (22, 70), (42, 130), (90, 90), (76, 130), (100, 90), (100, 130), (126, 40), (36, 33)])
 def test_streaming_kernels_against_oracle(device, N, w, mask):
     host = [seeded((1, 300, N), 330 + s, BF16) for s in range(4)]
     times = 257
