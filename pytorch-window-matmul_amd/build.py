@@ -36,6 +36,11 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
+# Sources whose kernels use more than 256 registers and look at most results of the matrix instructions once per use: with the
+# results in accumulation registers, the compiler's choice there, each has to be moved (key kernel at N = 64: 206 of 821
+# instructions of a block).
+FILE_FLAGS = {"wm_attention_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+
 
 def _newer(target, sources):
     if not os.path.exists(target):
@@ -67,7 +72,7 @@ def build_hip_library(force=False):
         objs.append(obj)
         if not force and _newer(obj, [src] + headers):
             continue  # this object is still current: only stale translation units are recompiled
-        cmd = [os.path.join(ROCM, "bin", "hipcc"), *HIPCC_FLAGS, "-c", src, "-o", obj]
+        cmd = [os.path.join(ROCM, "bin", "hipcc"), *HIPCC_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
         print("+", " ".join(cmd), flush=True)
         procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     for cmd, proc in procs:

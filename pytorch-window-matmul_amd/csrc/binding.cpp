@@ -456,14 +456,18 @@ bool ragged_rows_in_place(const torch::Tensor &t) {
   int64_t step, heads, group;
   return t.stride(-1) == 1 && batch_steps(t, &step, &heads, &group);
 }
-torch::Tensor attention_operand(const torch::Tensor &t, Heads &heads) {
-  if (!ragged_width(t)) return vector_friendly(t, heads);
+torch::Tensor attention_rows(const torch::Tensor &t, Heads &heads) {  // rows of any alignment
   return ragged_rows_in_place(t) && heads.admit(t) ? t : t.contiguous();
 }
-torch::Tensor attention_gradient(const torch::Tensor &t, Heads &heads) {
-  if (!ragged_width(t)) return empty_like_rows(t, t.size(-1), heads);
+torch::Tensor attention_rows_like(const torch::Tensor &t, Heads &heads) {
   auto g = torch::empty_like(t);
   return ragged_rows_in_place(g) && heads.admit(g) ? g : torch::empty(t.sizes(), t.options());
+}
+torch::Tensor attention_operand(const torch::Tensor &t, Heads &heads) {
+  return ragged_width(t) ? attention_rows(t, heads) : vector_friendly(t, heads);
+}
+torch::Tensor attention_gradient(const torch::Tensor &t, Heads &heads) {
+  return ragged_width(t) ? attention_rows_like(t, heads) : empty_like_rows(t, t.size(-1), heads);
 }
 
 void check_attention_inputs(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v) {
@@ -652,15 +656,80 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
   return WindowAttentionFunc::apply(q, k, v, window_size, scale, mask_out_of_range);
 }
 
-// Window attention in float32, where the recomputing kernels would need three times the matrix work: the separate ops
-// forward, and a backward that forms the gradient of the scores in one kernel.
-bool window_attention_f32_supported(const torch::Tensor &q, int64_t window_size, double scale) {
-  // From w = 128 on.  A training step through the separate ops / with the fused gradient of the scores, us, B96 M4096: N = 64
+// Window attention in float32.  Two routes beside the separate ops: the fused kernels (wm_attention_f32.hip), which recompute
+// everything from q, k and v with six bf16 products for every float32 one, and for training the separate ops forward
+// with a backward that forms the gradient of the scores in one kernel, which has the band in memory.
+//
+// Fused, us of the separate ops / of the fused kernels; T is tiles of 128 rows, and the route compared with in training
+// is the better of the other two:
+//   inference  T = 3072: N = 64 117 / 122 at w = 8, 149 / 113 at w = 16, 886 / 420 at w = 256; N = 128 323 / 317 at w = 16, 1249 / 710 at
+//              256.  Few tiles leave CUs idle where the separate ops share a tile out: N = 128 T = 32 39 / 29 at w = 64, 53 / 55 at w = 256,
+//              T = 64 138 / 167 at w = 1024, T = 128 196 / 170; N = 64 T = 32 105 / 92 at w = 1024.
+//   training   N <= 64: T = 3072 536 / 569 at w = 24, 678 / 561 at w = 32, 2096 / 1456 at w = 256; T = 32 96 / 66 at w = 64, 142 / 132 at
+//              w = 256, 177 / 200 at w = 400, T = 64 346 / 420 at w = 1024, T = 128 438 / 402.
+//              N > 64: the key kernel needs the registers of a whole SIMD per wavefront: T = 3072 N = 128 1540 / 1542 at w = 64,
+//              2252 / 2085 at w = 128, 3553 / 3130 at w = 256; N = 80 1609 / 1586 and 2516 / 2420; T = 256 N = 96 w = 1000 771 / 647; T = 168
+//              N = 80 239 / 240 at w = 300, 775 / 801 at w = 1500; T = 128 N = 128 203 / 251 at w = 256.
+//              Widths that 8 does not divide, which the separate ops take to the tile kernels: T = 3072 N = 60 616 / 602
+//              at w = 16, 748 / 580 at w = 32, N = 75 5062 / 2346 at w = 256; T = 32 N = 75 216 / 216 at w = 300.
+// Below 8 tiles all routes are a handful of launches, and what a problem of that size gives, traced or not, stays as it was bit for bit.
+// An infinite operand gives NaN in both routes, as in the separate ops from w = 16 on (wm_f32_split.hip).
+bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool training) {
+  const int64_t N = q.size(-1), M = q.size(-2);
+  if (N < 8 || N > kMaxWidth || M > (1 << 30) || window_size < 16 || window_size > (1 << 28) || !(scale > 0.0 && scale < 1.0e30)) return false;
+  const int64_t tiles = q.numel() / (N * M) * ((M + 127) / 128);
+  if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && (training || N > 64))) return false;
+  if (!training) return true;
+  return N > 64 && N % 8 == 0 ? window_size >= 128 && tiles >= 256 : window_size >= 32;
+}
+
+bool window_attention_f32_supported(const torch::Tensor &q, int64_t window_size, double scale, bool training) {
+  if (q.dim() < 2 || !q.device().is_cuda() || q.scalar_type() != at::kFloat || q.numel() == 0) return false;
+  if (f32_fused(q, window_size, scale, training)) return true;
+  // The gradient of the scores in one kernel, from w = 128 on.  A training step through the separate ops / with it, us, B96 M4096: N = 64
   // 931 / 953 at w = 64, 1251 / 1257 at w = 100, 2313 / 2093 at w = 256; N = 128 1521 / 1572, 2044 / 2027, 3609 / 3438; B8 M3001
   // N = 16 191 / 174 at w = 256.  In a narrow band the pieces at its two edges, read element by element, cost more than
   // the passes that are saved (N = 80, w = 32: 802 / 880).
-  return q.dim() >= 2 && q.device().is_cuda() && q.scalar_type() == at::kFloat && q.size(-1) >= 8 && q.size(-1) <= kMaxWidth &&
-         q.size(-1) % 8 == 0 && window_size >= 128 && window_size <= (1 << 28) && scale == scale && q.numel() > 0;
+  return training && q.size(-1) >= 8 && q.size(-1) <= kMaxWidth && q.size(-1) % 8 == 0 && window_size >= 128 && window_size <= (1 << 28) &&
+         scale == scale;
+}
+
+std::tuple<torch::Tensor, torch::Tensor> f32_fused_forward(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v,
+                                                           int64_t window_size, double scale, bool mask_out_of_range, bool training) {
+  at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+  const int64_t B = batch_of(q), M = q.size(-2), N = q.size(-1);
+  Heads heads;
+  auto qq = attention_rows(q, heads), kk = attention_rows(k, heads), vv = attention_rows(v, heads);
+  auto o = torch::empty(q.sizes(), q.options());
+  auto stats = training ? torch::empty({2, B, M}, q.options()) : torch::Tensor();
+  const wm_grouped_operand oq = grouped(qq), ok = grouped(kk), ov = grouped(vv), oo = grouped(o);
+  raise_on_error(wm_grouped_window_attention_f32_forward(&oq, &ok, &ov, &oo, training ? stats.data_ptr<float>() : nullptr, B, M, N,
+                                                         window_size, scale, mask_out_of_range, WM_DTYPE_F32, 0, current_stream(q)),
+                 "window_attention_f32");
+  return std::make_tuple(o, stats);
+}
+
+variable_list f32_fused_backward(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v, const torch::Tensor &o,
+                                 const torch::Tensor &stats, const torch::Tensor &grad, int64_t window_size, double scale, bool need_q,
+                                 bool need_k, bool need_v) {
+  variable_list g(7);
+  if (!need_q && !need_k && !need_v) return g;
+  at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+  const int64_t B = batch_of(q), M = q.size(-2), N = q.size(-1);
+  Heads heads;
+  auto qq = attention_rows(q, heads), kk = attention_rows(k, heads), vv = attention_rows(v, heads), oo = attention_rows(o, heads),
+       go = attention_rows(grad, heads);
+  wm_grouped_operand x{}, y{}, z{};
+  if (need_q) g[0] = attention_rows_like(q, heads), x = grouped(g[0]);
+  if (need_k) g[1] = attention_rows_like(k, heads), y = grouped(g[1]);
+  if (need_v) g[2] = attention_rows_like(v, heads), z = grouped(g[2]);
+  auto delta = torch::empty({B, M}, q.options());
+  const wm_grouped_operand a = grouped(qq), b = grouped(kk), c = grouped(vv), d = grouped(oo), e = grouped(go);
+  raise_on_error(wm_grouped_window_attention_f32_backward(&a, &b, &c, &d, stats.data_ptr<float>(), &e, need_q ? &x : nullptr,
+                                                          need_k ? &y : nullptr, need_v ? &z : nullptr, delta.data_ptr<float>(), B, M, N,
+                                                          window_size, scale, WM_DTYPE_F32, 0, current_stream(q)),
+                 "window_attention_f32 backward");
+  return g;
 }
 
 // An undefined result: the kernel does not take the problem (more workgroups than a launch can have; layouts are made to fit).
@@ -681,12 +750,19 @@ torch::Tensor score_gradient(const torch::Tensor &probs, const torch::Tensor &v,
 
 struct WindowAttentionF32Func : torch::autograd::Function<WindowAttentionF32Func> {
   static torch::Tensor forward(AutogradContext *ctx, const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v,
-                               int64_t window_size, double scale, bool mask_out_of_range) {
+                               int64_t window_size, double scale, bool mask_out_of_range, bool training) {
     check_attention_inputs(q, k, v);
+    const bool fused = f32_fused(q, window_size, scale, training);
+    ctx->saved_data["fused"] = fused;
     ctx->saved_data["window_size"] = window_size;
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["mask_out_of_range"] = mask_out_of_range;
     at::AutoDispatchBelowADInplaceOrView below;
+    if (fused) {
+      auto [out, stats] = f32_fused_forward(q, k, v, window_size, scale, mask_out_of_range, training);
+      if (training) ctx->save_for_backward({q, k, v, stats, keep_changeable(ctx, out)});
+      return out;
+    }
     auto probs = band_softmax_forward(window_matmul_forward(q, k.transpose(-1, -2), window_size), scale, mask_out_of_range);
     auto out = unwindow_matmul_forward(probs, v, window_size);
     ctx->save_for_backward({q, k, v, probs, keep_changeable(ctx, out)});
@@ -695,19 +771,26 @@ struct WindowAttentionF32Func : torch::autograd::Function<WindowAttentionF32Func
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     at::NoGradGuard no_grad;
     const auto t = ctx->get_saved_variables();
-    const auto &q = t[0], &k = t[1], &v = t[2], &probs = t[3], &grad = grads[0];
+    const auto &q = t[0], &k = t[1], &v = t[2], &grad = grads[0];
     const int64_t window_size = ctx->saved_data["window_size"].toInt();
     const double scale = ctx->saved_data["scale"].toDouble();
+    const bool mask_out_of_range = ctx->saved_data["mask_out_of_range"].toBool();
     const bool need_q = ctx->needs_input_grad(0), need_k = ctx->needs_input_grad(1), need_v = ctx->needs_input_grad(2);
     check_grad(grad, v, v.size(-1));
-    variable_list g(6);
+    if (ctx->saved_data["fused"].toBool()) {
+      auto stats = t[3], out = t[4];
+      if (changed_since(ctx)) std::tie(out, stats) = f32_fused_forward(q, k, v, window_size, scale, mask_out_of_range, true);  // again, bit for bit
+      return f32_fused_backward(q, k, v, out, stats, grad, window_size, scale, need_q, need_k, need_v);
+    }
+    const auto &probs = t[3];
+    variable_list g(7);
     if (need_v) g[2] = or_none(std::get<1>(unwindow_matmul_backward(probs, v, window_size, grad, false, true)));
     if (!need_q && !need_k) return g;
     const auto out = changed_since(ctx) ? unwindow_matmul_forward(probs, v, window_size) : t[4];  // again, bit for bit
     auto gs = score_gradient(probs, v, out, grad, window_size, scale);
     if (!gs.defined())
       gs = band_softmax_backward(probs, *std::get<0>(unwindow_matmul_backward(probs, v, window_size, grad, true, false)), scale,
-                                 ctx->saved_data["mask_out_of_range"].toBool());
+                                 mask_out_of_range);
     auto qk = window_matmul_backward(q, k.transpose(-1, -2), window_size, gs, need_q, need_k);
     if (need_q) g[0] = *std::get<0>(qk);
     if (need_k) g[1] = std::get<1>(qk)->transpose(-1, -2);
@@ -718,7 +801,8 @@ struct WindowAttentionF32Func : torch::autograd::Function<WindowAttentionF32Func
 torch::Tensor window_attention_f32(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v, int64_t window_size,
                                    double scale, bool mask_out_of_range) {
   refuse_tangents({&q, &k, &v});
-  return WindowAttentionF32Func::apply(q, k, v, window_size, scale, mask_out_of_range);
+  const bool training = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+  return WindowAttentionF32Func::apply(q, k, v, window_size, scale, mask_out_of_range, training);
 }
 
 // What Python shows as the grad_fn of a result: an object of a class of this name.
@@ -767,7 +851,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   name_node<WindowAttentionFunc>("WindowAttentionFuncBackward");
   name_node<WindowAttentionF32Func>("WindowAttentionF32FuncBackward");
   m.def("window_attention_f32_supported", &window_attention_f32_supported, "whether window_attention_f32 covers q", py::arg("q"),
-        py::arg("window_size"), py::arg("scale"));
+        py::arg("window_size"), py::arg("scale"), py::arg("training") = true);
   m.def("window_attention_f32", torch::wrap_pybind_function(window_attention_f32), "window attention in float32, differentiable", py::arg("q"), py::arg("k"),
         py::arg("v"), py::arg("window_size"), py::arg("scale"), py::arg("mask_out_of_range"));
   m.def("window_matmul", torch::wrap_pybind_function(window_matmul), "WindowMatmul, differentiable", py::arg("src"), py::arg("other"), py::arg("window_size"));

@@ -324,6 +324,36 @@ int wm_grouped_score_gradient(const wm_grouped_operand *grad_o, const wm_grouped
   return to_status(err);
 }
 
+int wm_grouped_window_attention_f32_forward(const wm_grouped_operand *q, const wm_grouped_operand *k, const wm_grouped_operand *v, const wm_grouped_operand *o, float *stats, int64_t B, int64_t M, int64_t N, int64_t w, double scale, int mask_out_of_range, int dtype, unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
+  if (B == 0 || M == 0) return WM_OK;
+  if (missing(q) || missing(k) || missing(v) || missing(o)) return WM_ERR_NULL_POINTER;
+  const Problem prob{B, M, N, w, dtype, flags, static_cast<hipStream_t>(stream)};
+  View vq = make_view(q), vk = make_view(k), vv = make_view(v), vo = make_view(o);
+  if (!common_heads({&vq, &vk, &vv, &vo})) return WM_ERR_BAD_SHAPE;
+  hipError_t err = hipSuccess;
+  if (!try_launch_attention_f32_forward(prob, vq, vk, vv, vo, stats, scale, mask_out_of_range, &err)) return WM_ERR_UNSUPPORTED;
+  return to_status(err);
+}
+
+int wm_grouped_window_attention_f32_backward(const wm_grouped_operand *q, const wm_grouped_operand *k, const wm_grouped_operand *v, const wm_grouped_operand *o, const float *stats, const wm_grouped_operand *grad_o, const wm_grouped_operand *grad_q, const wm_grouped_operand *grad_k, const wm_grouped_operand *grad_v, float *delta, int64_t B, int64_t M, int64_t N, int64_t w, double scale, int dtype, unsigned flags, void *stream) {
+  if (int st = check_common(B, M, N, w, dtype, flags)) return st;
+  if (!(scale == scale)) return WM_ERR_BAD_SHAPE;
+  if (B == 0 || M == 0) return WM_OK;
+  if (missing(q) || missing(k) || missing(v) || missing(o) || missing(grad_o) || stats == nullptr || delta == nullptr)
+    return WM_ERR_NULL_POINTER;
+  if (grad_q == nullptr && grad_k == nullptr && grad_v == nullptr) return WM_OK;
+  if ((grad_q && missing(grad_q)) || (grad_k && missing(grad_k)) || (grad_v && missing(grad_v))) return WM_ERR_NULL_POINTER;
+  const Problem prob{B, M, N, w, dtype, flags, static_cast<hipStream_t>(stream)};
+  View vq = make_view(q), vk = make_view(k), vv = make_view(v), vo = make_view(o), vgo = make_view(grad_o),
+       vgq = view_or_none(grad_q), vgk = view_or_none(grad_k), vgv = view_or_none(grad_v);
+  if (!common_heads({&vq, &vk, &vv, &vo, &vgo, &vgq, &vgk, &vgv})) return WM_ERR_BAD_SHAPE;
+  hipError_t err = hipSuccess;
+  if (!try_launch_attention_f32_backward(prob, vq, vk, vv, vo, vgo, stats, delta, vgq, vgk, vgv, scale, &err)) return WM_ERR_UNSUPPORTED;
+  return to_status(err);
+}
+
 int wm_window_attention_backward_static(const wm_operand *q, const wm_operand *k, const wm_operand *v,
                                         const wm_operand *o, const float *lse, const wm_operand *grad_o,
                                         const wm_operand *grad_q, const wm_operand *grad_k, const wm_operand *grad_v,

@@ -171,6 +171,15 @@ bool try_launch_attention_backward(const Problem &p, const View &q, const View &
                                    const View &go, const float *lse, float *delta, const View &gq, const View &gk,
                                    const View &gv, double scale, hipError_t *err);
 
+// Fused window attention in float32 (wm_attention_f32.hip): stats is a float32 (2,B,M) buffer that the forward fills (it may be
+// null) and the backward reads, delta a float32 (B,M) workspace of the backward.
+bool attention_f32_supports(const Problem &p, double scale);
+bool try_launch_attention_f32_forward(const Problem &p, const View &q, const View &k, const View &v, const View &o, float *stats,
+                                      double scale, int mask, hipError_t *err);
+bool try_launch_attention_f32_backward(const Problem &p, const View &q, const View &k, const View &v, const View &o, const View &go,
+                                       const float *stats, float *delta, const View &gq, const View &gk, const View &gv,
+                                       double scale, hipError_t *err);
+
 // Batched transpose of the last two dimensions (wm_transpose.hip): src (B,R,C) with unit column stride and
 // batch / row strides ssb / ssr (elements), dst contiguous (B,C,R).  Returns false, nothing launched,
 // unless dst is 16-byte aligned, R is a multiple of 16 bytes and elem_size is 2, 4 or 8.

@@ -5,8 +5,8 @@ themselves (reference tests/test_attention.py:57-63).  This function is that cha
 same semantics, as an addition next to the unchanged two-function API.  For float16 /
 bfloat16 inputs whose last dimension is 8 to 128 it runs fused kernels that
 never write the ``(…, M, 2w+1)`` band to memory (forward keeps only the log-sum-exp of every
-row, backward recomputes the probabilities); everything else runs the chain of the separate
-ops of this package, on the GPU as well.
+row, backward recomputes the probabilities), and for float32 inputs of such widths kernels that do the same at
+float32 accuracy where they are faster; everything else runs the chain of the separate ops of this package, on the GPU as well.
 """
 import math
 from typing import Optional
@@ -93,7 +93,7 @@ def window_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
             training and _chain_is_faster(window_size, query.shape[-1], query.numel())):
         fused = WindowAttentionFunc.apply if tracing else _native.window_attention
         return fused(query, key, value, window_size, scale, bool(mask_out_of_range))
-    if training and not autocast and not tracing and _native.window_attention_f32_supported(query, window_size, scale):
+    if not autocast and not tracing and _native.window_attention_f32_supported(query, window_size, scale, training):
         return _native.window_attention_f32(query, key, value, window_size, scale, bool(mask_out_of_range))
     att = window_matmul(query, key.transpose(-1, -2), window_size)
     return unwindow_matmul(band_softmax(att, scale, mask_out_of_range), value, window_size)

@@ -84,6 +84,10 @@ def lib():
         L.wm_grouped_window_attention_backward.argtypes = [G, G, G, G, vp, G, G, G, G, vp, i64, i64, i64, i64,
                                                            ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_grouped_score_gradient.argtypes = [G, G, G, P, P, i64, i64, i64, i64, ctypes.c_double, ctypes.c_int, u32, vp]
+        L.wm_grouped_window_attention_f32_forward.argtypes = [G, G, G, G, vp, i64, i64, i64, i64, ctypes.c_double, ctypes.c_int,
+                                                              ctypes.c_int, u32, vp]
+        L.wm_grouped_window_attention_f32_backward.argtypes = [G, G, G, G, vp, G, G, G, G, vp, i64, i64, i64, i64,
+                                                               ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_window_attention_backward_static.argtypes = [P, P, P, P, vp, P, P, P, P, i64, i64, i64, i64,
                                                           ctypes.c_double, ctypes.c_int, u32, vp]
         L.wm_window_attention_supported.argtypes = [i64, i64, i64, ctypes.c_int, ctypes.c_double]
@@ -227,3 +231,31 @@ def attention_backward(q, k, v, o, lse, go, w, scale=1.0, flags=0, want=(True, T
                                              float(scale), DTYPES[q.dtype], flags, _stream()),
            "wm_window_attention_backward")
     return gq, gk, gv
+
+
+def _pointer(t):
+    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+
+
+def attention_f32_forward(q, k, v, w, scale=1.0, mask=False, flags=0, want_stats=True, out=None):
+    """q, k, v (B,M,N) or (batch,heads,M,N) float32 -> (o, stats (2,B,M) or None)."""
+    B, M, N = math.prod(q.shape[:-2]), q.shape[-2], q.shape[-1]
+    o = torch.empty_like(q) if out is None else out
+    stats = torch.empty(2, B, M, dtype=torch.float32, device=q.device) if want_stats else None
+    _check(lib().wm_grouped_window_attention_f32_forward(grouped_op(q), grouped_op(k), grouped_op(v), grouped_op(o), _pointer(stats),
+                                                         B, M, N, w, float(scale), int(mask), DTYPES[q.dtype], flags, _stream()),
+           "wm_grouped_window_attention_f32_forward")
+    return o, stats
+
+
+def attention_f32_backward(q, k, v, o, stats, go, w, scale=1.0, flags=0, want=(True, True, True)):
+    """Gradients (gq, gk, gv) laid out like their operands, None where not wanted."""
+    B, M, N = math.prod(q.shape[:-2]), q.shape[-2], q.shape[-1]
+    grads = [torch.empty_like(t) if x else None for t, x in zip((q, k, v), want)]
+    delta = torch.empty(B, M, dtype=torch.float32, device=q.device)
+    operands = [grouped_op(t) if t is not None else None for t in grads]
+    _check(lib().wm_grouped_window_attention_f32_backward(grouped_op(q), grouped_op(k), grouped_op(v), grouped_op(o), _pointer(stats),
+                                                          grouped_op(go), *operands, _pointer(delta), B, M, N, w, float(scale),
+                                                          DTYPES[q.dtype], flags, _stream()),
+           "wm_grouped_window_attention_f32_backward")
+    return tuple(grads)
