@@ -461,6 +461,9 @@ __global__ __launch_bounds__(kThreads) void attention_backward_stats_kernel(
 // (Three workgroups per CU up to N = 64: the kernel needs about 157 registers.  Forced into the 128 of a
 // fourth workgroup it spills 35 of them and takes 237 instead of 104 us at B96 M4096 N64 w256; with
 // three workgroups two stages do as well as three, 101 against 104 us, and are what it uses.)
+// A tile starts with three rows per lane from as many tensors.  All loads are issued before the first is waited for: us at B96
+// M4096 without / with that: N = 128 w = 40 149 / 141, N = 80 w = 64 96 / 90, N = 96 w = 256 167 / 162, N = 64 w = 100 72 / 69; the forward and
+// the key kernel, with a row or two per lane, gain nothing from it.
 template <typename T, int NK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_query_dma_kernel(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K, const uint16_t *__restrict__ V,
@@ -509,12 +512,16 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 3 : 2) void attention_backward_
     const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
     const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr;
     const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr;
+    u32x4 of[NK];
+    width.fetch_operands(gr, dO, q_ok, half, gf);
+    width.fetch_operands(orow, O, q_ok, half, of);
+    width.fetch_operands(qr, Q, q_ok, half, qf);
+    __builtin_amdgcn_sched_barrier(0);
+    width.mask_operands(gf, q_ok, tail);
+    width.mask_operands(of, q_ok, tail);
+    width.mask_operands(qf, q_ok, tail);
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      qf[ks] = width.load_operand(qr, Q, q_ok, ks, half, tail);
-      gf[ks] = width.load_operand(gr, dO, q_ok, ks, half, tail);
-      delta += dot8<T>(gf[ks], width.load_operand(orow, O, q_ok, ks, half, tail));
-    }
+    for (int ks = 0; ks < NK; ++ks) delta += dot8<T>(gf[ks], of[ks]);
   }
   delta = halves_sum(delta);
   const float l2 = (q_ok ? L[(int64_t)b * M + qi] : 0.0f) * kLog2e;
@@ -962,12 +969,16 @@ __global__ __launch_bounds__(512, 2) void attention_backward_query_split_kernel(
     const uint16_t *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
     const uint16_t *gr = dO + gsb.at(bp) + (int64_t)qi * gsr;
     const uint16_t *orow = O + osb.at(bp) + (int64_t)qi * osr;
+    u32x4 of[NK];
+    width.fetch_operands(gr, dO, q_ok, half, gf);
+    width.fetch_operands(orow, O, q_ok, half, of);
+    width.fetch_operands(qr, Q, q_ok, half, qf);
+    __builtin_amdgcn_sched_barrier(0);
+    width.mask_operands(gf, q_ok, tail);
+    width.mask_operands(of, q_ok, tail);
+    width.mask_operands(qf, q_ok, tail);
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      qf[ks] = width.load_operand(qr, Q, q_ok, ks, half, tail);
-      gf[ks] = width.load_operand(gr, dO, q_ok, ks, half, tail);
-      delta += dot8<T>(gf[ks], width.load_operand(orow, O, q_ok, ks, half, tail));
-    }
+    for (int ks = 0; ks < NK; ++ks) delta += dot8<T>(gf[ks], of[ks]);
   }
   delta = halves_sum(delta);
   const float l2 = (q_ok ? L[(int64_t)b * M + qi] : 0.0f) * kLog2e;

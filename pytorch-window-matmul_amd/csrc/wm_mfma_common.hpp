@@ -130,6 +130,18 @@ struct HeadWidth {
                                                 u32x4 tail) const {
     return mask_operand(fetch_piece(row, safe, valid, 2 * ks + half), valid, ks, tail);
   }
+  // All pieces of a row as such operands, one row per lane.  fetch_operands leaves them as loaded, so that a kernel can have
+  // every row it needs in flight before mask_operands makes it wait for the first: with load and mask side by side the
+  // compiler waits for the first load before it issues the last, one more memory latency at the start of a tile.
+  __device__ __forceinline__ void fetch_operands(const uint16_t *row, const uint16_t *safe, bool valid, int half,
+                                                 u32x4 (&v)[NK]) const {
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) v[ks] = fetch_piece(row, safe, valid, 2 * ks + half);
+  }
+  __device__ __forceinline__ void mask_operands(u32x4 (&v)[NK], bool valid, u32x4 tail) const {
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks) v[ks] = mask_operand(v[ks], valid, ks, tail);
+  }
   // The same operand read from an LDS tile of whole pieces.
   static __device__ __forceinline__ u32x4 tile_operand(u32x4 v, int ks, u32x4 tail) { return RAG && ks == NK - 1 ? v & tail : v; }
 };
