@@ -36,10 +36,10 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-# Sources whose kernels use more than 256 registers and look at most results of the matrix instructions once per use: with the
-# results in accumulation registers, the compiler's choice there, each has to be moved (key kernel at N = 64: 206 of 821
-# instructions of a block).
-FILE_FLAGS = {"wm_attention_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# The float32 attention key kernel for the widest heads uses more than 256 registers and works on most results of the matrix
+# instructions with the vector ALU once: with the results in accumulation registers, the compiler's choice there, it spills.  Where
+# such a kernel leaves the compiler room the choice is the better one (at N = 64 it moves 12 registers a block against 111).
+FILE_FLAGS = {"wm_attention_f32_key_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _newer(target, sources):

@@ -19,10 +19,15 @@
 //
 // Head widths: any N = 8 ... 128, in pieces of eight columns, the last one moved back to end with the row (HeadWidth).  The
 // columns it shares with the piece before are cleared in the stationary operands; as result columns they come out twice.
+//
+// With F32_KEY_WIDE set (wm_attention_f32_key_wide.hip) this translation unit holds the key kernel for N > 96 alone, which wants
+// a compiler option of its own (FILE_FLAGS in build.py).
+#include "wm_deal.hpp"
 #include "wm_f32_split_common.hpp"
 
-#include <type_traits>
-#include <utility>
+#ifndef F32_KEY_WIDE
+#define F32_KEY_WIDE 0
+#endif
 
 namespace wm {
 namespace {
@@ -33,12 +38,12 @@ constexpr float kRaiseBy = 8.0f;
 
 // Chunks in LDS.  With three, the first products of a chunk run one iteration ahead of the rest, their vector work dealt out among
 // the matrix instructions (deal() below).  That is for one wavefront per SIMD: us at B96 M4096 w256, two stages / three: forward
-// N = 32 191 / 203, N = 64 430 / 430 (B2 M4096 w1024, one wavefront per SIMD there too: 121 / 92), N = 128 735 / 709; query kernel
-// N = 64 520 / 595 (two wavefronts only on two stages), N = 96 876 / 794, N = 128 1087 / 998; key kernel N = 64 820 / 735, above
-// that its registers do not suffice.
+// N = 32 191 / 203, N = 64 430 / 430 (B2 M4096 w1024, one wavefront per SIMD there too: 121 / 92), N = 128 735 / 712; query kernel
+// N = 64 520 / 595 (two wavefronts only on two stages), N = 80 789 / 703, N = 128 1087 / 1005; key kernel and D N = 32 w = 64 166 / 237,
+// N = 64 853 / 782, N = 80 1073 / 959, N = 96 1146 / 1053, N = 128 1450 / 1817 (there its registers do not suffice).
 constexpr int forward_stages(int NK) { return NK <= 3 ? 2 : 3; }
 constexpr int query_stages(int NK) { return NK <= 4 ? 2 : 3; }
-constexpr int key_stages(int NK) { return NK == 3 || NK == 4 ? 3 : 2; }
+constexpr int key_stages(int NK) { return NK >= 3 && NK <= 6 ? 3 : 2; }
 
 // A chunk of two streamed tensors as it lies in LDS.
 template <int NK>
@@ -85,17 +90,28 @@ __device__ __forceinline__ void split_to_lds(char *plane0, int plane_bytes, int 
 }
 // Piece of a row that stays in registers: the columns it shares with the piece before are zeros, rows outside too.
 template <int NK>
-__device__ __forceinline__ Eight stationary_piece(HeadWidth<true, NK> width, const float *row, const float *safe, bool valid,
-                                                  int piece) {
+__device__ __forceinline__ Eight mask_piece(HeadWidth<true, NK> width, Eight v, bool valid, int piece) {
   const bool there = valid && piece < width.pieces();
   const int first = width.first(piece);
-  Eight v = load8(there ? row + width.column(piece) : safe);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     v.lo[e] = there && e >= first ? v.lo[e] : 0.0f;
     v.hi[e] = there && e + 4 >= first ? v.hi[e] : 0.0f;
   }
   return v;
+}
+// All pieces of the rows of two tensors, one row per lane: every load in flight before the first is waited for.
+template <int NK>
+__device__ __forceinline__ void fetch_pieces(HeadWidth<true, NK> width, const float *row, const float *safe, bool valid, int half,
+                                             Eight (&v)[NK]) {
+#pragma unroll
+  for (int ks = 0; ks < NK; ++ks)
+    v[ks] = load8(valid && 2 * ks + half < width.pieces() ? row + width.column(2 * ks + half) : safe);
+}
+template <int NK>
+__device__ __forceinline__ Eight stationary_piece(HeadWidth<true, NK> width, const float *row, const float *safe, bool valid,
+                                                  int piece) {
+  return mask_piece(width, load8(valid && piece < width.pieces() ? row + width.column(piece) : safe), valid, piece);
 }
 
 __device__ __forceinline__ float both_halves_max(float v) {
@@ -105,28 +121,6 @@ __device__ __forceinline__ float both_halves_max(float v) {
 __device__ __forceinline__ float both_halves_sum(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// Vector work that is dealt out among matrix instructions by hand.  A matrix instruction of 32 cycles leaves its SIMD free
-// for vector instructions, but the compiler puts the ones first and the others after them, and two wavefronts per SIMD do not make up
-// for it (the forward at N = 64: matrix pipe busy 42 % of the cycles, vector ALU 47 %, hardly ever both).  So the work comes as a
-// list of small steps, and deal() runs slot i of SLOTS with its share of them, fenced against reordering.
-template <int... I, typename F>
-__device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F &&f) {
-  (f(std::integral_constant<int, I>()), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void each(F &&f) {
-  each_of(std::make_integer_sequence<int, N>(), f);
-}
-template <int SLOTS, int STEPS, typename Slot, typename Step>
-__device__ __forceinline__ void deal(Slot &&slot, Step &&step) {
-  each<SLOTS>([&](auto i) {
-    constexpr int from = i * STEPS / SLOTS, to = (i + 1) * STEPS / SLOTS;
-    slot(i);
-    each<to - from>([&](auto j) { step(std::integral_constant<int, from + decltype(j)::value>()); });
-    __builtin_amdgcn_sched_barrier(0);
-  });
 }
 
 // split4 in three steps: two elements, the other two, the planes.
@@ -283,8 +277,11 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_f32_forwa
   u32x4 qop[NK][3];  // B operand of the first product: this lane's query, split
   {
     const float *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
+    Eight x[NK];
+    fetch_pieces(width, qr, Q, qi < M, half, x);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) split8(stationary_piece(width, qr, Q, qi < M, 2 * ks + half), qop[ks]);
+    for (int ks = 0; ks < NK; ++ks) split8(mask_piece(width, x[ks], qi < M, 2 * ks + half), qop[ks]);
   }
   const uint32_t row_at = Tile::row_at(lane), tr_at = Tile::tr_at(lane);
   f32x16 o[NB];
@@ -596,11 +593,16 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_f32_query
     const float inv_l = q_ok ? stats[((int64_t)B + b) * M + qi] : 0.0f;
     const float *qr = Q + qsb.at(bp) + (int64_t)qi * qsr, *gr = dO + gsb.at(bp) + (int64_t)qi * gsr,
                 *orow = O + osb.at(bp) + (int64_t)qi * osr;
+    Eight xs[NK], gs[NK], os[NK];
+    fetch_pieces(width, gr, dO, q_ok, half, gs);
+    fetch_pieces(width, orow, O, q_ok, half, os);
+    fetch_pieces(width, qr, Q, q_ok, half, xs);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      split8(stationary_piece(width, qr, Q, q_ok, 2 * ks + half), qop[ks]);
-      Eight g = stationary_piece(width, gr, dO, q_ok, 2 * ks + half);
-      const Eight x = stationary_piece(width, orow, O, q_ok, 2 * ks + half);
+      split8(mask_piece(width, xs[ks], q_ok, 2 * ks + half), qop[ks]);
+      Eight g = mask_piece(width, gs[ks], q_ok, 2 * ks + half);
+      const Eight x = mask_piece(width, os[ks], q_ok, 2 * ks + half);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         g.lo[e] *= inv_l, g.hi[e] *= inv_l;
@@ -832,10 +834,14 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
   u32x4 kop[NK][3], vop[NK][3];
   {
     const float *kr = K + ksb.at(bp) + (int64_t)kj * ksr, *vr = V + vsb.at(bp) + (int64_t)kj * vsr;
+    Eight x[NK], y[NK];
+    fetch_pieces(width, kr, K, k_ok, half, x);
+    fetch_pieces(width, vr, V, k_ok, half, y);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
-      split8(stationary_piece(width, kr, K, k_ok, 2 * ks + half), kop[ks]);
-      split8(stationary_piece(width, vr, V, k_ok, 2 * ks + half), vop[ks]);
+      split8(mask_piece(width, x[ks], k_ok, 2 * ks + half), kop[ks]);
+      split8(mask_piece(width, y[ks], k_ok, 2 * ks + half), vop[ks]);
     }
   }
   const uint32_t row_at = Tile::row_at(lane), tr_at = Tile::tr_at(lane);
@@ -1043,6 +1049,21 @@ hipError_t allow_lds(const void *kernel, int bytes) {
 constexpr double kLog2eD = 1.4426950408889634;
 
 template <int NK>
+hipError_t launch_key(const Problem &p, const View &q, const View &k, const View &v, const View &go, const float *stats, const float *delta,
+                      const View &gk, const View &gv, double scale) {
+  const int nblk = (int)((p.M + FA_TM - 1) / FA_TM);
+  constexpr int BYTES = key_stages(NK) * (PlaneTile<NK>::STAGE_BYTES + 2 * FA_KC * 4);
+  const auto kernel = attention_f32_key_kernel<NK>;
+  if (const hipError_t err = allow_lds(reinterpret_cast<const void *>(kernel), BYTES); err != hipSuccess) return err;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)tiled_grid(p.B, nblk)), dim3(kThreads), BYTES, p.stream, (const float *)q.data,
+                     (const float *)k.data, (const float *)v.data, (const float *)go.data, stats, delta, (float *)gk.data,
+                     (float *)gv.data, (int)p.B, (int)p.M, (int)p.w, nblk, (int)p.N, (float)scale, (float)(scale * kLog2eD), q.sb, q.sr,
+                     k.sb, k.sr, v.sb, v.sr, go.sb, go.sr, gk.sb, gk.sr, gv.sb, gv.sr);
+  return hipGetLastError();
+}
+
+#if !F32_KEY_WIDE
+template <int NK>
 hipError_t launch_forward(const Problem &p, const View &q, const View &k, const View &v, const View &o, float *stats, double scale,
                           int mask) {
   const int nblk = (int)((p.M + FA_TM - 1) / FA_TM);
@@ -1061,7 +1082,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
   const int nblk = (int)((p.M + FA_TM - 1) / FA_TM);
   const dim3 grid((unsigned)tiled_grid(p.B, nblk)), block(kThreads);
   const float c = (float)(scale * kLog2eD);
-  constexpr int BYTES = query_stages(NK) * PlaneTile<NK>::STAGE_BYTES, KEY_BYTES = key_stages(NK) * (PlaneTile<NK>::STAGE_BYTES + 2 * FA_KC * 4);
+  constexpr int BYTES = query_stages(NK) * PlaneTile<NK>::STAGE_BYTES;
   if (gq.data != nullptr) {
     const auto kernel = attention_f32_query_kernel<NK>;
     if (const hipError_t err = allow_lds(reinterpret_cast<const void *>(kernel), BYTES); err != hipSuccess) return err;
@@ -1074,13 +1095,8 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
   }
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess || (gk.data == nullptr && gv.data == nullptr)) return err;
-  const auto kernel = attention_f32_key_kernel<NK>;
-  if (const hipError_t e = allow_lds(reinterpret_cast<const void *>(kernel), KEY_BYTES); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, grid, block, KEY_BYTES, p.stream, (const float *)q.data, (const float *)k.data, (const float *)v.data,
-                     (const float *)go.data, stats, (const float *)delta, (float *)gk.data, (float *)gv.data, (int)p.B, (int)p.M,
-                     (int)p.w, nblk, (int)p.N, (float)scale, c, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, go.sb, go.sr, gk.sb, gk.sr,
-                     gv.sb, gv.sr);
-  return hipGetLastError();
+  if constexpr (NK >= 7) return launch_attention_f32_key_wide(p, q, k, v, go, stats, delta, gk, gv, scale);
+  else return launch_key<NK>(p, q, k, v, go, stats, delta, gk, gv, scale);
 }
 
 bool rows_ok(std::initializer_list<const View *> views) {
@@ -1089,8 +1105,16 @@ bool rows_ok(std::initializer_list<const View *> views) {
   return true;
 }
 
+#endif
+
 }  // namespace
 
+#if F32_KEY_WIDE
+hipError_t launch_attention_f32_key_wide(const Problem &p, const View &q, const View &k, const View &v, const View &go, const float *stats,
+                                         const float *delta, const View &gk, const View &gv, double scale) {
+  return p.N > 112 ? launch_key<8>(p, q, k, v, go, stats, delta, gk, gv, scale) : launch_key<7>(p, q, k, v, go, stats, delta, gk, gv, scale);
+}
+#else
 bool attention_f32_supports(const Problem &p, double scale) {
   if (p.dtype != WM_DTYPE_F32 || (p.flags & (WM_FLAG_FORCE_STRIDED | WM_FLAG_NO_SPLIT_F32))) return false;
   if (p.N < 8 || p.N > 128 || p.M < 1 || p.w < 1 || p.w > 0x3fffffff) return false;
@@ -1121,5 +1145,7 @@ bool try_launch_attention_f32_backward(const Problem &p, const View &q, const Vi
   }
   return true;
 }
+
+#endif
 
 }  // namespace wm

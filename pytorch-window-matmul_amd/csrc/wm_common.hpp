@@ -179,6 +179,8 @@ bool try_launch_attention_f32_forward(const Problem &p, const View &q, const Vie
 bool try_launch_attention_f32_backward(const Problem &p, const View &q, const View &k, const View &v, const View &o, const View &go,
                                        const float *stats, float *delta, const View &gq, const View &gk, const View &gv,
                                        double scale, hipError_t *err);
+hipError_t launch_attention_f32_key_wide(const Problem &p, const View &q, const View &k, const View &v, const View &go, const float *stats,
+                                         const float *delta, const View &gk, const View &gv, double scale);  // N > 96
 
 // Batched transpose of the last two dimensions (wm_transpose.hip): src (B,R,C) with unit column stride and
 // batch / row strides ssb / ssr (elements), dst contiguous (B,C,R).  Returns false, nothing launched,
