@@ -665,11 +665,12 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 //   inference  T = 3072: N = 64 117 / 122 at w = 8, 149 / 113 at w = 16, 886 / 420 at w = 256; N = 128 323 / 317 at w = 16, 1249 / 710 at
 //              256.  Few tiles leave CUs idle where the separate ops share a tile out: N = 128 T = 32 39 / 29 at w = 64, 53 / 55 at w = 256,
 //              T = 64 138 / 167 at w = 1024, T = 128 196 / 170; N = 64 T = 32 105 / 92 at w = 1024.
-//   training   N <= 64: T = 3072 536 / 569 at w = 24, 678 / 561 at w = 32, 2096 / 1456 at w = 256; T = 32 96 / 66 at w = 64, 142 / 132 at
-//              w = 256, 177 / 200 at w = 400, T = 64 346 / 420 at w = 1024, T = 128 438 / 402.
-//              N > 64: the key kernel needs the registers of a whole SIMD per wavefront: T = 3072 N = 128 1540 / 1542 at w = 64,
-//              2252 / 2085 at w = 128, 3553 / 3130 at w = 256; N = 80 1609 / 1586 and 2516 / 2420; T = 256 N = 96 w = 1000 771 / 647; T = 168
-//              N = 80 239 / 240 at w = 300, 775 / 801 at w = 1500; T = 128 N = 128 203 / 251 at w = 256.
+//   training   N <= 32: T = 3072 N = 32 259 / 288 at w = 16, 329 / 287 at w = 24, N = 16 276 / 227 at w = 24; T = 32 176 / 149 at w = 400, T = 64
+//              347 / 314 at w = 1000.  N = 64: T = 3072 567 / 576 at w = 24, 678 / 561 at w = 32, 2096 / 1456 at w = 256; T = 32 96 / 66 at
+//              w = 64, 142 / 132 at w = 256, 177 / 200 at w = 400, T = 64 346 / 420 at w = 1024, T = 128 438 / 402.
+//              N > 64: a wavefront of the key kernel needs the registers of a whole SIMD: T = 3072 N = 80 1096 / 1112 at w = 64, N = 96
+//              1551 / 1640 at w = 100, 2709 / 2390 at w = 256, N = 128 2090 / 2074 at w = 128, 3553 / 3130 at w = 256; T = 168 N = 80 226 / 212 at
+//              w = 300, 766 / 687 at w = 1500, T = 128 N = 80 477 / 514 at w = 1000; T = 256 N = 128 251 / 251 and 791 / 792 at w = 200 and 1000.
 //              Widths that 8 does not divide, which the separate ops take to the tile kernels: T = 3072 N = 60 616 / 602
 //              at w = 16, 748 / 580 at w = 32, N = 75 5062 / 2346 at w = 256; T = 32 N = 75 216 / 216 at w = 300.
 // Below 8 tiles all routes are a handful of launches, and what a problem of that size gives, traced or not, stays as it was bit for bit.
@@ -678,9 +679,10 @@ bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool t
   const int64_t N = q.size(-1), M = q.size(-2);
   if (N < 8 || N > kMaxWidth || M > (1 << 30) || window_size < 16 || window_size > (1 << 28) || !(scale > 0.0 && scale < 1.0e30)) return false;
   const int64_t tiles = q.numel() / (N * M) * ((M + 127) / 128);
-  if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && (training || N > 64))) return false;
+  if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && N > (training ? 32 : 64))) return false;
   if (!training) return true;
-  return N > 64 && N % 8 == 0 ? window_size >= 128 && tiles >= 256 : window_size >= 32;
+  if (N > 64 && N % 8 == 0) return window_size >= 128 && tiles >= (N <= 96 ? 160 : 256);
+  return window_size >= (N <= 32 ? 24 : 32);
 }
 
 bool window_attention_f32_supported(const torch::Tensor &q, int64_t window_size, double scale, bool training) {

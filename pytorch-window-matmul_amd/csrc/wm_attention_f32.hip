@@ -277,11 +277,8 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_f32_forwa
   u32x4 qop[NK][3];  // B operand of the first product: this lane's query, split
   {
     const float *qr = Q + qsb.at(bp) + (int64_t)qi * qsr;
-    Eight x[NK];
-    fetch_pieces(width, qr, Q, qi < M, half, x);
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < NK; ++ks) split8(mask_piece(width, x[ks], qi < M, 2 * ks + half), qop[ks]);
+    for (int ks = 0; ks < NK; ++ks) split8(stationary_piece(width, qr, Q, qi < M, 2 * ks + half), qop[ks]);
   }
   const uint32_t row_at = Tile::row_at(lane), tr_at = Tile::tr_at(lane);
   f32x16 o[NB];
