@@ -9,10 +9,10 @@
 namespace wm {
 namespace {
 
-// Vector work that is dealt out among matrix instructions by hand.  A matrix instruction of 32 cycles leaves its SIMD free
-// for vector instructions, but the compiler puts the ones first and the others after them, and two wavefronts per SIMD do not make up
-// for it (the forward at N = 64: matrix pipe busy 42 % of the cycles, vector ALU 47 %, hardly ever both).  So the work comes as a
-// list of small steps, and deal() runs slot i of SLOTS with its share of them, fenced against reordering.
+// A matrix instruction of 32 cycles leaves its wavefront free to issue five or six vector instructions beside it (measured: 35 cycles
+// alone, 42 with six), but the compiler puts the ones first and the others after them.  Where a SIMD holds one wavefront nothing
+// else fills the time.  So the vector work comes as a list of small steps, and deal() runs slot i of SLOTS with its share
+// of them, fenced against reordering.  What it brings stands at forward_stages() in wm_attention_f32.hip; with two wavefronts per SIMD nothing.
 template <int... I, typename F>
 __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F &&f) {
   (f(std::integral_constant<int, I>()), ...);
