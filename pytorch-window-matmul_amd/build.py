@@ -12,6 +12,7 @@ Run ``python build.py`` (add ``--force`` to rebuild up-to-date targets).
 """
 import glob
 import os
+import re
 import subprocess
 import sys
 import sysconfig
@@ -42,6 +43,21 @@ HIPCC_FLAGS = [
 FILE_FLAGS = {"wm_attention_f32_key_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
+def _files_of(source):
+    """`source` and every file it includes by a quoted name, at any depth: headers, and the sources that a wrapper includes."""
+    seen, open_ = set(), [os.path.abspath(source)]
+    while open_:
+        path = open_.pop()
+        if path in seen:
+            continue
+        seen.add(path)
+        with open(path) as f:
+            names = re.findall(r'^[ \t]*#[ \t]*include[ \t]+"([^"]+)"', f.read(), re.M)
+        found = (os.path.abspath(os.path.join(d, n)) for n in names for d in (os.path.dirname(path), INCLUDE))
+        open_ += [f for f in found if os.path.exists(f)]
+    return sorted(seen)
+
+
 def _newer(target, sources):
     if not os.path.exists(target):
         return False
@@ -61,16 +77,16 @@ def _run(cmd):
 
 def build_hip_library(force=False):
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
-    deps = sources + glob.glob(os.path.join(CSRC, "*.hpp")) + glob.glob(os.path.join(INCLUDE, "*.h"))
-    if not force and _newer(HIP_LIB, deps):
+    this = os.path.abspath(__file__)  # the compiler flags stand here
+    deps = {src: [*_files_of(src), this] for src in sources}
+    if not force and _newer(HIP_LIB, {d for files in deps.values() for d in files}):
         return HIP_LIB
     objs = []
     procs = []
-    headers = [d for d in deps if d not in sources]
     for src in sources:
         obj = os.path.join(CSRC, os.path.basename(src)[:-4] + ".o")
         objs.append(obj)
-        if not force and _newer(obj, [src] + headers):
+        if not force and _newer(obj, deps[src]):
             continue  # this object is still current: only stale translation units are recompiled
         cmd = [os.path.join(ROCM, "bin", "hipcc"), *HIPCC_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
         print("+", " ".join(cmd), flush=True)
@@ -90,7 +106,7 @@ def build_extension(force=False):
     import torch
 
     src = os.path.join(CSRC, "binding.cpp")
-    deps = [src, HIP_LIB] + glob.glob(os.path.join(INCLUDE, "*.h"))
+    deps = [*_files_of(src), HIP_LIB, os.path.abspath(__file__)]
     if not force and _newer(EXT_LIB, deps):
         return EXT_LIB
     tdir = os.path.dirname(torch.__file__)
