@@ -267,9 +267,9 @@ int wm_grouped_score_gradient(const wm_grouped_operand *grad_o, const wm_grouped
 
 /* The fused attention for float32 storage, at float32 accuracy (products on the bf16 matrix instruction through an exact split
  * of every value).  As wm_grouped_window_attention_forward / _backward but for what the backward needs of the forward: stats,
- * float32 (2, B, M), per row the maximum the exponentials were taken against (log2 units) and 1 / their sum; NULL where no
+ * float32 (2, B, M), per row the score the exponentials were taken against and 1 / their sum; NULL where no
  * backward follows.  delta is a caller-owned float32 workspace of B * M values.  WM_ERR_UNSUPPORTED, nothing launched, unless
- * dtype is float32, 8 <= N <= 128, w >= 1, 0 < scale < 1e30 and the operands have unit column stride (rows of any alignment;
+ * dtype is float32, 8 <= N <= 128, w >= 1, 1.2e-38 < scale < 1e30 and the operands have unit column stride (rows of any alignment;
  * no byte outside them is touched).  Up to two kernels per call, no atomics: results are reproducible run to run.  An
  * infinite operand gives NaN where the exact result is infinite. */
 int wm_grouped_window_attention_f32_forward(const wm_grouped_operand *q, const wm_grouped_operand *k,

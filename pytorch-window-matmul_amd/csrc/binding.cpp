@@ -680,7 +680,7 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool training) {
   const int64_t N = q.size(-1), M = q.size(-2);
   if (q.numel() == 0) return false;
-  if (N < 8 || N > kMaxWidth || M > (1 << 30) || window_size < 16 || window_size > (1 << 28) || !(scale > 0.0 && scale < 1.0e30)) return false;
+  if (N < 8 || N > kMaxWidth || M > (1 << 30) || window_size < 16 || window_size > (1 << 28) || !(scale > 1.2e-38 && scale < 1.0e30)) return false;
   const int64_t tiles = batch_of(q) * ((M + 127) / 128);
   if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && N > (training ? 32 : 64))) return false;  // N = 32: T = 64 347 / 314 at w = 1000
   if (!training) return true;
