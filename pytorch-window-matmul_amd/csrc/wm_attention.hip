@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? (RAG ? 3 : 4) : 2) void attenti
     const int n_out = max(0, w - qi) + max(0, qi + w - (M - 1));
     const float m_new = n_out > 0 ? fmaxf(m_used, 0.0f) : m_used;
     alpha = __builtin_amdgcn_exp2f(m_used - m_new);
-    l = l * alpha + (float)n_out * __builtin_amdgcn_exp2f(-m_new);
+    l = l * alpha + (float)n_out * __builtin_amdgcn_exp2f(fminf(-m_new, 0.0f));
     m_used = m_new;
   }
   if (qi >= M) l = 1.0f;  // rows past the end: keep the arithmetic finite, nothing is stored
@@ -606,11 +606,12 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 4 : 2) void attention_forward_d
   float alpha = 1.0f;  // what the accumulated O still has to be scaled by (folded into the division by l)
   if (!MASK) {
     // Band entries outside the sequence: score 0 each, no value row.  Branch-free: a row without such
-    // entries keeps its maximum, alpha = 1 and adds 0 to the sum.
+    // entries keeps its maximum, alpha = 1 and adds 0 to the sum (the exponent is bounded for it: with a maximum
+    // below -128 the exponential would be infinite).
     const int n_out = max(0, w - qi) + max(0, qi + w - (M - 1));
     const float m_new = n_out > 0 ? fmaxf(m_used, 0.0f) : m_used;
     alpha = __builtin_amdgcn_exp2f(m_used - m_new);
-    l = l * alpha + (float)n_out * __builtin_amdgcn_exp2f(-m_new);
+    l = l * alpha + (float)n_out * __builtin_amdgcn_exp2f(fminf(-m_new, 0.0f));
     m_used = m_new;
   }
   if (qi >= M) l = 1.0f;  // rows past the end: keep the arithmetic finite, nothing is stored
@@ -828,7 +829,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void attention_forward_split_kernel(
     const int n_out = max(0, w - qi) + max(0, qi + w - (M - 1));
     const float m_new = n_out > 0 ? fmaxf(m_all, 0.0f) : m_all;
     alpha = __builtin_amdgcn_exp2f(m_all - m_new);
-    l = l * alpha + (float)n_out * __builtin_amdgcn_exp2f(-m_new);
+    l = l * alpha + (float)n_out * __builtin_amdgcn_exp2f(fminf(-m_new, 0.0f));
     m_all = m_new;
   }
   if (qi >= M) l = 1.0f;  // rows past the end: keep the arithmetic finite, nothing is stored

@@ -326,3 +326,26 @@ def test_one_kernel_and_two_kernel_backward_agree(device, case, dtype):
                 assert (x is None) == (not wanted)
                 if wanted:
                     assert torch.equal(x, y)
+
+
+# batch * heads, M, N, w, flags: every forward kernel (whole window in LDS, streamed through LDS, streamed through registers, streamed with
+# the tile shared out), whole and ragged head widths
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,M,N,w,flags", [(24, 1500, 64, 20, 0), (24, 1500, 64, 200, 0), (24, 1500, 64, 200, abi.NO_LDS_DIRECT), (2, 1500, 64, 200, 0), (2, 1500, 128, 200, 0),
+                                           (24, 1500, 128, 200, 0), (24, 1500, 60, 200, 0), (2, 1500, 75, 200, 0)])
+def test_rows_of_large_negative_scores(device, B, M, N, w, flags, dtype):
+    """A row whose neighbours all score far below zero (with them the largest score, -100 to -1000) is as finite as any other."""
+    q, k, v = (seeded((B, M, N), 40 + s, dtype) for s in range(3))
+    q, k = q.abs(), -k.abs()
+    scale = 30.0 if N == 64 else 15.0
+    if N % 16:
+        flags |= abi.ANY_HEAD_WIDTH
+    out, lse = abi.attention_forward(q.to(device), k.to(device), v.to(device), w, scale, False, flags)
+    want, want_lse = ao.window_attention_forward(q[:1], k[:1], v[:1], w, scale, False)
+    assert float(want_lse[0, M // 2]) < -100.0
+    assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(lse).all())
+    want = torch.from_numpy(want)
+    # scores of this size carry an error of 1000 * 2^-24 * a few: the result's rounding is what is left
+    error = float((out[:1].cpu().double() - want).norm() / want.norm())
+    assert error < (2e-3 if dtype == torch.float16 else 1e-2)
