@@ -10,7 +10,7 @@
 //                 value around 10 that is 5e-7, a relative error of every probability of the row; m and 1 / l are exact and
 //                 correctly rounded.
 //   query kernel  128 queries: S^T, dP^T = V dO^T, dS^T, dQ^T += K^T dS^T.  Also writes D / l, D = sum_h dO O, for
-//   key kernel    128 keys, walks over the queries: S, dP, dV^T += dO^T P, dK^T += Q^T dS.
+//   key kernel    128 keys, walks over the queries: S, dP, dV^T += dO^T P, dK^T += Q^T dS, or what one of the two needs.
 // The backward works on exp2(c (S - m)), not yet divided by l: dO is multiplied by 1 / l on its way in instead.
 //
 // Layouts are those of the 16-bit kernels: in a 32 x 32 score tile a lane owns one stationary row and sixteen streamed ones, the
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_f32_forwa
 }
 
 // ---------------------------------------------------------------------------------------------
-// backward: D / l of every row, when grad_q is not wanted (else the query kernel writes it)
+// backward: D / l of every row, when grad_k is wanted and grad_q is not (else the query kernel writes it)
 // ---------------------------------------------------------------------------------------------
 template <int NK>
 __global__ __launch_bounds__(kThreads) void attention_f32_delta_kernel(const float *__restrict__ O, const float *__restrict__ dO,
@@ -777,7 +777,11 @@ __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_f32_query
 // ---------------------------------------------------------------------------------------------
 // backward: key kernel
 // ---------------------------------------------------------------------------------------------
-template <int NK>
+// DK, DV: the results that are wanted.  Without dK neither dP nor D is needed, nor the values; without dV P is not split.  A training
+// step for grad_v alone / grad_q and grad_k, us at B96 M4096, separate ops, fused with all four products, fused with those needed:
+// N = 64 w = 32 345, 446, 252 / 586, 561, 527; N = 80 w = 256 1290, 1505, 1095 / 2192, 2177, 2021; N = 128 w = 128 1114, 1470, 1008 / 1922,
+// 2148, 1944, w = 256 1787, 2147, 1513 / 2986, 3150, 2852.
+template <int NK, bool DK, bool DV>
 __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_kernel(
     const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, const float *__restrict__ dO,
     const float *__restrict__ stats, const float *__restrict__ D, float *__restrict__ dK, float *__restrict__ dV, int B, int M,
@@ -815,7 +819,7 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
       greg[u] = load8(Gb + (int64_t)row * gsr + mine.column[u]);
       inv_reg[u] = inv_rows[row];
     }
-    stat_reg = ((tid & 32) ? d_rows : m_rows)[min(qc * FA_KC + (tid & 31), M - 1)];
+    stat_reg = (DK && (tid & 32) ? d_rows : m_rows)[min(qc * FA_KC + (tid & 31), M - 1)];
   };
   auto stash = [&](int buf) {
 #pragma unroll
@@ -834,17 +838,17 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
     __syncthreads();
   }
 
-  u32x4 kop[NK][3], vop[NK][3];
+  u32x4 kop[NK][3], vop[DK ? NK : 1][3];
   {
     const float *kr = K + ksb.at(bp) + (int64_t)kj * ksr, *vr = V + vsb.at(bp) + (int64_t)kj * vsr;
     Eight x[NK], y[NK];
     fetch_pieces(width, kr, K, k_ok, half, x);
-    fetch_pieces(width, vr, V, k_ok, half, y);
+    if constexpr (DK) fetch_pieces(width, vr, V, k_ok, half, y);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
       split8(mask_piece(width, x[ks], k_ok, 2 * ks + half), kop[ks]);
-      split8(mask_piece(width, y[ks], k_ok, 2 * ks + half), vop[ks]);
+      if constexpr (DK) split8(mask_piece(width, y[ks], k_ok, 2 * ks + half), vop[ks]);
     }
   }
   const uint32_t row_at = Tile::row_at(lane), tr_at = Tile::tr_at(lane);
@@ -863,9 +867,12 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
     for (int ks = 0; ks < NK; ++ks) {
       u32x4 qa[3], ga[3];
 #pragma unroll
-      for (int p = 0; p < 3; ++p) qa[p] = Tile::rows(tile(buf, 0, p), row_at, 0, ks), ga[p] = Tile::rows(tile(buf, 1, p), row_at, 0, ks);
+      for (int p = 0; p < 3; ++p) {
+        qa[p] = Tile::rows(tile(buf, 0, p), row_at, 0, ks);
+        if constexpr (DK) ga[p] = Tile::rows(tile(buf, 1, p), row_at, 0, ks);
+      }
       mma_split_two<true>(qa, kop[ks], s, s1);
-      mma_split_two(ga, vop[ks], dp, dp1);
+      if constexpr (DK) mma_split_two(ga, vop[ks], dp, dp1);
     }
 #pragma unroll
     for (int v = 0; v < 16; ++v) s[v] += s1[v], dp[v] += dp1[v];
@@ -880,7 +887,7 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
       Eight pr, ds;
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
-        const f32x4 m4 = row_stats(buf, 0, 2 * t + g), d4 = row_stats(buf, 1, 2 * t + g);
+        const f32x4 m4 = row_stats(buf, 0, 2 * t + g), d4 = DK ? row_stats(buf, 1, 2 * t + g) : m4;
         f32x4 p4, s4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -892,15 +899,18 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
         else pr.hi = p4, ds.hi = s4;
       }
       u32x4 pf[3], df[3];
-      split8(pr, pf);
-      split8(ds, df);
+      if constexpr (DV) split8(pr, pf);
+      if constexpr (DK) split8(ds, df);
 #pragma unroll
       for (int hb = 0; hb < NB; ++hb) {
         u32x4 ga[3], qa[3];
 #pragma unroll
-        for (int p = 0; p < 3; ++p) ga[p] = Tile::cols(tile(buf, 1, p), tr_at, 16 * t, hb), qa[p] = Tile::cols(tile(buf, 0, p), tr_at, 16 * t, hb);
-        dv[hb] = mma_split(ga, pf, dv[hb]);
-        dk[hb] = mma_split(qa, df, dk[hb]);
+        for (int p = 0; p < 3; ++p) {
+          if constexpr (DV) ga[p] = Tile::cols(tile(buf, 1, p), tr_at, 16 * t, hb);
+          if constexpr (DK) qa[p] = Tile::cols(tile(buf, 0, p), tr_at, 16 * t, hb);
+        }
+        if constexpr (DV) dv[hb] = mma_split(ga, pf, dv[hb]);
+        if constexpr (DK) dk[hb] = mma_split(qa, df, dk[hb]);
       }
     }
   };
@@ -950,27 +960,31 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
-          for (int p = 0; p < 3; ++p) ra[ks % 2][x][p] = Tile::rows(tile(next, x, p), row_at, 0, ks);
+          for (int p = 0; p < 3; ++p)
+            if (x == 0 || DK) ra[ks % 2][x][p] = Tile::rows(tile(next, x, p), row_at, 0, ks);
       };
       auto read_cols = [&](auto y) {  // y = NB t + hb
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
-          for (int p = 0; p < 3; ++p) ca[y % 2][x][p] = Tile::cols(tile(buf, x, p), tr_at, 16 * (y / NB), y % NB);
+          for (int p = 0; p < 3; ++p)
+            if (x == 0 ? DK : DV) ca[y % 2][x][p] = Tile::cols(tile(buf, x, p), tr_at, 16 * (y / NB), y % NB);
       };
-      f32x4 m4 = row_stats(buf, 0, 0), d4 = row_stats(buf, 1, 0), p4, s4;
+      auto row_delta = [&](int g) { return DK ? row_stats(buf, 1, g) : f32x4{0.0f, 0.0f, 0.0f, 0.0f}; };
+      f32x4 m4 = row_stats(buf, 0, 0), d4 = row_delta(0), p4, s4;
       read_rows(std::integral_constant<int, 0>());
       __builtin_amdgcn_sched_barrier(0);
       Split4Steps sp, sd;
-      deal<12 * NK, 32>(
+      constexpr int FIRST = DK ? 2 : 1, SECOND = DK && DV ? 2 : 1;  // products of either kind
+      deal<6 * FIRST * NK, 32>(
           [&](auto i) {
-            constexpr int ks = i / 12, r = i % 12;
+            constexpr int ks = i / (6 * FIRST), r = i % (6 * FIRST);
             if constexpr (r == 0 && ks + 1 < NK) read_rows(std::integral_constant<int, ks + 1>());
-            if constexpr (i == 12 * NK - 12) read_cols(std::integral_constant<int, 0>());
-            if constexpr (r % 2 == 0)
-              mma_step_two<r / 2, true>(ra[ks % 2][0], kop[ks], ns, ns1);
+            if constexpr (r == 0 && ks + 1 == NK) read_cols(std::integral_constant<int, 0>());
+            if constexpr (r % FIRST == 0)
+              mma_step_two<r / FIRST, true>(ra[ks % 2][0], kop[ks], ns, ns1);
             else
-              mma_step_two<r / 2>(ra[ks % 2][1], vop[ks], ndp, ndp1);
+              mma_step_two<r / FIRST>(ra[ks % 2][1], vop[ks], ndp, ndp1);
           },
           [&](auto j) {
             constexpr int g = j / 8, r = j % 8;
@@ -980,22 +994,22 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
                 p4[e] = exp2_above(s[4 * g + e], m4[e], c);
                 s4[e] = p4[e] * (dp[4 * g + e] - d4[e]);
               }
-              if constexpr (r == 1 && g < 3) m4 = row_stats(buf, 0, g + 1), d4 = row_stats(buf, 1, g + 1);
+              if constexpr (r == 1 && g < 3) m4 = row_stats(buf, 0, g + 1), d4 = row_delta(g + 1);
             } else if constexpr (r < 5) {
-              sp.run<r - 2>(p4, pf[g / 2], g % 2);
-            } else {
+              if constexpr (DV) sp.run<r - 2>(p4, pf[g / 2], g % 2);
+            } else if constexpr (DK) {
               sd.run<r - 5>(s4, df[g / 2], g % 2);
             }
           });
       StashSteps st;
-      deal<24 * NB, 8 + 15 * SLOTS>(
+      deal<12 * SECOND * NB, 8 + 15 * SLOTS>(
           [&](auto i) {
-            constexpr int y = i / 12, r = i % 12;
+            constexpr int y = i / (6 * SECOND), r = i % (6 * SECOND);
             if constexpr (r == 0 && y + 1 < 2 * NB) read_cols(std::integral_constant<int, y + 1>());
-            if constexpr (r % 2 == 0)
-              mma_step<r / 2>(ca[y % 2][1], pf[y / NB], dv[y % NB]);
+            if constexpr (DV && r % SECOND == 0)
+              mma_step<r / SECOND>(ca[y % 2][1], pf[y / NB], dv[y % NB]);
             else
-              mma_step<r / 2>(ca[y % 2][0], df[y / NB], dk[y % NB]);
+              mma_step<r / SECOND>(ca[y % 2][0], df[y / NB], dk[y % NB]);
           },
           [&](auto j) {
             if constexpr (j < 8) {
@@ -1037,8 +1051,8 @@ __global__ __launch_bounds__(kThreads, NK <= 2 ? 2 : 1) void attention_f32_key_k
     }
   }
   float *stage = reinterpret_cast<float *>(fa_lds) + wave * (32 * kStage);
-  if (dK != nullptr) store_f32_rows<NK>(stage, dk, scale, dK + dksb.at(bp), dksr, kw0, M, width, lane);
-  if (dV != nullptr) store_f32_rows<NK>(stage, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, width, lane);
+  if constexpr (DK) store_f32_rows<NK>(stage, dk, scale, dK + dksb.at(bp), dksr, kw0, M, width, lane);
+  if constexpr (DV) store_f32_rows<NK>(stage, dv, 1.0f, dV + dvsb.at(bp), dvsr, kw0, M, width, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1056,7 +1070,9 @@ hipError_t launch_key(const Problem &p, const View &q, const View &k, const View
                       const View &gk, const View &gv, double scale) {
   const int nblk = (int)((p.M + FA_TM - 1) / FA_TM);
   constexpr int BYTES = key_stages(NK) * (PlaneTile<NK>::STAGE_BYTES + 2 * FA_KC * 4);
-  const auto kernel = attention_f32_key_kernel<NK>;
+  const auto kernel = gv.data == nullptr   ? attention_f32_key_kernel<NK, true, false>
+                      : gk.data == nullptr ? attention_f32_key_kernel<NK, false, true>
+                                           : attention_f32_key_kernel<NK, true, true>;
   if (const hipError_t err = allow_lds(reinterpret_cast<const void *>(kernel), BYTES); err != hipSuccess) return err;
   hipLaunchKernelGGL(kernel, dim3((unsigned)tiled_grid(p.B, nblk)), dim3(kThreads), BYTES, p.stream, (const float *)q.data,
                      (const float *)k.data, (const float *)v.data, (const float *)go.data, stats, delta, (float *)gk.data,
@@ -1092,7 +1108,7 @@ hipError_t launch_backward(const Problem &p, const View &q, const View &k, const
     hipLaunchKernelGGL(kernel, grid, block, BYTES, p.stream, (const float *)q.data, (const float *)k.data, (const float *)v.data,
                        (const float *)o.data, (const float *)go.data, stats, (float *)gq.data, delta, (int)p.B, (int)p.M, (int)p.w,
                        nblk, (int)p.N, (float)scale, c, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr, o.sb, o.sr, go.sb, go.sr, gq.sb, gq.sr);
-  } else {
+  } else if (gk.data != nullptr) {
     hipLaunchKernelGGL(attention_f32_delta_kernel<NK>, grid, block, 0, p.stream, (const float *)o.data, (const float *)go.data, stats,
                        delta, (int)p.B, (int)p.M, nblk, (int)p.N, o.sb, o.sr, go.sb, go.sr);
   }
