@@ -665,9 +665,11 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 //   inference  T = 3072: N = 64 117 / 122 at w = 8, 149 / 113 at w = 16, 886 / 420 at w = 256; N = 128 323 / 317 at w = 16, 1249 / 710 at
 //              256.  Few tiles leave CUs idle where the separate ops share a tile out: N = 128 T = 32 39 / 29 at w = 64, 53 / 55 at w = 256,
 //              T = 64 138 / 167 at w = 1024, T = 128 196 / 170; N = 64 T = 32 105 / 92 at w = 1024.
-//   training   Narrow heads would gain as well (N = 32 329 / 287 at w = 24, N = 16 276 / 227), but there the separate ops, whose row sums of P dP
-//              have 2 w + 1 terms, are the more accurate: distance of grad_k to float64 in 1e-7, theirs / fused, N = 16 2.30 / 2.57 at
-//              w = 40, N = 24 2.07 / 2.11, N = 32 2.30 / 2.34 at w = 24, 3.08 / 3.09 at w = 100, N = 40 2.81 / 2.48 at w = 40.
+//   training   Narrow heads would gain as well (N = 32 329 / 287 at w = 24, 707 / 360 at w = 64, N = 16 276 / 227), but up to N = 32 the separate ops,
+//              whose row sums of P dP have 2 w + 1 terms, are the more accurate: distance to float64 in 1e-7, theirs / fused, grad_k N = 16
+//              2.30 / 2.57 at w = 40, N = 24 2.07 / 2.11, N = 32 2.77 / 2.81 at w = 64; with scores three times as large N = 32 w = 64 grad_q
+//              3.97 / 4.20, grad_k 3.90 / 4.07.  From N = 33 on none is worse (N = 33 ... 128, w = 32 ... 300, scores of one, three and six times
+//              the size, four inputs each).
 //              N = 64: T = 3072 567 / 576 at w = 24, 678 / 561 at w = 32, 2096 / 1456 at w = 256; T = 32 96 / 66 at
 //              w = 64, 142 / 132 at w = 256, 177 / 200 at w = 400, T = 64 346 / 420 at w = 1024, T = 128 438 / 402.
 //              N > 64: a wavefront of the key kernel needs the registers of a whole SIMD: T = 3072 N = 80 1096 / 1112 at w = 64, N = 96
@@ -682,10 +684,10 @@ bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool t
   if (q.numel() == 0) return false;
   if (N < 8 || N > kMaxWidth || M > (1 << 30) || window_size < 16 || window_size > (1 << 28) || !(scale > 1.2e-38 && scale < 1.0e30)) return false;
   const int64_t tiles = batch_of(q) * ((M + 127) / 128);
-  if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && N > (training ? 32 : 64))) return false;  // N = 32: T = 64 347 / 314 at w = 1000
+  if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && (training || N > 64))) return false;
   if (!training) return true;
   if (N > 64 && N % 8 == 0) return window_size >= 128 && tiles >= (N <= 96 ? 160 : 256);
-  return N >= 40 ? window_size >= 32 : N >= 32 && window_size >= 64;
+  return N >= 40 ? window_size >= 32 : N > 32 && window_size >= 64;
 }
 
 bool window_attention_f32_supported(const torch::Tensor &q, int64_t window_size, double scale, bool training) {

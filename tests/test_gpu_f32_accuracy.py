@@ -1,0 +1,51 @@
+"""float32 attention as training takes it: whichever route a head width goes, no gradient is farther from float64 than the separate ops'."""
+import math
+
+import pytest
+import torch
+
+from window_matmul import band_softmax, unwindow_matmul, window_attention, window_matmul
+
+B, M = 32, 1024
+
+
+def _float64(q, k, v, go, w, scale, mask):
+    """One sequence after the other: (out, grad_q, grad_k, grad_v) of dense masked attention."""
+    i = torch.arange(M, device=q.device)
+    outside = (i[None] - i[:, None]).abs() > w
+    zeros = (w - i).clamp(min=0) + (i + w - (M - 1)).clamp(min=0) if not mask else torch.zeros_like(i)  # neighbours outside: score 0
+    results = []
+    for q, k, v, go in zip(*(t.double() for t in (q, k, v, go))):
+        s = (q @ k.T * scale).masked_fill(outside, -math.inf)
+        top = s.amax(-1, keepdim=True).clamp(min=0.0)
+        p = torch.exp(s - top)
+        p = p / (p.sum(-1, keepdim=True) + zeros[:, None] * torch.exp(-top))
+        out = p @ v
+        ds = scale * p * (go @ v.T - (go * out).sum(-1, keepdim=True))
+        results.append((out, ds @ k, ds.T @ q, p.T @ go))
+    return [torch.stack(t) for t in zip(*results)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("factor", [1.0, 3.0])
+@pytest.mark.parametrize("w", [64, 100])
+@pytest.mark.parametrize("N", [24, 32, 33, 40, 41, 48, 60, 64, 75, 101, 127])
+def test_training_is_no_less_accurate_than_the_separate_ops(device, N, w, factor):
+    """Root mean square of the relative distance over four inputs, with and without mask.  Over other inputs of these sizes the
+    quotient was 0.49 to 1.001 where the fused kernels train (1.06 at N = 32, which therefore does not)."""
+    mine, theirs = [0.0] * 4, [0.0] * 4
+    for seed in range(4):
+        g = torch.Generator(device=device).manual_seed(9000 + seed)
+        q, k, v, go = (torch.randn((B, M, N), generator=g, device=device) for _ in range(4))
+        q, scale, mask = q * factor, 1.0 / math.sqrt(N), bool(seed % 2)
+        want = _float64(q, k, v, go, w, scale, mask)
+        for total, separate in ((mine, False), (theirs, True)):
+            xs = [t.detach().requires_grad_(True) for t in (q, k, v)]
+            if separate:
+                out = unwindow_matmul(band_softmax(window_matmul(xs[0], xs[1].transpose(-1, -2), w), scale, mask), xs[2], w)
+            else:
+                out = window_attention(*xs, w, scale, mask)
+            for i, (x, y) in enumerate(zip((out.detach(), *torch.autograd.grad(out, xs, go)), want)):
+                total[i] += float(((x.double() - y).norm() / y.norm()) ** 2)
+    for x, y in zip(mine, theirs):
+        assert x ** 0.5 <= 1.02 * y ** 0.5, [(a / b) ** 0.5 for a, b in zip(mine, theirs)]

@@ -170,7 +170,7 @@ def test_in_a_captured_graph(device):
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,M,N,w,fused", [(8, 128, 64, 32, True), (7, 128, 64, 32, False), (8, 128, 64, 31, False), (2, 4096, 64, 257, False),
                                                (8, 128, 80, 128, False), (256, 128, 80, 127, False), (256, 128, 80, 128, True),
-                                               (8, 128, 75, 32, True), (8, 128, 32, 64, True),
+                                               (8, 128, 75, 32, True), (8, 128, 33, 64, True), (8, 128, 33, 63, False), (8, 128, 32, 64, False),
                                                (8, 128, 32, 63, False), (64, 128, 24, 100, False), (159, 128, 96, 128, False), (160, 128, 96, 128, True), (255, 128, 104, 128, False)])
 def test_route_of_training_and_of_a_result_changed_in_place(device, heads, M, N, w, fused):
     from window_matmul import window_attention
