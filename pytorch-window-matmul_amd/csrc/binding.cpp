@@ -457,6 +457,7 @@ bool ragged_rows_in_place(const torch::Tensor &t) {
   return t.stride(-1) == 1 && batch_steps(t, &step, &heads, &group);
 }
 torch::Tensor attention_rows(const torch::Tensor &t, Heads &heads) {  // rows of any alignment
+  if (t.stride(-1) != 1 && t.stride(-2) == 1) return key_rows(t.transpose(-2, -1), heads);  // keys of a channels-first projection
   return ragged_rows_in_place(t) && heads.admit(t) ? t : t.contiguous();
 }
 torch::Tensor attention_rows_like(const torch::Tensor &t, Heads &heads) {
