@@ -665,7 +665,8 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 // is the better of the other two:
 //   inference  T = 3072: N = 64 117 / 122 at w = 8, 149 / 113 at w = 16, 886 / 420 at w = 256; N = 128 323 / 317 at w = 16, 1249 / 710 at
 //              256.  Few tiles leave CUs idle where the separate ops share a tile out: N = 128 T = 32 39 / 29 at w = 64, 53 / 55 at w = 256,
-//              T = 64 138 / 167 at w = 1024, T = 128 196 / 170; N = 64 T = 32 105 / 92 at w = 1024.
+//              T = 64 138 / 167 at w = 1024, T = 128 196 / 170; N = 64 T = 32 105 / 92 at w = 1024.  T = 8 of one sequence: N = 128 49 / 46 at w =
+//              160, 50 / 51 at 180, 53 / 59 at 256, N = 96 52 / 50 at 256, N = 127 104 / 59 at 256; T = 32 N = 128 59 / 60 at 256.
 //   training   Narrow heads would gain as well (N = 32 329 / 287 at w = 24, 707 / 360 at w = 64, N = 16 276 / 227), but up to N = 32 the separate ops,
 //              whose row sums of P dP have 2 w + 1 terms, are the more accurate: distance to float64 in 1e-7, theirs / fused, grad_k N = 16
 //              2.30 / 2.57 at w = 40, N = 24 2.07 / 2.11, N = 32 2.77 / 2.81 at w = 64; with scores three times as large N = 32 w = 64 grad_q
@@ -686,7 +687,7 @@ bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool t
   if (N < 8 || N > kMaxWidth || M > (1 << 30) || window_size < 16 || window_size > (1 << 28) || !(scale > 1.2e-38 && scale < 1.0e30)) return false;
   const int64_t tiles = batch_of(q) * ((M + 127) / 128);
   if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && (training || N > 64))) return false;
-  if (!training) return true;
+  if (!training) return tiles >= 32 || N <= 96 || N % 8 != 0 || std::min(window_size, M / 4) <= 160;
   if (N > 64 && N % 8 == 0) return window_size >= 128 && tiles >= (N <= 96 ? 160 : 256);
   return N >= 40 ? window_size >= 32 : N > 32 && window_size >= 64;
 }
