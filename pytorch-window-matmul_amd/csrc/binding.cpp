@@ -679,6 +679,9 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 //              w = 300, 766 / 687 at w = 1500, T = 128 N = 80 477 / 514 at w = 1000; T = 256 N = 128 251 / 251 and 791 / 792 at w = 200 and 1000.
 //              Widths that 8 does not divide, which the separate ops take to the tile kernels: T = 3072 N = 60 616 / 602
 //              at w = 16, 748 / 580 at w = 32, N = 75 5062 / 2346 at w = 256; T = 32 N = 75 216 / 216 at w = 300.
+//              N = 127 T = 1536 694 / 720 at w = 32, 879 / 885 at 48, 971 / 882 at 64, T = 256 156 / 131 at w = 32, 182 / 148 at 48; N = 110 T = 1536
+//              658 / 655 at w = 32.  With few tiles the separate ops wait for the host, 105 to 145 us by the machine: T = 8 N = 127
+//              143 / 101 at w = 32, 139 / 133 at 64, 142 / 150 at 80, 158 / 169 at 100, 188 / 189 at 140.
 // Below 8 tiles all routes are a handful of launches, and what a problem of that size gives, traced or not, stays as it was bit for bit.
 // An infinite operand gives NaN in both routes, as in the separate ops from w = 16 on (wm_f32_split.hip).
 bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool training) {
@@ -689,6 +692,7 @@ bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool t
   if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && (training || N > 64))) return false;
   if (!training) return tiles >= 32 || N <= 96 || N % 8 != 0 || std::min(window_size, M / 4) <= 160;
   if (N > 64 && N % 8 == 0) return window_size >= 128 && tiles >= (N <= 96 ? 160 : 256);
+  if (N > 112 && tiles >= 1024) return window_size >= 40;
   return N >= 40 ? window_size >= 32 : N > 32 && window_size >= 64;
 }
 

@@ -25,3 +25,10 @@ def _takes_the_fused_kernels(views, w, training):
 def test_inference(device, heads, M, N, w, fused):
     with torch.no_grad():
         assert _takes_the_fused_kernels(_views(1, heads, M, N, device), w, False) == fused
+
+
+# widths beyond 112 that 8 does not divide (the other lines: test_route_of_training_and_of_a_result_changed_in_place)
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,M,N,w,fused", [(8, 128, 127, 32, True), (1023, 128, 127, 32, True), (1024, 128, 127, 39, False), (1024, 128, 127, 40, True), (1024, 128, 111, 32, True)])
+def test_training(device, heads, M, N, w, fused):
+    assert _takes_the_fused_kernels(_views(1, heads, M, N, device), w, True) == fused
