@@ -146,18 +146,17 @@ def test_last_head_of_a_large_projection(device, batch, heads, M, N, w, dtype):
         return _rand((batch, M, heads * N), dtype, device, seed).view(batch, M, heads, N).transpose(1, 2)
 
     q, k, v, go = (projection(s) for s in (41, 42, 43, 44))
-    if dtype != torch.float32:
-        leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
-        alone = [t[-1:, -1:].contiguous().requires_grad_(True) for t in (q, k, v)]
-        for xs, grad in ((leaves, go), (alone, go[-1:, -1:].contiguous())):
-            out = window_attention(*xs, w)
-            out.backward(grad)
-            xs.append(out.detach())
-        for name, x, y in zip(("out", "grad_v", "grad_k", "grad_q"), [leaves[3]] + [t.grad for t in leaves[2::-1]],
-                              [alone[3]] + [t.grad for t in alone[2::-1]]):
-            _close(x[-1:, -1:], y, name)
-        del leaves, alone, out, xs, grad, x, y
-        torch.cuda.empty_cache()
+    leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    alone = [t[-1:, -1:].contiguous().requires_grad_(True) for t in (q, k, v)]
+    for xs, grad in ((leaves, go), (alone, go[-1:, -1:].contiguous())):
+        out = window_attention(*xs, w)
+        out.backward(grad)
+        xs.append(out.detach())
+    for name, x, y in zip(("out", "grad_v", "grad_k", "grad_q"), [leaves[3]] + [t.grad for t in leaves[2::-1]],
+                          [alone[3]] + [t.grad for t in alone[2::-1]]):
+        _close(x[-1:, -1:], y, name)
+    del leaves, alone, out, xs, grad, x, y
+    torch.cuda.empty_cache()
     if w <= 40:  # the separate ops, whose band still fits the card
         def last(fn, *xs):
             return fn(*xs)[-1:, -1:], fn(*(t[-1:, -1:].contiguous() for t in xs))
