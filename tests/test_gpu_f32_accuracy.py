@@ -29,11 +29,12 @@ def _float64(q, k, v, go, w, scale, mask):
 @pytest.mark.gpu
 @pytest.mark.parametrize("factor", [1.0, 3.0])
 @pytest.mark.parametrize("w", [64, 100])
-@pytest.mark.parametrize("N", [24, 32, 33, 40, 41, 48, 60, 64, 75, 101, 127])
-def test_training_is_no_less_accurate_than_the_separate_ops(device, N, w, factor):
-    """Root mean square of the relative distance over four inputs, with and without mask.  Over other inputs of these sizes the
-    quotient was 0.49 to 1.001 where the fused kernels train (1.06 at N = 32, which therefore does not)."""
-    mine, theirs = [0.0] * 4, [0.0] * 4
+@pytest.mark.parametrize("N", [8, 24, 32, 33, 40, 41, 48, 60, 64, 75, 101, 127])
+def test_no_less_accurate_than_the_separate_ops(device, N, w, factor):
+    """Root mean square of the relative distance over four inputs, with and without mask: result and gradients of a training step, and
+    the result without a graph.  The quotients were 0.44 to 0.947 where the fused kernels run (training at N = 32 would have 1.06 and
+    goes through the separate ops)."""
+    mine, theirs = [0.0] * 5, [0.0] * 5
     for seed in range(4):
         g = torch.Generator(device=device).manual_seed(9000 + seed)
         q, k, v, go = (torch.randn((B, M, N), generator=g, device=device) for _ in range(4))
@@ -45,7 +46,10 @@ def test_training_is_no_less_accurate_than_the_separate_ops(device, N, w, factor
                 out = unwindow_matmul(band_softmax(window_matmul(xs[0], xs[1].transpose(-1, -2), w), scale, mask), xs[2], w)
             else:
                 out = window_attention(*xs, w, scale, mask)
-            for i, (x, y) in enumerate(zip((out.detach(), *torch.autograd.grad(out, xs, go)), want)):
+            grads = torch.autograd.grad(out, xs, go)
+            with torch.no_grad():
+                plain = out if separate else window_attention(q, k, v, w, scale, mask)
+            for i, (x, y) in enumerate(zip((out.detach(), *grads, plain.detach()), (*want, want[0]))):
                 total[i] += float(((x.double() - y).norm() / y.norm()) ** 2)
-    for x, y in zip(mine, theirs):
-        assert x ** 0.5 <= 1.02 * y ** 0.5, [(a / b) ** 0.5 for a, b in zip(mine, theirs)]
+    quotients = [(x / y) ** 0.5 for x, y in zip(mine, theirs)]
+    assert max(quotients) <= (1.0 if N <= 32 else 0.97) and quotients[4] <= 0.97, quotients
