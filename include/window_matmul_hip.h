@@ -165,7 +165,7 @@ const char *wm_band_softmax_kernel_choice(int64_t w, int dtype, int contiguous, 
  * row as float32 (B * M values, contiguous) for use by a backward pass; the sum is taken over
  * the probabilities as rounded to the storage type, the values that multiply v.
  * Returns WM_ERR_UNSUPPORTED, having launched nothing, unless dtype is float16 / bfloat16,
- * N is a multiple of 16 up to 128, w >= 1, scale > 0 and all four operands have unit column
+ * N is a multiple of 16 up to 128, w >= 1, 1.2e-38 < scale < 1e30 and all four operands have unit column
  * stride and 16-byte aligned rows (see wm_window_attention_supported); with WM_FLAG_ANY_HEAD_WIDTH also
  * for every other N from 8 on, with rows of any alignment (no byte outside the rows is touched). */
 int wm_window_attention_forward(const wm_operand *q, const wm_operand *k, const wm_operand *v,

@@ -938,7 +938,7 @@ bool attention_supports(int64_t M, int64_t N, int64_t w, int dtype, double scale
   if (N % 16 != 0 || N < 16 || N > 128) return false;
   if (M < 1 || w < 1 || w > 0x3fffffff) return false;
   if (M > 0x7fffffff - w - 2 * AT_TM) return false;  // row and key indices are 32-bit in the kernels
-  return scale > 0.0 && scale < 1.0e30;
+  return scale > 1.2e-38 && scale < 1.0e30;  // as a float32 a normal number: a masked score times 0 would be NaN
 }
 
 bool try_launch_attention_forward(const Problem &p, const View &q, const View &k, const View &v, const View &o,

@@ -349,3 +349,19 @@ def test_rows_of_large_negative_scores(device, B, M, N, w, flags, dtype):
     # scores of this size carry an error of 1000 * 2^-24 * a few: the result's rounding is what is left
     error = float((out[:1].cpu().double() - want).norm() / want.norm())
     assert error < (2e-3 if dtype == torch.float16 else 1e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N", [60, 64])
+@pytest.mark.parametrize("mask", [False, True])
+def test_a_scale_that_vanishes_as_float32(device, N, mask, dtype):
+    """Equal weights, by the separate ops: the fused kernels would multiply the score of a masked neighbour, minus infinity, by zero."""
+    from window_matmul import window_attention
+
+    xs = [seeded((2, 300, N), 60 + s, dtype) for s in range(3)]
+    for scale in (1e-46, 1e-40):
+        out = window_attention(*(x.to(device) for x in xs), 20, scale, mask)
+        want = torch.from_numpy(ao.window_attention_forward(*xs, 20, scale, mask)[0])
+        # the band of weights is rounded once more than the result: 2^-11 or 2^-8 each
+        assert float((out.cpu().double() - want).norm() / want.norm()) < (2e-3 if dtype == torch.float16 else 1e-2)
