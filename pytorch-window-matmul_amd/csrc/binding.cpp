@@ -671,7 +671,10 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 //              whose row sums of P dP have 2 w + 1 terms, are the more accurate: distance to float64 in 1e-7, theirs / fused, grad_k N = 16
 //              2.30 / 2.57 at w = 40, N = 24 2.07 / 2.11, N = 32 2.77 / 2.81 at w = 64; with scores three times as large N = 32 w = 64 grad_q
 //              3.97 / 4.20, grad_k 3.90 / 4.07.  From N = 33 on none is worse (N = 33 ... 128, w = 32 ... 300, scores of one, three and six times
-//              the size, four inputs each).
+//              the size, four inputs each), up to w = 256.  Beyond, the separate ops pad widths that 8 does not divide and take the split products
+//              as well, and the row sums tell again: quotients of the distances, fused / theirs, N = 36 1.01 at w = 300, 1.07 at 600, N = 47 0.99 and
+//              1.04, N = 54 0.94 at w = 600, 1.01 at 1000, N = 63 0.97 at w = 1000, 1.02 at 1500, N = 70 0.98 at w = 1500, 1.02 at 3000, N = 85 0.99 at
+//              6000.  Widths that 8 divides had D = sum dO O from w = 128 on before: 0.92 ... 0.99 at w = 1500 ... 6000.
 //              N = 64: T = 3072 567 / 576 at w = 24, 678 / 561 at w = 32, 2096 / 1456 at w = 256; T = 32 96 / 66 at
 //              w = 64, 142 / 132 at w = 256, 177 / 200 at w = 400, T = 64 346 / 420 at w = 1024, T = 128 438 / 402.
 //              N > 64: a wavefront of the key kernel needs the registers of a whole SIMD: T = 3072 N = 80 1096 / 1112 at w = 64, N = 96
@@ -682,8 +685,12 @@ torch::Tensor window_attention(const torch::Tensor &q, const torch::Tensor &k, c
 //              N = 127 T = 1536 694 / 720 at w = 32, 879 / 885 at 48, 971 / 882 at 64, T = 256 156 / 131 at w = 32, 182 / 148 at 48; N = 110 T = 1536
 //              658 / 655 at w = 32.  With few tiles the separate ops wait for the host, 105 to 145 us by the machine: T = 8 N = 127
 //              143 / 101 at w = 32, 139 / 133 at 64, 142 / 150 at 80, 158 / 169 at 100, 188 / 189 at 140.
-// Below 8 tiles all routes are a handful of launches, and what a problem of that size gives, traced or not, stays as it was bit for bit.
-// An infinite operand gives NaN in both routes, as in the separate ops from w = 16 on (wm_f32_split.hip).
+// Below 8 tiles, whose routes differ in launches alone, a problem gives what it gave before these kernels, traced or not, bit for bit.  That
+// costs time: T = 8 takes 144 / 86 us for a step and 38 / 17 for inference (8 x M128 N64 w40); one sequence with T = 8, N = 64 at w = 257
+// 56 / 40 for inference and at w = 1000 66 / 51, T = 16 103 / 90.
+// An infinite operand gives NaN where the exact result is infinite, as in the separate ops on split products (wm_f32_split.hip); where those
+// run on the float32 instruction, which gives the infinity, that is a difference between the routes: widths that 8 does not divide
+// up to w = 256, values of N <= 32, and up to w = 28 (queries and keys: 31) widths of 16, 32, 48 and 64.
 bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool training) {
   const int64_t N = q.size(-1), M = q.size(-2);
   if (q.numel() == 0) return false;
@@ -691,6 +698,7 @@ bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool t
   const int64_t tiles = batch_of(q) * ((M + 127) / 128);
   if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && (training || N > 64))) return false;
   if (!training) return tiles >= 32 || N <= 96 || N % 8 != 0 || std::min(window_size, M / 4) <= 160;
+  if (N % 8 != 0 && std::min(window_size, M) > std::max<int64_t>(256, 60 * (N - 44))) return false;
   if (N > 64 && N % 8 == 0) return window_size >= 128 && tiles >= (N <= 96 ? 160 : 256);
   if (N > 112 && tiles >= 1024) return window_size >= 40;
   return N >= 40 ? window_size >= 32 : N > 32 && window_size >= 64;
