@@ -17,7 +17,8 @@
 // stationary operands stay in registers as planes, P and dS come out arranged as B operands.  A streamed chunk goes through
 // registers, is split once per workgroup and stored as swizzled bf16 planes (LdsTile), read by rows and transposed.
 //
-// Head widths: any N = 8 ... 128, in pieces of eight columns, the last one moved back to end with the row (HeadWidth).  The
+// Head widths (training through window_attention begins at N = 33, f32_fused() in binding.cpp; the backward of narrower ones is for
+// callers of the C ABI): any N = 8 ... 128, in pieces of eight columns, the last one moved back to end with the row (HeadWidth).  The
 // columns it shares with the piece before are cleared in the stationary operands; as result columns they come out twice.
 //
 // With F32_KEY_WIDE set (wm_attention_f32_key_wide.hip) this translation unit holds the key kernel for N > 96 alone, which wants
@@ -37,7 +38,8 @@ constexpr int FA_KC = 32;   // streamed rows per chunk
 constexpr float kRaiseBy = 8.0f;
 
 // Chunks in LDS.  With three, the first products of a chunk run one iteration ahead of the rest, their vector work dealt out among
-// the matrix instructions (deal() below).  That is for one wavefront per SIMD: us at B96 M4096 w256, two stages / three: forward
+// the matrix instructions (deal() below).  That is for one wavefront per SIMD: us at B96 M4096 w256, two stages / three, each kernel over and
+// over (the clock falls under that load: the forward at N = 64 takes 326 with pauses and 304-312 in a training step): forward
 // N = 32 191 / 203, N = 64 430 / 430 (B2 M4096 w1024, one wavefront per SIMD there too: 121 / 92), N = 128 735 / 712; query kernel
 // N = 64 520 / 595 (two wavefronts only on two stages), N = 80 789 / 703, N = 128 1087 / 1005; key kernel and D N = 32 w = 64 166 / 237,
 // N = 64 853 / 782, N = 80 1073 / 959, N = 96 1146 / 1053, N = 128 1450 / 1817 (there its registers do not suffice).
@@ -539,6 +541,8 @@ __global__ __launch_bounds__(kThreads) void attention_f32_delta_kernel(const flo
 // ---------------------------------------------------------------------------------------------
 // backward: query kernel
 // ---------------------------------------------------------------------------------------------
+// Above N = 64 the masks of the three rows that are loaded together take more scalar registers than there are: 20 to 91 of them go
+// through vector lanes, once per tile before its loop.
 template <int NK>
 __global__ __launch_bounds__(kThreads, NK <= 4 ? 2 : 1) void attention_f32_query_kernel(
     const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, const float *__restrict__ O,
