@@ -698,6 +698,7 @@ bool f32_fused(const torch::Tensor &q, int64_t window_size, double scale, bool t
   const int64_t tiles = batch_of(q) * ((M + 127) / 128);
   if (tiles < 8 || tiles > 0x7fffff00 || (tiles < 128 && window_size > 256 && (training || N > 64))) return false;
   if (!training) return tiles >= 32 || N <= 96 || N % 8 != 0 || std::min(window_size, M / 4) <= 160;
+  if (M < 16) return false;  // few neighbours: gradients of scores that cancel, with a single neighbour to exact zeros in the separate ops
   if (N % 8 != 0 && std::min(window_size, M) > std::max<int64_t>(256, 60 * (N - 44))) return false;
   if (N > 64 && N % 8 == 0) return window_size >= 128 && tiles >= (N <= 96 ? 160 : 256);
   if (N > 112 && tiles >= 1024) return window_size >= 40;

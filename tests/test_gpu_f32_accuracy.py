@@ -58,6 +58,14 @@ def test_no_less_accurate_than_the_separate_ops(device, N, w, factor):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N", [60, 64])
+def test_a_row_with_one_neighbour_has_no_gradient_of_its_score(device, N):
+    q, k, v = (torch.randn((16, 1, N), device=device, requires_grad=True) for _ in range(3))
+    grads = torch.autograd.grad(window_attention(q, k, v, 40, None, True).sum(), (q, k, v))
+    assert not grads[0].any() and not grads[1].any() and torch.equal(grads[2], torch.ones_like(v))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,w", [(33, 256), (33, 257), (36, 600), (39, 1500), (47, 256), (47, 600), (54, 600), (54, 601), (63, 1140), (70, 1500)])
 def test_wide_windows_of_widths_that_8_does_not_divide(device, N, w):
     """The separate ops pad these beyond w = 256; the fused kernels would be at 1.04 to 1.13 up to N = 47, at 1.02 at N = 63, w = 1500."""
